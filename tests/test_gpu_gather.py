@@ -96,3 +96,13 @@ def test_gather_reuses_buffers_and_is_idempotent():
     second = [plan.perm, plan.chunk_start[:n], plan.chunk_len[:n], plan.chunk_adapter[:n], plan.counters, plan.work]
     for a, b in zip(first, second):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,N", [(63, 2047), (65, 2048), (2048, 2047), (2049, 2047), (2048, 8191), (1025, 8192), (2049, 8192)])
+def test_gather_at_the_limits_of_its_forms(T, N):
+    """Wavefront and workgroup remainders, and pools on either side of the adapter counts at which the launcher
+    changes the form (counting with 2048 or 8192 counters, sorting beyond)."""
+    rng = np.random.default_rng(T + N)
+    pool = _pool(N, rng.choice([8, 16, 24], N), 8, rng)
+    say(f"gather form limits T={T} N={N}")
+    _check(np.append(rng.integers(-1, N, T - 2), [N - 1, 0]).astype(np.int32), pool, 4)
