@@ -73,6 +73,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 
 class MloraError(RuntimeError):
@@ -96,6 +97,20 @@ def lib() -> C.CDLL:
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+def host():
+    """The native launch path of the eager calls (module ``mlora._host``, built next to the library), imported once."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise ImportError(f"{os.path.join(_HERE, '_host.so')} is missing or stale: build it with "
+                              f"`make -C {os.path.join(CSRC_DIR, 'host')}`") from e
+        _host = mod
+    return _host
 
 
 def check(rc: int) -> None:

@@ -138,14 +138,9 @@ def plan_decode(tok_adapter: torch.Tensor, pool: AdapterPool, group: Optional[in
     else:
         out.tok_adapter = tok_adapter
         out.group = group
-    rc = _ext.lib().mlora_pool_gather(
-        _ext.ptr(tok_adapter), T, _ext.ptr(pool.page_tbl), _ext.ptr(pool.rank), _ext.ptr(pool.scaling),
-        pool.n_slots, pool.max_pages, pool.page_rows, pool.n_pages,
-        _ext.ptr(out.row_off), _ext.ptr(out.tok_rank), _ext.ptr(out.tok_scale),
-        _ext.ptr(out.perm), _ext.ptr(out.seg_start), _ext.ptr(out.seg_len), _ext.ptr(out.seg_adapter),
-        _ext.ptr(out.chunk_start), _ext.ptr(out.chunk_len), _ext.ptr(out.chunk_adapter), group,
-        _ext.ptr(out.counters), _ext.ptr(out.work), _ext.current_stream_ptr())
-    _ext.check(rc)
+    rc = _ext.host().gather(pool, out, tok_adapter, group)
+    if rc:
+        _ext.check(rc)
     return out
 
 
@@ -193,53 +188,12 @@ def bgmv(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], pool: AdapterPo
     intermediate in a buffer owned by the plan, allocated on the first call that needs it (so
     run one call before capturing a HIP graph); calls that share a plan must therefore follow each
     other on one stream, not overlap on several."""
-    n = len(projs)
-    if not (len(ys) == len(xs) == n) or not 1 <= n <= _ext.MAX_PROJ:
-        raise ValueError(f"need 1..{_ext.MAX_PROJ} projections with one y and one x each")
-    _need_cuda(tok_adapter, *ys, *xs)
-    _need_contig(tok_adapter, *ys, *xs)
-    if tok_adapter.dtype != torch.int32:
-        raise TypeError("tok_adapter must be int32")
-    T = tok_adapter.numel()
-    # the slab pointers and widths of a (layer, projections) pair never change: their argument arrays are kept
-    key = (layer, tuple(projs))
-    cached = pool._call_args.get(key)
-    if cached is None:
-        av, bv, hi, ho = _VoidArr(), _VoidArr(), _IntArr(), _IntArr()
-        for i, p in enumerate(projs):
-            hi[i], ho[i] = pool.projections[p]
-            av[i], bv[i] = pool.slab_ptrs(layer, p)
-        cached = pool._call_args[key] = (av, bv, hi, ho, max(hi[i] for i in range(n)))
-    av, bv, hi, ho, max_hin = cached
-    yv, xv = _VoidArr(), _VoidArr()
-    for i in range(n):
-        if xs[i].dtype != pool.dtype or ys[i].dtype != pool.dtype:
-            raise TypeError(f"x and y must have the pool dtype {pool.dtype}")
-        if xs[i].shape[0] != T or xs[i].shape[1] != hi[i] or ys[i].shape[0] != T or ys[i].shape[1] != ho[i] or xs[i].dim() != 2 or ys[i].dim() != 2:
-            raise ValueError(f"projection {projs[i]}: expected x [{T}, {hi[i]}] and y [{T}, {ho[i]}], "
-                             f"got {tuple(xs[i].shape)} and {tuple(ys[i].shape)}")
-        yv[i], xv[i] = ys[i].data_ptr(), xs[i].data_ptr()
-    pool.sync()
-    if plan is not None and plan.T != T:
-        raise ValueError("plan was built for a different batch size")
     if fused is None:
-        fused = plan is None or decode_fused(T, plan.group, n, pool.n_slots)
-    if not fused and plan is None:
-        raise ValueError("the two-launch form needs a plan")
-    ws, ws_bytes = None, 0
-    if not fused:
-        ws_bytes = _ext.lib().mlora_bgmv_workspace_bytes(n, T, max_hin, pool.max_rank)
-        if plan.vws is None or plan.vws.numel() < ws_bytes:
-            plan.vws = torch.empty(ws_bytes, dtype=torch.uint8, device=tok_adapter.device)
-        ws = plan.vws
-    rc = _ext.lib().mlora_bgmv_multi(
-        n, yv, xv, av, bv, hi, ho, _ext.ptr(tok_adapter), T,
-        _ext.ptr(pool.page_tbl), _ext.ptr(pool.rank), _ext.ptr(pool.scaling),
-        pool.n_slots, pool.max_pages, pool.page_rows, pool.n_pages, pool.max_rank,
-        _ext.ptr(plan.work) if plan else None, plan.group if plan else 1,
-        _ext.ptr(ws), ws_bytes,
-        pool.dtype_code, int(accumulate), _ext.current_stream_ptr())
-    _ext.check(rc)
+        fused = plan is None or decode_fused(plan.T, plan.group, len(projs), pool.n_slots)
+    pool.sync()
+    rc = _ext.host().bgmv(pool, layer, projs, ys, xs, tok_adapter, plan, bool(fused), bool(accumulate))
+    if rc:
+        _ext.check(rc)
 
 
 def add_lora_bgmv(y: torch.Tensor, x: torch.Tensor, wa_T_all: torch.Tensor, wb_T_all: torch.Tensor,
@@ -324,34 +278,9 @@ def add_lora_bgmv_multi(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], 
     was[p] [N, L, r, Hin], wbs[p] [N, L, Hout, r] and idx the index vector the plan was made from
     (``lora_gpu.py:137-138,149-150,161-162`` in one go).  ``accumulate=False`` defines ys as the delta alone
     (zeros for indices outside the pool), which saves the ``torch.zeros`` of ``lora_gpu.py:137``."""
-    n = len(ys)
-    if not (len(xs) == len(was) == len(wbs) == n) or not 1 <= n <= _ext.MAX_PROJ:
-        raise ValueError(f"need 1..{_ext.MAX_PROJ} projections with one y, x, wa and wb each")
-    _need_cuda(*ys, *xs, *was, *wbs)
-    _need_contig(*ys, *xs, *was, *wbs)
-    T = plan.T
-    yv, xv, av, bv, hi, ho = _VoidArr(), _VoidArr(), _VoidArr(), _VoidArr(), _IntArr(), _IntArr()
-    dt = ys[0].dtype
-    for i in range(n):
-        if was[i].dim() != 4 or wbs[i].dim() != 4:
-            raise ValueError("wa_T_all must be [N, L, r, Hin] and wb_T_all [N, L, Hout, r]")
-        N, L, r, hin = was[i].shape
-        N2, L2, hout, r2 = wbs[i].shape
-        if (N2, L2, r2) != (N, L, r) or (N, L, r) != (plan.N, plan.L, plan.r):
-            raise ValueError("pool tensors disagree with each other or with the plan on N, L or r")
-        if tuple(xs[i].shape) != (T, hin) or tuple(ys[i].shape) != (T, hout):
-            raise ValueError("x must be [B, Hin] and y [B, Hout] for the plan's batch")
-        if not (ys[i].dtype == xs[i].dtype == was[i].dtype == wbs[i].dtype == dt):
-            raise TypeError("y, x and the pools must share one 16-bit dtype")
-        yv[i], xv[i], av[i], bv[i], hi[i], ho[i] = ys[i].data_ptr(), xs[i].data_ptr(), was[i].data_ptr(), wbs[i].data_ptr(), hin, hout
-    lib = _ext.lib()
-    ws_bytes = lib.mlora_bgmv_workspace_bytes(n, T, max(hi[i] for i in range(n)), plan.r)
-    if plan.vws is None or plan.vws.numel() < ws_bytes:
-        plan.vws = torch.empty(ws_bytes, dtype=torch.uint8, device=ys[0].device)
-    rc = lib.mlora_bgmv_reflayout_multi(n, yv, xv, av, bv, hi, ho, plan.buf.data_ptr(), T, plan.N, plan.L, plan.r, layer_idx,
-                                        float(scale), plan.group, _ext.dtype_code(dt), int(accumulate),
-                                        plan.vws.data_ptr(), plan.vws.numel(), _ext.current_stream_ptr())
-    _ext.check(rc)
+    rc = _ext.host().bgmv_ref(plan, ys, xs, was, wbs, layer_idx, float(scale), bool(accumulate), plan.T, plan.N, plan.L, plan.r)
+    if rc:
+        _ext.check(rc)
 
 
 # ---------------------------------------------------------------------- prefill
@@ -392,16 +321,12 @@ def plan_prefill(seg_start: torch.Tensor, seg_len: torch.Tensor, seg_adapter: to
     ``sgmv_multi(..., plan=plan)``, ``gemm_lora(..., plan)`` for up to `n_proj` projections per call).
     ``aligned`` cuts the tiles at multiples of 64 tokens (and at segment ends) rather than every 64 tokens of a
     segment: fewer tiles per 256-row block of ``gemm_lora``, a few more tiles overall."""
-    n_seg = _check_segments(seg_start, seg_len, seg_adapter)
     if workspace is None:
-        workspace = sgmv_workspace(T, n_seg, seg_start.device, n_proj)
+        workspace = sgmv_workspace(T, _check_segments(seg_start, seg_len, seg_adapter), seg_start.device, n_proj)
     pool.sync()
-    plan_fn = _ext.lib().mlora_sgmv_plan_aligned if aligned else _ext.lib().mlora_sgmv_plan
-    rc = plan_fn(
-        seg_start.data_ptr(), seg_len.data_ptr(), seg_adapter.data_ptr(), n_seg,
-        _ext.ptr(pool.page_tbl), _ext.ptr(pool.rank), _ext.ptr(pool.scaling), T, pool.n_slots, pool.max_pages,
-        pool.page_rows, pool.n_pages, pool.max_rank, workspace.data_ptr(), workspace.numel(), _ext.current_stream_ptr())
-    _ext.check(rc)
+    rc = _ext.host().prefill_plan(pool, seg_start, seg_len, seg_adapter, T, workspace, bool(aligned))
+    if rc:
+        _ext.check(rc)
     return PrefillPlan(seg_start, seg_len, seg_adapter, T, workspace)
 
 
@@ -442,29 +367,10 @@ def sgmv_multi(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], pool: Ada
     """Prefill LoRA apply for up to 8 projections of one layer against one plan, three launches in all.
     Projections listed next to each other with the same x tensor (q, k, v; gate, up) share its reads.
     The plan's workspace must have been sized for this many projections (``plan_prefill(..., n_proj=)``)."""
-    n = len(projs)
-    if not (len(ys) == len(xs) == n) or not 1 <= n <= _ext.MAX_PROJ:
-        raise ValueError(f"need 1..{_ext.MAX_PROJ} projections with one y and one x each")
-    _need_cuda(*ys, *xs)
-    _need_contig(*ys, *xs)
-    T = plan.T
-    yv, xv, av, bv, hi, ho = _VoidArr(), _VoidArr(), _VoidArr(), _VoidArr(), _IntArr(), _IntArr()
-    for i, p in enumerate(projs):
-        hin, hout = pool.projections[p]
-        if xs[i].dtype != pool.dtype or ys[i].dtype != pool.dtype:
-            raise TypeError(f"x and y must have the pool dtype {pool.dtype}")
-        if tuple(xs[i].shape) != (T, hin) or tuple(ys[i].shape) != (T, hout):
-            raise ValueError(f"projection {p}: expected x [{T}, {hin}] and y [{T}, {hout}]")
-        a_ptr, b_ptr = pool.slab_ptrs(layer, p)
-        yv[i], xv[i], av[i], bv[i], hi[i], ho[i] = ys[i].data_ptr(), xs[i].data_ptr(), a_ptr, b_ptr, hin, hout
-    n_seg = _check_segments(plan.seg_start, plan.seg_len, plan.seg_adapter)
     pool.sync()
-    rc = _ext.lib().mlora_sgmv_multi_planned(
-        n, yv, xv, av, bv, hi, ho, plan.seg_start.data_ptr(), plan.seg_len.data_ptr(), plan.seg_adapter.data_ptr(),
-        n_seg, _ext.ptr(pool.page_tbl), _ext.ptr(pool.rank), _ext.ptr(pool.scaling), T, pool.n_slots, pool.max_pages,
-        pool.page_rows, pool.n_pages, pool.max_rank, pool.dtype_code, int(accumulate),
-        plan.workspace.data_ptr(), plan.workspace.numel(), _ext.current_stream_ptr())
-    _ext.check(rc)
+    rc = _ext.host().sgmv_multi(pool, layer, projs, ys, xs, plan, bool(accumulate))
+    if rc:
+        _ext.check(rc)
 
 
 def gemm_lora(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], ws: Sequence[torch.Tensor], pool: Optional[AdapterPool],
