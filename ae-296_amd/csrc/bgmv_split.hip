@@ -58,6 +58,8 @@ __device__ __forceinline__ typename RecPtr<BIG>::type record_at(const int32_t *w
     else return work + (size_t)b * WORK_WORDS;
 }
 
+constexpr int FINE_CHUNKS = 64;                                // slice width of a small launch, shrink and expand (512 columns)
+
 struct ItemId { int b, q; };
 
 __device__ __forceinline__ ItemId split_id(unsigned id, int nq)
@@ -391,6 +393,145 @@ __global__ __launch_bounds__(NTE) void bgmv_expand_kernel(const BgmvArgs p)
     } while (BIG && (b += p.rec_stride_ex) < p.items_cap);
 }
 
+// Expand of a small launch.  The kernel above gives a lane all rank rows of its columns, eight at a time, so an item
+// of rank 64 is a chain of eight round trips to memory; that costs nothing while other workgroups of the unit fill
+// the gaps, and everything in a launch that leaves the chip half empty.  Here the four wavefronts of a workgroup
+// split the rank rows of one 512-column slice between them: all rows are requested at once, the wavefronts' sums are
+// added through LDS in wavefront order, and a slice is half or a quarter as wide, which spreads a small batch over
+// more units.  Llama-7B widths, shrink + expand: one token at rank 64 16.8 -> 10.0 us (one projection), 20.0 -> 11.8
+// (seven); 8 tokens x 7 projections of ranks 8..64 23.3 -> 18.8 us.  Where the line to the wider slices lies, and why:
+// prefer_sliced in c_api.hip.
+template <int DT, int G, int RMAX, int KSC>
+__global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
+{
+    constexpr int SLICE = FINE_CHUNKS * 8;                      // columns per workgroup
+    constexpr int NQ = 256 / RMAX;                              // threads that share the slices of one intermediate
+    __shared__ __attribute__((aligned(16))) float s_vp[NQ][G][RMAX];
+    __shared__ __attribute__((aligned(16))) float s_o[4][G][SLICE];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const ItemId id = split_id(blockIdx.x, p.ex_end[p.n_proj - 1]);
+    int proj = 0;
+    while (proj + 1 < p.n_proj && id.q >= p.ex_end[proj]) proj++;
+    const int cs = id.q - (proj ? p.ex_end[proj - 1] : 0);
+    const int hout = p.hout[proj];
+    const int ncc_out = hout >> 3;
+    const int cc = cs * FINE_CHUNKS + lane;
+    const bool active = cc < ncc_out;
+    uint16_t *__restrict__ y = static_cast<uint16_t *>(p.y[proj]);
+    const uint16_t *__restrict__ brows = static_cast<const uint16_t *>(p.b_rows[proj]);
+    const int n_ks = ((p.hin[proj] >> 3) + KSC - 1) / KSC;
+
+    const int32_t *__restrict__ rec = p.work + (size_t)id.b * WORK_WORDS;
+    int ntok = rec[0];
+    if (ntok <= 0) return;
+    ntok = ntok < G ? ntok : G;
+    const int adapter = rec[1];
+    int r = rec[2];
+    r = r < 0 ? 0 : (r > RMAX ? RMAX : r);
+    const float scale = __builtin_bit_cast(float, rec[3]);
+    int tok[G];
+    int ytok = -1;                                              // wavefront k finishes token k
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+        const int t = k < ntok ? rec[4 + k] : -1;
+        tok[k] = (t >= 0 && t < p.T) ? t : -1;
+        ytok = wave == k ? tok[k] : ytok;
+    }
+    uint16_t *yp = y + (size_t)(ytok >= 0 ? ytok : 0) * hout + (size_t)(active ? cc : 0) * 8;
+    if (adapter < 0) {
+        if (!p.accumulate && active && ytok >= 0) stg16(yp, zero16());
+        return;
+    }
+    const int32_t *__restrict__ rows = rec + WORK_ROWS_AT;
+    uint4 yv = zero16();
+    float o[G][8];
+#pragma unroll
+    for (int k = 0; k < G; k++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[k][e] = 0.f;
+
+    // n rank rows of this wavefront from row j0 on, the slices' partial sums behind them
+    auto run = [&](auto n_tag) {
+        constexpr int N = decltype(n_tag)::value;
+        const int j0 = wave * N;
+        uint4 bv[N];
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int row = rows[j0 + i];
+            const bool ok = active && row >= 0 && row < p.pool.n_rows_b;
+            bv[i] = ok ? ldg16_stream(brows + (size_t)row * hout + (size_t)cc * 8) : zero16();
+        }
+        if (p.accumulate && active && ytok >= 0) yv = ldg16_stream(yp);
+        // sums of the shrink's slices: thread (q, j) adds slices q, q + NQ, ... of rank row j in ascending order, for
+        // every token; how many tokens share the item does not change the order of a token's sum
+        const int kstep = slice_factor<RMAX, false>(r);
+        const int q = tid / RMAX, j = tid - q * RMAX;
+        float sum[G];
+#pragma unroll
+        for (int k = 0; k < G; k++) sum[k] = 0.f;
+        if (j < r) {
+            for (int ks0 = q * kstep; ks0 < n_ks; ks0 += 4 * NQ * kstep) {
+                float t[G][4];
+#pragma unroll
+                for (int k = 0; k < G; k++) {
+                    const float *src = p.vws + (((size_t)proj * p.T + (tok[k] >= 0 ? tok[k] : 0)) * p.ks_max) * RMAX + j;
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const int ks = ks0 + u * NQ * kstep;
+                        t[k][u] = (ks < n_ks && tok[k] >= 0) ? src[(size_t)ks * RMAX] : 0.f;
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < G; k++)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) sum[k] += t[k][u];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < G; k++) s_vp[q][k][j] = sum[k];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            float f[8];
+            unpack8<DT>(bv[i], f);
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                float vk = 0.f;
+#pragma unroll
+                for (int q4 = 0; q4 < NQ; q4++) vk += s_vp[q4][k][j0 + i];
+                vk *= scale;
+#pragma unroll
+                for (int e = 0; e < 8; e++) o[k][e] = fmaf(vk, f[e], o[k][e]);
+            }
+        }
+    };
+    if constexpr (RMAX >= 64) { if (r > 32) run(std::integral_constant<int, 16>{}); }
+    if constexpr (RMAX >= 32) { if (r > 16 && r <= 32) run(std::integral_constant<int, 8>{}); }
+    if (r > 8 && r <= 16) run(std::integral_constant<int, 4>{});
+    if (r <= 8) run(std::integral_constant<int, 2>{});
+
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+        *reinterpret_cast<float4_t *>(&s_o[wave][k][lane * 8]) = float4_t{o[k][0], o[k][1], o[k][2], o[k][3]};
+        *reinterpret_cast<float4_t *>(&s_o[wave][k][lane * 8 + 4]) = float4_t{o[k][4], o[k][5], o[k][6], o[k][7]};
+    }
+    __syncthreads();
+    if (wave < G && active && ytok >= 0) {
+        float s[8];
+        unpack8<DT>(yv, s);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float4_t d0 = *reinterpret_cast<const float4_t *>(&s_o[w][wave][lane * 8]);
+            const float4_t d1 = *reinterpret_cast<const float4_t *>(&s_o[w][wave][lane * 8 + 4]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) { s[e] += d0[e]; s[4 + e] += d1[e]; }
+        }
+        stg16_stream(yp, pack8<DT>(s));
+    }
+}
+
 // Slice sizes per rank bucket, in 16-byte chunks (8 columns): the bytes of a shrink workgroup grow
 // with rank x slice width, so wider ranks take narrower slices (measured over 64 / 128 / 256 chunks
 // on rank-16, rank-32, rank-64 and mixed-rank batches).  Expand slices: 2048 columns (256 threads) at
@@ -621,16 +762,34 @@ static int launch_pair(const BgmvArgs &a0, hipStream_t s)
 }
 
 template <int DT, int G, int RMAX>
+static int launch_fine(const BgmvArgs &a, hipStream_t s)
+{
+    const long long n_sh = (long long)a.sh_end[a.n_proj - 1] * a.items_cap;
+    const long long n_ex = (long long)a.ex_end[a.n_proj - 1] * a.items_cap;
+    if (n_sh <= 0 || n_ex <= 0) return 0;
+    if (n_sh > 0x7fffffffLL || n_ex > 0x7fffffffLL) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, FINE_CHUNKS, false>), dim3((unsigned)n_sh), dim3(256), 0, s, a);
+    const int rc = (int)hipGetLastError();
+    if (rc) return rc;
+    hipLaunchKernelGGL((bgmv_expand_fine_kernel<DT, G, RMAX, FINE_CHUNKS>), dim3((unsigned)n_ex), dim3(256), 0, s, a);
+    return (int)hipGetLastError();
+}
+
+template <int DT, int G, int RMAX>
 static int launch_sliced(const BgmvArgs &a, hipStream_t s)
 {
+    if constexpr (G <= 4) {
+        if (a.fine) return launch_fine<DT, G, RMAX>(a, s);
+    }
     // Rounds of shrink workgroups the launch may need (host's upper bound on the work items, three workgroups per
     // compute unit): from about sixteen on, the items of a much-used adapter no longer run side by side.
     const long long rounds = (long long)a.sh_end[a.n_proj - 1] * a.items_cap / (3 * device_compute_units());
     if (rounds >= 16) return launch_pair<DT, G, RMAX, Slices<RMAX>::KSC, Slices<RMAX>::NTE, true>(a, s);
     return launch_pair<DT, G, RMAX, Slices<RMAX>::KSC, Slices<RMAX>::NTE, false>(a, s);
 }
-void bgmv_split_slices(int max_rank, int *ksc, int *nte, bool transposed_b)
+void bgmv_split_slices(int max_rank, int *ksc, int *nte, bool transposed_b, bool fine)
 {
+    if (fine) { *ksc = *nte = FINE_CHUNKS; return; }
     if (max_rank <= 16) { *ksc = Slices<16>::KSC; *nte = Slices<16>::NTE; }
     else if (max_rank <= 32) { *ksc = Slices<32>::KSC; *nte = Slices<32>::NTE; }
     else { *ksc = Slices<64>::KSC; *nte = Slices<64>::NTE; }

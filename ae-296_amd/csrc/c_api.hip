@@ -285,6 +285,99 @@ int64_t mlora_bgmv_workspace_bytes(int n_proj, int T, int max_hin, int max_rank)
     return (int64_t)n_proj * T * ks * mlora::bgmv_split_rank_stride(max_rank) * (int64_t)sizeof(float);
 }
 
+// Work items in use <= T/group + segments + 1 (one short piece per adapter present, one for the adapter-less
+// tokens), rounded up to the eight record residues; the gather packs them into the first records, so the rest
+// needs no workgroup.
+static int items_bound(int T, int n_adapters, int group)
+{
+    const int64_t segs = T < n_adapters ? T : n_adapters;
+    const int64_t bound = ((int64_t)(T + group - 1) / group + segs + 1 + 7) / 8 * 8;
+    const int64_t cap = MLORA_WORK_CAP(T);
+    return (int)(bound < cap ? bound : cap);
+}
+
+static int64_t fine_workspace_bytes(int n_proj, int T, int max_hin, int max_rank)
+{
+    int ksc, nte;
+    mlora::bgmv_split_slices(max_rank, &ksc, &nte, false, true);
+    const int64_t ks = (max_hin + ksc * 8 - 1) / (ksc * 8);
+    return (int64_t)n_proj * T * ks * mlora::bgmv_split_rank_stride(max_rank) * (int64_t)sizeof(float);
+}
+
+// 512-column workgroups a call makes in the larger of its two launches.
+static int64_t fine_workgroups(int n_proj, const int32_t *hin, const int32_t *hout, int items)
+{
+    int ksc, nte;
+    mlora::bgmv_split_slices(16, &ksc, &nte, false, true);
+    int64_t sh = 0, ex = 0;
+    for (int p = 0; p < n_proj; p++) {
+        sh += (hin[p] + ksc * 8 - 1) / (ksc * 8);
+        ex += (hout[p] + nte * 8 - 1) / (nte * 8);
+    }
+    return (sh > ex ? sh : ex) * items;
+}
+
+// Two-launch form: 512-column slices with the rank rows split over wavefronts (fine) while they make at most four
+// workgroups per compute unit, the wider slices beyond.  Measured on Llama-7B widths, wide -> fine, us per call: 8
+// tokens x 7 projections (560 workgroups) 26.6 -> 21.9 at rank 64, 12.5 -> 11.7 at rank 16; 32 tokens x 3 (768)
+// 23.5 -> 20.8; 16 x 7 (1120) 34.6 -> 34.8; 32 x 7 (2240) 52.4 -> 59.6.
+static bool prefer_sliced(int n_proj, const int32_t *hin, const int32_t *hout, int items, int group)
+{
+    return group > 4 || fine_workgroups(n_proj, hin, hout, items) > 4LL * mlora::device_compute_units();
+}
+
+// How a planned decode call runs best, and the workspace its two-launch form takes (mlora_bgmv_form).
+//
+// Fused, one launch: every item on one compute unit, whose chain of loads grows with the bytes of an item; it saves
+// a launch, which is 1.6 us of a graph and 2.6 us of host time of an eager call.  Eight layers of Llama-7B attention
+// projections, fused / two fine launches, us: rank 16 (256 KiB an item), 32 tokens x 1 projection eager 72 / 76, in a
+// graph 72 / 65; 8 tokens x 3 eager 75 / 75, graph 75 / 65; 64 tokens x 3 83 / 117; rank 32 (512 KiB), 8 tokens x 1 eager
+// 114 / 78, 32 x 3 126 / 109, 64 x 3 (more workgroups than the fine form likes) 136 / 152.  So: fused up to 320 KiB an
+// item, up to 640 KiB where the slices have filled the chip, and never where one item is much longer than the others
+// (MLP widths: rank 16, 16 tokens x 7 projections 17.4 us a call fused, 14.7 fine).
+static int decode_form(int n_proj, const int32_t *hin, const int32_t *hout, int T, int n_adapters, int max_rank, int group)
+{
+    const int64_t cus = mlora::device_compute_units();
+    int64_t item_bytes = 0;
+    int widest = 0;
+    for (int p = 0; p < n_proj; p++) {
+        const int64_t b = 2LL * max_rank * ((int64_t)hin[p] + hout[p]);
+        item_bytes = b > item_bytes ? b : item_bytes;
+        widest = hin[p] > widest ? hin[p] : widest;
+        widest = hout[p] > widest ? hout[p] : widest;
+    }
+    const int64_t segs = T < n_adapters ? T : n_adapters;
+    // groups of two leave one odd item for about every other adapter
+    const int64_t items = group == 1 ? T : (T + 1) / 2 + segs / 2;
+    const bool one_round = group <= 2 && items * n_proj <= cus;
+    const bool sliced = prefer_sliced(n_proj, hin, hout, items_bound(T, n_adapters, group), group);
+    if (one_round && widest <= 8192 && item_bytes <= (sliced ? 640 << 10 : 320 << 10)) return MLORA_FORM_FUSED;
+    return sliced ? MLORA_FORM_SLICED : MLORA_FORM_FINE;
+}
+
+int mlora_bgmv_form(int n_proj, const int32_t *hin, const int32_t *hout, int T, int n_adapters, int max_rank, int group,
+                    int64_t *workspace_bytes)
+{
+    if (n_proj < 1 || n_proj > MLORA_MAX_PROJ) return fail(MLORA_ERANGE, "n_proj must be in 1..%d (got %d)", MLORA_MAX_PROJ, n_proj);
+    if (!hin || !hout || !workspace_bytes) return fail(MLORA_EINVAL, "NULL pointer");
+    if (T < 0 || n_adapters <= 0) return fail(MLORA_EINVAL, "T must be >= 0 and n_adapters positive (got %d, %d)", T, n_adapters);
+    if (max_rank < 1 || max_rank > MLORA_MAX_RANK) return fail(MLORA_ERANGE, "max_rank must be in 1..%d (got %d)", MLORA_MAX_RANK, max_rank);
+    if (group != 1 && group != 2 && group != 4 && group != 8) return fail(MLORA_EINVAL, "group must be 1, 2, 4 or 8 (got %d)", group);
+    int max_hin = 0;
+    for (int p = 0; p < n_proj; p++) {
+        const int rc = check_dims(hin[p], hout[p]);
+        if (rc) return rc;
+        max_hin = hin[p] > max_hin ? hin[p] : max_hin;
+    }
+    *workspace_bytes = 0;
+    if (T == 0) return MLORA_FORM_FUSED;
+    const bool sliced = prefer_sliced(n_proj, hin, hout, items_bound(T, n_adapters, group), group);
+    const int64_t coarse = mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
+    const int64_t fine = sliced ? 0 : fine_workspace_bytes(n_proj, T, max_hin, max_rank);
+    *workspace_bytes = coarse > fine ? coarse : fine;
+    return decode_form(n_proj, hin, hout, T, n_adapters, max_rank, group);
+}
+
 // use_scratch: the two-launch form with the library's own per-device scratch array as its workspace
 static int bgmv_multi_impl(int n_proj, void *const *y, const void *const *x, const void *const *a_rows,
                      const void *const *b_rows, const int32_t *hin, const int32_t *hout,
@@ -326,12 +419,8 @@ static int bgmv_multi_impl(int n_proj, void *const *y, const void *const *x, con
     a.tok_adapter = tok_adapter; a.tok_adapter64 = nullptr;
     a.work = work; a.work_cap = MLORA_WORK_CAP(T);
     {
-        // Work items in use <= T/group + segments + 1 (one short piece per adapter present, one for the
-        // adapter-less tokens); the gather packs them into the first records, so the rest needs no workgroup.
-        const int g = group > 0 ? group : 1;
-        const int64_t segs = T < n_adapters ? T : n_adapters;
-        const int64_t bound = ((int64_t)(T + g - 1) / g + segs + 1 + 7) / 8 * 8;
-        a.items_cap = bound < a.work_cap ? (int)bound : a.work_cap;
+        const int bound = items_bound(T, n_adapters, group > 0 ? group : 1);
+        a.items_cap = bound < a.work_cap ? bound : a.work_cap;
     }
     a.T = T; a.n_proj = n_proj; a.accumulate = accumulate ? 1 : 0;
     if (use_scratch) {
@@ -349,8 +438,10 @@ static int bgmv_multi_impl(int n_proj, void *const *y, const void *const *x, con
             return fail(MLORA_ENOSPACE, "workspace holds %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
         if (!aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be 16-byte aligned");
         a.vws = static_cast<float *>(workspace);
+        const int64_t fine_need = fine_workspace_bytes(n_proj, T, max_hin, max_rank);
+        a.fine = workspace_bytes >= fine_need && !use_scratch && !prefer_sliced(n_proj, hin, hout, a.items_cap, group);
         int ksc, nte;
-        mlora::bgmv_split_slices(max_rank, &ksc, &nte);
+        mlora::bgmv_split_slices(max_rank, &ksc, &nte, false, a.fine != 0);
         a.ks_max = (max_hin + ksc * 8 - 1) / (ksc * 8);
         a.cs_max = (max_hout + nte * 8 - 1) / (nte * 8);
         int sh = 0, ex = 0;

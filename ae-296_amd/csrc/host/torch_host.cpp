@@ -185,14 +185,15 @@ PyObject *gather(PyObject *const *v, Py_ssize_t nargs)
     return PyLong_FromLong(rc);
 }
 
-// bgmv(pool, layer, projs, ys, xs, tok_adapter, plan or None, fused, accumulate)
+// bgmv(pool, layer, projs, ys, xs, tok_adapter, plan or None, fused: True, False or None (by the sizes), accumulate)
 PyObject *bgmv(PyObject *const *v, Py_ssize_t nargs)
 {
     if (nargs != 9) raise(PyExc_TypeError, "bgmv takes 9 arguments");
     PyObject *pool = v[0], *plan = v[6] == Py_None ? nullptr : v[6];
     const List ys(v[3]), xs(v[4]);
     const at::Tensor &tok = tensor(v[5]);
-    const bool fused = v[7] == Py_True, accumulate = v[8] == Py_True;
+    const bool accumulate = v[8] == Py_True;
+    bool fused = v[7] != Py_None && PyObject_IsTrue(v[7]) == 1;
     need_device(tok);
     need_contiguous(tok);
     if (tok.scalar_type() != at::kInt) raise(PyExc_TypeError, "tok_adapter must be int32");
@@ -201,22 +202,25 @@ PyObject *bgmv(PyObject *const *v, Py_ssize_t nargs)
     if (plan) {
         Ref made_for(PyObject_GetAttr(plan, s_tok_adapter));
         if (tensor(made_for.o).numel() != T) raise(PyExc_ValueError, "plan was built for a different batch size");
+    } else if (v[7] == Py_None) {
+        fused = true;
     } else if (!fused) {
         raise(PyExc_ValueError, "the two-launch form needs a plan");
     }
     const Tables tb = tables(pool);
+    const int group = plan ? (int)attr_int(plan, s_group) : 1;
     void *ws = nullptr;
     int64_t ws_bytes = 0;
     if (!fused && T > 0) {
-        int max_hin = 0;
-        for (int i = 0; i < c.n; i++) max_hin = c.hin[i] > max_hin ? c.hin[i] : max_hin;
-        ws_bytes = mlora_bgmv_workspace_bytes(c.n, (int)T, max_hin, tb.max_rank);
-        ws = intermediate(plan, ws_bytes, tok);
+        const int form = mlora_bgmv_form(c.n, c.hin, c.hout, (int)T, tb.n_slots, tb.max_rank, group, &ws_bytes);
+        if (form < 0) return PyLong_FromLong(form);
+        if (v[7] == Py_None && form == MLORA_FORM_FUSED) fused = true;
+        else ws = intermediate(plan, ws_bytes, tok);
     }
     const int rc = mlora_bgmv_multi(
         c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, static_cast<const int32_t *>(tok.data_ptr()), (int)T, tb.page_tbl, tb.rank, tb.scaling,
         tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, tb.max_rank, plan ? static_cast<const int32_t *>(attr_ptr(plan, s_work)) : nullptr,
-        plan ? (int)attr_int(plan, s_group) : 1, ws, ws_bytes, c.dtype, accumulate, stream());
+        group, ws, fused ? 0 : ws_bytes, c.dtype, accumulate, stream());
     return PyLong_FromLong(rc);
 }
 

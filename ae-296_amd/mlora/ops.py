@@ -89,10 +89,9 @@ def default_group(T: int) -> int:
 
 
 def decode_fused(T: int, group: int, n_proj: int, n_slots: int) -> bool:
-    """Form of a planned decode call when the caller does not say: the single fused launch while its
-    work items, one 512-thread workgroup each, fit the device in one round (the call is then bound by
-    the dependent loads of one workgroup, and a second launch only adds to that); the shrink and expand
-    launches beyond, where spreading one item over many workgroups is what fills the memory system.
+    """Whether a planned decode call could run as the single fused launch: its work items, one 512-thread
+    workgroup each, fit the device in one round.  Whether it does is decided by the bytes of an item as well
+    (`mlora_bgmv_form`); here it decides the tokens per item.
     The item count is the host's estimate: groups of two leave one odd item for about every other adapter."""
     if group > 2:
         return False
@@ -183,15 +182,13 @@ def bgmv(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], pool: AdapterPo
     ys[p][t] (+)= scaling[a] * (xs[p][t] . A_{p,a}) . B_{p,a},  a = tok_adapter[t].
 
     With a plan the call runs as a shrink launch and an expand launch over column slices
-    (``fused=False``) or as one fused launch (``fused=True``), by default whichever `decode_fused`
-    names for the batch; without a plan it is always the fused launch with one token per work item.  The two-launch form keeps its fp32
+    (``fused=False``) or as one fused launch (``fused=True``), by default whichever `mlora_bgmv_form`
+    names for the sizes; without a plan it is always the fused launch with one token per work item.  The two-launch form keeps its fp32
     intermediate in a buffer owned by the plan, allocated on the first call that needs it (so
     run one call before capturing a HIP graph); calls that share a plan must therefore follow each
     other on one stream, not overlap on several."""
-    if fused is None:
-        fused = plan is None or decode_fused(plan.T, plan.group, len(projs), pool.n_slots)
     pool.sync()
-    rc = _ext.host().bgmv(pool, layer, projs, ys, xs, tok_adapter, plan, bool(fused), bool(accumulate))
+    rc = _ext.host().bgmv(pool, layer, projs, ys, xs, tok_adapter, plan, fused, bool(accumulate))
     if rc:
         _ext.check(rc)
 

@@ -388,3 +388,39 @@ def test_bgmv_many_round_launch_walks_several_records(group, rank_set, hin, T, N
     want = oracle_apply(pp, x, tok, None)
     assert_close_bits(got, want, dtype, "delta")
     assert not np.any(f32_of(got, dtype)[tok < 0]), "rows of tokens without an adapter must be zeros in y = delta mode"
+
+
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("T,group,ranks,hin,hout", [
+    (1, 1, [64], 512, 520), (3, 1, [9, 64, 33], 1032, 504), (7, 2, [8, 16, 17, 24, 64], 4096, 11008),
+    (13, 4, [8, 32, 25], 2056, 1032), (33, 4, [16, 8, 1], 520, 2048), (5, 1, [40, 8], 20488, 64)])
+def test_bgmv_fine_slices(dtype, T, group, ranks, hin, hout):
+    """The two-launch form of a small batch: slices that end inside 512 columns, every rank bucket in launches sized
+    for rank 16, 32 and 64, more slices than one pass of the summation takes, both modes; the sum of a token does not
+    depend on the group."""
+    from mlora import _ext
+    rng = np.random.default_rng(T * 31 + hin)
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
+    pool = upload_pool(pp)
+    tok = rng.integers(-1, len(ranks), T).astype(np.int32)
+    tok[0] = 0
+    t = torch.from_numpy(tok).cuda()
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
+    import ctypes
+    need = ctypes.c_int64()
+    hi, ho = (ctypes.c_int32 * 1)(hin), (ctypes.c_int32 * 1)(hout)
+    assert _ext.lib().mlora_bgmv_form(1, hi, ho, T, pool.n_slots, pool.max_rank, group, ctypes.byref(need)) in (_ext.FORM_FUSED, _ext.FORM_FINE)
+    assert need.value > _ext.lib().mlora_bgmv_workspace_bytes(1, T, hin, pool.max_rank) or hin <= 512
+    outs = {}
+    for g in (group, 1):
+        for accumulate in (True, False):
+            say(f"bgmv fine dtype={dtype} T={T} group={g} ranks={ranks} {hin}->{hout} accumulate={accumulate}")
+            plan = plan_decode(t, pool, group=g)
+            y = bits_to_torch(y0, dtype, "cuda")
+            bgmv([y], [bits_to_torch(x, dtype, "cuda")], pool, 0, ["p"], t, plan=plan, accumulate=accumulate, fused=False)
+            torch.cuda.synchronize()
+            outs[g, accumulate] = torch_to_bits(y)
+            assert_close_bits(outs[g, accumulate], oracle_apply(pp, x, tok, y0 if accumulate else None), dtype, "fine")
+    for accumulate in (True, False):
+        assert np.array_equal(outs[group, accumulate], outs[1, accumulate])
