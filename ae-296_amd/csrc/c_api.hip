@@ -665,10 +665,14 @@ SgmvWs sgmv_layout(int T, int n_seg, int n_proj)
     const long long per_split = (long long)w.max_tiles * n_proj;
     const long long target = n_proj > 1 ? 1024 : 768;
     long long ks = (target + per_split - 1) / per_split;
-    w.ksplit = ks < 1 ? 1 : (ks > 8 ? 8 : (int)ks);
+    // A prompt of a tile or two takes up to sixteen splits, two stages of 128 columns each at hidden 4096: the launch
+    // is a chain of loads and more workgroups shorten it (one prompt of 64 tokens, three projections at rank 64: 20.0 us a
+    // call with eight splits, 18.6 with sixteen, 21.0 with thirty-two; 512 tokens 24.9, 26.9, 30.9: partial sums).
+    const int most = w.max_tiles <= 6 ? 16 : 8;
+    w.ksplit = ks < 1 ? 1 : (ks > most ? most : (int)ks);
     // a projection with a longer K than the others of its call gets proportionally more splits (up to three
     // times as many, at most 8), so that every shrink workgroup walks about the same number of columns
-    w.ks_cap = n_proj > 1 ? (3 * w.ksplit < 8 ? 3 * w.ksplit : 8) : w.ksplit;
+    w.ks_cap = n_proj > 1 && w.ksplit < 8 ? (3 * w.ksplit < 8 ? 3 * w.ksplit : 8) : w.ksplit;
     size_t off = ((size_t)w.max_tiles * 3 + 4) * sizeof(int32_t);
     off = (off + 255) & ~(size_t)255;
     w.off_cover = off;                              // int32 [T]: 1 where a token belongs to some segment
@@ -686,14 +690,13 @@ SgmvWs sgmv_layout(int T, int n_seg, int n_proj)
 }
 
 // Columns of y one expand workgroup covers, and the column blocks per tile that follow from it.
-// 512 columns amortise the V operand; fewer when that leaves the chip idle (single-projection calls), and a block
+// 512 columns amortise the V operand; fewer when that leaves the chip idle (few tiles or projections), and a block
 // count per tile that the tile-major order of the expand can use (a multiple of eight or just below one):
 // otherwise the width that gives the nearest multiple of eight blocks, in whole cache lines.
 int expand_block_cols(int n_proj, int max_tiles, int hout, int *ncb_out)
 {
     int cols = 512;
-    if (n_proj == 1)
-        while (cols > 128 && (long long)max_tiles * ((hout + cols - 1) / cols) < 1024) cols >>= 1;
+    while (cols > 128 && (long long)max_tiles * n_proj * ((hout + cols - 1) / cols) < 1024) cols >>= 1;
     int ncb = (hout + cols - 1) / cols;
     if (!mlora::tile_major(ncb) && ncb >= 6) {
         const int n8 = ((ncb + 3) / 8) * 8 > 0 ? ((ncb + 3) / 8) * 8 : 8;
@@ -721,16 +724,22 @@ void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w)
         a.pr[p].vhi = reinterpret_cast<uint16_t *>(pb + w.off_hi);
         a.pr[p].vlo = reinterpret_cast<uint16_t *>(pb + w.off_lo);
         int ks = (int)(((long long)w.ksplit * a.pr[p].hin + hin_min / 2) / (hin_min > 0 ? hin_min : 1));
-        a.pr[p].ksplit = ks < w.ksplit ? w.ksplit : (ks > w.ks_cap ? w.ks_cap : ks);
+        ks = ks < w.ksplit ? w.ksplit : (ks > w.ks_cap ? w.ks_cap : ks);
+        const int nst = (a.pr[p].hin + 127) / 128;             // stages of the shrink: more splits than that would be empty
+        a.pr[p].ksplit = ks < nst ? ks : nst;
         int ncb = 0;
         const int cols = expand_block_cols(a.n_proj, w.max_tiles, a.pr[p].hout, &ncb);
         a.pr[p].cols = cols;
         a.pr[p].ncb = ncb;
     }
-    // shrink groups: up to three consecutive projections that read the same activations (one workgroup serves a group)
+    // shrink groups: up to three consecutive projections that read the same activations (one workgroup serves a group).
+    // A launch that leaves the chip half empty keeps them apart: x comes from L2 then, and three times as many
+    // workgroups share the work (three projections at rank 64, together / apart: 64 tokens 25.6 / 19.7 us a call, 1024
+    // tokens 41 / 36; four prompts of 512 52 / 52; seven projections, eight prompts of 100 tokens 76 / 83).
+    const bool share_x = (long long)w.max_tiles * a.n_proj * w.ksplit >= 704;
     a.n_grp = 0;
     for (int p = 0; p < a.n_proj; p++) {
-        if (p > 0 && a.pr[p].x == a.pr[p - 1].x && a.pr[p].hin == a.pr[p - 1].hin && a.grp_n[a.n_grp - 1] < 3) a.grp_n[a.n_grp - 1]++;
+        if (p > 0 && share_x && a.pr[p].x == a.pr[p - 1].x && a.pr[p].hin == a.pr[p - 1].hin && a.grp_n[a.n_grp - 1] < 3) a.grp_n[a.n_grp - 1]++;
         else { a.grp_first[a.n_grp] = p; a.grp_n[a.n_grp] = 1; a.n_grp++; }
     }
 }
@@ -960,6 +969,7 @@ int mlora_prefill_reflayout(void *y, const void *x, const void *A_T, const void 
     a.pr[0].hin = hin; a.pr[0].hout = hout;
     a.n_seg = B; a.T = T; a.accumulate = 0; a.b_transposed = 1; a.seg_uniform_len = Lpad;
     carve(a, workspace, w);
+    a.max_tiles = B * ((Lpad + SG_TM - 1) / SG_TM);
     rc = mlora::launch_sgmv(a, dtype, r, mlora::SGMV_PLAN | mlora::SGMV_APPLY, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "prefill launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;

@@ -64,14 +64,7 @@ __global__ __launch_bounds__(256) void gemm_lora_reduce_kernel(const GemmLoraArg
     for (int idx = threadIdx.x; idx < ntok * CPT; idx += 256) {
         const int t = tok0 + idx / CPT, c0 = (idx % CPT) * 8;
         float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = 0.f;
-        for (int sp = 0; sp < pj.ksplit; sp++) {
-            const float4_t *vp = reinterpret_cast<const float4_t *>(pj.v + ((size_t)sp * p.T + t) * MAX_RANK + c0);
-            const float4_t a = vp[0], b = vp[1];
-            v[0] += a[0]; v[1] += a[1]; v[2] += a[2]; v[3] += a[3];
-            v[4] += b[0]; v[5] += b[1]; v[6] += b[2]; v[7] += b[3];
-        }
+        sum_splits_any(pj.v + (size_t)t * MAX_RANK + c0, (size_t)p.T * MAX_RANK, pj.ksplit, v);
         uint32_t h[8], l[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) {

@@ -133,6 +133,35 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8])
     return make_uint4(pack2<DT>(f[0], f[1]), pack2<DT>(f[2], f[3]), pack2<DT>(f[4], f[5]), pack2<DT>(f[6], f[7]));
 }
 
+// v = sum over n K splits of eight neighbouring partial sums, in ascending order; the loads of U splits leave together.
+template <int U>
+__device__ __forceinline__ void sum_splits(const float *__restrict__ src, size_t stride, int n, float (&v)[8])
+{
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = 0.f;
+    for (int s0 = 0; s0 < n; s0 += U) {
+        float4_t a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float4_t *vp = reinterpret_cast<const float4_t *>(src + (size_t)(s0 + u < n ? s0 + u : s0) * stride);
+            a[u] = vp[0]; b[u] = vp[1];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) { v[e] += s0 + u < n ? a[u][e] : 0.f; v[4 + e] += s0 + u < n ? b[u][e] : 0.f; }
+        }
+    }
+}
+
+// The same with the loads of all splits in one batch, up to sixteen of them (n is uniform over the launch).
+__device__ __forceinline__ void sum_splits_any(const float *__restrict__ src, size_t stride, int n, float (&v)[8])
+{
+    if (n <= 2) sum_splits<2>(src, stride, n, v);
+    else if (n <= 8) sum_splits<8>(src, stride, n, v);
+    else sum_splits<16>(src, stride, n, v);
+}
+
 // Sum over each aligned group of 16 lanes (a DPP "row"); every lane of the row gets the sum.
 __device__ __forceinline__ float row16_sum(float v)
 {

@@ -73,6 +73,20 @@ __host__ __device__ inline long long xcd_grid(int max_tiles, int n_second)
     return 8LL * ((runs + 7) / 8) * n_second * XRUN;
 }
 
+// Launches of few tiles number the second index fastest, without padding: the runs above would leave most ids of a
+// batch of a tile or two without work (512 workgroups for 8 at one tile and eight splits), and what runs together
+// is everything anyway.
+__host__ __device__ inline bool few_tiles(int max_tiles) { return max_tiles < XRUN * 8; }
+__device__ __forceinline__ void place(int w, int n_second, int max_tiles, int &tile, int &second)
+{
+    if (few_tiles(max_tiles)) { tile = w / n_second; second = w - tile * n_second; }
+    else xcd_remap(w, n_second, tile, second);
+}
+__host__ __device__ inline long long place_grid(int max_tiles, int n_second)
+{
+    return few_tiles(max_tiles) ? (long long)max_tiles * n_second : xcd_grid(max_tiles, n_second);
+}
+
 // Expand launches use a second order where it fits: tile-major, the column blocks of a tile next to each other, so
 // that the eight workgroups running side by side (one per XCD) update one contiguous stretch of 64 y rows instead
 // of the same 1 KiB column block of 64 different tiles (DRAM pages stay open: a bare read-modify-write walk over
@@ -84,7 +98,48 @@ __host__ __device__ inline long long xcd_grid(int max_tiles, int n_second)
 // blocks; the host therefore picks the block width so that the count fits, see tile_major in mlora_args.hpp).
 __host__ __device__ inline long long expand_grid(int max_tiles, int ncb)
 {
-    return tile_major(ncb) ? (long long)max_tiles * ((ncb + 7) & ~7) : xcd_grid(max_tiles, ncb);
+    return tile_major(ncb) && !few_tiles(max_tiles) ? (long long)max_tiles * ((ncb + 7) & ~7) : place_grid(max_tiles, ncb);
+}
+
+// What a workgroup needs to know about its tile: from the plan's record, or, for equally long segments on a dense
+// pool (the reference's prefill, segment s = adapter s), computed, which needs no plan at all.
+// (A compile-time choice: a branch on it around the row lookups made the shrink wait for each of its twelve in turn,
+// which doubled the whole call.)
+template <bool UNIFORM>
+struct Tile {
+    int ntok, adapter, rank, tok0;
+    float scale;
+    const int32_t *__restrict__ rows;   // record: row of every rank row, -1 = absent
+    long long row0;                     // uniform: row of rank row 0
+    __device__ __forceinline__ int row(int j, long long n_rows) const
+    {
+        if constexpr (!UNIFORM) return rows[j];
+        const long long r = row0 + j;
+        return j < rank && r < n_rows ? (int)r : -1;
+    }
+};
+
+template <bool UNIFORM>
+__device__ __forceinline__ Tile<UNIFORM> tile_of(const SgmvArgs &p, int tile)
+{
+    Tile<UNIFORM> t;
+    if constexpr (UNIFORM) {
+        const int len = p.seg_uniform_len, per_seg = (len + TM - 1) / TM;
+        const int seg = tile / per_seg, i = tile - seg * per_seg;
+        t.ntok = len - i * TM < TM ? len - i * TM : TM;
+        t.adapter = seg;
+        t.rank = p.pool.uniform_rank < MAX_RANK ? p.pool.uniform_rank : MAX_RANK;
+        t.scale = p.pool.uniform_scale;
+        t.tok0 = seg * len + i * TM;
+        t.rows = nullptr;
+        t.row0 = (long long)seg * p.pool.a_dense_stride;
+    } else {
+        const int32_t *__restrict__ rec = p.tile_rec + (size_t)tile * TILE_WORDS;
+        t.ntok = rec[0]; t.adapter = rec[1]; t.rank = rec[2]; t.scale = __builtin_bit_cast(float, rec[3]); t.tok0 = rec[4];
+        t.rows = rec + TILE_ROWS_AT;
+        t.row0 = 0;
+    }
+    return t;
 }
 
 // ------------------------------------------------------------------ plan
@@ -140,6 +195,9 @@ __global__ __launch_bounds__(1024) void sgmv_plan_kernel(const SgmvArgs p)
     // Per-tile records: everything a shrink / expand workgroup needs, so that it starts from one load.
     // Headers of up to 1024 tiles at a time go through LDS (one tile per thread), then all threads
     // fill the 80-word records of that batch with one table lookup per row word.
+    // Records beyond the tiles in use are marked empty, so that a workgroup starts from its record alone and does not
+    // wait for the count first.
+    for (int t = n_tiles + tid; t < p.max_tiles; t += 1024) { p.tile_rec[(size_t)t * TILE_WORDS] = 0; p.tile_rec[(size_t)t * TILE_WORDS + 1] = -1; }
     const PoolView &pv = p.pool;
     __shared__ int s_hdr[1024][6];
     for (int t0 = 0; t0 < n_tiles; t0 += 1024) {
@@ -185,9 +243,11 @@ __device__ __forceinline__ float4_t mfma16(const uint4 &a, const uint4 &b, float
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf168_t, a), __builtin_bit_cast(bf168_t, b), c, 0, 0, 0);
 }
 
-constexpr int SG_NM = 3;     // projections of one x that a shrink workgroup serves (a larger group is cut by the host)
+constexpr int SG_NM = 3;     // projections of one x that a shrink workgroup serves at most (a larger group is cut by the host)
 
-template <int DT, int RMAX>
+// NM: the largest group of the launch (1 or SG_NM), which sizes the LDS: at rank 64 a launch whose groups are single
+// projections fits four workgroups on a unit instead of two.
+template <int DT, int RMAX, int NM, bool UNIFORM>
 __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
 {
     // One workgroup: 64 tokens x RMAX ranks over one K slice, for every projection of its group (up to SG_NM
@@ -204,20 +264,18 @@ __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
     constexpr int XP = TM * CPR / SG_NT;     // X loads per thread and stage (4)
     constexpr int AP = (RMAX * CPR + SG_NT - 1) / SG_NT;   // A loads per thread, projection and stage (1, 2 or 4)
     __shared__ __attribute__((aligned(16))) unsigned char s_x[TM * PITCH];
-    __shared__ __attribute__((aligned(16))) unsigned char s_a[SG_NM][RMAX * PITCH];
+    __shared__ __attribute__((aligned(16))) unsigned char s_a[NM][RMAX * PITCH];
     int grp = 0;
     while (grp + 1 < p.n_grp && blockIdx.x >= p.grp_end[grp]) grp++;
     int tile, split;
-    const int nm = p.grp_n[grp] < SG_NM ? p.grp_n[grp] : SG_NM; // projections this workgroup serves
-    xcd_remap((int)(blockIdx.x - (grp ? p.grp_end[grp - 1] : 0u)), p.pr[p.grp_first[grp]].ksplit, tile, split);
+    const int nm = p.grp_n[grp] < NM ? p.grp_n[grp] : NM;       // projections this workgroup serves
+    place((int)(blockIdx.x - (grp ? p.grp_end[grp - 1] : 0u)), p.pr[p.grp_first[grp]].ksplit, p.max_tiles, tile, split);
     const int p0 = p.grp_first[grp];
     const SgmvProj &pj = p.pr[p0];
-    if (tile >= p.n_tiles[0]) return;
-    const int32_t *__restrict__ rec = p.tile_rec + (size_t)tile * TILE_WORDS;
-    const int ntok = rec[0], adapter = rec[1];
-    const int tok0 = rec[4];
-    if (adapter < 0 || ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
-    const int32_t *__restrict__ rows = rec + TILE_ROWS_AT;     // -1 for every rank row that does not exist
+    if (tile >= p.max_tiles) return;                            // records beyond the tiles in use hold no tokens
+    const Tile<UNIFORM> tl = tile_of<UNIFORM>(p, tile);
+    const int ntok = tl.ntok, tok0 = tl.tok0;
+    if (tl.adapter < 0 || ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m = lane & 15, g = lane >> 4;
@@ -232,20 +290,20 @@ __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
         t = t < ntok ? t : ntok - 1;                            // tail rows repeat the last token; never stored
         xp[q] = reinterpret_cast<const uint4 *>(x + (size_t)(tok0 + t) * hin);
     }
-    const uint4 *ap[SG_NM][AP];
+    const uint4 *ap[NM][AP];
 #pragma unroll
-    for (int mm = 0; mm < SG_NM; mm++) {
+    for (int mm = 0; mm < NM; mm++) {
         const uint16_t *arows = static_cast<const uint16_t *>(p.pr[p0 + (mm < nm ? mm : 0)].a_rows);
 #pragma unroll
         for (int q = 0; q < AP; q++) {
             const int j = lrow + 16 * q;
-            const int row = j < RMAX ? rows[j] : -1;
+            const int row = j < RMAX ? tl.row(j, p.pool.n_rows_a) : -1;
             ap[mm][q] = reinterpret_cast<const uint4 *>(arows + (size_t)(row >= 0 ? row : 0) * hin);
         }
     }
-    float4_t acc[SG_NM][NB];
+    float4_t acc[NM][NB];
 #pragma unroll
-    for (int mm = 0; mm < SG_NM; mm++)
+    for (int mm = 0; mm < NM; mm++)
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) acc[mm][nb] = float4_t{0.f, 0.f, 0.f, 0.f};
 
@@ -254,7 +312,7 @@ __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
     const int per = (nstage + pj.ksplit - 1) / pj.ksplit;
     const int st0 = split * per;
     const int st1 = st0 + per < nstage ? st0 + per : nstage;
-    uint4 xr[XP], ar[SG_NM][AP];
+    uint4 xr[XP], ar[NM][AP];
     auto load_stage = [&](int st) {
         const int c = st * CPR + lchk;
         const bool ok = c < ncc;                                // K tail: both operands become zero
@@ -265,7 +323,7 @@ __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
             if (!ok) xr[q] = zero16();
         }
 #pragma unroll
-        for (int mm = 0; mm < SG_NM; mm++)
+        for (int mm = 0; mm < NM; mm++)
             if (mm < nm) {
 #pragma unroll
                 for (int q = 0; q < AP; q++) { ar[mm][q] = ldg16(ap[mm][q] + cs); if (!ok) ar[mm][q] = zero16(); }
@@ -279,7 +337,7 @@ __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
         for (int q = 0; q < XP; q++)
             *reinterpret_cast<uint4 *>(s_x + (lrow + 16 * q) * PITCH + lchk * 16) = xr[q];
 #pragma unroll
-        for (int mm = 0; mm < SG_NM; mm++)
+        for (int mm = 0; mm < NM; mm++)
             if (mm < nm) {
 #pragma unroll
                 for (int q = 0; q < AP; q++)
@@ -291,7 +349,7 @@ __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
         for (int ks = 0; ks < KB / 32; ks++) {
             const uint4 xf = *reinterpret_cast<const uint4 *>(s_x + (wave * 16 + m) * PITCH + (ks * 4 + g) * 16);
 #pragma unroll
-            for (int mm = 0; mm < SG_NM; mm++)
+            for (int mm = 0; mm < NM; mm++)
                 if (mm < nm) {
 #pragma unroll
                     for (int nb = 0; nb < NB; nb++) {
@@ -303,13 +361,13 @@ __global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
     }
     // D[token 4g+i][rank m] per 16x16 block; rank columns that do not exist are stored as zero.
 #pragma unroll
-    for (int mm = 0; mm < SG_NM; mm++)
+    for (int mm = 0; mm < NM; mm++)
         if (mm < nm) {
             float *vout = p.pr[p0 + mm].v + ((size_t)split * p.T + tok0 + wave * 16) * VSTRIDE;
 #pragma unroll
             for (int nb = 0; nb < NB; nb++) {
                 const int col = nb * 16 + m;
-                const bool col_ok = rows[col] >= 0;
+                const bool col_ok = tl.row(col, p.pool.n_rows_a) >= 0;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const int trow_o = wave * 16 + 4 * g + i;
@@ -345,7 +403,7 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
     const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (long long)p.T * CPT) return;
     const int t = (int)(idx / CPT), c0 = (int)(idx - (long long)t * CPT) * 8;
-    if (p.tok_cover[t] == 0) {
+    if (p.seg_uniform_len == 0 && p.tok_cover[t] == 0) {
         // token outside every segment: no tile touches its row.  y = delta mode defines it as zeros
         // (the CPT threads of the token share the row); accumulate mode keeps it.
         if (!p.accumulate) {
@@ -355,14 +413,7 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
         return;
     }
     float v[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = 0.f;
-    for (int sp = 0; sp < pj.ksplit; sp++) {
-        const float4_t *vp = reinterpret_cast<const float4_t *>(pj.v + ((size_t)sp * p.T + t) * VSTRIDE + c0);
-        const float4_t a = vp[0], b = vp[1];
-        v[0] += a[0]; v[1] += a[1]; v[2] += a[2]; v[3] += a[3];
-        v[4] += b[0]; v[5] += b[1]; v[6] += b[2]; v[7] += b[3];
-    }
+    sum_splits_any(pj.v + (size_t)t * VSTRIDE + c0, (size_t)p.T * VSTRIDE, pj.ksplit, v);
     uint4 hi, lo;
     split_hi_lo<DT>(v, hi, lo);
     stg16(pj.vhi + (size_t)t * VSTRIDE + c0, hi);
@@ -370,6 +421,12 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
 }
 
 // ------------------------------------------------------------------ expand
+// Up to rank 32 the expand sums up to eight K splits itself and the reduce launch falls away: seven projections at rank
+// 16, 16 tokens 28.8 -> 26.6 us a call, 8 x 512 tokens 184.6 -> 179.4.  At rank 64 the sums are four times as long and
+// every column block of a tile repeats them: 8 x 512 tokens 221 -> 232 us, 16 ragged prompts 375 -> 417 us of expand.
+template <int RMAX> constexpr bool FOLD_RANK = RMAX <= 32;
+constexpr int FOLD_SPLITS = 8;
+
 template <int DT, int RMAX, bool BT>
 __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
 {
@@ -399,20 +456,19 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     int tile, colblk;
     {
         const int w = (int)(blockIdx.x - (proj ? p.ex_end[proj - 1] : 0u));
-        if (tile_major(pj.ncb)) {
+        if (tile_major(pj.ncb) && !few_tiles(p.max_tiles)) {
             const int ncb8 = (pj.ncb + 7) & ~7;
             tile = w / ncb8;
             colblk = (w - tile * ncb8 + ncb8 - ((tile >> 3) & 7)) % ncb8;
             if (colblk >= pj.ncb) return;
         } else {
-            xcd_remap(w, pj.ncb, tile, colblk);
+            place(w, pj.ncb, p.max_tiles, tile, colblk);
         }
     }
-    if (tile >= p.n_tiles[0]) return;
-    const int32_t *__restrict__ rec = p.tile_rec + (size_t)tile * TILE_WORDS;
-    const int ntok = rec[0], adapter = rec[1], r = rec[2];
-    const float scale = __builtin_bit_cast(float, rec[3]);
-    const int tok0 = rec[4];
+    if (tile >= p.max_tiles) return;
+    const Tile<BT> tl = tile_of<BT>(p, tile);        // the reference layout and equal segments go together
+    const int ntok = tl.ntok, adapter = tl.adapter, r = tl.rank, tok0 = tl.tok0;
+    const float scale = tl.scale;
     const PoolView &pv = p.pool;
     if (ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
     const int hout = pj.hout;
@@ -437,13 +493,13 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     if constexpr (!BT) {
         // B rows share the page table with the A rows
         for (int j = tid; j < KP; j += SG_NT) {
-            const int row = j < MAX_RANK ? rec[TILE_ROWS_AT + j] : -1;
+            const int row = j < MAX_RANK ? tl.row(j, pv.n_rows_a) : -1;
             s_brow[j] = (row >= 0 && row < pv.n_rows_b) ? row : -1;
         }
     }
 
-    // ---- V operand: 16 tokens of this wavefront x KP ranks as a hi + lo pair of 16-bit values
-    // (written by the reduce kernel); rank columns beyond the adapter's rank are zero.
+    // ---- V operand: 16 tokens of this wavefront x KP ranks as a hi + lo pair of 16-bit values (written by the reduce
+    // kernel, or made here out of a few splits' partial sums); rank columns beyond the adapter's rank are zero.
     int trow = wave * 16 + m;
     trow = trow < ntok ? trow : ntok - 1;
     uint4 vhi[KS], vlo[KS];
@@ -451,6 +507,14 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     for (int ks = 0; ks < KS; ks++) {
         const int c0 = ks * 32 + 8 * g;
         vhi[ks] = zero16(); vlo[ks] = zero16();
+        if constexpr (FOLD_RANK<RMAX>) {
+            if (c0 < RMAX && p.fold) {
+                float v[8];
+                sum_splits<8>(pj.v + (size_t)(tok0 + trow) * VSTRIDE + c0, (size_t)p.T * VSTRIDE, pj.ksplit, v);
+                split_hi_lo<DT>(v, vhi[ks], vlo[ks]);
+                continue;
+            }
+        }
         if (c0 < RMAX) {
             vhi[ks] = ldg16(pj.vhi + ((size_t)(tok0 + trow) * VSTRIDE + c0));
             vlo[ks] = ldg16(pj.vlo + ((size_t)(tok0 + trow) * VSTRIDE + c0));
@@ -586,7 +650,7 @@ template <int DT, int RMAX>
 static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
 {
     int rc = 0;
-    if (phases & SGMV_PLAN) {
+    if ((phases & SGMV_PLAN) && a.seg_uniform_len == 0) {
         hipLaunchKernelGGL(sgmv_plan_kernel, dim3(1), dim3(1024), 0, s, a);
         rc = (int)hipGetLastError();
         if (rc) return rc;
@@ -596,7 +660,7 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     SgmvArgs g = a;
     unsigned end = 0;
     for (int q = 0; q < g.n_grp; q++) {
-        end += (unsigned)xcd_grid(g.max_tiles, g.pr[g.grp_first[q]].ksplit);
+        end += (unsigned)place_grid(g.max_tiles, g.pr[g.grp_first[q]].ksplit);
         g.grp_end[q] = end;
     }
     const unsigned sgrid = end;
@@ -606,10 +670,19 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
         g.ex_end[q] = end;
     }
     const unsigned egrid = end;
-    hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX>), dim3(sgrid), dim3(SG_NT), 0, s, g);
+    int nm = 1;
+    for (int q = 0; q < g.n_grp; q++) nm = g.grp_n[q] > nm ? g.grp_n[q] : nm;
+    if ((g.seg_uniform_len > 0) != (g.b_transposed != 0) || (g.b_transposed && nm != 1)) return (int)hipErrorInvalidValue;
+    if (g.seg_uniform_len > 0) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, 1, true>), dim3(sgrid), dim3(SG_NT), 0, s, g);
+    else if (nm == 1) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, 1, false>), dim3(sgrid), dim3(SG_NT), 0, s, g);
+    else hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, SG_NM, false>), dim3(sgrid), dim3(SG_NT), 0, s, g);
     rc = (int)hipGetLastError();
     if (rc || !(phases & SGMV_APPLY)) return rc;
-    {
+    // Few K splits are summed by the expand itself (FOLD_RANK); rows outside every segment are zeroed by the reduce launch only.
+    int most = 1;
+    for (int q = 0; q < g.n_proj; q++) most = g.pr[q].ksplit > most ? g.pr[q].ksplit : most;
+    g.fold = FOLD_RANK<RMAX> && most <= FOLD_SPLITS && (g.accumulate || g.seg_uniform_len > 0);
+    if (!g.fold) {
         const long long n = (long long)g.T * (RMAX / 8);
         hipLaunchKernelGGL((sgmv_reduce_kernel<DT, RMAX>), dim3((unsigned)((n + 255) / 256), (unsigned)g.n_proj), dim3(256), 0, s, g);
         rc = (int)hipGetLastError();
