@@ -869,6 +869,20 @@ int mlora_sgmv_multi_planned(int n_proj, void *const *y, const void *const *x, c
                        workspace_bytes, mlora::SGMV_APPLY, stream);
 }
 
+int64_t mlora_gemm_lora_partial_bytes(int n_proj, const int32_t *hin, const int32_t *hout, int T)
+{
+    if (n_proj < 1 || n_proj > MLORA_MAX_PROJ || !hin || !hout || T <= 0) return 0;
+    mlora::GemmLoraArgs g;
+    mlora::GemmShape sh;
+    memset(&g, 0, sizeof(g));
+    g.n_proj = n_proj; g.T = T;
+    for (int p = 0; p < n_proj; p++) {
+        if (hin[p] <= 0 || hout[p] <= 0) return 0;
+        g.pr[p].hin = hin[p]; g.pr[p].hout = hout[p];
+    }
+    return mlora::gemm_lora_shape(g, true, &sh);
+}
+
 int mlora_gemm_lora_planned(int n_proj, void *const *y, const void *const *x, const void *const *w,
                             const void *const *a_rows, const void *const *b_rows, const int32_t *hin,
                             const int32_t *hout, const int32_t *seg_start, const int32_t *seg_len,
@@ -876,6 +890,19 @@ int mlora_gemm_lora_planned(int n_proj, void *const *y, const void *const *x, co
                             const float *scaling, int T, int n_adapters, int max_pages, int page_rows,
                             int64_t n_pages, int max_rank, int dtype, void *workspace, int64_t workspace_bytes,
                             void *stream)
+{
+    return mlora_gemm_lora_split(n_proj, y, x, w, a_rows, b_rows, hin, hout, seg_start, seg_len, seg_adapter, n_seg, page_tbl,
+                                 rank, scaling, T, n_adapters, max_pages, page_rows, n_pages, max_rank, dtype, workspace,
+                                 workspace_bytes, nullptr, 0, stream);
+}
+
+int mlora_gemm_lora_split(int n_proj, void *const *y, const void *const *x, const void *const *w,
+                          const void *const *a_rows, const void *const *b_rows, const int32_t *hin,
+                          const int32_t *hout, const int32_t *seg_start, const int32_t *seg_len,
+                          const int32_t *seg_adapter, int n_seg, const int32_t *page_tbl, const int32_t *rank,
+                          const float *scaling, int T, int n_adapters, int max_pages, int page_rows,
+                          int64_t n_pages, int max_rank, int dtype, void *workspace, int64_t workspace_bytes,
+                          void *partials, int64_t partial_bytes, void *stream)
 {
     if (dtype != MLORA_F16 && dtype != MLORA_BF16) return fail(MLORA_EDTYPE, "dtype must be MLORA_F16 or MLORA_BF16 (got %d)", dtype);
     if (T < 0 || n_seg < 0) return fail(MLORA_EINVAL, "T and n_seg must be >= 0 (got %d, %d)", T, n_seg);
@@ -912,6 +939,12 @@ int mlora_gemm_lora_planned(int n_proj, void *const *y, const void *const *x, co
         }
     }
     g.n_proj = n_proj; g.T = T; g.lora = lora ? 1 : 0;
+    if (partials) {
+        const int64_t need = mlora_gemm_lora_partial_bytes(n_proj, hin, hout, T);
+        if (partial_bytes < need) return fail(MLORA_ENOSPACE, "partials hold %lld bytes, %lld needed", (long long)partial_bytes, (long long)need);
+        if (!aligned16(partials)) return fail(MLORA_EALIGN, "partials must be 16-byte aligned");
+        if (need > 0) { g.partials = static_cast<float *>(partials); g.partial_bytes = need; }
+    }
     if (lora) {
         const SgmvWs ws = sgmv_layout(T, n_seg, n_proj);
         if (!workspace || !aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be a 16-byte aligned device pointer");

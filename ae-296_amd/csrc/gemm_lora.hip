@@ -16,27 +16,35 @@
 // that global memory fills directly (buffer_load ... lds): while the MFMAs of step k run from one stage, the
 // loads of steps k+1 .. k+3 are in flight or landed.  x is K-contiguous, so its operand is a plain 16-byte
 // LDS read; W is N-contiguous and is read back with the transposing LDS read.
+//
+// A short batch runs the same loop on tiles of 64, 128 or 192 rows with K cut into ranges (gemm_lora_shape): its bound is
+// the weights' way from HBM up to about 64 tokens (Llama-7B layer, 405 MB: 78 us at 16 tokens) and the feed of the compute
+// units beyond.  A range leaves fp32 partial sums; one more launch adds them in K order and rounds once.
 #include "mlora_args.hpp"
 #include "mlora_dev.hpp"
 #include <type_traits>
 
 namespace mlora {
 
-constexpr int GM = 256;                 // rows (tokens) per tile
 constexpr int GN = 256;                 // output columns per tile
 constexpr int GK = 32;                  // K columns per stage
 constexpr int NST = 4;                  // stages in flight (a ring)
 constexpr int G_NT = 256;
-constexpr int A_BYTES = GM * GK * 2;    // x tile of a stage, rows unpadded and chunk-swizzled
-constexpr int B_BYTES = GK * GN * 2;    // W tile of a stage, likewise
-constexpr int STAGE = A_BYTES + B_BYTES;
+constexpr int B_BYTES = GK * GN * 2;    // W tile of a stage, chunk-swizzled like the x tile, rows unpadded
 constexpr int OPITCH = 128 * 2 + 16;    // bytes per row of a wavefront's 32 x 128 output staging tile
 constexpr int GROUP_M = 4;              // row tiles that share W column tiles back to back on one XCD
 typedef short gl_short4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) gl_short4 gl_lds_short4;
 
-static_assert(NST * STAGE <= 160 * 1024 - 4096, "the stages and the small tables must fit the LDS of a compute unit");
-static_assert(32 * OPITCH <= STAGE && MAX_RANK * GN * 2 <= STAGE, "a wavefront's output staging and the parked B rows each reuse one stage");
+// Bytes of one stage of the ring: an x tile of 64 * MI rows and a W tile; the parked B rows and a wavefront's output
+// staging reuse one stage each.
+template <int RMAX, int MI> constexpr int stage_bytes()
+{
+    constexpr int ab = 64 * MI * GK * 2 + B_BYTES, rows = RMAX * GN * 2;
+    return ab > rows ? ab : rows;
+}
+static_assert(NST * stage_bytes<64, 4>() <= 160 * 1024 - 4096, "the stages and the small tables must fit the LDS of a compute unit");
+static_assert(32 * OPITCH <= stage_bytes<16, 1>(), "a wavefront's output staging reuses one stage");
 
 template <int DT>
 __device__ __forceinline__ float16_t mfma32(const uint4 &a, const uint4 &b, float16_t c)
@@ -80,9 +88,14 @@ __global__ __launch_bounds__(256) void gemm_lora_reduce_kernel(const GemmLoraArg
 }
 
 // ------------------------------------------------------------------ GEMM + expand
-template <int DT, int RMAX>
-__global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p)
+// MI: 32-row MFMA blocks per wavefront, a tile has 64 * MI rows.  SPLIT: a workgroup walks one of the projection's
+// K ranges; where there are several it leaves fp32 partial sums for gemm_lora_sum_kernel, and the last one adds the LoRA part.
+template <int DT, int RMAX, int MI, bool SPLIT>
+__device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
 {
+    constexpr int GM = 64 * MI;
+    constexpr int A_BYTES = GM * GK * 2;
+    constexpr int STAGE = stage_bytes<RMAX, MI>();
     // one array per stage: the compiler then knows that loads into one stage cannot alias the operand reads of another
     __shared__ __attribute__((aligned(16))) unsigned char smem[STAGE];
     __shared__ __attribute__((aligned(16))) unsigned char smem1[STAGE];
@@ -101,14 +114,16 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
     while (proj + 1 < p.n_proj && blockIdx.x >= p.pr[proj].end) proj++;
     const GemmProj &pj = p.pr[proj];
     const int w = (int)(blockIdx.x - (proj ? p.pr[proj - 1].end : 0u));
-    const int ntn = pj.ntn, ntm = p.ntm;
+    const int nsplit = SPLIT ? pj.nsplit : 1;
+    const int ntn = pj.ntn * nsplit, ntm = p.ntm;               // the K ranges of a column tile follow each other
     const int n_tiles_out = ntm * ntn;
     const int per_xcd = (n_tiles_out + 7) >> 3;
     const int L = (w & 7) * per_xcd + (w >> 3);
     if ((w >> 3) >= per_xcd || L >= n_tiles_out) return;
     const int grp = L / (GROUP_M * ntn), within = L - grp * (GROUP_M * ntn);
     const int rows_in_grp = ntm - grp * GROUP_M < GROUP_M ? ntm - grp * GROUP_M : GROUP_M;
-    const int mt = grp * GROUP_M + within % rows_in_grp, nt = within / rows_in_grp;
+    const int mt = grp * GROUP_M + within % rows_in_grp, vt = within / rows_in_grp;
+    const int nt = SPLIT ? vt / nsplit : vt, split = SPLIT ? vt - nt * nsplit : 0;
     const int m0 = mt * GM, n0 = nt * GN;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -131,7 +146,8 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
         seg = rec[5];
         return h.y >= 0 && h.z > 0 && h.x > 0 && tok0 >= 0 && tok0 + h.x <= T && tok0 < m0 + GM && tok0 + h.x > m0;
     };
-    const int n_plan = p.lora ? p.n_tiles[0] : 0;
+    const bool lora = p.lora && split == nsplit - 1;
+    const int n_plan = lora ? p.n_tiles[0] : 0;
     // s_list / s_last = first and last tile of every run among plan tiles b0 .. b0 + 255, in order (a run that
     // crosses the window's end is cut there); s_list[G_NT] = how many (two barriers inside)
     auto list_tiles = [&](int b0) {
@@ -168,7 +184,7 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
             }
         }
     };
-    if (p.lora) {
+    if (lora) {
         // the first four runs: their records are fetched now, behind the K loop
         list_tiles(0);
         fill_rows(0, s_list[G_NT]);                // visible after the barrier that opens the K loop
@@ -185,13 +201,14 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
     // One load of wavefront w covers 16 rows of x (rows 16 (4 q + w) ..) or 2 rows of W (rows 2 (4 q + w) ..).
     // Rows beyond T and columns beyond hout are clamped to valid addresses; what they produce is never stored.
     const int rows_here = T - m0 < GM ? T - m0 : GM;
-    unsigned aoff[4], boff[4];
+    const int k0 = SPLIT ? split * pj.ksteps : 0;               // first K step of this workgroup
+    unsigned aoff[MI], boff[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
+    for (int q = 0; q < MI; q++) {
         const int row = 16 * (4 * q + wave) + (lane >> 2);
         const int c = (lane & 3) ^ ((row >> 2) & 3);
         const int r = row < rows_here ? row : rows_here - 1;
-        aoff[q] = ((unsigned)r * (unsigned)hin + (unsigned)c * 8u) * 2u;
+        aoff[q] = ((unsigned)r * (unsigned)hin + (unsigned)(k0 * GK) + (unsigned)c * 8u) * 2u;
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -199,7 +216,7 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
         const int c = (lane & 31) ^ ((k & 3) << 2);
         int col = n0 + c * 8;
         col = col < hout ? col : hout - 8;
-        boff[q] = ((unsigned)k * (unsigned)hout + (unsigned)col) * 2u;
+        boff[q] = ((unsigned)(k0 * GK + k) * (unsigned)hout + (unsigned)col) * 2u;
     }
     // A uniform descriptor per operand, a fixed 32-bit offset per load in a VGPR and the K advance as the scalar
     // offset: the loop spends no vector instructions on addresses.  The x descriptor starts at this tile's first
@@ -230,30 +247,30 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :: "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff) : "memory");
     };
-    // the 8 loads of one K step: 4 of x, 4 of W
+    // the loads of one K step: MI of x, 4 of W
     auto dma = [&](unsigned char *stage, int ks) {
         const unsigned soff_a = (unsigned)ks * (GK * 2), soff_b = (unsigned)ks * GK * (unsigned)hout * 2u;
         const unsigned base = (unsigned)(__UINTPTR_TYPE__)(lds_byte *)stage + (unsigned)wave * 1024u;
 #pragma unroll
-        for (int q = 0; q < 4; q++) dma1(xrw, base + q * 4096, aoff[q], soff_a);
+        for (int q = 0; q < MI; q++) dma1(xrw, base + q * 4096, aoff[q], soff_a);
 #pragma unroll
         for (int q = 0; q < 4; q++) dma1(wrw, base + A_BYTES + q * 4096, boff[q], soff_b);
     };
 
-    float16_t acc[4][4];
+    float16_t acc[MI][4];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < MI; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
 
-    // Operand addresses inside a stage.  x: lane (row wm * 128 + 32 i + lane % 32, chunk 2 kk + lane / 32); the key
+    // Operand addresses inside a stage.  x: lane (row wm * 32 MI + 32 i + lane % 32, chunk 2 kk + lane / 32); the key
     // of the row does not depend on i.  W: lane group g = lane / 16, m = lane % 16 reads rows 16 kk + 8 (g / 2) +
     // m / 4 (+ 4), bytes of columns wn * 128 + 32 j + 16 (g % 2) + 4 (m % 4) ..; the key (m / 4) * 4 flips bits of j.
     unsigned a_at[2], b_at[4];
     {
-        const int row = wm * 128 + l32, key = (l32 >> 2) & 3;
+        const int row = wm * (32 * MI) + l32, key = (l32 >> 2) & 3;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) a_at[kk] = (unsigned)(row * (GK * 2) + (((2 * kk + lh) ^ key) << 4));
         const int g = lane >> 4, m = lane & 15;
@@ -278,31 +295,33 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
                                __builtin_bit_cast(uint2, hi).x, __builtin_bit_cast(uint2, hi).y);
         }
     };
-    // Operands of one K = 16 slice (4 x fragments, 4 W fragments), read one slice ahead of the MFMAs that use them.
-    uint4 fa[2][4], fb[2][4];
-    auto frags = [&](const unsigned char *stage, auto kk_c, uint4 (&af)[4], uint4 (&bf)[4]) {
+    // Operands of one K = 16 slice (MI x fragments, 4 W fragments), read one slice ahead of the MFMAs that use them.
+    uint4 fa[2][MI], fb[2][4];
+    auto frags = [&](const unsigned char *stage, auto kk_c, uint4 (&af)[MI], uint4 (&bf)[4]) {
         constexpr int kk = decltype(kk_c)::value;
 #pragma unroll
-        for (int i = 0; i < 4; i++) af[i] = *reinterpret_cast<const uint4 *>(stage + a_at[kk] + i * 32 * (GK * 2));
+        for (int i = 0; i < MI; i++) af[i] = *reinterpret_cast<const uint4 *>(stage + a_at[kk] + i * 32 * (GK * 2));
         w_frags(stage + A_BYTES, kk, bf);
     };
-    auto mfma16x = [&](const uint4 (&af)[4], const uint4 (&bf)[4]) {
+    auto mfma16x = [&](const uint4 (&af)[MI], const uint4 (&bf)[4]) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < MI; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++) acc[i][j] = mfma32<DT>(af[i], bf[j], acc[i][j]);
     };
     using K0 = std::integral_constant<int, 0>;
     using K1 = std::integral_constant<int, 1>;
 #define GL_FENCE() __builtin_amdgcn_sched_barrier(0)
-    // Scheduling hints: one MFMA, then at most one operand read and at most one global load, so that the memory
+    // A slice is NM MFMAs; NR operand reads and NL global loads are dealt out over them.
+    constexpr int NM = 4 * MI, NR = MI + 8, NL = MI + 4;
+    constexpr int RPM = (NR + NM - 1) / NM, LPM = (NL + NM - 1) / NM;
+    // Scheduling hints: one MFMA, then its share of the operand reads, so that the memory
     // instructions issue in the shadow of the MFMAs instead of in a burst between them (an MFMA occupies its pipe
     // for 32 cycles, issuing it takes 4).
-#define GL_MIX(n_ds_read, n_load)                                                  \
-    _Pragma("unroll") for (int n_ = 0; n_ < 16; n_++) {                              \
+#define GL_MIX()                                                                   \
+    _Pragma("unroll") for (int n_ = 0; n_ < NM; n_++) {                              \
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          \
-        if (n_ < (n_ds_read)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    \
-        if (n_ < (n_load)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);       \
+        if (n_ * RPM < NR) __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0);     \
     }
     // s_waitcnt with only the vector-memory counter set: at most n loads of this wavefront still in flight
     // (loads complete in order).
@@ -330,32 +349,39 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
         unsigned char *nxt = cur_i == 0 ? smem1 : cur_i == 1 ? smem2 : cur_i == 2 ? smem3 : smem;
         frags(cur, K1{}, fa[1], fb[1]);
         mfma16x(fa[0], fb[0]);
-        GL_MIX(12, 0)
+        GL_MIX()
         GL_FENCE();
         const bool more_loads = steady || ks + 4 < ns, more_steps = steady || ks + 1 < ns;
-        GL_WAIT_LOADS(steady ? 16 : 0);            // steady: the loads of steps ks + 2 and ks + 3 may still be in flight
+        GL_WAIT_LOADS(steady ? 2 * NL : 0);        // steady: the loads of steps ks + 2 and ks + 3 may still be in flight
         __syncthreads();
         // Second slice, scheduled by hand (the loads are assembly, which the scheduler will not interleave):
-        // after MFMA n comes operand read n of the next step's first slice (4 of x, then 8 halves of W) and,
-        // for n < 8, load n of step ks + 4 into the stage that has just been released.
+        // after MFMA n come the operand reads n * RPM .. of the next step's first slice (MI of x, then 8 halves of W)
+        // and the loads n * LPM .. of step ks + 4 into the stage that has just been released.
         const unsigned soff_a = (unsigned)(ks + 4) * (GK * 2), soff_b = (unsigned)(ks + 4) * GK * (unsigned)hout * 2u;
         const unsigned lbase = (unsigned)(__UINTPTR_TYPE__)(lds_byte *)cur + (unsigned)wave * 1024u;
 #pragma unroll
-        for (int n = 0; n < 16; n++) {
+        for (int n = 0; n < NM; n++) {
             acc[n >> 2][n & 3] = mfma32<DT>(fa[1][n >> 2], fb[1][n & 3], acc[n >> 2][n & 3]);
             if (more_steps) {
-                if (n < 4) {
-                    fa[0][n] = *reinterpret_cast<const uint4 *>(nxt + a_at[0] + n * 32 * (GK * 2));
-                } else if (n < 12) {
-                    const int j = (n - 4) >> 1;
-                    const unsigned char *src = nxt + A_BYTES + b_at[j] + ((n & 1) ? 4 * (GN * 2) : 0);
-                    const uint2 h = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((gl_lds_short4 *)src));
-                    if (n & 1) { fb[0][j].z = h.x; fb[0][j].w = h.y; } else { fb[0][j].x = h.x; fb[0][j].y = h.y; }
+#pragma unroll
+                for (int t = n * RPM; t < n * RPM + RPM; t++) {
+                    if (t < MI) {
+                        fa[0][t] = *reinterpret_cast<const uint4 *>(nxt + a_at[0] + t * 32 * (GK * 2));
+                    } else if (t < NR) {
+                        const int j = (t - MI) >> 1;
+                        const bool second = ((t - MI) & 1) != 0;
+                        const unsigned char *src = nxt + A_BYTES + b_at[j] + (second ? 4 * (GN * 2) : 0);
+                        const uint2 h = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((gl_lds_short4 *)src));
+                        if (second) { fb[0][j].z = h.x; fb[0][j].w = h.y; } else { fb[0][j].x = h.x; fb[0][j].y = h.y; }
+                    }
                 }
             }
-            if (more_loads && n < 8) {
-                if (n < 4) dma1(xrw, lbase + n * 4096, aoff[n], soff_a);
-                else dma1(wrw, lbase + A_BYTES + (n - 4) * 4096, boff[n - 4], soff_b);
+            if (more_loads) {
+#pragma unroll
+                for (int t = n * LPM; t < n * LPM + LPM; t++) {
+                    if (t < MI) dma1(xrw, lbase + t * 4096, aoff[t], soff_a);
+                    else if (t < NL) dma1(wrw, lbase + A_BYTES + (t - MI) * 4096, boff[t - MI], soff_b);
+                }
             }
             GL_FENCE();
         }
@@ -368,7 +394,8 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
     using No = std::false_type;
 
     // Full K steps run through the pipeline; a partial last step follows on its own.
-    const int ns = hin / GK;
+    const int ns_all = hin / GK;
+    const int ns = !SPLIT ? ns_all : (ns_all - k0 < pj.ksteps ? ns_all - k0 : pj.ksteps);
     if (ns > 0) {
         dma(smem, 0);
         if (ns > 1) dma(smem1, 1);
@@ -393,31 +420,31 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
             if (ks + 3 < ns) k_step(S3{}, No{}, ks + 3, ns);
         }
     }
-    if (ns * GK < hin) {
+    if (ns_all * GK < hin && split == nsplit - 1) {
         // Partial last K step: through registers, with chunks of x and rows of W beyond hin replaced by zeros,
         // parked in the same swizzled layout, in the stage after the one the last full step read (some wavefronts
         // may still be reading that one; the one after it was released four steps ago).
         unsigned char *st = (ns & 3) == 0 ? smem : (ns & 3) == 1 ? smem1 : (ns & 3) == 2 ? smem2 : smem3;
         const int ncc = hin >> 3;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < MI; q++) {
             const int row = 16 * (4 * q + wave) + (lane >> 2);
             const int c = (lane & 3) ^ ((row >> 2) & 3);
-            const bool ok = ns * 4 + c < ncc;
-            const unsigned back = ok ? 0u : (unsigned)(ns * 4 + c - (ncc - 1)) * 16u;
+            const bool ok = ns_all * 4 + c < ncc;
+            const unsigned back = ok ? 0u : (unsigned)(ns_all * 4 + c - (ncc - 1)) * 16u;
             const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)(aoff[q] - back), ns * (GK * 2), 0);
             *reinterpret_cast<uint4 *>(st + (4 * q + wave) * 1024 + lane * 16) = ok ? make_uint4(v.x, v.y, v.z, v.w) : zero16();
         }
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int k = ns * GK + 2 * (4 * q + wave) + (lane >> 5);
+            const int k = ns_all * GK + 2 * (4 * q + wave) + (lane >> 5);
             const bool ok = k < hin;
             const unsigned back = ok ? 0u : (unsigned)(k - (hin - 1)) * (unsigned)hout * 2u;
             const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(wrs, (int)(boff[q] - back), (int)((unsigned)ns * GK * (unsigned)hout * 2u), 0);
             *reinterpret_cast<uint4 *>(st + A_BYTES + (4 * q + wave) * 1024 + lane * 16) = ok ? make_uint4(v.x, v.y, v.z, v.w) : zero16();
         }
         __syncthreads();
-        const int rem = hin - ns * GK;
+        const int rem = hin - ns_all * GK;
         frags(st, K0{}, fa[0], fb[0]); mfma16x(fa[0], fb[0]);
         if (rem > 16) { frags(st, K1{}, fa[0], fb[0]); mfma16x(fa[0], fb[0]); }
     }
@@ -431,12 +458,12 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
     // of two MFMAs per 32 columns with (hi, lo) of the intermediate of the tile's rows as the x operand (zero
     // for the other rows).  The intermediate depends on the row only, so a block's operands are read once,
     // one block ahead, whatever tiles cover it.
-    if (p.lora) {
+    if (lora) {
         constexpr int NSL = RMAX / 16;             // rank rows an adapter does not have read as zeros on both sides,
                                                    // so every tile runs the same RMAX / 16 slices
         // (hi, lo) of rank columns 16 s + 8 (lane / 32) .. + 7 of this lane's row in 32-row block i
         auto load_v = [&](int i, uint4 (&vh)[NSL], uint4 (&vl)[NSL]) {
-            int row = m0 + wm * 128 + i * 32 + l32;
+            int row = m0 + wm * (32 * MI) + i * 32 + l32;
             row = row < T ? row : T - 1;
             const size_t at = (size_t)row * MAX_RANK + 8 * lh;
 #pragma unroll
@@ -468,9 +495,9 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
             GL_WAIT_LOADS(0);
             __syncthreads();
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                if (i + 1 < 4) load_v(i + 1, vh[(i + 1) & 1], vl[(i + 1) & 1]);
-                const int R0 = wm * 128 + i * 32, my = R0 + l32;
+            for (int i = 0; i < MI; i++) {
+                if (i + 1 < MI) load_v(i + 1, vh[(i + 1) & 1], vl[(i + 1) & 1]);
+                const int R0 = wm * (32 * MI) + i * 32, my = R0 + l32;
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     if (q >= nrun || R0 + 32 <= i0[q] || R0 >= i1[q]) continue;       // uniform per wavefront
@@ -506,7 +533,26 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
     }
 #undef GL_WAIT_LOADS
 
-    // ---- y: every wavefront passes its 128 x 128 block through a private LDS tile, 32 rows at a time, so
+    if constexpr (SPLIT) {
+        if (nsplit > 1) {
+            // partial sums of this K range: a wavefront's store covers 128 contiguous bytes of two rows
+            float *__restrict__ part = pj.part + (size_t)split * T * hout;
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int gc = n0 + wn * 128 + j * 32 + l32;
+#pragma unroll
+                    for (int e = 0; e < 16; e++) {
+                        const int gr = m0 + wm * (32 * MI) + i * 32 + 8 * (e >> 2) + 4 * lh + (e & 3);
+                        if (gr < T && gc < hout) part[(size_t)gr * hout + gc] = acc[i][j][e];
+                    }
+                }
+            return;
+        }
+    }
+
+    // ---- y: every wavefront passes its 32 MI x 128 block through a private LDS tile, 32 rows at a time, so
     // that the stores are 16 bytes wide and a 16-lane row covers 256 contiguous bytes of one token.
     // D layout of the 32x32 MFMA: lane holds column lane % 32, rows 8 * (e / 4) + 4 * (lane / 32) + e % 4.
     // The tile is private to the wavefront and LDS operations of one wavefront complete in order, so no
@@ -517,7 +563,7 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
         typedef __attribute__((address_space(3))) volatile u32x4_t lds_vu32x4;
         uint16_t *__restrict__ y = static_cast<uint16_t *>(pj.y);
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < MI; i++) {
 #pragma unroll
             for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -532,7 +578,7 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
             for (int q = 0; q < 8; q++) {
                 const int pp = lane + 64 * q, row = pp >> 4, c = pp & 15;
                 const u32x4_t v = *(lds_vu32x4 *)(so + row * OPITCH + c * 16);
-                const int gr = m0 + wm * 128 + i * 32 + row, gc = n0 + wn * 128 + c * 8;
+                const int gr = m0 + wm * (32 * MI) + i * 32 + row, gc = n0 + wn * 128 + c * 8;
                 if (gr < T && gc < hout) stg16_stream(y + (size_t)gr * hout + gc, make_uint4(v.x, v.y, v.z, v.w));
             }
         }
@@ -540,33 +586,137 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
 }
 
 template <int DT, int RMAX>
+__global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p)
+{
+    gemm_lora_body<DT, RMAX, 4, false>(p);
+}
+
+// Batches of few tiles (shape_of): tiles of 64 to 256 rows, K cut into ranges.
+template <int DT, int RMAX, int MI>
+__global__ __launch_bounds__(G_NT, 1) void gemm_lora_short_kernel(const GemmLoraArgs p)
+{
+    gemm_lora_body<DT, RMAX, MI, true>(p);
+}
+
+// y = round16(sum of a projection's partial sums, in ascending K order); blockIdx.y counts the projections that have any.
+template <int DT>
+__global__ __launch_bounds__(256) void gemm_lora_sum_kernel(const GemmLoraArgs p)
+{
+    int proj = -1;
+    for (int q = 0, n = 0; q < p.n_proj; q++)
+        if (p.pr[q].nsplit > 1 && n++ == (int)blockIdx.y) proj = q;
+    if (proj < 0) return;
+    const GemmProj &pj = p.pr[proj];
+    const size_t n8 = (size_t)p.T * pj.hout / 8, idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= n8) return;
+    float v[8];
+    sum_splits_any(pj.part + idx * 8, n8 * 8, pj.nsplit, v);
+    stg16_stream(static_cast<uint16_t *>(pj.y) + idx * 8, pack8<DT>(v));
+}
+
+// ------------------------------------------------------------------ shape of a launch
+// Rows per tile (64 * mi) and K ranges per projection for a batch of T tokens.
+//
+// Tiles of 256 rows with K whole are right once they fill the chip several times over.  A short batch makes a few
+// hundred tiles or fewer: most units idle, the longest K (the MLP's second product) is a chain several times as long as
+// the rest, and rows past T are multiplied for nothing.  The rule estimates, for every tile height and number of
+// ranges, rounds of workgroups x mean time of one (or the longest chain) plus the cost of the partial sums, and takes
+// the least; the plain shape stays within 5 % of it, where the estimate does not tell them apart.  Step times are those
+// measured with one workgroup on each unit.  Base products at Llama-7B widths, fp16, us, plain -> chosen (best of the 28
+// shapes tried): q/k/v 16 tokens 77 -> 30 (28), 120 tokens 83 -> 41 (40), 351 tokens 85 -> 64 (63), 700 tokens 95 -> 84 (84);
+// all seven 16 tokens 196 -> 78 (78; 5.2 TB/s of weights), 192 tokens 249 -> 111 (111), 351 tokens 268 -> 199 (191), 500
+// tokens 292 -> 265 (258); from 1024 tokens on the plain shape is the fastest or within 2 % of it (q/k/v at 1500: 203 -> 170).
+// Tiles of 256 rows are never cut: with the ranges the compiler spills accumulators.
+int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out)
+{
+    static const double step_us[4] = {0.42, 0.55, 0.68, 0.85};                // one K step, by mi
+    const double ends_us = 6.0, launch_us = 4.0, byte_us = 2.0 / 4.0e6;         // a workgroup's start and end; one more launch; a byte written and read
+    const double cus = device_compute_units();
+    int longest = 1;
+    for (int q = 0; q < a.n_proj; q++) longest = a.pr[q].hin / GK > longest ? a.pr[q].hin / GK : longest;
+    double best = 0.0;
+    int64_t best_bytes = 0;
+    GemmShape cand;
+    for (int mi = 4; mi >= 1; mi--) {
+        const int64_t ntm = ((int64_t)a.T + 64 * mi - 1) / (64 * mi);
+        for (int k = 1; k <= (may_split && mi < 4 ? 8 : 1); k++) {
+            const int target = (longest + k - 1) / k;
+            double items = 0, total = 0, chain = 0;
+            int64_t bytes = 0;
+            cand.mi = mi;
+            for (int q = 0; q < a.n_proj; q++) {
+                const int ns = a.pr[q].hin / GK > 0 ? a.pr[q].hin / GK : 1;
+                int n = k == 1 ? 1 : (ns + target / 2) / target;
+                n = n < 1 ? 1 : n;
+                const int per = (ns + n - 1) / n;
+                n = (ns + per - 1) / per;                                       // no range is empty
+                cand.nsplit[q] = n;
+                cand.ksteps[q] = per;
+                const double t = per * step_us[mi - 1] + ends_us;
+                const double it = (double)ntm * ((a.pr[q].hout + GN - 1) / GN) * n;
+                items += it; total += it * t; chain = t > chain ? t : chain;
+                if (n > 1) bytes += (int64_t)n * a.T * a.pr[q].hout * (int64_t)sizeof(float);
+            }
+            double us = __builtin_ceil(items / cus) * (total / items);
+            us = us > chain ? us : chain;
+            if (bytes > 0) us += launch_us + (double)bytes * byte_us;
+            if (mi == 4) {
+                *out = cand; best = 0.95 * us;
+                if (items >= 8 * cus) return 0;                                 // many rounds: nothing to gain
+            } else if (us < best) { best = us; *out = cand; best_bytes = bytes; }
+        }
+    }
+    return best_bytes;
+}
+
+template <int DT, int RMAX>
 static int launch_gl(const GemmLoraArgs &a, hipStream_t s)
 {
     GemmLoraArgs g = a;
     g.rmax = RMAX;
-    g.ntm = (g.T + GM - 1) / GM;
-    // projections with the longest K loop first: their tiles take longest, and a long tile started last
+    GemmShape sh;
+    if (gemm_lora_shape(g, g.partials != nullptr, &sh) > g.partial_bytes) return (int)hipErrorInvalidValue;
+    const int gm = 64 * sh.mi;
+    g.ntm = (g.T + gm - 1) / gm;
+    float *part = g.partials;
+    for (int q = 0; q < g.n_proj; q++) {
+        g.pr[q].nsplit = sh.nsplit[q];
+        g.pr[q].ksteps = sh.ksteps[q];
+        g.pr[q].part = part;
+        if (sh.nsplit[q] > 1) part += (size_t)sh.nsplit[q] * g.T * g.pr[q].hout;
+    }
+    // projections with the longest K range first: their tiles take longest, and a long tile started last
     // would leave the rest of the device idle at the end of the launch
     for (int q = 1; q < g.n_proj; q++)
-        for (int r = q; r > 0 && g.pr[r].hin > g.pr[r - 1].hin; r--) {
+        for (int r = q; r > 0 && g.pr[r].ksteps > g.pr[r - 1].ksteps; r--) {
             const GemmProj t = g.pr[r]; g.pr[r] = g.pr[r - 1]; g.pr[r - 1] = t;
         }
-    unsigned end = 0;
+    unsigned end = 0, n_sum = 0;
+    long long widest = 0;
     for (int q = 0; q < g.n_proj; q++) {
         g.pr[q].ntn = (g.pr[q].hout + GN - 1) / GN;
-        const long long tiles = (long long)g.ntm * g.pr[q].ntn;
+        const long long tiles = (long long)g.ntm * g.pr[q].ntn * g.pr[q].nsplit;
         const long long padded = (tiles + 7) / 8 * 8;
         if (end + padded > 0x7fffffffLL) return (int)hipErrorInvalidValue;
         end += (unsigned)padded;
         g.pr[q].end = end;
+        if (g.pr[q].nsplit > 1) { n_sum++; widest = g.pr[q].hout > widest ? g.pr[q].hout : widest; }
     }
     if (end == 0) return 0;
+    int rc = 0;
     if (g.lora) {
         hipLaunchKernelGGL((gemm_lora_reduce_kernel<DT, RMAX>), dim3((unsigned)g.max_tiles, (unsigned)g.n_proj), dim3(256), 0, s, g);
-        const int rc = (int)hipGetLastError();
+        rc = (int)hipGetLastError();
         if (rc) return rc;
     }
-    hipLaunchKernelGGL((gemm_lora_kernel<DT, RMAX>), dim3(end), dim3(G_NT), 0, s, g);
+    if (sh.mi == 4) hipLaunchKernelGGL((gemm_lora_kernel<DT, RMAX>), dim3(end), dim3(G_NT), 0, s, g);
+    else if (sh.mi == 3) hipLaunchKernelGGL((gemm_lora_short_kernel<DT, RMAX, 3>), dim3(end), dim3(G_NT), 0, s, g);
+    else if (sh.mi == 2) hipLaunchKernelGGL((gemm_lora_short_kernel<DT, RMAX, 2>), dim3(end), dim3(G_NT), 0, s, g);
+    else hipLaunchKernelGGL((gemm_lora_short_kernel<DT, RMAX, 1>), dim3(end), dim3(G_NT), 0, s, g);
+    rc = (int)hipGetLastError();
+    if (rc || n_sum == 0) return rc;
+    const long long blocks = (g.T * widest / 8 + 255) / 256;
+    hipLaunchKernelGGL((gemm_lora_sum_kernel<DT>), dim3((unsigned)blocks, n_sum), dim3(256), 0, s, g);
     return (int)hipGetLastError();
 }
 

@@ -171,6 +171,8 @@ struct GemmProj {
     int ksplit;
     int ntn;               // column tiles (set by the launcher)
     unsigned end;          // first workgroup id after this projection (set by the launcher)
+    int nsplit, ksteps;    // K ranges of a tile, and the 32-column steps of each (set by the launcher)
+    float *part;           // [nsplit, T, hout] partial sums when there are several (set by the launcher)
 };
 
 struct GemmLoraArgs {
@@ -184,7 +186,12 @@ struct GemmLoraArgs {
     const int32_t *n_tiles;    // [1]
     int max_tiles;
     long long n_rows_b;
+    float *partials;       // room for the partial sums of tiles whose K is cut (null: none is)
+    long long partial_bytes;
 };
+
+// Shape of a base GEMM + LoRA launch: tiles of 64 * mi rows, and the K ranges per projection.
+struct GemmShape { int mi, nsplit[MAX_PROJ], ksteps[MAX_PROJ]; };
 
 // launchers (defined next to their kernels); return hipError_t as int
 int launch_bgmv(const BgmvArgs &a, int dtype, int group, int max_rank, bool b_transposed, hipStream_t s);
@@ -200,6 +207,8 @@ constexpr int SGMV_APPLY = 2;   // shrink, reduce, expand (the workspace already
 constexpr int SGMV_SHRINK = 4;  // the shrink launch alone: its partial sums feed the base GEMM + LoRA kernel
 int launch_sgmv(const SgmvArgs &a, int dtype, int max_rank, int phases, hipStream_t s);
 int launch_gemm_lora(const GemmLoraArgs &a, int dtype, int max_rank, hipStream_t s);
+// the shape for a.T, a.n_proj and the projections' hin and hout; returns the bytes of partial sums it takes
+int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out);
 // compute units of the current device (asked once per device; 256 when the query fails)
 int device_compute_units();
 

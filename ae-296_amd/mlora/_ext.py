@@ -71,6 +71,9 @@ SIGNATURES = {
                                         _i32, _i32, _i64, _i32, _i32, _i32, _vp, _i64, _vp]),
     "mlora_gemm_lora_planned": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32,
                                        _i32, _i32, _i64, _i32, _i32, _vp, _i64, _vp]),
+    "mlora_gemm_lora_partial_bytes": (_i64, [_i32, _vp, _vp, _i32]),
+    "mlora_gemm_lora_split": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32,
+                                     _i32, _i32, _i64, _i32, _i32, _vp, _i64, _vp, _i64, _vp]),
     "mlora_prefill_reflayout": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp]),
 }
 

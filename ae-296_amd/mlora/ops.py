@@ -398,17 +398,21 @@ def gemm_lora(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], ws: Sequen
         yv[i], xv[i], wv[i], hi[i], ho[i] = ys[i].data_ptr(), xs[i].data_ptr(), ws[i].data_ptr(), hin, hout
         if plan is not None:
             av[i], bv[i] = pool.slab_ptrs(layer, p)
+    # room for the partial sums of a batch that is cut along K (a short one)
+    room = _ext.lib().mlora_gemm_lora_partial_bytes(n, hi, ho, T)
+    partials = torch.empty(room, dtype=torch.uint8, device=xs[0].device) if room else None
     if plan is None:
-        rc = _ext.lib().mlora_gemm_lora_planned(n, yv, xv, wv, None, None, hi, ho, None, None, None, 0, None, None, None, T,
-                                                0, 0, 0, 0, 16, _ext.dtype_code(dtype), None, 0, _ext.current_stream_ptr())
+        rc = _ext.lib().mlora_gemm_lora_split(n, yv, xv, wv, None, None, hi, ho, None, None, None, 0, None, None, None, T,
+                                              0, 0, 0, 0, 16, _ext.dtype_code(dtype), None, 0, _ext.ptr(partials), room,
+                                              _ext.current_stream_ptr())
     else:
         n_seg = _check_segments(plan.seg_start, plan.seg_len, plan.seg_adapter)
         pool.sync()
-        rc = _ext.lib().mlora_gemm_lora_planned(
+        rc = _ext.lib().mlora_gemm_lora_split(
             n, yv, xv, wv, av, bv, hi, ho, plan.seg_start.data_ptr(), plan.seg_len.data_ptr(), plan.seg_adapter.data_ptr(),
             n_seg, _ext.ptr(pool.page_tbl), _ext.ptr(pool.rank), _ext.ptr(pool.scaling), T, pool.n_slots, pool.max_pages,
             pool.page_rows, pool.n_pages, pool.max_rank, pool.dtype_code,
-            plan.workspace.data_ptr(), plan.workspace.numel(), _ext.current_stream_ptr())
+            plan.workspace.data_ptr(), plan.workspace.numel(), _ext.ptr(partials), room, _ext.current_stream_ptr())
     _ext.check(rc)
 
 

@@ -366,6 +366,22 @@ int mlora_gemm_lora_planned(int n_proj, void *const *y, const void *const *x, co
                             int dtype, void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
+ * The same with room for partial sums: a batch of few output tiles is then cut along K as well, the pieces are summed
+ * in fp32 in a fixed order by one more launch and rounded once.  mlora_gemm_lora_partial_bytes says how much room such a
+ * call takes (0: it is not cut); `partials` is a 16-byte aligned device pointer to at least that much, or NULL.
+ * Calls that share it must be ordered on one stream.
+ */
+int64_t mlora_gemm_lora_partial_bytes(int n_proj, const int32_t *hin, const int32_t *hout, int T);
+int mlora_gemm_lora_split(int n_proj, void *const *y, const void *const *x, const void *const *w,
+                          const void *const *a_rows, const void *const *b_rows,
+                          const int32_t *hin, const int32_t *hout,
+                          const int32_t *seg_start, const int32_t *seg_len, const int32_t *seg_adapter, int n_seg,
+                          const int32_t *page_tbl, const int32_t *rank, const float *scaling,
+                          int T, int n_adapters, int max_pages, int page_rows, int64_t n_pages, int max_rank,
+                          int dtype, void *workspace, int64_t workspace_bytes, void *partials, int64_t partial_bytes,
+                          void *stream);
+
+/*
  * The reference's prefill call on its own layout (lora_gpu.py:125-128): request b uses
  * adapter slot b; x [B, Lpad, hin]; A_T [>=B, L, r, hin]; B_T [>=B, L, hout, r];
  * y [B, Lpad, hout] = (x[b] . A_T[b, layer]^T) . B_T[b, layer]^T   (y is overwritten).

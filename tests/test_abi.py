@@ -96,6 +96,15 @@ def test_validation_errors_without_gpu():
     rc = lib.mlora_sgmv(one, one, one, one, one, one, one, 2, one, one, one, 100, 64, 64, 4, 8, 8, 10, 64, 1, 1,
                         one, 16, None)
     assert rc == _ext.MLORA_ENOSPACE
+    # base products: a short batch may be cut along K and says how much room that takes, a long one is not
+    wide = (C.c_int32 * 8)(*([4096] * 8))
+    need = lib.mlora_gemm_lora_partial_bytes(3, wide, wide, 64)
+    assert need >= 2 * 3 * 64 * 4096 * 4
+    assert lib.mlora_gemm_lora_partial_bytes(7, wide, wide, 8192) == 0
+    assert lib.mlora_gemm_lora_partial_bytes(3, wide, wide, 0) == 0
+    rc = lib.mlora_gemm_lora_split(3, P, P, P, None, None, wide, wide, None, None, None, 0, None, None, None, 64, 0, 0, 0, 0, 16, 0,
+                                   None, 0, 16, need - 1, None)
+    assert rc == _ext.MLORA_ENOSPACE
     rc = lib.mlora_bgmv_reflayout(one, one, one, one, one, 4, 8, 32, 16, 64, 64, 32, 1.0, 0, None)
     assert rc == _ext.MLORA_ERANGE                     # layer_idx == L
     # grouped reference-layout call: ranks 8 / 16 / 32 / 64 only, plan buffer and workspace sizes checked

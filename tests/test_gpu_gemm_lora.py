@@ -217,3 +217,62 @@ def test_plan_tile_list_matches_oracle(aligned):
     assert np.array_equal(words[:n], want_s)
     assert np.array_equal(words[max_tiles:max_tiles + n], want_t0)
     assert np.array_equal(words[2 * max_tiles:2 * max_tiles + n], want_n)
+
+
+@pytest.mark.parametrize("T,hin,hout,n_proj,ranks,dtype", [
+    (1, 2056, 264, 1, [64, 8], FP16),          # one row of a 64-row tile, uneven K ranges and a partial last step
+    (64, 2088, 4104, 3, [16, 8], BF16),        # a full 64-row tile, a column tile of eight columns
+    (65, 2056, 4096, 3, [64, 24], FP16),       # 128-row tiles, one row in the upper half's first block
+    (128, 3080, 4096, 3, [32, 17], BF16),
+    (129, 4104, 4096, 3, [32, 16], FP16),      # 192-row tiles, one row in the third block
+    (192, 4096, 4352, 3, [64, 40], BF16),
+    (351, 4104, 1288, 7, [16, 8], FP16),       # two row tiles, the second with a ragged end
+])
+def test_gemm_lora_short_batches(T, hin, hout, n_proj, ranks, dtype):
+    """Tiles of 64 to 192 rows with K cut into ranges: the rows at the tiles' edges against the oracle, every projection
+    alike, and the same result as the call without room for partial sums up to the last rounding."""
+    from mlora import _ext
+    import ctypes as C
+    rng = np.random.default_rng(T * 7 + hin)
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
+    names = [f"p{i}" for i in range(n_proj)]
+    pool = upload_pool(pp, projections={nm: (hin, hout) for nm in names})
+    for nm in names:
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, dtype))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, dtype))
+    cut = max(1, T // 3)
+    lens = [cut] + ([T - cut] if T > cut else [])
+    ss, sl, sa, _ = _layout(lens, [0] * len(lens), [0, 1][:len(lens)])
+    tok = _tok_of(ss, sl, sa, T)
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
+    w = bits_of((rng.standard_normal((hin, hout)) / np.sqrt(hin)).astype(np.float32), dtype)
+    xt, wt = bits_to_torch(x, dtype, "cuda"), bits_to_torch(w, dtype, "cuda")
+    arr = [(C.c_int32 * 8)(*([v] * n_proj)) for v in (hin, hout)]
+    assert _ext.lib().mlora_gemm_lora_partial_bytes(n_proj, *arr, T) > 0          # K is cut
+    plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in (ss, sl, sa)), T, pool, n_proj=n_proj)
+    ys = [torch.full((T, hout), float("nan"), dtype=tdtype(dtype), device="cuda") for _ in names]
+    say(f"gemm_lora short T={T} {hin}x{hout} n_proj={n_proj} ranks={ranks} dtype={dtype}")
+    gemm_lora(ys, [xt] * n_proj, [wt] * n_proj, pool, 0, names, plan)
+    torch.cuda.synchronize()
+    got = torch_to_bits(ys[0])
+    rows = np.unique(np.clip([0, cut - 1, cut, 31, 32, 63, 64, 65, 127, 128, 191, 192, T - 2, T - 1], 0, T - 1))
+    assert_close_bits(got[rows], _oracle(pp, x[rows], w, tok[rows]), dtype, "rows at the edges")
+    for y in ys[1:]:
+        assert torch.equal(y, ys[0])
+    # without room for partial sums: K whole, the same products summed in another order.  Both round one fp32 sum to 16
+    # bits; sums differ by no more than hin roundings of 2^-24 of their terms' size, about one, so by less than 1e-3 at
+    # these widths, and the results by that and one rounding step.
+    ptr = lambda ts: (C.c_void_p * 8)(*[t.data_ptr() for t in ts])
+    whole = [torch.empty_like(y) for y in ys]
+    rc = _ext.lib().mlora_gemm_lora_planned(
+        n_proj, ptr(whole), ptr([xt] * n_proj), ptr([wt] * n_proj), ptr([pool.a_rows[nm][0] for nm in names]),
+        ptr([pool.b_rows[nm][0] for nm in names]), *arr, plan.seg_start.data_ptr(), plan.seg_len.data_ptr(),
+        plan.seg_adapter.data_ptr(), len(lens), pool.page_tbl.data_ptr(), pool.rank.data_ptr(), pool.scaling.data_ptr(), T,
+        pool.n_slots, pool.max_pages, pool.page_rows, pool.n_pages, pool.max_rank, pool.dtype_code,
+        plan.workspace.data_ptr(), plan.workspace.numel(), _ext.current_stream_ptr())
+    _ext.check(rc)
+    torch.cuda.synchronize()
+    ulp = 2.0 ** (-10 if dtype == FP16 else -7)
+    for y in whole:
+        a, b = y.double(), ys[0].double()
+        assert bool(((a - b).abs() <= ulp * b.abs() + 1e-3).all())
