@@ -32,7 +32,6 @@ FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-featu
 LIMITS = [
     ("gemm_lora.hip", r"gemm_lora_kernel<", {"scratch": (0, 0), "vgpr_spill": (0, 0), "agprs": (256, 256), "vgprs": (0, 256),
                                              "occupancy": (1, 1), "lds": (0, 160 * 1024), "accvgpr_moves": (0, 1300)}),
-    ("gemm_lora.hip", r"gemm_lora_short_kernel<", {"lds": (0, 160 * 1024), "accvgpr_moves": (0, 800)}),
     ("gemm_lora.hip", r".", {"scratch": (0, 0), "vgpr_spill": (0, 0)}),
     ("bgmv_split.hip", r".", {"scratch": (0, 0), "vgpr_spill": (0, 0)}),
     ("bgmv_split.hip", r"bgmv_shrink_kernel<\d, [124], 16, 256, false>", {"occupancy": (4, 8)}),
