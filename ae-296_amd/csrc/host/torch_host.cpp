@@ -85,6 +85,22 @@ struct List {       // a list or tuple of the caller
 
 void *stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+// Other Python threads run while a launch is made (it waits when the device's queue is full).
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    Unlocked() = default;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+    Unlocked(const Unlocked &) = delete;
+    Unlocked &operator=(const Unlocked &) = delete;
+};
+
+template <typename F, typename... A>
+int launch(F entry_point, A... args)                 // args are read before the lock goes
+{
+    const Unlocked u;
+    return entry_point(args...);
+}
+
 // ---------------------------------------------------------------- a call over projections of one pool layer
 struct Call {
     int n = 0, dtype = 0;
@@ -177,8 +193,8 @@ PyObject *gather(PyObject *const *v, Py_ssize_t nargs)
     const at::Tensor &tok = tensor(v[2]);
     const Tables tb = tables(pool);
     auto i32 = [&](PyObject *name) { return static_cast<int32_t *>(attr_ptr(plan, name)); };
-    const int rc = mlora_pool_gather(
-        static_cast<const int32_t *>(tok.data_ptr()), (int)tok.numel(), tb.page_tbl, tb.rank, tb.scaling,
+    const int rc = launch(
+        mlora_pool_gather, static_cast<const int32_t *>(tok.data_ptr()), (int)tok.numel(), tb.page_tbl, tb.rank, tb.scaling,
         tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, i32(s_row_off), i32(s_tok_rank), static_cast<float *>(attr_ptr(plan, s_tok_scale)), i32(s_perm), i32(s_seg_start),
         i32(s_seg_len), i32(s_seg_adapter), i32(s_chunk_start), i32(s_chunk_len), i32(s_chunk_adapter), (int)as_int(v[3]),
         i32(s_counters), i32(s_work), stream());
@@ -217,8 +233,8 @@ PyObject *bgmv(PyObject *const *v, Py_ssize_t nargs)
         if (v[7] == Py_None && form == MLORA_FORM_FUSED) fused = true;
         else ws = intermediate(plan, ws_bytes, tok);
     }
-    const int rc = mlora_bgmv_multi(
-        c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, static_cast<const int32_t *>(tok.data_ptr()), (int)T, tb.page_tbl, tb.rank, tb.scaling,
+    const int rc = launch(
+        mlora_bgmv_multi, c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, static_cast<const int32_t *>(tok.data_ptr()), (int)T, tb.page_tbl, tb.rank, tb.scaling,
         tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, tb.max_rank, plan ? static_cast<const int32_t *>(attr_ptr(plan, s_work)) : nullptr,
         group, ws, fused ? 0 : ws_bytes, c.dtype, accumulate, stream());
     return PyLong_FromLong(rc);
@@ -261,7 +277,7 @@ PyObject *bgmv_ref(PyObject *const *v, Py_ssize_t nargs)
     static PyObject *s_buf = PyUnicode_InternFromString("buf");
     const int64_t bytes = mlora_bgmv_workspace_bytes(n, (int)T, max_hin, (int)r);
     void *ws = bytes > 0 ? intermediate(plan, bytes, ys[0]) : nullptr;
-    const int rc = mlora_bgmv_reflayout_multi(n, y, x, a, b, hin, hout, attr_ptr(plan, s_buf), (int)T, (int)N, (int)L, (int)r,
+    const int rc = launch(mlora_bgmv_reflayout_multi, n, y, x, a, b, hin, hout, attr_ptr(plan, s_buf), (int)T, (int)N, (int)L, (int)r,
                                               (int)as_int(v[5]), (float)PyFloat_AsDouble(v[6]), (int)attr_int(plan, s_group),
                                               type == at::kHalf ? MLORA_F16 : MLORA_BF16, v[7] == Py_True, ws, bytes, stream());
     return PyLong_FromLong(rc);
@@ -292,7 +308,7 @@ PyObject *prefill_plan(PyObject *const *v, Py_ssize_t nargs)
     const at::Tensor &ws = tensor(v[5]);
     const Tables tb = tables(pool);
     const auto plan = v[6] == Py_True ? mlora_sgmv_plan_aligned : mlora_sgmv_plan;
-    const int rc = plan(sg.start, sg.len, sg.adapter, (int)sg.n, tb.page_tbl, tb.rank, tb.scaling, (int)as_int(v[4]),
+    const int rc = launch(plan, sg.start, sg.len, sg.adapter, (int)sg.n, tb.page_tbl, tb.rank, tb.scaling, (int)as_int(v[4]),
                         tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, tb.max_rank, ws.data_ptr(), ws.numel(), stream());
     return PyLong_FromLong(rc);
 }
@@ -310,7 +326,7 @@ PyObject *sgmv_multi(PyObject *const *v, Py_ssize_t nargs)
     const Segments sg = segments(tensor(start.o), tensor(len.o), tensor(adapter.o));
     const at::Tensor &ws = tensor(wsp.o);
     const Tables tb = tables(pool);
-    const int rc = mlora_sgmv_multi_planned(c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, sg.start, sg.len, sg.adapter, (int)sg.n, tb.page_tbl,
+    const int rc = launch(mlora_sgmv_multi_planned, c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, sg.start, sg.len, sg.adapter, (int)sg.n, tb.page_tbl,
                                             tb.rank, tb.scaling, (int)T, tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, tb.max_rank,
                                             c.dtype, v[6] == Py_True, ws.data_ptr(), ws.numel(), stream());
     return PyLong_FromLong(rc);
