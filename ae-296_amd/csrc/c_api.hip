@@ -655,7 +655,7 @@ struct SgmvWs { int max_tiles; int ksplit; int ks_cap; size_t off_cover, off_rec
 
 // Workspace: the plan (tile list, tile records: depends on T and n_seg only), then per projection the
 // K-split partial sums and the hi / lo halves of their sum.
-SgmvWs sgmv_layout(int T, int n_seg, int n_proj)
+SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int most)
 {
     SgmvWs w;
     w.max_tiles = T / SG_TM + 2 * n_seg + 1;       // aligned cuts can add one partial tile at either end of a segment
@@ -665,10 +665,6 @@ SgmvWs sgmv_layout(int T, int n_seg, int n_proj)
     const long long per_split = (long long)w.max_tiles * n_proj;
     const long long target = n_proj > 1 ? 1024 : 768;
     long long ks = (target + per_split - 1) / per_split;
-    // A prompt of a tile or two takes up to sixteen splits, two stages of 128 columns each at hidden 4096: the launch
-    // is a chain of loads and more workgroups shorten it (one prompt of 64 tokens, three projections at rank 64: 20.0 us a
-    // call with eight splits, 18.6 with sixteen, 21.0 with thirty-two; 512 tokens 24.9, 26.9, 30.9: partial sums).
-    const int most = w.max_tiles <= 6 ? 16 : 8;
     w.ksplit = ks < 1 ? 1 : (ks > most ? most : (int)ks);
     // a projection with a longer K than the others of its call gets proportionally more splits (up to three
     // times as many, at most 8), so that every shrink workgroup walks about the same number of columns
@@ -687,6 +683,20 @@ SgmvWs sgmv_layout(int T, int n_seg, int n_proj)
     w.per_proj = (w.off_lo + (size_t)T * MLORA_MAX_RANK * sizeof(uint16_t) + 255) & ~(size_t)255;
     w.total = off + w.per_proj * n_proj;
     return w;
+}
+
+// The layout for a workspace of `have` bytes (negative: as large as the call can use).
+// A prompt of a tile or two takes up to sixteen splits, two stages of 128 columns each at hidden 4096: the launch
+// is a chain of loads and more workgroups shorten it (one prompt of 64 tokens, three projections at rank 64: 20.0 us a
+// call with eight splits, 18.6 with sixteen, 21.0 with thirty-two; 512 tokens 24.9, 26.9, 30.9: partial sums).
+// Where they do not fit, eight do: a workspace sized for a longer batch serves its shorter ones.
+SgmvWs sgmv_layout(int T, int n_seg, int n_proj, int64_t have = -1)
+{
+    if (T / SG_TM + 2 * n_seg + 1 <= 6) {
+        const SgmvWs w = sgmv_layout_splits(T, n_seg, n_proj, 16);
+        if (have < 0 || (int64_t)w.total <= have) return w;
+    }
+    return sgmv_layout_splits(T, n_seg, n_proj, 8);
 }
 
 // Columns of y one expand workgroup covers, and the column blocks per tile that follow from it.
@@ -797,7 +807,7 @@ static int sgmv_common(int n_proj, void *const *y, const void *const *x, const v
     } else {
         a.pr[0].hin = 8; a.pr[0].hout = 8;
     }
-    const SgmvWs w = sgmv_layout(T, n_seg, n_proj);
+    const SgmvWs w = sgmv_layout(T, n_seg, n_proj, workspace_bytes < 0 ? 0 : workspace_bytes);
     if (!workspace || !aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be a 16-byte aligned device pointer");
     if (workspace_bytes < (int64_t)w.total)
         return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)w.total);
@@ -946,7 +956,7 @@ int mlora_gemm_lora_split(int n_proj, void *const *y, const void *const *x, cons
         if (need > 0) { g.partials = static_cast<float *>(partials); g.partial_bytes = need; }
     }
     if (lora) {
-        const SgmvWs ws = sgmv_layout(T, n_seg, n_proj);
+        const SgmvWs ws = sgmv_layout(T, n_seg, n_proj, workspace_bytes < 0 ? 0 : workspace_bytes);
         if (!workspace || !aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be a 16-byte aligned device pointer");
         if (workspace_bytes < (int64_t)ws.total)
             return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)ws.total);
@@ -982,7 +992,7 @@ int mlora_prefill_reflayout(void *y, const void *x, const void *A_T, const void 
         return fail(MLORA_EALIGN, "device pointers must be 16-byte aligned");
     if ((int64_t)B * L * r > 0x7fffffffLL) return fail(MLORA_ERANGE, "pool has more than 2^31-1 rank rows");
     const int T = B * Lpad;
-    const SgmvWs w = sgmv_layout(T, B, 1);
+    const SgmvWs w = sgmv_layout(T, B, 1, workspace_bytes < 0 ? 0 : workspace_bytes);
     if (!workspace || !aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be a 16-byte aligned device pointer");
     if (workspace_bytes < (int64_t)w.total)
         return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)w.total);

@@ -305,3 +305,25 @@ def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj):
         want = oracle_apply(pp, x, tok, y0 if accumulate else None)
         for nm, y in zip(names, ys):
             assert_close_bits(torch_to_bits(y), want, FP16, nm)
+
+
+def test_sgmv_workspace_of_a_longer_batch():
+    """A workspace sized for one prompt of 400 tokens takes a shorter prompt, though that one has a use for more."""
+    from mlora import _ext, sgmv_multi
+    from mlora.ops import sgmv_workspace
+    rng = np.random.default_rng(5)
+    T, hin, hout = 255, 4096, 264
+    pp = PagedPool(rng, [64], hin, hout, page_rows=8, dtype=FP16)
+    pool = upload_pool(pp)
+    seg = _segments([T], [0])
+    dev = [torch.from_numpy(a).cuda() for a in seg]
+    ws = sgmv_workspace(400, 1, "cuda", 1)
+    assert ws.numel() < _ext.lib().mlora_sgmv_workspace_bytes(T, 1)
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), FP16)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), FP16)
+    y = bits_to_torch(y0, FP16, "cuda")
+    say(f"sgmv workspace of a longer batch T={T} {hin}->{hout}")
+    plan = plan_prefill(*dev, T, pool, workspace=ws)
+    sgmv_multi([y], [bits_to_torch(x, FP16, "cuda")], pool, 0, ["p"], plan)
+    torch.cuda.synchronize()
+    assert_close_bits(torch_to_bits(y), oracle_apply(pp, x, _tok_of(*seg, T), y0), FP16, "short prompt")
