@@ -185,6 +185,20 @@ void *intermediate(PyObject *plan, int64_t bytes, const at::Tensor &like)
 }
 
 // ---------------------------------------------------------------- decode
+// A plan's buffer: data pointer (null for None), after a check that a launch on `like` may write `n` values of its type there.
+void *buffer(PyObject *plan, PyObject *name, at::ScalarType type, int64_t n, const at::Tensor &like)
+{
+    Ref a(PyObject_GetAttr(plan, name));
+    if (a.o == Py_None) return nullptr;
+    const at::Tensor &t = tensor(a.o);
+    if (t.numel() < n)
+        raise(PyExc_ValueError, "the plan's %U holds %lld values, %lld needed: it was made for a smaller batch or pool", name,
+              (long long)t.numel(), (long long)n);
+    if (t.scalar_type() != type || !t.is_contiguous() || t.device() != like.device())
+        raise(PyExc_ValueError, "the plan's %U must be a contiguous buffer of its type on the batch's device", name);
+    return t.data_ptr();
+}
+
 // gather(pool, plan, tok_adapter, group)
 PyObject *gather(PyObject *const *v, Py_ssize_t nargs)
 {
@@ -192,12 +206,18 @@ PyObject *gather(PyObject *const *v, Py_ssize_t nargs)
     PyObject *pool = v[0], *plan = v[1];
     const at::Tensor &tok = tensor(v[2]);
     const Tables tb = tables(pool);
-    auto i32 = [&](PyObject *name) { return static_cast<int32_t *>(attr_ptr(plan, name)); };
-    const int rc = launch(
-        mlora_pool_gather, static_cast<const int32_t *>(tok.data_ptr()), (int)tok.numel(), tb.page_tbl, tb.rank, tb.scaling,
-        tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, i32(s_row_off), i32(s_tok_rank), static_cast<float *>(attr_ptr(plan, s_tok_scale)), i32(s_perm), i32(s_seg_start),
-        i32(s_seg_len), i32(s_seg_adapter), i32(s_chunk_start), i32(s_chunk_len), i32(s_chunk_adapter), (int)as_int(v[3]),
-        i32(s_counters), i32(s_work), stream());
+    const int64_t T = tok.numel(), segs = T < tb.n_slots ? T : tb.n_slots;
+    auto i32 = [&](PyObject *name, int64_t n) { return static_cast<int32_t *>(buffer(plan, name, at::kInt, n, tok)); };
+    // the per-token view, which is None unless the caller asked for it
+    int32_t *row_off = i32(s_row_off, T * tb.max_pages), *tok_rank = i32(s_tok_rank, T);
+    float *tok_scale = static_cast<float *>(buffer(plan, s_tok_scale, at::kFloat, T, tok));
+    int32_t *perm = i32(s_perm, T), *seg_start = i32(s_seg_start, segs), *seg_len = i32(s_seg_len, segs), *seg_adapter = i32(s_seg_adapter, segs);
+    int32_t *chunk_start = i32(s_chunk_start, T), *chunk_len = i32(s_chunk_len, T), *chunk_adapter = i32(s_chunk_adapter, T);
+    int32_t *counters = i32(s_counters, MLORA_CNT_WORDS), *work = i32(s_work, (int64_t)MLORA_WORK_CAP(T) * MLORA_WORK_WORDS);
+    need_device(tok);
+    const int rc = launch(mlora_pool_gather, static_cast<const int32_t *>(tok.data_ptr()), (int)T, tb.page_tbl, tb.rank, tb.scaling, tb.n_slots,
+                          tb.max_pages, tb.page_rows, tb.n_pages, row_off, tok_rank, tok_scale, perm, seg_start, seg_len, seg_adapter,
+                          chunk_start, chunk_len, chunk_adapter, (int)as_int(v[3]), counters, work, stream());
     return PyLong_FromLong(rc);
 }
 

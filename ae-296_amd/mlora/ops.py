@@ -112,7 +112,8 @@ def plan_decode(tok_adapter: torch.Tensor, pool: AdapterPool, group: Optional[in
     """Index/offset gather for a decode batch: groups tokens by adapter (stable) and cuts the
     groups into work items of at most `group` tokens (1, 2, 4 or 8; default by batch size and, when the
     caller says how many projections its calls will carry (`n_proj`), by the launch form those take).  Pass
-    `out` to reuse a plan's buffers (no allocation; safe under graph capture)."""
+    `out` to reuse a plan's buffers (no allocation; safe under graph capture; a batch or pool larger than the one it
+    was made for is refused)."""
     _need_cuda(tok_adapter)
     if tok_adapter.dtype != torch.int32:
         raise TypeError("tok_adapter must be int32")
@@ -134,12 +135,12 @@ def plan_decode(tok_adapter: torch.Tensor, pool: AdapterPool, group: Optional[in
             out.row_off = torch.empty((max(T, 1), pool.max_pages), **i32)
             out.tok_rank = torch.empty(max(T, 1), **i32)
             out.tok_scale = torch.empty(max(T, 1), dtype=torch.float32, device=dev)
-    else:
-        out.tok_adapter = tok_adapter
-        out.group = group
     rc = _ext.host().gather(pool, out, tok_adapter, group)
     if rc:
         _ext.check(rc)
+    # only now: a batch that the plan's buffers do not hold was refused and must not be taken for the plan's own
+    out.tok_adapter = tok_adapter
+    out.group = group
     return out
 
 

@@ -71,3 +71,16 @@ def test_slabs_are_read_from_the_pool_on_every_call():
     want = oracle_apply(pp, torch_to_bits(x), tok.cpu().numpy())
     assert_close_bits(torch_to_bits(y), want, FP16, "first slab")
     assert torch.equal(y2, (y.float() * 2).half())           # doubling is exact in fp16
+
+
+def test_a_plan_refuses_a_larger_batch_and_stays_usable():
+    """A batch larger than the plan's buffers is refused before anything is launched, and leaves the plan its own batch."""
+    pp, pool, tok, x, y = _setup(T=4)
+    plan = mlora.plan_decode(tok, pool)
+    with pytest.raises(ValueError):
+        mlora.plan_decode(torch.zeros(300, dtype=torch.int32, device="cuda"), pool, out=plan)
+    assert plan.tok_adapter is tok
+    say("bgmv on a plan that refused a larger batch")
+    mlora.bgmv([y], [x], pool, 0, ["p"], tok, plan=plan, accumulate=False)
+    torch.cuda.synchronize()
+    assert_close_bits(torch_to_bits(y), oracle_apply(pp, torch_to_bits(x), tok.cpu().numpy()), FP16, "own batch")
