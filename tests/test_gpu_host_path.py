@@ -70,7 +70,11 @@ def test_slabs_are_read_from_the_pool_on_every_call():
     torch.cuda.synchronize()
     want = oracle_apply(pp, torch_to_bits(x), tok.cpu().numpy())
     assert_close_bits(torch_to_bits(y), want, FP16, "first slab")
-    assert torch.equal(y2, (y.float() * 2).half())           # doubling is exact in fp16
+    # Doubling is exact where y is a normal fp16 number.  Below 2^-14 the spacing no longer falls with the value: y is up
+    # to half a step (2^-25) from its sum, which doubling doubles, and y2 up to half a step from twice that sum.
+    normal = y.abs() >= 2.0 ** -14
+    assert torch.equal(y2[normal], (y * 2)[normal])
+    assert bool(((y2.float() - 2 * y.float())[~normal].abs() <= 3 * 2.0 ** -25).all())
 
 
 def test_a_plan_refuses_a_larger_batch_and_stays_usable():
