@@ -326,6 +326,8 @@ PyObject *prefill_plan(PyObject *const *v, Py_ssize_t nargs)
     PyObject *pool = v[0];
     const Segments sg = segments(tensor(v[1]), tensor(v[2]), tensor(v[3]));
     const at::Tensor &ws = tensor(v[5]);
+    need_device(ws);
+    need_contiguous(ws);
     const Tables tb = tables(pool);
     const auto plan = v[6] == Py_True ? mlora_sgmv_plan_aligned : mlora_sgmv_plan;
     const int rc = launch(plan, sg.start, sg.len, sg.adapter, (int)sg.n, tb.page_tbl, tb.rank, tb.scaling, (int)as_int(v[4]),
@@ -345,6 +347,8 @@ PyObject *sgmv_multi(PyObject *const *v, Py_ssize_t nargs)
         wsp(PyObject_GetAttr(plan, s_workspace));
     const Segments sg = segments(tensor(start.o), tensor(len.o), tensor(adapter.o));
     const at::Tensor &ws = tensor(wsp.o);
+    need_device(ws);
+    need_contiguous(ws);
     const Tables tb = tables(pool);
     const int rc = launch(mlora_sgmv_multi_planned, c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, sg.start, sg.len, sg.adapter, (int)sg.n, tb.page_tbl,
                                             tb.rank, tb.scaling, (int)T, tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, tb.max_rank,

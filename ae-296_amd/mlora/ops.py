@@ -349,6 +349,8 @@ def sgmv(y: torch.Tensor, x: torch.Tensor, pool: AdapterPool, layer: int, proj: 
         raise TypeError(f"x and y must have the pool dtype {pool.dtype}")
     if workspace is None:
         workspace = sgmv_workspace(T, n_seg, x.device)
+    _need_cuda(workspace)
+    _need_contig(workspace)
     pool.sync()
     a_ptr, b_ptr = pool.slab_ptrs(layer, proj)
     fn = _ext.lib().mlora_sgmv_planned if plan is not None else _ext.lib().mlora_sgmv
@@ -408,6 +410,8 @@ def gemm_lora(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], ws: Sequen
                                               _ext.current_stream_ptr())
     else:
         n_seg = _check_segments(plan.seg_start, plan.seg_len, plan.seg_adapter)
+        _need_cuda(plan.workspace)
+        _need_contig(plan.workspace)
         pool.sync()
         rc = _ext.lib().mlora_gemm_lora_split(
             n, yv, xv, wv, av, bv, hi, ho, plan.seg_start.data_ptr(), plan.seg_len.data_ptr(), plan.seg_adapter.data_ptr(),
@@ -439,6 +443,8 @@ def lora_prefill_ref(x: torch.Tensor, A_T: torch.Tensor, B_T: torch.Tensor, laye
             raise ValueError("out must be a contiguous device tensor [bsz, Lpad, Hout] of x's dtype")
     if workspace is None:
         workspace = sgmv_workspace(bsz * lpad, bsz, x.device)
+    _need_cuda(workspace)
+    _need_contig(workspace)
     rc = _ext.lib().mlora_prefill_reflayout(y.data_ptr(), x.data_ptr(), A_T.data_ptr(), B_T.data_ptr(), bsz, lpad, L, r,
                                             hin, hout, layer_idx, _ext.dtype_code(x.dtype), workspace.data_ptr(),
                                             workspace.numel(), _ext.current_stream_ptr())

@@ -88,3 +88,21 @@ def test_a_plan_refuses_a_larger_batch_and_stays_usable():
     mlora.bgmv([y], [x], pool, 0, ["p"], tok, plan=plan, accumulate=False)
     torch.cuda.synchronize()
     assert_close_bits(torch_to_bits(y), oracle_apply(pp, torch_to_bits(x), tok.cpu().numpy()), FP16, "own batch")
+
+
+def test_a_prefill_workspace_in_host_memory_is_refused():
+    """Every prefill entry point writes its workspace from the device: one in host memory is refused before a launch."""
+    pp, pool, tok, x, y = _setup()
+    seg = tuple(torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([0], [5], [1]))
+    host = mlora.sgmv_workspace(5, 1, "cpu")
+    strided = torch.empty((host.numel(), 2), dtype=torch.uint8, device="cuda")[:, 0]
+    w = torch.zeros(64, 96, device="cuda").half()
+    for ws in (host, strided):
+        plan = mlora.PrefillPlan(*seg, 5, ws)
+        for call in (lambda: mlora.plan_prefill(*seg, 5, pool, workspace=ws), lambda: mlora.sgmv_multi([y], [x], pool, 0, ["p"], plan),
+                     lambda: mlora.sgmv(y, x, pool, 0, "p", plan=plan), lambda: mlora.sgmv(y, x, pool, 0, "p", *seg, workspace=ws),
+                     lambda: mlora.gemm_lora([y], [x], [w], pool, 0, ["p"], plan),
+                     lambda: mlora.lora_prefill_ref(x[None], torch.zeros(1, 1, 8, 64, device="cuda").half(),
+                                                    torch.zeros(1, 1, 96, 8, device="cuda").half(), 0, workspace=ws)):
+            with pytest.raises(ValueError):
+                call()
