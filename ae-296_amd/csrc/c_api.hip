@@ -378,8 +378,8 @@ int mlora_bgmv_form(int n_proj, const int32_t *hin, const int32_t *hout, int T, 
     return decode_form(n_proj, hin, hout, T, n_adapters, max_rank, group);
 }
 
-// use_scratch: the two-launch form with the library's own per-device scratch array as its workspace
-static int bgmv_multi_impl(int n_proj, void *const *y, const void *const *x, const void *const *a_rows,
+// form: MLORA_FORM_*; use_scratch: with the library's own per-device scratch array as its workspace
+static int bgmv_multi_impl(int form, int n_proj, void *const *y, const void *const *x, const void *const *a_rows,
                      const void *const *b_rows, const int32_t *hin, const int32_t *hout,
                      const int32_t *tok_adapter, int T, const int32_t *page_tbl, const int32_t *rank,
                      const float *scaling, int n_adapters, int max_pages, int page_rows, int64_t n_pages,
@@ -403,7 +403,8 @@ static int bgmv_multi_impl(int n_proj, void *const *y, const void *const *x, con
     } else if (group != 1) {
         return fail(MLORA_EINVAL, "group must be 1 when work is NULL (got %d)", group);
     }
-    if ((workspace || use_scratch) && !work) return fail(MLORA_EINVAL, "the two-launch form needs the work records");
+    if (form != MLORA_FORM_FUSED && !work) return fail(MLORA_EINVAL, "the two-launch form needs the work records");
+    if (form == MLORA_FORM_FINE && group > 4) return fail(MLORA_EINVAL, "MLORA_FORM_FINE takes groups of 1, 2 or 4 (got %d)", group);
     int max_hin = 0, max_hout = 0;
     for (int p = 0; p < n_proj; p++) {
         if (!y[p] || !x[p] || !a_rows[p] || !b_rows[p]) return fail(MLORA_EINVAL, "projection %d: NULL device pointer", p);
@@ -432,14 +433,15 @@ static int bgmv_multi_impl(int n_proj, void *const *y, const void *const *x, con
         if (!workspace) return MLORA_ELAUNCH;
         workspace_bytes = (int64_t)SCRATCH_BYTES;
     }
-    if (workspace) {
-        const int64_t need = mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
+    if (form != MLORA_FORM_FUSED) {
+        a.fine = form == MLORA_FORM_FINE || (form == MLORA_FORM_PAIR && !prefer_sliced(n_proj, hin, hout, a.items_cap, group));
+        const int64_t need = a.fine ? fine_workspace_bytes(n_proj, T, max_hin, max_rank)
+                                    : mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
+        if (!workspace) return fail(MLORA_EINVAL, "the two-launch form needs a workspace");
         if (workspace_bytes < need)
             return fail(MLORA_ENOSPACE, "workspace holds %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);
         if (!aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be 16-byte aligned");
         a.vws = static_cast<float *>(workspace);
-        const int64_t fine_need = fine_workspace_bytes(n_proj, T, max_hin, max_rank);
-        a.fine = workspace_bytes >= fine_need && !use_scratch && !prefer_sliced(n_proj, hin, hout, a.items_cap, group);
         int ksc, nte;
         mlora::bgmv_split_slices(max_rank, &ksc, &nte, false, a.fine != 0);
         a.ks_max = (max_hin + ksc * 8 - 1) / (ksc * 8);
@@ -465,9 +467,22 @@ int mlora_bgmv_multi(int n_proj, void *const *y, const void *const *x, const voi
                      int max_rank, const int32_t *work, int group, void *workspace, int64_t workspace_bytes,
                      int dtype, int accumulate, void *stream)
 {
-    return bgmv_multi_impl(n_proj, y, x, a_rows, b_rows, hin, hout, tok_adapter, T, page_tbl, rank, scaling, n_adapters,
-                           max_pages, page_rows, n_pages, max_rank, work, group, workspace, workspace_bytes, false,
-                           dtype, accumulate, stream);
+    return bgmv_multi_impl(workspace ? MLORA_FORM_SLICED : MLORA_FORM_FUSED, n_proj, y, x, a_rows, b_rows, hin, hout, tok_adapter, T,
+                           page_tbl, rank, scaling, n_adapters, max_pages, page_rows, n_pages, max_rank, work, group, workspace,
+                           workspace_bytes, false, dtype, accumulate, stream);
+}
+
+int mlora_bgmv_multi_form(int form, int n_proj, void *const *y, const void *const *x, const void *const *a_rows,
+                          const void *const *b_rows, const int32_t *hin, const int32_t *hout,
+                          const int32_t *tok_adapter, int T, const int32_t *page_tbl, const int32_t *rank,
+                          const float *scaling, int n_adapters, int max_pages, int page_rows, int64_t n_pages,
+                          int max_rank, const int32_t *work, int group, void *workspace, int64_t workspace_bytes,
+                          int dtype, int accumulate, void *stream)
+{
+    if (form < MLORA_FORM_FUSED || form > MLORA_FORM_PAIR) return fail(MLORA_EINVAL, "form must be one of MLORA_FORM_* (got %d)", form);
+    return bgmv_multi_impl(form, n_proj, y, x, a_rows, b_rows, hin, hout, tok_adapter, T, page_tbl, rank, scaling, n_adapters,
+                           max_pages, page_rows, n_pages, max_rank, work, group, workspace, workspace_bytes, false, dtype,
+                           accumulate, stream);
 }
 
 int mlora_bgmv_multi_noalloc(int n_proj, void *const *y, const void *const *x, const void *const *a_rows,
@@ -477,9 +492,9 @@ int mlora_bgmv_multi_noalloc(int n_proj, void *const *y, const void *const *x, c
                              int max_rank, const int32_t *work, int group, int dtype, int accumulate, void *stream)
 {
     if (!work) return fail(MLORA_EINVAL, "mlora_bgmv_multi_noalloc needs the work records of mlora_pool_gather");
-    return bgmv_multi_impl(n_proj, y, x, a_rows, b_rows, hin, hout, tok_adapter, T, page_tbl, rank, scaling, n_adapters,
-                           max_pages, page_rows, n_pages, max_rank, work, group, nullptr, 0, true,
-                           dtype, accumulate, stream);
+    return bgmv_multi_impl(MLORA_FORM_SLICED, n_proj, y, x, a_rows, b_rows, hin, hout, tok_adapter, T, page_tbl, rank, scaling,
+                           n_adapters, max_pages, page_rows, n_pages, max_rank, work, group, nullptr, 0, true, dtype, accumulate,
+                           stream);
 }
 
 int mlora_bgmv(void *y, const void *x, const void *a_rows, const void *b_rows, const int32_t *tok_adapter,

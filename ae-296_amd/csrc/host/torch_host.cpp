@@ -59,6 +59,13 @@ long long as_int(PyObject *o)
     return v;
 }
 
+bool is_true(PyObject *o)
+{
+    const int v = PyObject_IsTrue(o);
+    if (v < 0) throw PyFail();
+    return v != 0;
+}
+
 long long attr_int(PyObject *o, PyObject *name)
 {
     Ref a(PyObject_GetAttr(o, name));
@@ -229,7 +236,7 @@ PyObject *bgmv(PyObject *const *v, Py_ssize_t nargs)
     const List ys(v[3]), xs(v[4]);
     const at::Tensor &tok = tensor(v[5]);
     const bool accumulate = v[8] == Py_True;
-    bool fused = v[7] != Py_None && PyObject_IsTrue(v[7]) == 1;
+    bool fused = v[7] != Py_None && is_true(v[7]);
     need_device(tok);
     need_contiguous(tok);
     if (tok.scalar_type() != at::kInt) raise(PyExc_TypeError, "tok_adapter must be int32");
@@ -247,16 +254,17 @@ PyObject *bgmv(PyObject *const *v, Py_ssize_t nargs)
     const int group = plan ? (int)attr_int(plan, s_group) : 1;
     void *ws = nullptr;
     int64_t ws_bytes = 0;
+    int form = MLORA_FORM_FUSED;
     if (!fused && T > 0) {
-        const int form = mlora_bgmv_form(c.n, c.hin, c.hout, (int)T, tb.n_slots, tb.max_rank, group, &ws_bytes);
+        form = mlora_bgmv_form(c.n, c.hin, c.hout, (int)T, tb.n_slots, tb.max_rank, group, &ws_bytes);
         if (form < 0) return PyLong_FromLong(form);
-        if (v[7] == Py_None && form == MLORA_FORM_FUSED) fused = true;
-        else ws = intermediate(plan, ws_bytes, tok);
+        if (v[7] != Py_None) form = MLORA_FORM_PAIR;
+        if (form != MLORA_FORM_FUSED) ws = intermediate(plan, ws_bytes, tok);
     }
     const int rc = launch(
-        mlora_bgmv_multi, c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, static_cast<const int32_t *>(tok.data_ptr()), (int)T, tb.page_tbl, tb.rank, tb.scaling,
+        mlora_bgmv_multi_form, form, c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, static_cast<const int32_t *>(tok.data_ptr()), (int)T, tb.page_tbl, tb.rank, tb.scaling,
         tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, tb.max_rank, plan ? static_cast<const int32_t *>(attr_ptr(plan, s_work)) : nullptr,
-        group, ws, fused ? 0 : ws_bytes, c.dtype, accumulate, stream());
+        group, ws, ws_bytes, c.dtype, accumulate, stream());
     return PyLong_FromLong(rc);
 }
 

@@ -19,7 +19,7 @@ MLORA_OK = 0
 MLORA_EINVAL, MLORA_ERANGE, MLORA_EALIGN, MLORA_EDTYPE, MLORA_ELAUNCH, MLORA_ENOSPACE = -1, -2, -3, -4, -5, -6
 MLORA_F16, MLORA_BF16 = 0, 1
 MAX_PROJ = 8
-FORM_FUSED, FORM_SLICED, FORM_FINE = 0, 1, 2
+FORM_FUSED, FORM_SLICED, FORM_FINE, FORM_PAIR = 0, 1, 2, 3
 MAX_RANK = 64
 GATHER_MAX_T = 8192
 CNT_NSEG, CNT_NVALID, CNT_NCHUNK, CNT_BAD, CNT_WORDS = 0, 1, 2, 3, 8
@@ -49,6 +49,8 @@ SIGNATURES = {
     "mlora_bgmv_form": (_i32, [_i32, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "mlora_bgmv_multi": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32,
                                 _i64, _i32, _vp, _i32, _vp, _i64, _i32, _i32, _vp]),
+    "mlora_bgmv_multi_form": (_i32, [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32,
+                                     _i64, _i32, _vp, _i32, _vp, _i64, _i32, _i32, _vp]),
     "mlora_bgmv_multi_noalloc": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32,
                                         _i64, _i32, _vp, _i32, _i32, _i32, _vp]),
     "mlora_bgmv": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i64,

@@ -168,8 +168,8 @@ int mlora_assist_import(int n_proj, void *const *res, const void *const *out_slo
  * With work == NULL every token is its own work item and group must be 1.
  * Two-launch form: with a `workspace` of mlora_bgmv_workspace_bytes(n_proj, T, max hin, max_rank)
  * bytes (and work records) the call runs as a shrink launch and an expand launch over
- * column slices of the items (1024 or 2048 columns, by max_rank; 512 for a small batch, which takes more workspace:
- * mlora_bgmv_form), the fp32 intermediate passing through the workspace; on a
+ * column slices of the items (1024 or 2048 columns, by max_rank), the fp32 intermediate passing through
+ * the workspace; how large the workspace is beyond that changes nothing.  On a
  * decode batch with about one item per compute unit this balances the load far better than the
  * fused launch.  workspace == NULL selects the fused launch.  Calls that share a workspace must be
  * ordered on one stream.  Both forms accumulate in fp32 and
@@ -180,19 +180,6 @@ int mlora_assist_import(int n_proj, void *const *res, const void *const *out_slo
  * makes that valid; a caller that fills `work` itself must keep it.
  */
 int64_t mlora_bgmv_workspace_bytes(int n_proj, int T, int max_hin, int max_rank);
-
-/*
- * Which form of mlora_bgmv_multi is fastest for a batch of these sizes: MLORA_FORM_FUSED (workspace == NULL),
- * MLORA_FORM_SLICED or MLORA_FORM_FINE (the two-launch form, fine: 512-column slices), or a negative error code.
- * Arguments as for that call (host arrays hin, hout).  *workspace_bytes receives what the two-launch form can use,
- * whichever form is returned: a workspace that large lets a small batch run fine, one of
- * mlora_bgmv_workspace_bytes always suffices.
- */
-#define MLORA_FORM_FUSED 0
-#define MLORA_FORM_SLICED 1
-#define MLORA_FORM_FINE 2
-int mlora_bgmv_form(int n_proj, const int32_t *hin, const int32_t *hout, int T, int n_adapters, int max_rank,
-                    int group, int64_t *workspace_bytes);
 
 int mlora_bgmv_multi(int n_proj, void *const *y, const void *const *x,
                      const void *const *a_rows, const void *const *b_rows,
@@ -205,6 +192,34 @@ int mlora_bgmv_multi(int n_proj, void *const *y, const void *const *x,
                      int dtype, int accumulate, void *stream);
 
 /*
+ * Which form of mlora_bgmv_multi_form is fastest for a batch of these sizes, or a negative error code.  Arguments as
+ * for that call (host arrays hin, hout).  *workspace_bytes receives what its two-launch forms take, whichever form
+ * is returned.
+ *   MLORA_FORM_FUSED   one launch, no workspace
+ *   MLORA_FORM_SLICED  two launches over slices of 1024 or 2048 columns, as mlora_bgmv_multi with a workspace
+ *   MLORA_FORM_FINE    two launches over 512-column slices with the rank rows split over wavefronts (group <= 4): small batches
+ *   MLORA_FORM_PAIR    two launches, fine or sliced by the sizes (mlora_bgmv_form does not return it)
+ * The forms differ in the order the fp32 sums are added.
+ */
+#define MLORA_FORM_FUSED 0
+#define MLORA_FORM_SLICED 1
+#define MLORA_FORM_FINE 2
+#define MLORA_FORM_PAIR 3
+int mlora_bgmv_form(int n_proj, const int32_t *hin, const int32_t *hout, int T, int n_adapters, int max_rank,
+                    int group, int64_t *workspace_bytes);
+
+/* mlora_bgmv_multi in the form the caller names: workspace is unused for MLORA_FORM_FUSED, needed for the others. */
+int mlora_bgmv_multi_form(int form, int n_proj, void *const *y, const void *const *x,
+                          const void *const *a_rows, const void *const *b_rows,
+                          const int32_t *hin, const int32_t *hout,
+                          const int32_t *tok_adapter, int T,
+                          const int32_t *page_tbl, const int32_t *rank, const float *scaling,
+                          int n_adapters, int max_pages, int page_rows, int64_t n_pages, int max_rank,
+                          const int32_t *work, int group,
+                          void *workspace, int64_t workspace_bytes,
+                          int dtype, int accumulate, void *stream);
+
+/*
  * mlora_bgmv_multi in its two-launch form with no workspace argument and no allocation anywhere on its
  * path.  No counterpart in the reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc) and so cannot provide the
@@ -212,7 +227,7 @@ int mlora_bgmv_multi(int n_proj, void *const *y, const void *const *x,
  * MLORA_NOALLOC_SCRATCH_BYTES that every GPU the library runs on holds until the process ends; a call that
  * needs more (mlora_bgmv_workspace_bytes(n_proj, T, max hin, max_rank): n_proj x T x column slices x rank
  * stride x 4 bytes) returns MLORA_ENOSPACE.  `work` (the records of mlora_pool_gather) is required.  Results
- * are those of mlora_bgmv_multi with a workspace of exactly those bytes, bit for bit.  The array keeps the previous call's contents;
+ * are those of mlora_bgmv_multi with a workspace, bit for bit.  The array keeps the previous call's contents;
  * nothing in it has to start at zero (the shrink launch writes every value the expand launch reads).  All
  * calls on one GPU share the one array: calls that overlap on a GPU (two streams, two threads) race; order
  * them on one stream.  The array's device address is looked up on the first call on each device (a runtime

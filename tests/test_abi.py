@@ -71,6 +71,18 @@ def test_validation_errors_without_gpu():
         _ext.check(bgmv(dtype=7))
     assert e.value.code == _ext.MLORA_EDTYPE
 
+    # the form named by the caller: what each form needs
+    def form(which, ws=16, ws_bytes=1 << 20, work=one, group=4, max_rank=32):
+        return lib.mlora_bgmv_multi_form(which, 1, P, P, P, P, H, H, one, 4, one, one, one, 4, 8, 8, 10, max_rank, work, group, ws,
+                                         ws_bytes, 0, 1, None)
+    assert form(4) == _ext.MLORA_EINVAL and form(-1) == _ext.MLORA_EINVAL
+    for which in (_ext.FORM_SLICED, _ext.FORM_FINE, _ext.FORM_PAIR):
+        assert form(which, work=None, group=1) == _ext.MLORA_EINVAL
+        assert form(which, ws=None, ws_bytes=0) == _ext.MLORA_EINVAL
+        assert form(which, ws_bytes=64) == _ext.MLORA_ENOSPACE
+        assert form(which, ws=8) == _ext.MLORA_EALIGN
+    assert form(_ext.FORM_FINE, group=8) == _ext.MLORA_EINVAL
+
     # the allocation-free form: needs work records, and refuses a batch whose intermediate exceeds its fixed array
     def noalloc(T=4, work=one, n_proj=1, hin=H, max_rank=64):
         return lib.mlora_bgmv_multi_noalloc(n_proj, P, P, P, P, hin, H, one, T, one, one, one, 4, 8, 8, 10, max_rank,

@@ -66,6 +66,32 @@ def test_noalloc_matches_workspace_form_on_two_calls():
             assert_close_bits(got, oracle_apply(pp, x_bits[i], tok_np, y0_bits[i]), FP16, f"noalloc T={T}")
 
 
+@pytest.mark.parametrize("T", [1, 5, 24])
+def test_results_do_not_depend_on_the_size_of_the_workspace(T):
+    """A small batch, which mlora_bgmv_form would run in 512-column slices: mlora_bgmv_multi gives the same bits with a
+    workspace of the size it asks for and with one many times as large, and so does the allocation-free form."""
+    rng = np.random.default_rng(779 + T)
+    hin, hout, ranks = 4096, 4096, [16, 64, 32]
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=FP16)
+    pool = upload_pool(pp)
+    tok_np = rng.integers(-1, len(ranks), T).astype(np.int32)
+    tok = torch.from_numpy(tok_np).cuda()
+    plan = plan_decode(tok, pool, group=1)
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), FP16)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), FP16)
+    need = _ext.lib().mlora_bgmv_workspace_bytes(1, T, hin, pool.max_rank)
+    outs = []
+    for size in (need, 64 * need, None):
+        y = bits_to_torch(y0, FP16, "cuda")
+        ws = None if size is None else torch.empty(size, dtype=torch.uint8, device="cuda")
+        say(f"decode T={T} with a workspace of {size} bytes")
+        _call(pool, plan, tok, [bits_to_torch(x, FP16, "cuda")], [y], [hin], [hout], noalloc=size is None, ws=ws)
+        torch.cuda.synchronize()
+        outs.append(torch_to_bits(y))
+    assert_close_bits(outs[0], oracle_apply(pp, x, tok_np, y0), FP16, f"workspace form T={T}")
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+
+
 def test_noalloc_rejects_a_batch_beyond_its_array():
     rng = np.random.default_rng(778)
     pp = PagedPool(rng, [64] * 4, 64, 64, page_rows=8, dtype=FP16)
