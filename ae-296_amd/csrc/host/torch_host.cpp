@@ -174,23 +174,6 @@ Tables tables(PyObject *pool)
             (int)attr_int(pool, s_page_rows), (int)attr_int(pool, s_max_rank), attr_int(pool, s_n_pages)};
 }
 
-// The plan's intermediate: at least `bytes` on the device of `like`, allocated when it is missing or too small.
-void *intermediate(PyObject *plan, int64_t bytes, const at::Tensor &like)
-{
-    {
-        Ref have(PyObject_GetAttr(plan, s_vws));
-        if (have.o != Py_None) {
-            const at::Tensor &t = tensor(have.o);
-            if (t.numel() >= bytes) return t.data_ptr();
-        }
-    }
-    at::Tensor t = at::empty({bytes}, like.options().dtype(at::kByte));
-    void *p = t.data_ptr();
-    Ref made(THPVariable_Wrap(std::move(t)));
-    if (PyObject_SetAttr(plan, s_vws, made.o)) throw PyFail();
-    return p;
-}
-
 // ---------------------------------------------------------------- decode
 // A plan's buffer: data pointer (null for None), after a check that a launch on `like` may write `n` values of its type there.
 void *buffer(PyObject *plan, PyObject *name, at::ScalarType type, int64_t n, const at::Tensor &like)
@@ -252,20 +235,36 @@ PyObject *bgmv(PyObject *const *v, Py_ssize_t nargs)
     }
     const Tables tb = tables(pool);
     const int group = plan ? (int)attr_int(plan, s_group) : 1;
-    void *ws = nullptr;
+    // The intermediate of the two-launch forms is this call's own, from torch's allocator: calls that share a plan may
+    // overlap on several streams or threads, and a captured graph keeps what its launches write.  It may be given back
+    // when the launches are queued (the allocator hands it out again in stream order).
+    at::Tensor room;
     int64_t ws_bytes = 0;
     int form = MLORA_FORM_FUSED;
     if (!fused && T > 0) {
         form = mlora_bgmv_form(c.n, c.hin, c.hout, (int)T, tb.n_slots, tb.max_rank, group, &ws_bytes);
         if (form < 0) return PyLong_FromLong(form);
         if (v[7] != Py_None) form = MLORA_FORM_PAIR;
-        if (form != MLORA_FORM_FUSED) ws = intermediate(plan, ws_bytes, tok);
+        if (form != MLORA_FORM_FUSED) room = at::empty({ws_bytes}, tok.options().dtype(at::kByte));
     }
     const int rc = launch(
         mlora_bgmv_multi_form, form, c.n, c.y, c.x, c.a, c.b, c.hin, c.hout, static_cast<const int32_t *>(tok.data_ptr()), (int)T, tb.page_tbl, tb.rank, tb.scaling,
         tb.n_slots, tb.max_pages, tb.page_rows, tb.n_pages, tb.max_rank, plan ? static_cast<const int32_t *>(attr_ptr(plan, s_work)) : nullptr,
-        group, ws, ws_bytes, c.dtype, accumulate, stream());
+        group, room.defined() ? room.data_ptr() : nullptr, ws_bytes, c.dtype, accumulate, stream());
     return PyLong_FromLong(rc);
+}
+
+// The reference-layout plan's intermediate: at least `bytes` on the device of `like`, allocated when it is missing or too small.
+at::Tensor intermediate(PyObject *plan, int64_t bytes, const at::Tensor &like)
+{
+    {
+        Ref have(PyObject_GetAttr(plan, s_vws));
+        if (have.o != Py_None && tensor(have.o).numel() >= bytes) return tensor(have.o);
+    }
+    at::Tensor t = at::empty({bytes}, like.options().dtype(at::kByte));
+    Ref made(THPVariable_Wrap(t));
+    if (PyObject_SetAttr(plan, s_vws, made.o)) throw PyFail();
+    return t;
 }
 
 // bgmv_ref(plan, ys, xs, was, wbs, layer, scale, accumulate, T, N, L, r)
@@ -304,7 +303,8 @@ PyObject *bgmv_ref(PyObject *const *v, Py_ssize_t nargs)
     if (type != at::kHalf && type != at::kBFloat16) raise(PyExc_TypeError, "mlora kernels take float16 or bfloat16 tensors");
     static PyObject *s_buf = PyUnicode_InternFromString("buf");
     const int64_t bytes = mlora_bgmv_workspace_bytes(n, (int)T, max_hin, (int)r);
-    void *ws = bytes > 0 ? intermediate(plan, bytes, ys[0]) : nullptr;
+    const at::Tensor room = bytes > 0 ? intermediate(plan, bytes, ys[0]) : at::Tensor();
+    void *ws = room.defined() ? room.data_ptr() : nullptr;
     const int rc = launch(mlora_bgmv_reflayout_multi, n, y, x, a, b, hin, hout, attr_ptr(plan, s_buf), (int)T, (int)N, (int)L, (int)r,
                                               (int)as_int(v[5]), (float)PyFloat_AsDouble(v[6]), (int)attr_int(plan, s_group),
                                               type == at::kHalf ? MLORA_F16 : MLORA_BF16, v[7] == Py_True, ws, bytes, stream());

@@ -57,7 +57,6 @@ class DecodePlan:
     row_off: Optional[torch.Tensor] = None   # int32 [T, max_pages]
     tok_rank: Optional[torch.Tensor] = None
     tok_scale: Optional[torch.Tensor] = None
-    vws: Optional[torch.Tensor] = None       # uint8: fp32 intermediate of the two-launch decode form
 
     @property
     def T(self) -> int:
@@ -184,10 +183,9 @@ def bgmv(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], pool: AdapterPo
 
     With a plan the call runs as a shrink launch and an expand launch over column slices
     (``fused=False``) or as one fused launch (``fused=True``), by default whichever `mlora_bgmv_form`
-    names for the sizes; without a plan it is always the fused launch with one token per work item.  The two-launch form keeps its fp32
-    intermediate in a buffer owned by the plan, allocated on the first call that needs it (so
-    run one call before capturing a HIP graph); calls that share a plan must therefore follow each
-    other on one stream, not overlap on several."""
+    names for the sizes; without a plan it is always the fused launch with one token per work item.  The two-launch
+    forms take their fp32 intermediate from torch's allocator for the length of the call (under capture from the
+    graph's pool); a plan is only read, so calls that share one may overlap on several streams."""
     pool.sync()
     rc = _ext.host().bgmv(pool, layer, projs, ys, xs, tok_adapter, plan, fused, bool(accumulate))
     if rc:

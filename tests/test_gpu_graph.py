@@ -1,6 +1,6 @@
 """HIP graph replays of the decode and prefill steps give the eager results bit for bit, replay after
-replay, with eager work and synchronisations in between (nothing in the library records a memset node
-or allocates during capture once the plan's buffers exist)."""
+replay, with eager work and synchronisations in between (nothing in the library records a memset node;
+what a call allocates during capture comes from the graph's own pool)."""
 import numpy as np
 import pytest
 import torch
@@ -42,7 +42,7 @@ def test_graph_replays_match_eager():
         sgmv_multi(y_pre, [x, x], pool, 0, ["p", "o"], pplan)
 
     say("graph: eager reference step")
-    step()                                        # also allocates the plan's intermediate buffer
+    step()
     torch.cuda.synchronize()
     want = [t.clone() for t in y_dec + y_pre]
     assert not torch.equal(want[0], y0)

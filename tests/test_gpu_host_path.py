@@ -106,3 +106,97 @@ def test_a_prefill_workspace_in_host_memory_is_refused():
                                                     torch.zeros(1, 1, 96, 8, device="cuda").half(), 0, workspace=ws)):
             with pytest.raises(ValueError):
                 call()
+
+
+def _small_batch(n_proj, T=6, hin=2048, hout=1536, ranks=(64, 16, 40)):
+    """A batch that mlora_bgmv_form runs as two launches, and its projections' names."""
+    pp = PagedPool(np.random.default_rng(17), list(ranks), hin, hout, page_rows=8, dtype=FP16)
+    names = [f"p{i}" for i in range(n_proj)]
+    pool = upload_pool(pp, projections={nm: (hin, hout) for nm in names})
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    for nm in names:
+        pool.a_rows[nm].copy_(torch.randn(pool.a_rows[nm].shape, device="cuda", generator=gen) * 0.02)
+        pool.b_rows[nm].copy_(torch.randn(pool.b_rows[nm].shape, device="cuda", generator=gen) * 0.02)
+    tok = torch.tensor([i % (len(ranks) + 1) - 1 for i in range(T)], dtype=torch.int32, device="cuda")
+    xs = [torch.randn(T, hin, device="cuda", generator=gen).half() for _ in range(8)]
+    return pool, names, tok, xs, lambda: [torch.zeros(T, hout, device="cuda").half() for _ in names]
+
+
+@pytest.mark.parametrize("fused", [None, False, True])
+def test_a_call_leaves_its_plan_as_it_was(fused):
+    pool, names, tok, xs, zeros = _small_batch(3)
+    plan = mlora.plan_decode(tok, pool)
+    before = dict(vars(plan))
+    say(f"bgmv on a plan that stays as it was, fused={fused}")
+    mlora.bgmv(zeros(), xs[:3], pool, 0, names, tok, plan=plan, fused=fused)
+    torch.cuda.synchronize()
+    assert vars(plan).keys() == before.keys() and all(v is before[k] for k, v in vars(plan).items())
+
+
+def test_small_batches_that_share_a_plan_on_several_streams_and_threads():
+    """Calls of one plan that overlap, from one thread on two streams and from four threads on a stream each."""
+    import threading
+    pool, names, tok, xs, zeros = _small_batch(3)
+    plan = mlora.plan_decode(tok, pool)
+    want = []
+    for x in xs:
+        y = zeros()
+        mlora.bgmv(y, [x] * 3, pool, 0, names, tok, plan=plan, accumulate=False)
+        want.append(y)
+    torch.cuda.synchronize()
+
+    def run(which, stream, out, reps=40):
+        with torch.cuda.stream(stream):
+            for i in range(reps):
+                k = (which + i) % len(xs)
+                mlora.bgmv(out[i], [xs[k]] * 3, pool, 0, names, tok, plan=plan, accumulate=False)
+
+    say("bgmv on two streams and one plan")
+    outs = [[zeros() for _ in range(40)] for _ in range(4)]
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    torch.cuda.synchronize()
+    for i in range(40):
+        for j in range(2):
+            with torch.cuda.stream(streams[j]):
+                mlora.bgmv(outs[j][i], [xs[(j + i) % len(xs)]] * 3, pool, 0, names, tok, plan=plan, accumulate=False)
+    torch.cuda.synchronize()
+    for j in range(2):
+        for i in range(40):
+            assert all(torch.equal(a, b) for a, b in zip(outs[j][i], want[(j + i) % len(xs)])), (j, i)
+    say("bgmv from four threads and one plan")
+    threads = [threading.Thread(target=run, args=(j, streams[j], outs[j])) for j in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for j in range(4):
+        for i in range(40):
+            assert all(torch.equal(a, b) for a, b in zip(outs[j][i], want[(j + i) % len(xs)])), (j, i)
+
+
+def test_a_captured_step_keeps_its_intermediate():
+    """Eager calls of other sizes on the plan of a captured step, and new tensors after them: the replay gives the same
+    bits and writes to none of the new tensors."""
+    pool, names, tok, xs, zeros = _small_batch(7)
+    plan = mlora.plan_decode(tok, pool, n_proj=7)
+    y = zeros()
+    step = lambda: mlora.bgmv(y, xs[:7], pool, 0, names, tok, plan=plan, accumulate=False)  # noqa: E731
+    say("bgmv captured, then eager calls on the same plan")
+    step()
+    torch.cuda.synchronize()
+    want = [t.clone() for t in y]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        step()
+    for n in (1, 3, 7):
+        mlora.bgmv(zeros()[:n], xs[:n], pool, 0, names[:n], tok, plan=plan, fused=False)
+    fresh = [torch.full((1 << 20,), 7.0, device="cuda") for _ in range(8)]
+    for rep in range(3):
+        for t in y:
+            t.fill_(float(rep))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(y, want)), rep
+        assert all(bool((t == 7.0).all()) for t in fresh), rep
