@@ -363,7 +363,7 @@ __global__ __launch_bounds__(NTE) void bgmv_expand_kernel(const BgmvArgs p)
                     for (int u = 0; u < 8; u++) s += t[u];
                 }
             }
-            s_v[k][j] = s * scale;
+            s_v[k][j] = j < r ? s * scale : 0.f;                        // an infinite scale must not reach rows that are not there
         }
         __syncthreads();
         if (active) {
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
         ytok = wave == k ? tok[k] : ytok;
     }
     uint16_t *yp = y + (size_t)(ytok >= 0 ? ytok : 0) * hout + (size_t)(active ? cc : 0) * 8;
-    if (adapter < 0) {
+    if (adapter < 0 || r == 0) {
         if (!p.accumulate && active && ytok >= 0) stg16(yp, zero16());
         return;
     }
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
                 float vk = 0.f;
 #pragma unroll
                 for (int q4 = 0; q4 < NQ; q4++) vk += s_vp[q4][k][j0 + i];
-                vk *= scale;
+                vk = j0 + i < r ? vk * scale : 0.f;             // rows of the bucket that the adapter does not have
 #pragma unroll
                 for (int e = 0; e < 8; e++) o[k][e] = fmaf(vk, f[e], o[k][e]);
             }

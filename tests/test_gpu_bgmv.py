@@ -424,3 +424,66 @@ def test_bgmv_fine_slices(dtype, T, group, ranks, hin, hout):
             assert_close_bits(outs[g, accumulate], oracle_apply(pp, x, tok, y0 if accumulate else None), dtype, "fine")
     for accumulate in (True, False):
         assert np.array_equal(outs[group, accumulate], outs[1, accumulate])
+
+
+def _run_form(pp, x_bits, tok, y0_bits, group, form):
+    """One projection through mlora_bgmv_multi_form."""
+    import ctypes as C
+    from mlora import _ext
+    lib, pool = _ext.lib(), upload_pool(pp)
+    x, y, t = bits_to_torch(x_bits, pp.dtype, "cuda"), bits_to_torch(y0_bits, pp.dtype, "cuda"), torch.from_numpy(tok).cuda()
+    plan = plan_decode(t, pool, group=group)
+    a, b = pool.slab_ptrs(0, "p")
+    P, I = C.c_void_p * 1, C.c_int32 * 1
+    need = C.c_int64()
+    _ext.check(min(0, lib.mlora_bgmv_form(1, I(pp.hin), I(pp.hout), len(tok), pool.n_slots, pool.max_rank, group, C.byref(need))))
+    ws = torch.empty(max(need.value, 16), dtype=torch.uint8, device="cuda")
+    _ext.check(lib.mlora_bgmv_multi_form(
+        form, 1, P(y.data_ptr()), P(x.data_ptr()), P(a), P(b), I(pp.hin), I(pp.hout), t.data_ptr(), len(tok),
+        pool.page_tbl.data_ptr(), pool.rank.data_ptr(), pool.scaling.data_ptr(), pool.n_slots, pool.max_pages, pool.page_rows,
+        pool.n_pages, pool.max_rank, plan.work.data_ptr(), group, ws.data_ptr(), ws.numel(), pool.dtype_code, 1,
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    return torch_to_bits(y)
+
+
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("form", ["FUSED", "SLICED", "FINE"])
+@pytest.mark.parametrize("group", [1, 2])
+def test_bgmv_infinities_and_nan(form, dtype, group):
+    """Infinite scaling at a rank below every rank bucket (the rows that pad the bucket must not make NaN of it), an
+    infinity and a NaN in x, both in B, a rank-0 adapter whose row stays as it is: the same infinities and NaN as in 64
+    bits, the finite values within the tolerance."""
+    from mlora import _ext
+    rng = np.random.default_rng(77)
+    ranks = [1, 9, 17, 33, 64, 24, 0]
+    hin, hout = 1024, 520
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
+    pp.a_rows = bits_of(np.abs(f32_of(pp.a_rows, dtype)) + 0.001, dtype)
+    pp.b_rows = bits_of(np.abs(f32_of(pp.b_rows, dtype)) + 0.001, dtype)
+    pp.scaling[:4] = np.inf
+    pp.scaling[6] = np.nan
+    brow = f32_of(pp.b_rows, dtype).copy()
+    brow[pp.rows(5)[3], 7], brow[pp.rows(5)[23], 515] = np.inf, np.nan
+    pp.b_rows = bits_of(brow, dtype)
+    tok = np.array([0, 1, 2, 3, 4, 4, 4, 5, -1, 6, 0, 5, 3], np.int32)
+    x = np.abs(rng.standard_normal((len(tok), hin))).astype(np.float32) * 0.1
+    x[5, 1000], x[6, 3] = np.inf, np.nan
+    xb = bits_of(x, dtype)
+    y0 = rng.standard_normal((len(tok), hout)).astype(np.float32)
+    y0[9, :5] = -0.0
+    y0b = bits_of(y0, dtype)
+    want = f32_of(y0b, dtype).astype(np.float64)
+    with np.errstate(all="ignore"):
+        for t, a in enumerate(tok):
+            if a >= 0 and ranks[a] > 0:
+                v = (f32_of(xb[t], dtype).astype(np.float64)[:, None] * pp.A(a)).sum(0) * np.float64(pp.scaling[a])
+                want[t] += (v[:, None] * pp.B(a)).sum(0)
+    say(f"bgmv infinities and NaN form={form} group={group} dtype={dtype}")
+    bits = _run_form(pp, xb, tok, y0b, group, getattr(_ext, "FORM_" + form))
+    got = f32_of(bits, dtype)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0))
+    fine = np.isfinite(want)
+    assert (np.abs(got[fine] - want[fine]) <= ATOL + RTOL * np.abs(want[fine])).all()
+    assert np.array_equal(bits[8], y0b[8]) and np.array_equal(bits[9], y0b[9])
