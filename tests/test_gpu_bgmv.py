@@ -487,3 +487,33 @@ def test_bgmv_infinities_and_nan(form, dtype, group):
     fine = np.isfinite(want)
     assert (np.abs(got[fine] - want[fine]) <= ATOL + RTOL * np.abs(want[fine])).all()
     assert np.array_equal(bits[8], y0b[8]) and np.array_equal(bits[9], y0b[9])
+
+
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+def test_bgmv_forms_are_equally_exact(dtype):
+    """Share of results that are not the correctly rounded 64-bit sum, per form: the forms add the same fp32 products in
+    other orders, so none may have more than its share of the fp32 rounding that the others show (rank 64, where the
+    sums are longest; shares of about 1e-4, 2^19 results: a factor of two is far outside their scatter)."""
+    from mlora import _ext
+    rng = np.random.default_rng(78)
+    T, hin, hout = 16, 4096, 32768
+    pp = PagedPool(rng, [64, 64], hin, hout, page_rows=8, dtype=dtype)
+    tok = rng.integers(0, 2, T).astype(np.int32)
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
+    exact = f32_of(y0, dtype).astype(np.float64)
+    for t in range(T):
+        a = tok[t]
+        exact[t] += (f32_of(x[t], dtype).astype(np.float64) @ pp.A(a) * np.float64(pp.scaling[a])) @ pp.B(a)
+    f = exact.astype(np.float32)                             # 64 -> 16 bits in one rounding: to odd in 32 bits first
+    over = np.abs(f.astype(np.float64)) > np.abs(exact)
+    odd = f.view(np.int32) - over.astype(np.int32)
+    odd = np.where(f.astype(np.float64) != exact, odd | 1, odd).view(np.float32)
+    want = bits_of(odd, dtype)
+    share = {}
+    for form in ("FUSED", "SLICED", "FINE"):
+        say(f"bgmv exactness form={form} dtype={dtype}")
+        share[form] = float((_run_form(pp, x, tok, y0, 1, getattr(_ext, "FORM_" + form)) != want).mean())
+    print(share)
+    assert max(share.values()) < 1e-3
+    assert share["FINE"] <= 2 * min(share["FUSED"], share["SLICED"])
