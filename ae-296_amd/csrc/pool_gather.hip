@@ -301,6 +301,9 @@ __global__ __launch_bounds__(1024) void gather_count_kernel(const GatherArgs g, 
                     const int in_wave = __popcll(same & ((1ull << lane) - 1ull));
                     int at = 0;
                     if (act && in_wave == 0) { at = s_at[wave][r]; s_at[wave][r] = at + __popcll(same); }
+                    // the next 64 chunks' leaders are other lanes of this wavefront: they read what was written here
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
                     at = __shfl(at, act ? __builtin_ctzll(same) : lane) + in_wave;
                     if (act) s_ord[at] = (uint16_t)c;
                 }

@@ -106,3 +106,12 @@ def test_gather_at_the_limits_of_its_forms(T, N):
     pool = _pool(N, rng.choice([8, 16, 24], N), 8, rng)
     say(f"gather form limits T={T} N={N}")
     _check(np.append(rng.integers(-1, N, T - 2), [N - 1, 0]).astype(np.int32), pool, 4)
+
+
+@pytest.mark.parametrize("ranks", [[8, 64], [8, 16, 24, 32, 40, 48, 56, 64]])
+def test_gather_order_by_rank_over_many_chunks(ranks):
+    """256 chunks per eighth of the records, few ranks: every 64 chunks continue the counts of the 64 before them."""
+    rng = np.random.default_rng(len(ranks))
+    pool = _pool(1500, rng.choice(ranks, 1500), 8, rng)
+    say(f"gather order by rank, ranks {ranks}")
+    _check(rng.integers(-1, 1500, 2048).astype(np.int32), pool, 1)
