@@ -669,8 +669,8 @@ constexpr int SG_TM = 64;   // tokens per tile, as in sgmv_prefill.hip
 struct SgmvWs { int max_tiles; int ksplit; int ks_cap; size_t off_cover, off_rec, off_proj, per_proj, off_hi, off_lo, total; };
 
 // Workspace: the plan (tile list, tile records: depends on T and n_seg only), then per projection the
-// K-split partial sums and the hi / lo halves of their sum.
-SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int most)
+// K-split partial sums and the hi / lo halves of their sum.  `most`: splits of a projection, `cap`: of one with a longer K.
+SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int most, int cap)
 {
     SgmvWs w;
     w.max_tiles = T / SG_TM + 2 * n_seg + 1;       // aligned cuts can add one partial tile at either end of a segment
@@ -682,8 +682,11 @@ SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int most)
     long long ks = (target + per_split - 1) / per_split;
     w.ksplit = ks < 1 ? 1 : (ks > most ? most : (int)ks);
     // a projection with a longer K than the others of its call gets proportionally more splits (up to three
-    // times as many, at most 8), so that every shrink workgroup walks about the same number of columns
+    // times as many, at most 8 or as many as the others have), so that every shrink workgroup walks about the same
+    // number of columns
     w.ks_cap = n_proj > 1 && w.ksplit < 8 ? (3 * w.ksplit < 8 ? 3 * w.ksplit : 8) : w.ksplit;
+    w.ks_cap = w.ks_cap < cap ? w.ks_cap : cap;
+    w.ksplit = w.ksplit < w.ks_cap ? w.ksplit : w.ks_cap;
     size_t off = ((size_t)w.max_tiles * 3 + 4) * sizeof(int32_t);
     off = (off + 255) & ~(size_t)255;
     w.off_cover = off;                              // int32 [T]: 1 where a token belongs to some segment
@@ -704,14 +707,21 @@ SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int most)
 // A prompt of a tile or two takes up to sixteen splits, two stages of 128 columns each at hidden 4096: the launch
 // is a chain of loads and more workgroups shorten it (one prompt of 64 tokens, three projections at rank 64: 20.0 us a
 // call with eight splits, 18.6 with sixteen, 21.0 with thirty-two; 512 tokens 24.9, 26.9, 30.9: partial sums).
-// Where they do not fit, eight do: a workspace sized for a longer batch serves its shorter ones.
+// The number of splits steps up as a batch gets shorter, so a shorter batch can have a use for more workspace than a longer
+// one, and fewer projections for more than many; where `have` does not hold what the call would take, it takes the
+// splits that fit (eight of the sixteen first), down to one: with one split the size only grows with tokens, segments and
+// projections, so a workspace sized for a larger call always serves a smaller one.
 SgmvWs sgmv_layout(int T, int n_seg, int n_proj, int64_t have = -1)
 {
     if (T / SG_TM + 2 * n_seg + 1 <= 6) {
-        const SgmvWs w = sgmv_layout_splits(T, n_seg, n_proj, 16);
+        const SgmvWs w = sgmv_layout_splits(T, n_seg, n_proj, 16, 16);
         if (have < 0 || (int64_t)w.total <= have) return w;
     }
-    return sgmv_layout_splits(T, n_seg, n_proj, 8);
+    const SgmvWs w = sgmv_layout_splits(T, n_seg, n_proj, 8, 8);
+    if (have < 0 || (int64_t)w.total <= have) return w;
+    const int64_t split = (int64_t)T * MLORA_MAX_RANK * (int64_t)sizeof(float);        // as large as the hi / lo halves together
+    const int64_t fit = (have - (int64_t)w.off_proj) / n_proj / split - 1;
+    return sgmv_layout_splits(T, n_seg, n_proj, 8, fit < 1 ? 1 : (int)fit);
 }
 
 // Columns of y one expand workgroup covers, and the column blocks per tile that follow from it.
@@ -783,6 +793,13 @@ int mlora_sgmv_expand_cols(int T, int n_seg, int n_proj, int hout)
 {
     if (T <= 0 || n_seg <= 0 || n_proj < 1 || n_proj > MLORA_MAX_PROJ || hout <= 0) return 0;
     return expand_block_cols(n_proj, sgmv_layout(T, n_seg, n_proj).max_tiles, hout, nullptr);
+}
+
+int mlora_sgmv_splits(int T, int n_seg, int n_proj, int64_t workspace_bytes)
+{
+    if (T <= 0 || n_seg <= 0 || n_proj < 1 || n_proj > MLORA_MAX_PROJ || workspace_bytes < 0) return 0;
+    const SgmvWs w = sgmv_layout(T, n_seg, n_proj, workspace_bytes);
+    return (int64_t)w.total <= workspace_bytes ? w.ks_cap : 0;
 }
 
 int64_t mlora_sgmv_multi_workspace_bytes(int T, int n_seg, int n_proj)

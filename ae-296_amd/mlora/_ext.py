@@ -61,6 +61,7 @@ SIGNATURES = {
     "mlora_bgmv_reflayout_multi": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _f32, _i32,
                                           _i32, _i32, _vp, _i64, _vp]),
     "mlora_sgmv_workspace_bytes": (_i64, [_i32, _i32]),
+    "mlora_sgmv_splits": (_i32, [_i32, _i32, _i32, _i64]),
     "mlora_sgmv": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32,
                           _i32, _i64, _i32, _i32, _i32, _vp, _i64, _vp]),
     "mlora_sgmv_plan": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i64, _i32, _vp, _i64, _vp]),

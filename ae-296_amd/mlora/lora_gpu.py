@@ -49,6 +49,7 @@ class Lora_GPU:
         self.select_inds = [torch.randint(0, hi, (i + 1,), device=self.device, generator=self._gen)
                             for i in range(self.batch_size)]
         self._workspace = None
+        self._workspace_for = (0, 0)                   # rows and requests it was sized for
         # Grouping of the current decode batch by adapter.  It is served again only for the very tensor object it was
         # made from (`_plan_src`, kept alive here so that neither its address nor its Python identity can pass to
         # another tensor) at the same torch version counter: a serving loop builds `lora_ids` afresh every step
@@ -135,9 +136,9 @@ class Lora_GPU:
                 raise RuntimeError("prefill adapters are not loaded (call prepare_lora_prefill)")
             if not x.is_contiguous():
                 x = x.contiguous()
-            need = ops._ext.lib().mlora_sgmv_workspace_bytes(bsz * x.shape[1], bsz)
-            if self._workspace is None or self._workspace.numel() < need:
-                self._workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+            rows, reqs = max(bsz * x.shape[1], self._workspace_for[0]), max(bsz, self._workspace_for[1])
+            if (rows, reqs) != self._workspace_for:    # a shorter batch than it was sized for keeps it
+                self._workspace, self._workspace_for = ops.sgmv_workspace(rows, reqs, x.device), (rows, reqs)
             return ops.lora_prefill_ref(x, down, up, layer_id, workspace=self._workspace)
         if not ops.ref_rank_supported(self.lora_rank):
             return self._invoke_single(name, x, layer_id, lora_ids)

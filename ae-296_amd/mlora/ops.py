@@ -282,7 +282,8 @@ def add_lora_bgmv_multi(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], 
 # ---------------------------------------------------------------------- prefill
 def sgmv_workspace(T: int, n_seg: int, device, n_proj: int = 1) -> torch.Tensor:
     """Workspace for a prefill batch of T tokens in n_seg segments; n_proj > 1 sizes it for
-    ``sgmv_multi`` calls of up to that many projections (it then also serves single ``sgmv`` calls)."""
+    ``sgmv_multi`` calls of up to that many projections (it then also serves single ``sgmv`` calls).  It serves every
+    batch with no more tokens and segments; one that would use more K splits than it holds runs with those that fit."""
     lib = _ext.lib()
     nbytes = max(lib.mlora_sgmv_workspace_bytes(T, n_seg), lib.mlora_sgmv_multi_workspace_bytes(T, n_seg, n_proj))
     return torch.empty(nbytes, dtype=torch.uint8, device=device)

@@ -294,8 +294,15 @@ int mlora_bgmv_reflayout_multi(int n_proj, void *const *y, const void *const *x,
  * per-call weight transposes/copies or the padding to equal prompt length.
  * seg_* are device arrays of n_seg entries.  Segments must not overlap; tokens covered by no
  * segment keep y (accumulate) or get zeros.  workspace: mlora_sgmv_workspace_bytes(T, n_seg).
+ *
+ * The workspace holds the fp32 partial sums of the call's K splits.  One that was sized for more tokens, segments or
+ * projections serves every smaller call; where that holds fewer splits than the call would take by itself (a shorter
+ * batch takes more), it takes those that fit, which is slower and another order of the same fp32 sums: a result's
+ * last rounding can depend on the workspace's size, for every prefill call below.  mlora_sgmv_splits says how many
+ * splits a projection of a call can get in a workspace (the one with the longest K; 0: the call does not fit).
  */
 int64_t mlora_sgmv_workspace_bytes(int T, int n_seg);
+int mlora_sgmv_splits(int T, int n_seg, int n_proj, int64_t workspace_bytes);
 int mlora_sgmv(void *y, const void *x, const void *a_rows, const void *b_rows,
                const int32_t *seg_start, const int32_t *seg_len, const int32_t *seg_adapter, int n_seg,
                const int32_t *page_tbl, const int32_t *rank, const float *scaling,
@@ -337,7 +344,7 @@ int mlora_sgmv_planned(void *y, const void *x, const void *a_rows, const void *b
  * instead of three per projection.  y, x, a_rows, b_rows, hin, hout are HOST arrays of n_proj entries as
  * in mlora_bgmv_multi.  Consecutive projections that are given the same x pointer (q, k, v; gate, up)
  * share its reads in the shrink launch: their workgroups for the same tokens run back to back on one
- * XCD, so x comes from HBM once.  The workspace must hold mlora_sgmv_multi_workspace_bytes(T, n_seg,
+ * XCD, so x comes from HBM once.  The workspace: mlora_sgmv_multi_workspace_bytes(T, n_seg,
  * n_proj) bytes; a plan written by mlora_sgmv_plan into that workspace is valid for any n_proj.
  * Replaces the three torch.bmm pairs of lora_gpu.py:127-128,145-146,157-158 for one layer.
  */

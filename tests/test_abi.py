@@ -131,3 +131,24 @@ def test_validation_errors_without_gpu():
     assert rc == _ext.MLORA_ENOSPACE
     rc = lib.mlora_prefill_reflayout(one, one, one, one, 2, 16, 4, 12, 64, 64, 0, 0, one, 1 << 30, None)
     assert rc == _ext.MLORA_ERANGE                     # rank not a multiple of 8
+
+
+@pytest.mark.parametrize("T", [1, 63, 64, 255, 256, 400, 2880, 3648, 6144, 6848, 8192, 8256, 8320, 20000])
+def test_a_prefill_workspace_serves_every_smaller_call(T):
+    """The splits step up as a batch shrinks, so a shorter batch, fewer segments or fewer projections can ask for more
+    than a workspace sized for a larger call holds: the layout takes what fits, and never refuses it."""
+    lib = _ext.lib()
+    shorter = sorted({1, 40, 64, 100, 127, 255, 383, T // 3, T // 2, max(1, T - 64), max(1, T - 704), T})
+    grew = 0
+    for n_seg in (1, 2, 8, 16):
+        for n_proj in (1, 2, 3, 7, 8):
+            have = max(lib.mlora_sgmv_workspace_bytes(T, n_seg), lib.mlora_sgmv_multi_workspace_bytes(T, n_seg, n_proj))
+            assert lib.mlora_sgmv_splits(T, n_seg, n_proj, have) == lib.mlora_sgmv_splits(T, n_seg, n_proj, 1 << 50)
+            for t in [v for v in shorter if 0 < v <= T]:
+                for s in [v for v in (1, 2, 5, 8, 16) if v <= n_seg]:
+                    for p in [v for v in (1, 2, 3, 6, 7, 8) if v <= n_proj]:
+                        got, full = lib.mlora_sgmv_splits(t, s, p, have), lib.mlora_sgmv_splits(t, s, p, 1 << 50)
+                        assert 1 <= got <= full, (t, s, p, have)
+                        grew += got < full
+    assert grew > 0 or T <= 64                   # the sweep meets calls that would take more than they are given
+    assert lib.mlora_sgmv_splits(T, 1, 1, 256) == 0

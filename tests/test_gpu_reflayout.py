@@ -239,3 +239,20 @@ def test_prefill_ref_tiles_without_a_plan(B, Lpad, r, hin, hout):
     y = lora_prefill_ref(*(bits_to_torch(t, FP16, "cuda") for t in (x, A_T, B_T)), 1)
     torch.cuda.synchronize()
     assert_close_bits(torch_to_bits(y), orc.prefill_bmm_ref(x, A_T, B_T, 1, FP16, round_mid=False), FP16)
+
+
+def test_lora_gpu_keeps_its_workspace_for_a_shorter_prefill():
+    """One prompt of 300 tokens, then one of 250, which would take more K splits: the workspace that a captured call
+    may still use is not replaced, and both results meet the reference."""
+    cfg = dict(n_layers=1, batch_size=4, lora_rank=64, hidden_dim=1024, tp_degree=1, max_prefill_batch_size=1)
+    g = Lora_GPU(cfg, shared=True, device="cuda", seed=5)
+    say("Lora_GPU: a shorter prefill after a longer one")
+    seen = []
+    for length in (300, 250):
+        x = torch.randn(1, length, 1024, device="cuda").half()
+        y = g.invoke_one_layer_q(x, 0, True)
+        want = torch.bmm(torch.bmm(x.float(), g.q_down_prefill[:1, 0].float().transpose(-1, -2)),
+                         g.q_up_prefill[:1, 0].float().transpose(-1, -2))
+        assert torch.allclose(y.float(), want, rtol=RTOL, atol=ATOL)
+        seen.append(g._workspace)
+    assert seen[0] is seen[1]

@@ -327,3 +327,50 @@ def test_sgmv_workspace_of_a_longer_batch():
     sgmv_multi([y], [bits_to_torch(x, FP16, "cuda")], pool, 0, ["p"], plan)
     torch.cuda.synchronize()
     assert_close_bits(torch_to_bits(y), oracle_apply(pp, x, _tok_of(*seg, T), y0), FP16, "short prompt")
+
+
+@pytest.mark.parametrize("long,T,n_seg,n_proj", [(6848, 6144, 1, 1), (3648, 2880, 8, 7), (3648, 3648, 8, 6), (300, 250, 1, 1)])
+def test_a_workspace_of_a_larger_call_serves_a_smaller_one(long, T, n_seg, n_proj):
+    """Batches that would take more workspace than the larger call's holds (more K splits), through the LoRA call and the
+    one-pass base product; (3648, 3648): fewer projections than it was sized for."""
+    from mlora import _ext, gemm_lora, sgmv_multi, sgmv_workspace
+    rng = np.random.default_rng(long + T)
+    hin, hout = 1032, 72
+    names = [f"p{i}" for i in range(n_proj)]
+    pp = PagedPool(rng, [64, 16, 40], hin, hout, page_rows=8, dtype=FP16)
+    pool = upload_pool(pp, projections={nm: (hin, hout) for nm in names})
+    for nm in names:
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, FP16))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, FP16))
+    ws = sgmv_workspace(long, n_seg, "cuda", 7 if n_seg == 8 else n_proj)
+    lib = _ext.lib()
+    assert lib.mlora_sgmv_splits(T, n_seg, n_proj, ws.numel()) < lib.mlora_sgmv_splits(T, n_seg, n_proj, 1 << 50)
+    cuts = np.sort(rng.choice(np.arange(1, T), n_seg - 1, replace=False)) if n_seg > 1 else np.empty(0, np.int64)
+    lens = np.diff(np.concatenate([[0], cuts, [T]])).astype(int)
+    seg = _segments(lens, rng.integers(0, 3, n_seg))
+    dev = [torch.from_numpy(a).cuda() for a in seg]
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), FP16)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), FP16)
+    xt = bits_to_torch(x, FP16, "cuda")
+    ys = [bits_to_torch(y0, FP16, "cuda") for _ in names]
+    say(f"sgmv_multi T={T} in a workspace for {long}")
+    plan = plan_prefill(*dev, T, pool, workspace=ws)
+    sgmv_multi(ys, [xt] * n_proj, pool, 0, names, plan)
+    torch.cuda.synchronize()
+    tok = _tok_of(*seg, T)
+    want = oracle_apply(pp, x, tok, y0)
+    for y in ys:
+        assert_close_bits(torch_to_bits(y), want, FP16, "sgmv_multi")
+    w = (torch.randn(hin, hout, device="cuda") / hin ** 0.5).half()
+    outs = [torch.zeros(T, hout, device="cuda").half() for _ in names]
+    say(f"gemm_lora T={T} in a workspace for {long}")
+    plan = plan_prefill(*dev, T, pool, workspace=ws, aligned=True)
+    gemm_lora(outs, [xt] * n_proj, [w] * n_proj, pool, 0, names, plan)
+    torch.cuda.synchronize()
+    base = xt.double().cpu().numpy() @ w.double().cpu().numpy()
+    for a in range(3):
+        v = (f32_of(x, FP16).astype(np.float64)[tok == a] @ pp.A(a)) * np.float64(pp.scaling[a])
+        base[tok == a] += v @ pp.B(a)
+    for y in outs:
+        got = y.double().cpu().numpy()
+        assert (np.abs(got - base) <= ATOL + RTOL * np.abs(base)).all()
