@@ -152,3 +152,14 @@ def test_a_prefill_workspace_serves_every_smaller_call(T):
                         grew += got < full
     assert grew > 0 or T <= 64                   # the sweep meets calls that would take more than they are given
     assert lib.mlora_sgmv_splits(T, 1, 1, 256) == 0
+
+
+def test_one_make_builds_what_the_package_imports():
+    """`make -C csrc` alone builds the library and the launch path that loads with it, and the launch path by itself the
+    library it links (make's dry run)."""
+    import subprocess
+    csrc = os.path.join(ROOT, "ae-296_amd", "csrc")
+    run = lambda *a: subprocess.run(["make", "-n", "-B", *a], capture_output=True, text=True, check=True).stdout  # noqa: E731
+    whole, alone = run("-C", csrc), run("-C", os.path.join(csrc, "host"))
+    for out in (whole, alone):
+        assert out.index("-o ../mlora/libmlora_hip.so") < out.index("-o ../../mlora/_host.so")
