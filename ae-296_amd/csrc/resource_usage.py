@@ -9,11 +9,12 @@ the limits below.  The limits say what the kernels were designed around:
   kernel, which no parity test can see);
 * `gemm_lora_kernel` keeps its 256 fp32 accumulators in AGPRs, runs one workgroup per compute unit and must not
   move accumulators between AGPRs and VGPRs inside the K loop (the epilogue reads each of them out: about a thousand
-  moves over its unrolled paths; the K loop gone wrong adds more than that again);
+  moves over its unrolled paths; the K loop gone wrong adds more than that again); `gemm_lora_short_kernel` of MI
+  32-row blocks keeps 64 MI of them and may move 320 MI times (the epilogue reads 256 MI; at -O1 400, 704 and 1008);
 * the decode shrink of a one-round launch needs at least four (rank <= 16) or three (rank 32) workgroups per
   compute unit, the expand three;
-* M0 in `gemm_lora_kernel` and `gemm_lora_short_kernel` is written only by the kernel's own LDS-bound loads: one `s_mov_b32 m0` per such load
-  and no other instruction that names M0.
+* M0 in `gemm_lora_kernel` and `gemm_lora_short_kernel` is written only by the kernel's own LDS-bound loads: one
+  `s_mov_b32 m0` per such load and no other instruction that names M0.
 """
 from __future__ import annotations
 
@@ -104,7 +105,7 @@ def compile_report(source: str, extra_flags=()):
 
 
 def violations(source: str, report):
-    """List of strings, one per (kernel, field) outside LIMITS, plus the M0 rule of gemm_lora_kernel."""
+    """List of strings, one per (kernel, field) outside LIMITS, plus the M0 rule and the accumulators of the GEMM kernels."""
     bad = []
     for src, pattern, limits in LIMITS:
         if src != source:
@@ -122,6 +123,12 @@ def violations(source: str, report):
             bad.append(f"{source}: no kernel matches {pattern!r}")
     if source == "gemm_lora.hip":
         for name, rec in report.items():
+            short = re.search(r"gemm_lora_short_kernel<\d, \d+, (\d)>", name)
+            if short:
+                mi = int(short.group(1))
+                for field, lo, hi in (("agprs", 64 * mi, 64 * mi), ("accvgpr_moves", 0, 320 * mi)):
+                    if not lo <= rec.get(field, -1) <= hi:
+                        bad.append(f"{source}: {name}: {field} = {rec.get(field)}, allowed {lo}..{hi}")
             if re.search(r"gemm_lora_(short_)?kernel<", name):
                 if rec.get("m0_other", 1) != 0 or rec.get("m0_writes", 0) != rec.get("lds_loads", -1):
                     bad.append(f"{source}: {name}: M0 is named by {rec.get('m0_other')} instructions besides its "

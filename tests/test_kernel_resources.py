@@ -46,6 +46,16 @@ def test_checker_flags_a_kernel_that_left_its_limits(field, value):
     assert bad and "gemm_lora_kernel<0, 64>" in bad[0]
 
 
+@pytest.mark.parametrize("field, value", [("scratch", 8), ("agprs", 144), ("accvgpr_moves", 704), ("m0_other", 1)])
+def test_checker_flags_a_short_batch_kernel_that_left_its_limits(field, value):
+    """The accumulators of the short-batch kernel, by its row blocks; the values are those of a build at -O1."""
+    short = dict(scratch=0, vgpr_spill=0, agprs=128, vgprs=152, occupancy=1, lds=101488, accvgpr_moves=512, m0_writes=80, m0_other=0,
+                 lds_loads=80)
+    assert ru.violations("gemm_lora.hip", {**GOOD, "gemm_lora_short_kernel<0, 16, 2>": short}) == []
+    bad = ru.violations("gemm_lora.hip", {**GOOD, "gemm_lora_short_kernel<0, 16, 2>": {**short, field: value}})
+    assert bad and "gemm_lora_short_kernel<0, 16, 2>" in bad[0]
+
+
 def test_checker_reads_the_compilers_remarks_and_assembly():
     remarks = "\n".join(f"k.hip:9:1: remark: {t} [-Rpass-analysis=kernel-resource-usage]" for t in (
         "Function Name: _Z1kv", "    TotalSGPRs: 20", "    VGPRs: 300", "    AGPRs: 12", "    ScratchSize [bytes/lane]: 96",
