@@ -419,10 +419,7 @@ static int bgmv_multi_impl(int form, int n_proj, void *const *y, const void *con
     }
     a.tok_adapter = tok_adapter; a.tok_adapter64 = nullptr;
     a.work = work; a.work_cap = MLORA_WORK_CAP(T);
-    {
-        const int bound = items_bound(T, n_adapters, group > 0 ? group : 1);
-        a.items_cap = bound < a.work_cap ? bound : a.work_cap;
-    }
+    a.items_cap = items_bound(T, n_adapters, group);
     a.T = T; a.n_proj = n_proj; a.accumulate = accumulate ? 1 : 0;
     if (use_scratch) {
         const int64_t need = mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
@@ -635,11 +632,7 @@ int mlora_bgmv_reflayout_multi(int n_proj, void *const *y, const void *const *x,
     a.b_transposed = 1; a.ref_layers = L;
     a.tok_adapter = nullptr; a.tok_adapter64 = nullptr;
     a.work = ref_plan_work(const_cast<void *>(plan), T); a.work_cap = MLORA_WORK_CAP(T);
-    {
-        const int64_t segs = T < N ? T : N;
-        const int64_t bound = ((int64_t)(T + group - 1) / group + segs + 1 + 7) / 8 * 8;
-        a.items_cap = bound < a.work_cap ? (int)bound : a.work_cap;
-    }
+    a.items_cap = items_bound(T, N, group);
     a.T = T; a.n_proj = n_proj; a.accumulate = accumulate ? 1 : 0;
     const int64_t need = mlora_bgmv_workspace_bytes(n_proj, T, max_hin, r);
     if (!workspace || !aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be a 16-byte aligned device pointer");

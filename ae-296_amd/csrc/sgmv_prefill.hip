@@ -30,23 +30,16 @@ constexpr int VSTRIDE = MAX_RANK;
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4;
 
-__device__ __forceinline__ int sg_pool_row(const int32_t *__restrict__ tbl, long long dense_stride, int adapter, int j,
-                                           const PoolView &pv, long long n_rows)
+__device__ __forceinline__ int sg_pool_row(const int32_t *__restrict__ tbl, int adapter, int j, const PoolView &pv, long long n_rows)
 {
-    long long row;
-    if (tbl) {
-        const int pg = tbl[(long long)adapter * pv.max_pages + (j >> pv.page_shift)];
-        row = pg < 0 ? -1 : (((long long)pg << pv.page_shift) + (j & ((1 << pv.page_shift) - 1)));
-    } else {
-        row = (long long)adapter * dense_stride + j;
-    }
+    const int pg = tbl[(long long)adapter * pv.max_pages + (j >> pv.page_shift)];
+    const long long row = pg < 0 ? -1 : (((long long)pg << pv.page_shift) + (j & ((1 << pv.page_shift) - 1)));
     return (row < 0 || row >= n_rows) ? -1 : (int)row;
 }
 
 __device__ __forceinline__ void seg_of(const SgmvArgs &p, int s, int &start, int &len, int &adapter)
 {
-    if (p.seg_uniform_len > 0) { start = s * p.seg_uniform_len; len = p.seg_uniform_len; adapter = s; }
-    else { start = p.seg_start[s]; len = p.seg_len[s]; adapter = p.seg_adapter[s]; }
+    start = p.seg_start[s]; len = p.seg_len[s]; adapter = p.seg_adapter[s];
     if (start < 0 || len < 0 || start > p.T) { start = 0; len = 0; }
     if (len > p.T - start) len = p.T - start;
 }
@@ -143,6 +136,7 @@ __device__ __forceinline__ Tile<UNIFORM> tile_of(const SgmvArgs &p, int tile)
 }
 
 // ------------------------------------------------------------------ plan
+// (segments on a paged pool; equally long ones on a dense pool need none, see Tile)
 __global__ __launch_bounds__(1024) void sgmv_plan_kernel(const SgmvArgs p)
 {
     __shared__ int s_wave[16];
@@ -209,10 +203,11 @@ __global__ __launch_bounds__(1024) void sgmv_plan_kernel(const SgmvArgs p)
             const bool real = adapter >= 0 && adapter < pv.n_adapters;
             int rk = 0, sc = 0;
             if (real) {
-                rk = pv.rank ? pv.rank[adapter] : pv.uniform_rank;
+                const int cap = pv.max_pages << pv.page_shift;
+                rk = pv.rank[adapter];
                 rk = rk < 0 ? 0 : (rk > MAX_RANK ? MAX_RANK : rk);
-                if (pv.a_tbl) { const int cap = pv.max_pages << pv.page_shift; rk = rk > cap ? cap : rk; }
-                sc = __builtin_bit_cast(int, pv.scaling ? pv.scaling[adapter] : pv.uniform_scale);
+                rk = rk > cap ? cap : rk;
+                sc = __builtin_bit_cast(int, pv.scaling[adapter]);
             }
             s_hdr[tid][0] = p.tile_ntok[t]; s_hdr[tid][1] = real ? adapter : -1; s_hdr[tid][2] = rk;
             s_hdr[tid][3] = sc; s_hdr[tid][4] = p.tile_tok0[t]; s_hdr[tid][5] = seg;
@@ -225,7 +220,7 @@ __global__ __launch_bounds__(1024) void sgmv_plan_kernel(const SgmvArgs p)
             if (w < 6) val = s_hdr[lt][w];
             else if (w >= TILE_ROWS_AT) {
                 const int j = w - TILE_ROWS_AT, adapter = s_hdr[lt][1];
-                val = (adapter >= 0 && j < s_hdr[lt][2]) ? sg_pool_row(pv.a_tbl, pv.a_dense_stride, adapter, j, pv, pv.n_rows_a) : -1;
+                val = (adapter >= 0 && j < s_hdr[lt][2]) ? sg_pool_row(pv.a_tbl, adapter, j, pv, pv.n_rows_a) : -1;
             }
             p.tile_rec[(size_t)(t0 + lt) * TILE_WORDS + w] = val;
         }
