@@ -196,7 +196,7 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     // 64 lanes x 16 bytes into 1 KiB of consecutive LDS, lane i to slot i.  The tiles therefore have no row
     // padding; bank conflicts are avoided by storing 16-byte chunk c of a row at position c ^ key(row), which
     // costs nothing on the way in (lane i simply fetches the chunk that belongs in slot i).
-    //   x tile [256 rows][4 chunks]:  key = (row / 4) % 4   (16 operand rows of one chunk column -> 16 bank groups)
+    //   x tile [64 MI rows][4 chunks]:  key = (row / 4) % 4   (16 operand rows of one chunk column -> 16 bank groups)
     //   W tile [32 k rows][32 chunks]: key = (k % 4) * 4     (the 4 rows of a transposing read -> 4 bank groups)
     // One load of wavefront w covers 16 rows of x (rows 16 (4 q + w) ..) or 2 rows of W (rows 2 (4 q + w) ..).
     // Rows beyond T and columns beyond hout are clamped to valid addresses; what they produce is never stored.
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(G_NT, 1) void gemm_lora_kernel(const GemmLoraArgs p
     gemm_lora_body<DT, RMAX, 4, false>(p);
 }
 
-// Batches of few tiles (shape_of): tiles of 64 to 256 rows, K cut into ranges.
+// Batches of few tiles (gemm_lora_shape): tiles of 64 to 192 rows, K cut into ranges or whole.
 template <int DT, int RMAX, int MI>
 __global__ __launch_bounds__(G_NT, 1) void gemm_lora_short_kernel(const GemmLoraArgs p)
 {
@@ -625,7 +625,9 @@ __global__ __launch_bounds__(256) void gemm_lora_sum_kernel(const GemmLoraArgs p
 // measured with one workgroup on each unit.  Base products at Llama-7B widths, fp16, us, plain -> chosen (best of the 28
 // shapes tried): q/k/v 16 tokens 77 -> 30 (28), 120 tokens 83 -> 41 (40), 351 tokens 85 -> 64 (63), 700 tokens 95 -> 84 (84);
 // all seven 16 tokens 196 -> 78 (78; 5.2 TB/s of weights), 192 tokens 249 -> 111 (111), 351 tokens 268 -> 199 (191), 500
-// tokens 292 -> 265 (258); from 1024 tokens on the plain shape is the fastest or within 2 % of it (q/k/v at 1500: 203 -> 170).
+// tokens 292 -> 265 (258).  K is cut up to 384 tokens; the plain shape is chosen for the seven from 577 tokens on, but for
+// 1025..1152 and 1793..1920, and for q/k/v at 961..1280, at 1921..2560 and from 3073 on: in between, 256 rows would leave a
+// last round nearly empty (1500 tokens 203 -> 170 with 192 rows).
 // Tiles of 256 rows are never cut: with the ranges the compiler spills accumulators.
 int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out)
 {
