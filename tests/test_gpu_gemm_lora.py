@@ -226,7 +226,7 @@ def test_plan_tile_list_matches_oracle(aligned):
     (128, 3080, 4096, 3, [32, 17], BF16),
     (129, 4104, 4096, 3, [32, 16], FP16),      # 192-row tiles, one row in the third block
     (192, 4096, 4352, 3, [64, 40], BF16),
-    (351, 4104, 1288, 7, [16, 8], FP16),       # two row tiles, the second with a ragged end
+    (351, 4104, 1288, 7, [16, 8], FP16),       # three tiles of 128 rows, the last with a ragged end
 ])
 def test_gemm_lora_short_batches(T, hin, hout, n_proj, ranks, dtype):
     """Tiles of 64 to 192 rows with K cut into ranges: the rows at the tiles' edges against the oracle, every projection
@@ -276,3 +276,41 @@ def test_gemm_lora_short_batches(T, hin, hout, n_proj, ranks, dtype):
     for y in whole:
         a, b = y.double(), ys[0].double()
         assert bool(((a - b).abs() <= ulp * b.abs() + 1e-3).all())
+
+
+@pytest.mark.parametrize("T,hins,houts,splits,ranks,dtype", [
+    # K ranges per projection, as the rule chooses them: cut and whole projections in one launch, the cut ones ...
+    (100, [4096, 512, 4104, 320, 2048], [264, 520, 256, 768, 512], [8, 1, 8, 1, 4], [16, 5], FP16),      # first, in the middle and last
+    (200, [352, 4104, 512, 2080, 416], [512, 264, 1032, 520, 768], [1, 8, 1, 4, 1], [64, 24], BF16),     # between whole ones
+    (260, [4104, 4096, 1024], [4096, 4096, 4104], [3, 3, 1], [32, 8], FP16),                             # two tiles of 192 rows
+])
+def test_gemm_lora_short_batches_of_unlike_projections(T, hins, houts, splits, ranks, dtype):
+    """Projections of other widths, each with its own number of K ranges: the room of the cut ones side by side, the sum
+    launch over them alone, the whole ones written by the product itself."""
+    from mlora import _ext
+    import ctypes as C
+    n = len(hins)
+    names = [f"p{i}" for i in range(n)]
+    pps = [PagedPool(np.random.default_rng(31), ranks, hi, ho, page_rows=8, dtype=dtype) for hi, ho in zip(hins, houts)]
+    pool = upload_pool(pps[0], projections={nm: (hi, ho) for nm, hi, ho in zip(names, hins, houts)})
+    rng = np.random.default_rng(T)
+    xs, ws = [], []
+    for nm, pp in zip(names, pps):
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, dtype))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, dtype))
+        xs.append(bits_of(rng.standard_normal((T, pp.hin)).astype(np.float32), dtype))
+        ws.append(bits_of((rng.standard_normal((pp.hin, pp.hout)) / np.sqrt(pp.hin)).astype(np.float32), dtype))
+    arr = [(C.c_int32 * 8)(*v) for v in (hins, houts)]
+    room = sum(s * T * ho * 4 for s, ho in zip(splits, houts) if s > 1)
+    assert _ext.lib().mlora_gemm_lora_partial_bytes(n, *arr, T) == room
+    ss, sl, sa, _ = _layout([T // 3, T - T // 3 - 7], [0, 7], [0, 1])
+    tok = _tok_of(ss, sl, sa, T)
+    plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in (ss, sl, sa)), T, pool, n_proj=n)
+    ys = [torch.full((T, ho), float("nan"), dtype=tdtype(dtype), device="cuda") for ho in houts]
+    say(f"gemm_lora short T={T} {hins}x{houts} ranges={splits}")
+    gemm_lora(ys, [bits_to_torch(x, dtype, "cuda") for x in xs], [bits_to_torch(w, dtype, "cuda") for w in ws], pool, 0, names, plan)
+    torch.cuda.synchronize()
+    rows = np.unique(np.clip([0, T // 3 - 1, T // 3, T // 3 + 6, T // 3 + 7, 63, 64, 127, 128, 191, 192, T - 1], 0, T - 1))
+    for nm, pp, x, w, y in zip(names, pps, xs, ws, ys):
+        assert bool(torch.isfinite(y).all())
+        assert_close_bits(torch_to_bits(y)[rows], _oracle(pp, x[rows], w, tok[rows]), dtype, nm)
