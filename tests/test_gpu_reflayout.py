@@ -227,18 +227,19 @@ def test_lora_gpu_mirror_calls():
     assert torch.equal(g.k_up[7], g.k_up_prefill[0]) and torch.equal(g.v_down[3], g.v_down_prefill[1])
 
 
+@pytest.mark.parametrize("dtype", [FP16, BF16])
 @pytest.mark.parametrize("B,Lpad,r,hin,hout", [(2, 1, 8, 4096, 264), (5, 65, 24, 392, 1032), (22, 130, 64, 128, 136), (40, 128, 16, 640, 128)])
-def test_prefill_ref_tiles_without_a_plan(B, Lpad, r, hin, hout):
+def test_prefill_ref_tiles_without_a_plan(B, Lpad, r, hin, hout, dtype):
     """Equal prompts need no plan launch: one and several tiles per prompt, last tiles of one and two tokens, and both
     numberings of the workgroups (fewer than 64 tiles, and more)."""
     rng = np.random.default_rng(B + Lpad)
-    A_T = bits_of((rng.standard_normal((B, 2, r, hin)) * 0.02).astype(np.float32), FP16)
-    B_T = bits_of((rng.standard_normal((B, 2, hout, r)) * 0.02).astype(np.float32), FP16)
-    x = bits_of(rng.standard_normal((B, Lpad, hin)).astype(np.float32), FP16)
+    A_T = bits_of((rng.standard_normal((B, 2, r, hin)) * 0.02).astype(np.float32), dtype)
+    B_T = bits_of((rng.standard_normal((B, 2, hout, r)) * 0.02).astype(np.float32), dtype)
+    x = bits_of(rng.standard_normal((B, Lpad, hin)).astype(np.float32), dtype)
     say(f"prefill ref without a plan B={B} Lpad={Lpad} r={r} {hin}x{hout}")
-    y = lora_prefill_ref(*(bits_to_torch(t, FP16, "cuda") for t in (x, A_T, B_T)), 1)
+    y = lora_prefill_ref(*(bits_to_torch(t, dtype, "cuda") for t in (x, A_T, B_T)), 1)
     torch.cuda.synchronize()
-    assert_close_bits(torch_to_bits(y), orc.prefill_bmm_ref(x, A_T, B_T, 1, FP16, round_mid=False), FP16)
+    assert_close_bits(torch_to_bits(y), orc.prefill_bmm_ref(x, A_T, B_T, 1, dtype, round_mid=False), dtype)
 
 
 def test_lora_gpu_keeps_its_workspace_for_a_shorter_prefill():

@@ -270,6 +270,7 @@ def test_sgmv_multi_projection_call():
             assert torch.allclose(y1.float(), ys["k"].float(), rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("dtype", [FP16, BF16])
 @pytest.mark.parametrize("lens,ranks,hin,hout,n_proj", [
     ([1], [64], 4096, 640, 3),                     # one tile, sixteen K splits, projections kept apart
     ([65, 3], [16, 32], 264, 1032, 3),             # fewer stages than splits; a width that ends inside a column block
@@ -278,33 +279,33 @@ def test_sgmv_multi_projection_call():
     ([64] * 25, [64], 512, 512, 2),                # 76 tiles at most: the numbering in runs
     ([64] * 30, [16], 384, 256, 3),                # projections that share x in one workgroup
 ])
-def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj):
+def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj, dtype):
     """Both sides of the size rules of the prefill launches: K splits, column blocks, numbering of the workgroups,
     shared x, and who sums the splits, with and without accumulation; a gap of rows no segment covers at the end."""
     from mlora import sgmv_multi
     rng = np.random.default_rng(sum(lens) + hin)
-    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=FP16)
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
     pool = upload_pool(pp, projections={f"p{i}": (hin, hout) for i in range(n_proj)})
     names = list(pool.projections)
     for nm in names:
-        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, FP16))
-        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, FP16))
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, dtype))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, dtype))
     seg = _segments(lens, rng.integers(0, len(ranks), len(lens)))
     T = sum(lens) + 5
     tok = _tok_of(*seg, T)
     dev = [torch.from_numpy(a).cuda() for a in seg]
-    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), FP16)
-    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), FP16)
-    xt = bits_to_torch(x, FP16, "cuda")
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
+    xt = bits_to_torch(x, dtype, "cuda")
     plan = plan_prefill(*dev, T, pool, n_proj=n_proj)
     for accumulate in (True, False):
-        say(f"sgmv launch shapes lens={lens[:4]}x{len(lens)} {hin}->{hout} n_proj={n_proj} accumulate={accumulate}")
-        ys = [bits_to_torch(y0, FP16, "cuda") for _ in names]
+        say(f"sgmv launch shapes lens={lens[:4]}x{len(lens)} {hin}->{hout} n_proj={n_proj} dtype={dtype} accumulate={accumulate}")
+        ys = [bits_to_torch(y0, dtype, "cuda") for _ in names]
         sgmv_multi(ys, [xt] * n_proj, pool, 0, names, plan, accumulate=accumulate)
         torch.cuda.synchronize()
         want = oracle_apply(pp, x, tok, y0 if accumulate else None)
         for nm, y in zip(names, ys):
-            assert_close_bits(torch_to_bits(y), want, FP16, nm)
+            assert_close_bits(torch_to_bits(y), want, dtype, nm)
 
 
 def test_sgmv_workspace_of_a_longer_batch():
