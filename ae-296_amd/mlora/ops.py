@@ -81,16 +81,24 @@ def n_cus(device=None) -> int:
 
 def default_group(T: int) -> int:
     """Tokens of one adapter per decode work item when the caller does not say: 1 up to 64 tokens and
-    2 up to 128 (the batch then fits one workgroup per compute unit and runs as the single fused launch,
-    see `decode_fused`), 4 beyond (measured per call, three projections: 8.5 us at 64 tokens against
-    9.9 for the two-launch form, 10.8 against 13.2 at 128, 20.5 against 20.9 with 2 at 256)."""
+    2 up to 128, where every item can have a compute unit of its own (see `decode_fused`), 4 beyond."""
     return 1 if T <= 64 else 2 if T <= 128 else 4
 
 
+def decode_form(widths: Sequence[tuple], T: int, group: int, pool: AdapterPool) -> int:
+    """The form (``_ext.FORM_*``) that ``bgmv`` takes by default for projections of these (hin, hout) widths, with a plan
+    of T tokens whose work items hold up to `group` of them."""
+    hi, ho = _IntArr(*(w[0] for w in widths)), _IntArr(*(w[1] for w in widths))
+    form = _ext.lib().mlora_bgmv_form(len(widths), hi, ho, T, pool.n_slots, pool.max_rank, group, C.byref(C.c_int64()))
+    if form < 0:
+        _ext.check(form)
+    return form
+
+
 def decode_fused(T: int, group: int, n_proj: int, n_slots: int) -> bool:
-    """Whether a planned decode call could run as the single fused launch: its work items, one 512-thread
-    workgroup each, fit the device in one round.  Whether it does is decided by the bytes of an item as well
-    (`mlora_bgmv_form`); here it decides the tokens per item.
+    """Whether the work items of a decode call, one 512-thread workgroup each, fit the device in one round, so that it
+    could run as the single fused launch.  This decides the tokens per item (`group_for`); the form of a call
+    is decided by the bytes and widths of its items as well (`decode_form`).
     The item count is the host's estimate: groups of two leave one odd item for about every other adapter."""
     if group > 2:
         return False
@@ -99,9 +107,9 @@ def decode_fused(T: int, group: int, n_proj: int, n_slots: int) -> bool:
 
 
 def group_for(T: int, n_proj: int, n_slots: int) -> int:
-    """Tokens per work item for calls of `n_proj` projections: `default_group(T)` while such a call runs as the
-    fused launch; once it runs as the shrink + expand pair, 4 from 65 tokens on (config 3, 128 tokens x 7
-    projections: 0.267 ms per step with 2, 0.260 with 4)."""
+    """Tokens per work item for calls of `n_proj` projections: `default_group(T)` while the items of such a call fit the
+    device in one round, 4 from 65 tokens on beyond (128 tokens x 7 projections of four ranks, shrink + expand pair:
+    0.267 ms per step with 2, 0.260 with 4)."""
     g = default_group(T)
     return 4 if (T > 64 and not decode_fused(T, g, n_proj, n_slots)) else g
 
@@ -110,7 +118,7 @@ def plan_decode(tok_adapter: torch.Tensor, pool: AdapterPool, group: Optional[in
                 out: Optional[DecodePlan] = None, n_proj: Optional[int] = None) -> DecodePlan:
     """Index/offset gather for a decode batch: groups tokens by adapter (stable) and cuts the
     groups into work items of at most `group` tokens (1, 2, 4 or 8; default by batch size and, when the
-    caller says how many projections its calls will carry (`n_proj`), by the launch form those take).  Pass
+    caller says how many projections its calls will carry (`n_proj`), by how many items those make).  Pass
     `out` to reuse a plan's buffers (no allocation; safe under graph capture; a batch or pool larger than the one it
     was made for is refused)."""
     _need_cuda(tok_adapter)

@@ -738,8 +738,9 @@ def bench_decode(args, dev, workload, steps, warmup, min_ms=0.0):
     xs = [{i: torch.randn(T, width[i], device=dev, generator=gen).half() for i in inputs} for _ in range(L)]
     ys = [[torch.randn(T, shapes[p][1], device=dev, generator=gen).half() for p in projs] for _ in range(L)]
     plan = mlora.plan_decode(tok, pool, group=group) if group else None
-    fused = bool(args.fused or plan is None or
-                 (not args.split and mlora.ops.decode_fused(T, group, len(projs), pool.n_slots)))
+    # the form is the product's choice unless the command line names one; `fused` says which it is
+    want = True if args.fused or plan is None else (False if args.split else None)
+    fused = want if want is not None else mlora.ops.decode_form([shapes[p] for p in projs], T, group, pool) == mlora._ext.FORM_FUSED
 
     # config 5 carries prefill segments through SGMV in the same step (activations shared by the layers:
     # they are larger than the last-level cache anyway)
@@ -760,7 +761,7 @@ def bench_decode(args, dev, workload, steps, warmup, min_ms=0.0):
 
     def bgmv_layers():
         for l in range(L):
-            mlora.bgmv(ys[l], [xs[l][_IN[p]] for p in projs], pool, l, projs, tok, plan=plan, fused=fused)
+            mlora.bgmv(ys[l], [xs[l][_IN[p]] for p in projs], pool, l, projs, tok, plan=plan, fused=want)
 
     def step():
         if plan is not None:
@@ -771,7 +772,7 @@ def bench_decode(args, dev, workload, steps, warmup, min_ms=0.0):
         pplan = mlora.plan_prefill(pre["ss"], pre["sl"], pre["sa"], pre["T"], pool, workspace=pre["ws"])
         for l in range(L):
             def decode_half(l=l):
-                mlora.bgmv(ys[l], [xs[l][_IN[p]] for p in projs], pool, l, projs, tok, plan=plan, fused=fused)
+                mlora.bgmv(ys[l], [xs[l][_IN[p]] for p in projs], pool, l, projs, tok, plan=plan, fused=want)
 
             def prefill_half(l=l):
                 mlora.sgmv_multi([pre["y"][p] for p in projs], [pre["x"][_IN[p]] for p in projs], pool, l, projs, pplan)

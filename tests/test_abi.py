@@ -163,3 +163,26 @@ def test_one_make_builds_what_the_package_imports():
     whole, alone = run("-C", csrc), run("-C", os.path.join(csrc, "host"))
     for out in (whole, alone):
         assert out.index("-o ../mlora/libmlora_hip.so") < out.index("-o ../../mlora/_host.so")
+
+
+def test_decode_form_on_both_sides_of_its_lines():
+    """mlora_bgmv_form at the sizes where its rule changes its mind (256 compute units, as also assumed without a GPU)."""
+    lib = _ext.lib()
+
+    def form(n, hin, hout, T, rank, group=1, slots=1000):
+        need = C.c_int64(-1)
+        rc = lib.mlora_bgmv_form(n, (C.c_int32 * 8)(*[hin] * n), (C.c_int32 * 8)(*[hout] * n), T, slots, rank, group, C.byref(need))
+        coarse = lib.mlora_bgmv_workspace_bytes(n, T, hin, rank)
+        assert rc < 0 or need.value >= coarse
+        assert rc != _ext.FORM_FINE or need.value > coarse
+        return rc
+
+    FUSED, SLICED, FINE = _ext.FORM_FUSED, _ext.FORM_SLICED, _ext.FORM_FINE
+    assert (form(1, 4096, 4096, 32, 20), form(1, 4096, 4096, 32, 21)) == (FUSED, FINE)          # 320 KiB an item
+    assert (form(3, 4096, 4096, 64, 40), form(3, 4096, 4096, 64, 41)) == (FUSED, SLICED)        # 640 KiB, the slices fill the chip
+    assert (form(1, 8192, 8192, 32, 8), form(1, 8200, 8192, 32, 8)) == (FUSED, FINE)            # the widest of a fused item
+    assert (form(1, 4096, 8192, 64, 64), form(1, 4096, 8192, 65, 64)) == (FINE, SLICED)         # four workgroups per unit
+    assert (form(1, 4096, 4096, 256, 16), form(1, 4096, 4096, 257, 16)) == (FUSED, SLICED)      # one round of fused items
+    assert (form(1, 1024, 512, 40, 16, group=4, slots=8), form(1, 1024, 512, 40, 16, group=8, slots=8)) == (FINE, SLICED)
+    assert form(0, 512, 512, 4, 16) == _ext.MLORA_ERANGE and form(1, 512, 512, 4, 65) == _ext.MLORA_ERANGE
+    assert form(1, 512, 512, 4, 16, group=3) == _ext.MLORA_EINVAL

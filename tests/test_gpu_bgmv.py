@@ -517,3 +517,22 @@ def test_bgmv_forms_are_equally_exact(dtype):
     print(share)
     assert max(share.values()) < 1e-3
     assert share["FINE"] <= 2 * min(share["FUSED"], share["SLICED"])
+
+
+@pytest.mark.parametrize("T,ranks,hin,hout,form", [(32, [16], 2048, 2048, "FUSED"), (9, [64, 8], 4096, 4096, "FINE"),
+                                                   (256, [64], 4096, 8192, "SLICED"), (300, [16], 1024, 1024, "FINE")])
+def test_bgmv_default_form_is_the_one_the_rule_names(T, ranks, hin, hout, form):
+    """Without `fused` a planned call is, bit for bit, the call in the form that `decode_form` names."""
+    from mlora import _ext, ops
+    rng = np.random.default_rng(T + hout)
+    pp = PagedPool(rng, ranks * 12, hin, hout, page_rows=8, dtype=FP16)
+    pool = upload_pool(pp)
+    tok = rng.integers(-1, pool.n_slots, T).astype(np.int32)
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), FP16)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), FP16)
+    group = ops.default_group(T)
+    assert ops.decode_form([(hin, hout)], T, group, pool) == getattr(_ext, "FORM_" + form)
+    say(f"bgmv default form T={T} {form}")
+    got = _run(pp, x, tok, y0, group)
+    assert_close_bits(got, oracle_apply(pp, x, tok, y0), FP16, form)
+    assert np.array_equal(got, _run_form(pp, x, tok, y0, group, getattr(_ext, "FORM_" + form)))
