@@ -407,6 +407,7 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
     constexpr int SLICE = FINE_CHUNKS * 8;                      // columns per workgroup
     constexpr int NQ = 256 / RMAX;                              // threads that share the slices of one intermediate
     __shared__ __attribute__((aligned(16))) float s_vp[NQ][G][RMAX];
+    __shared__ __attribute__((aligned(16))) float s_v[G][RMAX];
     __shared__ __attribute__((aligned(16))) float s_o[4][G][SLICE];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -492,16 +493,21 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
 #pragma unroll
         for (int k = 0; k < G; k++) s_vp[q][k][j] = sum[k];
         __syncthreads();
+        if (tid < G * RMAX) {
+            const int k = tid / RMAX, jj = tid - k * RMAX;
+            float v = 0.f;
+#pragma unroll
+            for (int q4 = 0; q4 < NQ; q4++) v += s_vp[q4][k][jj];
+            s_v[k][jj] = jj < r ? v * scale : 0.f;              // an infinite scale must not reach rows that are not there
+        }
+        __syncthreads();
 #pragma unroll
         for (int i = 0; i < N; i++) {
             float f[8];
             unpack8<DT>(bv[i], f);
 #pragma unroll
             for (int k = 0; k < G; k++) {
-                float vk = 0.f;
-#pragma unroll
-                for (int q4 = 0; q4 < NQ; q4++) vk += s_vp[q4][k][j0 + i];
-                vk = j0 + i < r ? vk * scale : 0.f;             // rows of the bucket that the adapter does not have
+                const float vk = s_v[k][j0 + i];
 #pragma unroll
                 for (int e = 0; e < 8; e++) o[k][e] = fmaf(vk, f[e], o[k][e]);
             }
