@@ -1,10 +1,11 @@
 // SGMV prefill kernels for gfx950: tokens are packed per segment (one adapter per segment)
 //     y[t] (+)= s_a * (x[t] . A_a) . B_a
-// computed on v_mfma_f32_16x16x32_{f16,bf16} tiles in four launches on one stream (the first can be shared by all projections and layers of a batch):
+// computed on v_mfma_f32_16x16x32_{f16,bf16} tiles in three or four launches on one stream (the first can be shared by all projections and layers of a batch):
 //   plan   : cuts every segment into tiles of at most 64 tokens (work list in the workspace);
 //   shrink : V[split][t][0..R) = x[t, Kslice] . A_a[:, Kslice]^T   (split-K, fp32 partials);
 //   reduce : sums the K splits and stores the result as a hi + lo pair of 16-bit values, so
-//            the intermediate keeps fp32 accuracy through the second MFMA;
+//            the intermediate keeps fp32 accuracy through the second MFMA (up to rank 32 and eight
+//            splits the expand does this itself where y accumulates);
 //   expand : y[t, cols] (+)= s_a * (Vhi + Vlo) . B_a[:, cols].
 // Both MFMA operands of the shrink are read straight from global memory in operand layout
 // (8 contiguous K values per lane).  The expand parks the B tile in LDS (rank must be the

@@ -754,6 +754,8 @@ def bench_decode(args, dev, workload, steps, warmup, min_ms=0.0):
         sa = torch.from_numpy(seg_adapter).to(dev)
         px = {i: torch.randn(Tp, width[i], device=dev, generator=gen).half() for i in inputs}
         py = {p: torch.randn(Tp, shapes[p][1], device=dev, generator=gen).half() for p in projs}
+        # two launches a layer where the expand sums the K splits itself (rank <= 32), three beyond
+        pre_launches = 2 if pool.max_rank <= 32 else 3
         pre = dict(ss=ss, sl=sl, sa=sa, T=Tp, x=px, y=py, ws=mlora.sgmv_workspace(Tp, n_seg, dev, n_proj=len(projs)),
                    adapters=seg_adapter)
 
@@ -815,7 +817,7 @@ def bench_decode(args, dev, workload, steps, warmup, min_ms=0.0):
         extra.update({"whole_step": {"achieved": alg_step / (ms_per_step * 1e-3) / 1e9,
                                      "frac": alg_step / (ms_per_step * 1e-3) / 1e9 / HBM_PEAK_GBS,
                                      "algorithmic_bytes_per_step": alg_step, "prefill_bytes_per_layer": alg_pre,
-                                     "kernels": "gather + prefill plan + 32 x (decode pair + SGMV shrink, reduce, expand over 7 projections)"}})
+                                     "kernels": f"gather + prefill plan + {L} x (decode pair + SGMV shrink, {'' if pre_launches == 2 else 'reduce, '}expand over {len(projs)} projections)"}})
     traffic, src = traffic_of(workload, group == mlora.ops.group_for(cfg["T"], len(projs), cfg["N"]) and L == cfg["layers"] and not fused)
 
     metric = "BGMV decode throughput (LoRA-applied token-projections per second)"
@@ -829,7 +831,7 @@ def bench_decode(args, dev, workload, steps, warmup, min_ms=0.0):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f16", "data": "synthetic",
         "config": {"workload": cfg["desc"], "layers": L, "projections_per_call": len(projs),
-                   "launches_per_step": L * (1 if fused else 2) + (1 if plan else 0) + ((1 + 3 * L) if pre else 0),
+                   "launches_per_step": L * (1 if fused else 2) + (1 if plan else 0) + ((1 + pre_launches * L) if pre else 0),
                    "form": "fused" if fused else "shrink + expand",
                    "tokens": T, "prefill_tokens": pre["T"] if pre else 0, "adapters": cfg["N"],
                    "adapters_touched": int(len(uniq)), "group": group,
@@ -1040,6 +1042,7 @@ def main():
                          "reference's arrival trace; swap = adapter swap-in from pinned host memory; assist = CPU-assist transport; "
                          "f1 = base projection + LoRA in one pass on the config-4 batch; reflayout = the reference's pool layout and call; "
                          "coldstart = prefill latency with the adapter cached, loading (CPU-assisted) and loaded on demand")
+    ap.add_argument("--case", help="run ten passes of this case of perf/cases.py and end, for a kernel trace (nothing is timed)")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (run with --gpus 1)", file=sys.stderr)
@@ -1055,6 +1058,14 @@ def main():
     mlora._ext.lib()
     dev = torch.device("cuda:0")
     torch.cuda.set_device(dev)
+    if args.case:
+        from perf import cases
+        state = cases.prepare(next(c for c in cases.listed() if c["name"] == args.case), 1)
+        for _ in range(10):
+            cases.run(state)
+        torch.cuda.synchronize()
+        print(f"ten passes of {args.case}")
+        return
     if args.calib_copy:
         src = torch.ones(128 << 20, dtype=torch.float16, device=dev)      # 256 MiB read + 256 MiB written per copy
         dst = torch.empty_like(src)
