@@ -3,9 +3,11 @@
 //
 // Why it is native: an eager decode or prefill step is a few calls per layer, each checking up to fourteen tensors.
 // In Python that took 6 to 22 us a call on top of the launches themselves (2.6 us each), more than the kernels of a
-// small batch run.  Host time per call before -> now: plan_decode 9.2 -> 3.6 us, bgmv over seven projections in two
-// launches 19.4 -> 6.1 us, sgmv_multi over seven (three launches) 34.5 -> 13.1 us.
-// Nothing is kept from one call for the next: every tensor is checked and every slab looked up on every call.  A negative code of the C ABI is returned, and raised by the caller.
+// small batch run.  Host time per call, launches included, in Python -> here: plan_decode 9.2 -> 4.5 us, bgmv over seven
+// projections in two launches 19.4 -> 9.1 us (0.5 of it the allocation of its intermediate), sgmv_multi over seven (three
+// launches) 34.5 -> 10.7 us.
+// Nothing is kept from one call for the next: every tensor is checked and every slab looked up on every call.  A negative
+// code of the C ABI is returned, and raised by the caller.
 #include <Python.h>
 
 #include <ATen/ATen.h>

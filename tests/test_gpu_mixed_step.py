@@ -1,5 +1,5 @@
 """The mixed step of config 5 on a multi-layer pool at its real row count: per layer one decode call
-(`bgmv`, two launches) and one prefill call (`sgmv_multi`, three launches) that share the pool and the plans,
+(`bgmv`, two launches) and one prefill call (`sgmv_multi`, two launches) that share the pool and the plans,
 side by side on two streams and joined before the next layer, as `bench.py --workload c5` runs it, eagerly and
 replayed from a HIP graph.
 
