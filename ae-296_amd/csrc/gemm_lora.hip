@@ -12,10 +12,14 @@
 // rank / 16 more MFMA steps with (intermediate, B rows of its adapter) as operands.
 //
 // One workgroup (256 threads, 2 x 2 wavefronts of 128 x 128 outputs each) computes a 256 x 256 tile of y
-// on v_mfma_f32_32x32x16_{f16,bf16}.  K advances 32 columns per step through a ring of four LDS stages
-// that global memory fills directly (buffer_load ... lds): while the MFMAs of step k run from one stage, the
-// loads of steps k+1 .. k+3 are in flight or landed.  x is K-contiguous, so its operand is a plain 16-byte
-// LDS read; W is N-contiguous and is read back with the transposing LDS read.
+// on v_mfma_f32_32x32x16_{f16,bf16}.  K advances 32 columns per step through LDS stages that global memory
+// fills directly (buffer_load ... lds): a ring of four W stages of 32 columns and one of two x stages of 64, so that
+// while the MFMAs of step k run, the loads of steps k+1 .. k+3 are in flight or landed.  x is K-contiguous, so its
+// operand is a plain 16-byte LDS read; W is N-contiguous and is read back with the transposing LDS read.
+// x stages hold 64 columns because a row's piece is then a whole 128-byte cache line: with 32 columns a line came from L2
+// twice (4096 x 4096 outputs over K = 16384: 50.3 -> 33.6 million L2 reads; 351 tokens x seven Llama-7B projections 224 -> 209
+// us a call, 9216 tokens of Llama-13B 5.27 -> 5.11 ms).  What bounds the loop now: the MFMA pipes, busy 0.77 of it, at the 1.7
+// GHz the card holds under this load; without any global load in the loop it would take 0.87 of the time.
 //
 // A short batch runs the same loop on tiles of 64, 128 or 192 rows with K cut into ranges (gemm_lora_shape): its bound is
 // the weights' way from HBM up to about 64 tokens (Llama-7B layer, 405 MB: 78 us at 16 tokens) and the feed of the compute
@@ -27,8 +31,9 @@
 namespace mlora {
 
 constexpr int GN = 256;                 // output columns per tile
-constexpr int GK = 32;                  // K columns per stage
-constexpr int NST = 4;                  // stages in flight (a ring)
+constexpr int GK = 32;                  // K columns per step, and per stage of the W ring
+constexpr int XK = 2 * GK;              // K columns per stage of the x ring
+constexpr int NXS = 2, NWS = 4;         // stages of the x ring and of the W ring
 constexpr int G_NT = 256;
 constexpr int B_BYTES = GK * GN * 2;    // W tile of a stage, chunk-swizzled like the x tile, rows unpadded
 constexpr int OPITCH = 128 * 2 + 16;    // bytes per row of a wavefront's 32 x 128 output staging tile
@@ -36,15 +41,16 @@ constexpr int GROUP_M = 4;              // row tiles that share W column tiles b
 typedef short gl_short4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) gl_short4 gl_lds_short4;
 
-// Bytes of one stage of the ring: an x tile of 64 * MI rows and a W tile; the parked B rows and a wavefront's output
-// staging reuse one stage each.
-template <int RMAX, int MI> constexpr int stage_bytes()
+// Bytes of one stage of the x ring: 64 * MI rows of XK columns.  The B rows of an adapter are parked in one x stage or
+// in two neighbouring W stages, a wavefront's output staging takes one W stage.
+template <int RMAX, int MI> constexpr int x_stage_bytes()
 {
-    constexpr int ab = 64 * MI * GK * 2 + B_BYTES, rows = RMAX * GN * 2;
-    return ab > rows ? ab : rows;
+    constexpr int x = 64 * MI * XK * 2, rows = RMAX * GN * 2;
+    return x > rows ? x : rows;
 }
-static_assert(NST * stage_bytes<64, 4>() <= 160 * 1024 - 4096, "the stages and the small tables must fit the LDS of a compute unit");
-static_assert(32 * OPITCH <= stage_bytes<16, 1>(), "a wavefront's output staging reuses one stage");
+static_assert(NXS * x_stage_bytes<64, 4>() + NWS * B_BYTES <= 160 * 1024 - 4096, "the stages and the small tables must fit the LDS of a compute unit");
+static_assert(MAX_RANK * GN * 2 <= 2 * B_BYTES, "the B rows of an adapter fit two W stages");
+static_assert(32 * OPITCH <= B_BYTES, "a wavefront's output staging reuses one W stage");
 
 template <int DT>
 __device__ __forceinline__ float16_t mfma32(const uint4 &a, const uint4 &b, float16_t c)
@@ -94,13 +100,11 @@ template <int DT, int RMAX, int MI, bool SPLIT>
 __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
 {
     constexpr int GM = 64 * MI;
-    constexpr int A_BYTES = GM * GK * 2;
-    constexpr int STAGE = stage_bytes<RMAX, MI>();
-    // one array per stage: the compiler then knows that loads into one stage cannot alias the operand reads of another
-    __shared__ __attribute__((aligned(16))) unsigned char smem[STAGE];
-    __shared__ __attribute__((aligned(16))) unsigned char smem1[STAGE];
-    __shared__ __attribute__((aligned(16))) unsigned char smem2[STAGE];
-    __shared__ __attribute__((aligned(16))) unsigned char smem3[STAGE];
+    constexpr int XSTAGE = x_stage_bytes<RMAX, MI>();
+    __shared__ __attribute__((aligned(16))) unsigned char sx0[XSTAGE];
+    __shared__ __attribute__((aligned(16))) unsigned char sx1[XSTAGE];
+    __shared__ __attribute__((aligned(16))) unsigned char sw01[2 * B_BYTES];       // W stages 0 and 1
+    __shared__ __attribute__((aligned(16))) unsigned char sw23[2 * B_BYTES];       // W stages 2 and 3
     __shared__ unsigned long long s_mask[2 * (G_NT / 64)];
     __shared__ int s_list[G_NT + 1];               // first plan tile of every run (of the 256 tiles looked at); [G_NT] = how many runs
     __shared__ int s_last[G_NT];                   // last plan tile of every run
@@ -196,22 +200,23 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     // 64 lanes x 16 bytes into 1 KiB of consecutive LDS, lane i to slot i.  The tiles therefore have no row
     // padding; bank conflicts are avoided by storing 16-byte chunk c of a row at position c ^ key(row), which
     // costs nothing on the way in (lane i simply fetches the chunk that belongs in slot i).
-    //   x tile [64 MI rows][4 chunks]:  key = (row / 4) % 4   (16 operand rows of one chunk column -> 16 bank groups)
+    //   x tile [64 MI rows][8 chunks]:  key = (row / 2) % 8   (16 operand rows of one chunk column -> 16 bank groups)
     //   W tile [32 k rows][32 chunks]: key = (k % 4) * 4     (the 4 rows of a transposing read -> 4 bank groups)
-    // One load of wavefront w covers 16 rows of x (rows 16 (4 q + w) ..) or 2 rows of W (rows 2 (4 q + w) ..).
+    // One load of wavefront w covers 8 rows of x (rows 8 (4 q + w) ..) or 2 rows of W (rows 2 (4 q + w) ..).
     // Rows beyond T and columns beyond hout are clamped to valid addresses; what they produce is never stored.
     const int rows_here = T - m0 < GM ? T - m0 : GM;
     const int k0 = SPLIT ? split * pj.ksteps : 0;               // first K step of this workgroup
-    unsigned aoff[MI], boff[4];
+    constexpr int NX = 2 * MI, NW = 4;                          // a wavefront's loads per x stage and per W stage
+    unsigned aoff[NX], boff[NW];
 #pragma unroll
-    for (int q = 0; q < MI; q++) {
-        const int row = 16 * (4 * q + wave) + (lane >> 2);
-        const int c = (lane & 3) ^ ((row >> 2) & 3);
+    for (int q = 0; q < NX; q++) {
+        const int row = 8 * (4 * q + wave) + (lane >> 3);
+        const int c = (lane & 7) ^ ((row >> 1) & 7);
         const int r = row < rows_here ? row : rows_here - 1;
         aoff[q] = ((unsigned)r * (unsigned)hin + (unsigned)(k0 * GK) + (unsigned)c * 8u) * 2u;
     }
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
+    for (int q = 0; q < NW; q++) {
         const int k = 2 * (4 * q + wave) + (lane >> 5);
         const int c = (lane & 31) ^ ((k & 3) << 2);
         int col = n0 + c * 8;
@@ -247,14 +252,18 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :: "s"(lds_addr), "v"(voff), "s"(rs), "s"(soff) : "memory");
     };
-    // the loads of one K step: MI of x, 4 of W
-    auto dma = [&](unsigned char *stage, int ks) {
-        const unsigned soff_a = (unsigned)ks * (GK * 2), soff_b = (unsigned)ks * GK * (unsigned)hout * 2u;
-        const unsigned base = (unsigned)(__UINTPTR_TYPE__)(lds_byte *)stage + (unsigned)wave * 1024u;
+    auto x_stage = [&](int j) -> unsigned char * { return (j & 1) ? sx1 : sx0; };
+    auto w_stage = [&](int k) -> unsigned char * { return ((k & 2) ? sw23 : sw01) + (k & 1) * B_BYTES; };
+    auto lds_of = [&](unsigned char *stage) { return (unsigned)(__UINTPTR_TYPE__)(lds_byte *)stage + (unsigned)wave * 1024u; };
+    // the loads of K steps 2 j and 2 j + 1 of x, and of K step k of W.  Columns of x past hin (the second half of the last
+    // stage) come from the next row, or as zeros from past the last one; no step reads them.
+    auto dma_x = [&](int j) {
 #pragma unroll
-        for (int q = 0; q < MI; q++) dma1(xrw, base + q * 4096, aoff[q], soff_a);
+        for (int q = 0; q < NX; q++) dma1(xrw, lds_of(x_stage(j)) + q * 4096, aoff[q], (unsigned)j * (XK * 2));
+    };
+    auto dma_w = [&](int k) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) dma1(wrw, base + A_BYTES + q * 4096, boff[q], soff_b);
+        for (int q = 0; q < NW; q++) dma1(wrw, lds_of(w_stage(k)) + q * 4096, boff[q], (unsigned)k * GK * (unsigned)hout * 2u);
     };
 
     float16_t acc[MI][4];
@@ -265,14 +274,14 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
 
-    // Operand addresses inside a stage.  x: lane (row wm * 32 MI + 32 i + lane % 32, chunk 2 kk + lane / 32); the key
-    // of the row does not depend on i.  W: lane group g = lane / 16, m = lane % 16 reads rows 16 kk + 8 (g / 2) +
+    // Operand addresses inside a stage.  x: lane (row wm * 32 MI + 32 i + lane % 32, chunk 4 (step % 2) + 2 kk + lane / 32);
+    // the key of the row does not depend on i.  W: lane group g = lane / 16, m = lane % 16 reads rows 16 kk + 8 (g / 2) +
     // m / 4 (+ 4), bytes of columns wn * 128 + 32 j + 16 (g % 2) + 4 (m % 4) ..; the key (m / 4) * 4 flips bits of j.
-    unsigned a_at[2], b_at[4];
+    unsigned a_at[4], b_at[4];                     // a_at: slice 0 and 1 of an even step, then of an odd one
     {
-        const int row = wm * (32 * MI) + l32, key = (l32 >> 2) & 3;
+        const int row = wm * (32 * MI) + l32, key = (l32 >> 1) & 7;
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++) a_at[kk] = (unsigned)(row * (GK * 2) + (((2 * kk + lh) ^ key) << 4));
+        for (int s4 = 0; s4 < 4; s4++) a_at[s4] = (unsigned)(row * (XK * 2) + (((2 * s4 + lh) ^ key) << 4));
         const int g = lane >> 4, m = lane & 15;
         const int krow = 8 * (g >> 1) + (m >> 2);
 #pragma unroll
@@ -297,11 +306,11 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     };
     // Operands of one K = 16 slice (MI x fragments, 4 W fragments), read one slice ahead of the MFMAs that use them.
     uint4 fa[2][MI], fb[2][4];
-    auto frags = [&](const unsigned char *stage, auto kk_c, uint4 (&af)[MI], uint4 (&bf)[4]) {
-        constexpr int kk = decltype(kk_c)::value;
+    auto frags = [&](const unsigned char *xs, const unsigned char *wst, auto odd_c, auto kk_c, uint4 (&af)[MI], uint4 (&bf)[4]) {
+        constexpr int odd = decltype(odd_c)::value, kk = decltype(kk_c)::value;
 #pragma unroll
-        for (int i = 0; i < MI; i++) af[i] = *reinterpret_cast<const uint4 *>(stage + a_at[kk] + i * 32 * (GK * 2));
-        w_frags(stage + A_BYTES, kk, bf);
+        for (int i = 0; i < MI; i++) af[i] = *reinterpret_cast<const uint4 *>(xs + a_at[2 * odd + kk] + i * 32 * (XK * 2));
+        w_frags(wst, kk, bf);
     };
     auto mfma16x = [&](const uint4 (&af)[MI], const uint4 (&bf)[4]) {
 #pragma unroll
@@ -312,9 +321,9 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     using K0 = std::integral_constant<int, 0>;
     using K1 = std::integral_constant<int, 1>;
 #define GL_FENCE() __builtin_amdgcn_sched_barrier(0)
-    // A slice is NM MFMAs; NR operand reads and NL global loads are dealt out over them.
-    constexpr int NM = 4 * MI, NR = MI + 8, NL = MI + 4;
-    constexpr int RPM = (NR + NM - 1) / NM, LPM = (NL + NM - 1) / NM;
+    // A slice is NM MFMAs; NR operand reads are dealt out over them.
+    constexpr int NM = 4 * MI, NR = MI + 8;
+    constexpr int RPM = (NR + NM - 1) / NM;
     // Scheduling hints: one MFMA, then its share of the operand reads, so that the memory
     // instructions issue in the shadow of the MFMAs instead of in a burst between them (an MFMA occupies its pipe
     // for 32 cycles, issuing it takes 4).
@@ -326,11 +335,14 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     // s_waitcnt with only the vector-memory counter set: at most n loads of this wavefront still in flight
     // (loads complete in order).
 #define GL_WAIT_LOADS(n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((n) & 15) | (((n) >> 4) << 14))
-    // One K step of 32 columns out of stage `ks % 4`, two slices of 16.  Operand reads run one slice ahead of
-    // the MFMAs.  The barrier sits between the slices: by then every wavefront has read all it needs from this
-    // stage and its loads of step ks + 1 (requested three steps earlier) have landed, so the second slice's
-    // operand prefetch reads the next stage, and this stage is free to receive step ks + 4 at once.
-    // `steady`: steps ks + 1 .. ks + 4 all exist; otherwise the ends of the pipeline are checked.
+    // One K step of 32 columns, two slices of 16; step k reads W stage k % 4 and one half of x stage (k / 2) % 2.
+    // Operand reads run one slice ahead of the MFMAs.  The barrier sits between the slices: by then every wavefront has
+    // read all it needs of this step, and its own loads of step k + 1 have landed, so the second slice's operand
+    // prefetch reads step k + 1.  The second slice also requests what goes into the stages just released: step k + 4 of W,
+    // and after an odd step steps k + 3 and k + 4 of x.
+    // In flight behind what step k + 1 needs, when all of it exists: W of steps k + 2 and k + 3, and, before the barrier of an
+    // even step, x of steps k + 2 and k + 3.
+    // `steady`: steps k + 1 .. k + 4 all exist; otherwise the ends of the pipeline are checked and all loads waited for.
     const gl_i32x4 brw = rsrc_words(pj.b_rows, (size_t)p.n_rows_b * hout * 2);   // the launcher guarantees < 4 GiB
     // one load = rank rows 2 jj and 2 jj + 1 (lanes 0..31 and 32..63) of tile q, jj = wave + 4 u, row indices from s_rows
     auto b_row_of = [&](int q, int u) { return s_rows[q][2 * (wave + 4 * u) + (lane >> 5)]; };
@@ -343,22 +355,22 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
         dma1(brw, lds_stage_wave + u * 4096, voff, 0u);
     };
     auto k_step = [&](auto cur_c, auto steady_c, int ks, int ns) {
-        constexpr int cur_i = decltype(cur_c)::value;
+        constexpr int cur = decltype(cur_c)::value, odd = cur & 1;
         constexpr bool steady = decltype(steady_c)::value;
-        unsigned char *cur = cur_i == 0 ? smem : cur_i == 1 ? smem1 : cur_i == 2 ? smem2 : smem3;
-        unsigned char *nxt = cur_i == 0 ? smem1 : cur_i == 1 ? smem2 : cur_i == 2 ? smem3 : smem;
-        frags(cur, K1{}, fa[1], fb[1]);
+        const unsigned char *nx = x_stage((cur + 1) >> 1), *nw = w_stage(cur + 1);       // of the next step
+        frags(x_stage(cur >> 1), w_stage(cur), std::integral_constant<int, odd>{}, K1{}, fa[1], fb[1]);
         mfma16x(fa[0], fb[0]);
         GL_MIX()
         GL_FENCE();
-        const bool more_loads = steady || ks + 4 < ns, more_steps = steady || ks + 1 < ns;
-        GL_WAIT_LOADS(steady ? 2 * NL : 0);        // steady: the loads of steps ks + 2 and ks + 3 may still be in flight
+        const bool more_w = steady || ks + 4 < ns, more_x = odd && (steady || ks + 3 < ns), more_steps = steady || ks + 1 < ns;
+        GL_WAIT_LOADS(!steady ? 0 : odd ? 2 * NW : 2 * NW + NX);
         __syncthreads();
         // Second slice, scheduled by hand (the loads are assembly, which the scheduler will not interleave):
         // after MFMA n come the operand reads n * RPM .. of the next step's first slice (MI of x, then 8 halves of W)
-        // and the loads n * LPM .. of step ks + 4 into the stage that has just been released.
-        const unsigned soff_a = (unsigned)(ks + 4) * (GK * 2), soff_b = (unsigned)(ks + 4) * GK * (unsigned)hout * 2u;
-        const unsigned lbase = (unsigned)(__UINTPTR_TYPE__)(lds_byte *)cur + (unsigned)wave * 1024u;
+        // and the loads n * LPM .. into the stages that have just been released (x first: it is needed first).
+        constexpr int NLX = odd ? NX : 0, NL = NLX + NW, LPM = (NL + NM - 1) / NM;
+        const unsigned soff_a = (unsigned)((ks + 3) >> 1) * (XK * 2), soff_b = (unsigned)(ks + 4) * GK * (unsigned)hout * 2u;
+        const unsigned xbase = lds_of(x_stage(cur >> 1)), wbase = lds_of(w_stage(cur));
 #pragma unroll
         for (int n = 0; n < NM; n++) {
             acc[n >> 2][n & 3] = mfma32<DT>(fa[1][n >> 2], fb[1][n & 3], acc[n >> 2][n & 3]);
@@ -366,22 +378,20 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
 #pragma unroll
                 for (int t = n * RPM; t < n * RPM + RPM; t++) {
                     if (t < MI) {
-                        fa[0][t] = *reinterpret_cast<const uint4 *>(nxt + a_at[0] + t * 32 * (GK * 2));
+                        fa[0][t] = *reinterpret_cast<const uint4 *>(nx + a_at[odd ? 0 : 2] + t * 32 * (XK * 2));
                     } else if (t < NR) {
                         const int j = (t - MI) >> 1;
                         const bool second = ((t - MI) & 1) != 0;
-                        const unsigned char *src = nxt + A_BYTES + b_at[j] + (second ? 4 * (GN * 2) : 0);
+                        const unsigned char *src = nw + b_at[j] + (second ? 4 * (GN * 2) : 0);
                         const uint2 h = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((gl_lds_short4 *)src));
                         if (second) { fb[0][j].z = h.x; fb[0][j].w = h.y; } else { fb[0][j].x = h.x; fb[0][j].y = h.y; }
                     }
                 }
             }
-            if (more_loads) {
 #pragma unroll
-                for (int t = n * LPM; t < n * LPM + LPM; t++) {
-                    if (t < MI) dma1(xrw, lbase + t * 4096, aoff[t], soff_a);
-                    else if (t < NL) dma1(wrw, lbase + A_BYTES + (t - MI) * 4096, boff[t - MI], soff_b);
-                }
+            for (int t = n * LPM; t < n * LPM + LPM; t++) {
+                if (t < NLX) { if (more_x) dma1(xrw, xbase + t * 4096, aoff[t], soff_a); }
+                else if (t < NL) { if (more_w) dma1(wrw, wbase + (t - NLX) * 4096, boff[t - NLX], soff_b); }
             }
             GL_FENCE();
         }
@@ -397,13 +407,15 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     const int ns_all = hin / GK;
     const int ns = !SPLIT ? ns_all : (ns_all - k0 < pj.ksteps ? ns_all - k0 : pj.ksteps);
     if (ns > 0) {
-        dma(smem, 0);
-        if (ns > 1) dma(smem1, 1);
-        if (ns > 2) dma(smem2, 2);
-        if (ns > 3) dma(smem3, 3);
-        GL_WAIT_LOADS(0);
+        dma_x(0);
+        dma_w(0);
+        if (ns > 1) dma_w(1);
+        if (ns > 2) { dma_x(1); dma_w(2); }
+        if (ns > 3) dma_w(3);
+        if (ns > 3) GL_WAIT_LOADS(NX + 3 * NW);    // the first step's
+        else GL_WAIT_LOADS(0);
         __syncthreads();
-        frags(smem, K0{}, fa[0], fb[0]);
+        frags(sx0, sw01, K0{}, K0{}, fa[0], fb[0]);
         int ks = 0;
 #pragma unroll 1
         for (; ks + 8 <= ns; ks += 4) {                                  // all four steps have steps ks + 4 .. behind them
@@ -422,31 +434,37 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     }
     if (ns_all * GK < hin && split == nsplit - 1) {
         // Partial last K step: through registers, with chunks of x and rows of W beyond hin replaced by zeros,
-        // parked in the same swizzled layout, in the stage after the one the last full step read (some wavefronts
-        // may still be reading that one; the one after it was released four steps ago).
-        unsigned char *st = (ns & 3) == 0 ? smem : (ns & 3) == 1 ? smem1 : (ns & 3) == 2 ? smem2 : smem3;
-        const int ncc = hin >> 3;
+        // parked in the same swizzled layout, in the stages after those that the last full step read (some wavefronts may
+        // still be reading these; the W stage was released four steps ago, and so was the half of an x stage, or it holds
+        // what was loaded past the last full step, which nothing reads).
+        unsigned char *xst = x_stage(ns >> 1), *wst = w_stage(ns);
+        const int odd = ns & 1, ncc = hin >> 3;
 #pragma unroll
-        for (int q = 0; q < MI; q++) {
-            const int row = 16 * (4 * q + wave) + (lane >> 2);
-            const int c = (lane & 3) ^ ((row >> 2) & 3);
+        for (int q = 0; q < NX; q++) {
+            const int row = 8 * (4 * q + wave) + (lane >> 3);
+            const int c = ((lane & 7) ^ ((row >> 1) & 7)) - 4 * odd;            // chunk of this step, 0 .. 3
+            if (c < 0 || c >= 4) continue;
             const bool ok = ns_all * 4 + c < ncc;
             const unsigned back = ok ? 0u : (unsigned)(ns_all * 4 + c - (ncc - 1)) * 16u;
-            const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)(aoff[q] - back), ns * (GK * 2), 0);
-            *reinterpret_cast<uint4 *>(st + (4 * q + wave) * 1024 + lane * 16) = ok ? make_uint4(v.x, v.y, v.z, v.w) : zero16();
+            const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)(aoff[q] - back), (ns >> 1) * (XK * 2), 0);
+            *reinterpret_cast<uint4 *>(xst + (4 * q + wave) * 1024 + lane * 16) = ok ? make_uint4(v.x, v.y, v.z, v.w) : zero16();
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < NW; q++) {
             const int k = ns_all * GK + 2 * (4 * q + wave) + (lane >> 5);
             const bool ok = k < hin;
             const unsigned back = ok ? 0u : (unsigned)(k - (hin - 1)) * (unsigned)hout * 2u;
             const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(wrs, (int)(boff[q] - back), (int)((unsigned)ns * GK * (unsigned)hout * 2u), 0);
-            *reinterpret_cast<uint4 *>(st + A_BYTES + (4 * q + wave) * 1024 + lane * 16) = ok ? make_uint4(v.x, v.y, v.z, v.w) : zero16();
+            *reinterpret_cast<uint4 *>(wst + (4 * q + wave) * 1024 + lane * 16) = ok ? make_uint4(v.x, v.y, v.z, v.w) : zero16();
         }
         __syncthreads();
         const int rem = hin - ns_all * GK;
-        frags(st, K0{}, fa[0], fb[0]); mfma16x(fa[0], fb[0]);
-        if (rem > 16) { frags(st, K1{}, fa[0], fb[0]); mfma16x(fa[0], fb[0]); }
+        if (odd) { frags(xst, wst, K1{}, K0{}, fa[0], fb[0]); } else { frags(xst, wst, K0{}, K0{}, fa[0], fb[0]); }
+        mfma16x(fa[0], fb[0]);
+        if (rem > 16) {
+            if (odd) { frags(xst, wst, K1{}, K1{}, fa[0], fb[0]); } else { frags(xst, wst, K0{}, K1{}, fa[0], fb[0]); }
+            mfma16x(fa[0], fb[0]);
+        }
     }
     __syncthreads();                               // every wavefront is done with the stages
 #undef GL_FENCE
@@ -485,8 +503,8 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 if (q >= nrun) continue;
-                unsigned char *stage = q == 0 ? smem : q == 1 ? smem1 : q == 2 ? smem2 : smem3;
-                const unsigned lbase = (unsigned)(__UINTPTR_TYPE__)(lds_byte *)stage + (unsigned)wave * 1024u;
+                unsigned char *stage = q == 0 ? sx0 : q == 1 ? sx1 : q == 2 ? sw01 : sw23;
+                const unsigned lbase = lds_of(stage);
 #pragma unroll
                 for (int u = 0; u < RMAX / 8; u++) b_rows_load(b_row_of(q, u), u, lbase);
             }
@@ -501,7 +519,7 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     if (q >= nrun || R0 + 32 <= i0[q] || R0 >= i1[q]) continue;       // uniform per wavefront
-                    const unsigned char *stage = q == 0 ? smem : q == 1 ? smem1 : q == 2 ? smem2 : smem3;
+                    const unsigned char *stage = q == 0 ? sx0 : q == 1 ? sx1 : q == 2 ? sw01 : sw23;
                     const unsigned keep = (my >= i0[q] && my < i1[q]) ? 0xffffffffu : 0u;
                     uint4 bf[2][4];                 // W-side operands, one slice ahead
                     w_frags(stage, 0, bf[0]);
@@ -558,7 +576,7 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     // The tile is private to the wavefront and LDS operations of one wavefront complete in order, so no
     // barrier is needed; the accesses are volatile so that they stay in program order.
     {
-        unsigned char *so = wave == 0 ? smem : wave == 1 ? smem1 : wave == 2 ? smem2 : smem3;
+        unsigned char *so = (wave < 2 ? sw01 : sw23) + (wave & 1) * B_BYTES;
         typedef __attribute__((address_space(3))) volatile uint16_t lds_vu16;
         typedef __attribute__((address_space(3))) volatile u32x4_t lds_vu32x4;
         uint16_t *__restrict__ y = static_cast<uint16_t *>(pj.y);
@@ -650,7 +668,8 @@ int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out)
                 const int ns = a.pr[q].hin / GK > 0 ? a.pr[q].hin / GK : 1;
                 int n = k == 1 ? 1 : (ns + target / 2) / target;
                 n = n < 1 ? 1 : n;
-                const int per = (ns + n - 1) / n;
+                int per = (ns + n - 1) / n;
+                if (n > 1) per += per & 1;                                      // a range starts at a whole 128-byte line of x
                 n = (ns + per - 1) / per;                                       // no range is empty
                 cand.nsplit[q] = n;
                 cand.ksteps[q] = per;
