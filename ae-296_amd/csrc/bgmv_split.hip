@@ -560,21 +560,24 @@ __device__ __forceinline__ float group_sum(float v)
 
 // Expand on the reference's layout: B is given as one [hout, R] block per adapter and layer (wb_T_all of
 // lightllm/models/lora_gpu.py:34,37,40), i.e. the R values of an output column lie next to each other and the
-// columns of a slice form one contiguous run.  A workgroup walks its 2048-column slice in sub-tiles of 256
-// columns: the sub-tile's run of 256 * R values is read with fully coalesced 16-byte loads (chunk q = 256 i + t
-// holds 8 ranks of column q / (R / 8)), every lane multiplies its 8 ranks with the matching 8 intermediates of
-// each token, the R / 8 lanes of a column are added with DPP moves, and the sums pass through LDS so that y is
-// updated with 16-byte, row-contiguous accesses.  The next sub-tile's loads are in flight during the arithmetic.
+// columns of a slice form one contiguous run.  A workgroup takes a run of 32 KiB (2048 columns at rank 8, 256 at rank 64):
+// chunk q = 256 i + t of the run holds 8 ranks of column q / (R / 8), every lane multiplies its 8 ranks with the matching
+// 8 intermediates of each token, the R / 8 lanes of a column are added with DPP moves, and the sums pass through LDS so
+// that y is updated with 16-byte, row-contiguous accesses.
+// What bounds it is how much of the run is in flight, not arithmetic: the whole of it is requested before anything is waited
+// for.  Walking 2048 columns in sub-tiles of 256 with a barrier each and one sub-tile ahead took, q / k / v of four layers
+// at hidden 4096, 256 tokens of 64 adapters, whole step: rank 16 99 us (now 91), rank 32 144 (130), rank 64 251 (227).
+constexpr int BT_CHUNKS = 8;                                    // 16-byte chunks of the run per thread
+template <int R> constexpr int BT_COLS = BT_CHUNKS * 256 * 8 / R;
 template <int DT, int G, int R, int KSC>
 __global__ __launch_bounds__(256) void bgmv_expand_bt_kernel(const BgmvArgs p)
 {
     constexpr int RMAX = R <= 16 ? 16 : (R <= 32 ? 32 : 64);   // rank stride of the shrink's partial sums
     constexpr int LPC = R / 8;                                  // lanes per column
-    constexpr int CPP = 256 / LPC;                              // columns per pass of 256 chunks
-    constexpr int SUB = 256;                                    // columns per sub-tile
-    constexpr int SLICE = 2048;                                 // columns per workgroup
+    constexpr int COLS = BT_COLS<R>;                            // columns per workgroup
+    constexpr int YQ = (G * COLS / 8 + 255) / 256;              // 16-byte pieces of y per thread
     __shared__ __attribute__((aligned(16))) float s_v[G][RMAX];
-    __shared__ __attribute__((aligned(16))) float s_out[2][G][SUB];
+    __shared__ __attribute__((aligned(16))) float s_out[G][COLS];
 
     const int tid = threadIdx.x;
     const ItemId id = split_id(blockIdx.x, p.ex_end[p.n_proj - 1]);
@@ -583,111 +586,99 @@ __global__ __launch_bounds__(256) void bgmv_expand_bt_kernel(const BgmvArgs p)
     const int cs = id.q - (proj ? p.ex_end[proj - 1] : 0);
     const int hout = p.hout[proj];
     uint16_t *__restrict__ y = static_cast<uint16_t *>(p.y[proj]);
-    const int col_begin = cs * SLICE;
-    const int col_end = col_begin + SLICE < hout ? col_begin + SLICE : hout;
-    // y rows are handled by the first G * 32 threads: thread t -> token t / 32, 8 columns from (t % 32) * 8 of the sub-tile
-    const int yk = tid >> 5, yc = (tid & 31) * 8;
-    const int part = tid % LPC;                                 // which 8 ranks of a column this lane multiplies
+    const int col0 = cs * COLS;
     const int n_ks = ((p.hin[proj] >> 3) + KSC - 1) / KSC;
 
-    const int b = id.b;
-    do {
-        const int32_t *__restrict__ rec = p.work + (size_t)b * WORK_WORDS;
-        int ntok = rec[0];
-        if (ntok <= 0) break;
-        ntok = ntok < G ? ntok : G;
-        const int adapter = rec[1];
-        int tok[G];
+    const int32_t *__restrict__ rec = p.work + (size_t)id.b * WORK_WORDS;
+    int ntok = rec[0];
+    if (ntok <= 0) return;
+    ntok = ntok < G ? ntok : G;
+    const int adapter = rec[1];
+    int tok[G];
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+        const int t = k < ntok ? rec[4 + k] : -1;
+        tok[k] = (t >= 0 && t < p.T) ? t : -1;
+    }
+    const float scale = __builtin_bit_cast(float, rec[3]) * p.pool.uniform_scale;
+    // piece n of this thread: 8 columns from yc[n] on of the row at yrow[n], -1 = none
+    long long yat[YQ];
+#pragma unroll
+    for (int n = 0; n < YQ; n++) {
+        const int e = n * 256 + tid, yk = e / (COLS / 8), c = col0 + (e - yk * (COLS / 8)) * 8;
+        int t = -1;
+#pragma unroll
+        for (int k = 0; k < G; k++) t = yk == k ? tok[k] : t;
+        yat[n] = (t >= 0 && c < hout) ? (long long)t * hout + c : -1;
+    }
+    if (adapter < 0 || adapter >= p.pool.n_adapters) {
+        if (!p.accumulate)
+#pragma unroll
+            for (int n = 0; n < YQ; n++)
+                if (yat[n] >= 0) stg16(y + yat[n], zero16());
+        return;
+    }
+    const uint16_t *__restrict__ bt = static_cast<const uint16_t *>(p.b_rows[proj]) +
+                                      (size_t)adapter * (size_t)p.ref_layers * (size_t)hout * R + (size_t)col0 * R;
+    uint4 bv[BT_CHUNKS];
+#pragma unroll
+    for (int i = 0; i < BT_CHUNKS; i++) {
+        const int q = i * 256 + tid;
+        bv[i] = col0 + q / LPC < hout ? ldg16_stream(bt + (size_t)q * 8) : zero16();
+    }
+    uint4 yv[YQ];
+#pragma unroll
+    for (int n = 0; n < YQ; n++) yv[n] = (p.accumulate && yat[n] >= 0) ? ldg16_stream(y + yat[n]) : zero16();
+
+    // v = scaling * (sum of the slices' partial sums), slices added in ascending order
+    for (int e = tid; e < G * RMAX; e += 256) {
+        const int k = e / RMAX, j = e - k * RMAX;
+        float s = 0.f;
+        if (j < R && tok[k] >= 0) {
+            const float *src = p.vws + (((size_t)proj * p.T + tok[k]) * p.ks_max) * RMAX + j;
+            for (int ks0 = 0; ks0 < n_ks; ks0 += 8) {
+                float t8[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) t8[u] = ks0 + u < n_ks ? src[(size_t)(ks0 + u) * RMAX] : 0.f;
+#pragma unroll
+                for (int u = 0; u < 8; u++) s += t8[u];
+            }
+        }
+        s_v[k][j] = s * scale;
+    }
+    __syncthreads();
+    const int part = tid % LPC;                                 // which 8 ranks of a column this lane multiplies
+    float vr[G][8];                                             // this lane's 8 intermediates of every token
+#pragma unroll
+    for (int k = 0; k < G; k++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) vr[k][e] = s_v[k][part * 8 + e];
+#pragma unroll
+    for (int i = 0; i < BT_CHUNKS; i++) {
+        float f[8];
+        unpack8<DT>(bv[i], f);
 #pragma unroll
         for (int k = 0; k < G; k++) {
-            const int t = k < ntok ? rec[4 + k] : -1;
-            tok[k] = (t >= 0 && t < p.T) ? t : -1;
+            float d = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) d = fmaf(vr[k][e], f[e], d);
+            d = group_sum<LPC>(d);
+            if (part == 0) s_out[k][(i * 256 + tid) / LPC] = d;
         }
-        int ytok = -1;
+    }
+    __syncthreads();
 #pragma unroll
-        for (int k = 0; k < G; k++) ytok = yk == k ? tok[k] : ytok;
-
-        if (adapter < 0 || adapter >= p.pool.n_adapters) {
-            if (!p.accumulate && ytok >= 0)
-                for (int c0 = col_begin; c0 < col_end; c0 += SUB)
-                    if (c0 + yc < col_end) stg16(y + (size_t)ytok * hout + c0 + yc, zero16());
-            continue;
+    for (int n = 0; n < YQ; n++)
+        if (yat[n] >= 0) {
+            const int e = n * 256 + tid, yk = e / (COLS / 8), c = (e - yk * (COLS / 8)) * 8;
+            float o[8];
+            unpack8<DT>(yv[n], o);                              // zeros when not accumulating
+            const float4_t d0 = *reinterpret_cast<const float4_t *>(&s_out[yk][c]);
+            const float4_t d1 = *reinterpret_cast<const float4_t *>(&s_out[yk][c + 4]);
+            o[0] += d0[0]; o[1] += d0[1]; o[2] += d0[2]; o[3] += d0[3];
+            o[4] += d1[0]; o[5] += d1[1]; o[6] += d1[2]; o[7] += d1[3];
+            stg16_stream(y + yat[n], pack8<DT>(o));
         }
-        const float scale = __builtin_bit_cast(float, rec[3]) * p.pool.uniform_scale;
-        const uint16_t *__restrict__ bt = static_cast<const uint16_t *>(p.b_rows[proj]) +
-                                          (size_t)adapter * (size_t)p.ref_layers * (size_t)hout * R;
-
-        uint4 bv[LPC], bn[LPC];
-        auto load_sub = [&](int c0, uint4 (&out)[LPC]) {
-            // chunk 256 i + t of the sub-tile's run: column c0 + i * CPP + t / LPC, ranks part * 8 ..
-#pragma unroll
-            for (int i = 0; i < LPC; i++) {
-                const int col = c0 + i * CPP + tid / LPC;
-                out[i] = col < col_end ? ldg16_stream(bt + (size_t)c0 * R + ((size_t)i * 256 + tid) * 8) : zero16();
-            }
-        };
-        load_sub(col_begin, bv);
-        uint4 yv = zero16();
-        if (p.accumulate && ytok >= 0 && col_begin + yc < col_end) yv = ldg16_stream(y + (size_t)ytok * hout + col_begin + yc);
-
-        // v = scaling * (sum of the slices' partial sums), slices added in ascending order
-        for (int e = tid; e < G * RMAX; e += 256) {
-            const int k = e / RMAX, j = e - k * RMAX;
-            float s = 0.f;
-            if (j < R && tok[k] >= 0) {
-                const float *src = p.vws + (((size_t)proj * p.T + tok[k]) * p.ks_max) * RMAX + j;
-                for (int ks0 = 0; ks0 < n_ks; ks0 += 8) {
-                    float t8[8];
-#pragma unroll
-                    for (int u = 0; u < 8; u++) t8[u] = ks0 + u < n_ks ? src[(size_t)(ks0 + u) * RMAX] : 0.f;
-#pragma unroll
-                    for (int u = 0; u < 8; u++) s += t8[u];
-                }
-            }
-            s_v[k][j] = s * scale;
-        }
-        __syncthreads();
-        float vr[G][8];                                             // this lane's 8 intermediates of every token
-#pragma unroll
-        for (int k = 0; k < G; k++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) vr[k][e] = s_v[k][part * 8 + e];
-
-        int buf = 0;
-#pragma unroll 1
-        for (int c0 = col_begin; c0 < col_end; c0 += SUB, buf ^= 1) {
-            const bool more = c0 + SUB < col_end;
-            if (more) load_sub(c0 + SUB, bn);
-            uint4 yn = zero16();
-            if (more && p.accumulate && ytok >= 0 && c0 + SUB + yc < col_end) yn = ldg16_stream(y + (size_t)ytok * hout + c0 + SUB + yc);
-#pragma unroll
-            for (int i = 0; i < LPC; i++) {
-                float f[8];
-                unpack8<DT>(bv[i], f);
-#pragma unroll
-                for (int k = 0; k < G; k++) {
-                    float d = 0.f;
-#pragma unroll
-                    for (int e = 0; e < 8; e++) d = fmaf(vr[k][e], f[e], d);
-                    d = group_sum<LPC>(d);
-                    if (part == 0) s_out[buf][k][i * CPP + tid / LPC] = d;
-                }
-            }
-            __syncthreads();                                        // also orders this buffer's reads of two steps ago before these writes
-            if (ytok >= 0 && c0 + yc < col_end) {
-                float o[8];
-                unpack8<DT>(yv, o);                                 // zeros when not accumulating
-                const float4_t d0 = *reinterpret_cast<const float4_t *>(&s_out[buf][yk][yc]);
-                const float4_t d1 = *reinterpret_cast<const float4_t *>(&s_out[buf][yk][yc + 4]);
-                o[0] += d0[0]; o[1] += d0[1]; o[2] += d0[2]; o[3] += d0[3];
-                o[4] += d1[0]; o[5] += d1[1]; o[6] += d1[2]; o[7] += d1[3];
-                stg16_stream(y + (size_t)ytok * hout + c0 + yc, pack8<DT>(o));
-            }
-#pragma unroll
-            for (int i = 0; i < LPC; i++) bv[i] = bn[i];
-            yv = yn;
-        }
-    } while (false);
 }
 
 // Records a launch covers (a multiple of 8, one per XCD residue): every workgroup walks records b, b + stride, ...
@@ -799,7 +790,7 @@ void bgmv_split_slices(int max_rank, int *ksc, int *nte, bool transposed_b, bool
     if (max_rank <= 16) { *ksc = Slices<16>::KSC; *nte = Slices<16>::NTE; }
     else if (max_rank <= 32) { *ksc = Slices<32>::KSC; *nte = Slices<32>::NTE; }
     else { *ksc = Slices<64>::KSC; *nte = Slices<64>::NTE; }
-    if (transposed_b) *nte = 256;              // bgmv_expand_bt_kernel walks 2048-column slices at every rank
+    if (transposed_b) *nte = BT_CHUNKS * 256 / max_rank;       // a run of 32 KiB of B (max_rank is the pool's rank)
 }
 
 template <int DT, int RMAX>
