@@ -735,7 +735,106 @@ int expand_block_cols(int n_proj, int max_tiles, int hout, int *ncb_out)
     return cols;
 }
 
-void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w)
+// K splits of a projection of `hin` columns where the narrowest of its call gets k: in proportion to the width, at least eight
+// stages of 64 columns a split, and what the workspace holds.
+int splits_of(int hin, int hin_min, int k, const SgmvWs &w)
+{
+    const int most = (hin + 511) / 512 < 8 ? (hin + 511) / 512 : 8;
+    int ks = (int)(((long long)k * hin + hin_min / 2) / hin_min);
+    ks = ks < 1 ? 1 : (ks > most ? most : ks);
+    return ks < w.ks_cap ? ks : w.ks_cap;
+}
+
+// Shape of a prefill call's shrink launch: whether a workgroup serves up to three projections of one x (share_x), the groups, and
+// the K splits.  More splits and single projections make more and shorter workgroups; fewer splits mean fewer partial
+// sums, shared x fewer lines from L2.  The rule estimates the launch for both kinds and six numbers of splits, and takes
+// the least: workgroups of known length (4 ns a 128-byte line and compute unit) are dealt, longest first, to the slots of
+// the device, but not below what all lines take together (6.4 TB/s); a split costs 0.05 ns a token and projection (written,
+// and read by the reduce launch or the expand).  Fitted to both kinds at 1, 2 and 4 splits over 46 batches of 16 to 9216
+// tokens (ranks 16 to 64; one, three, four and seven projections): the shape it names is within 5 % of the best of the six
+// everywhere and 0.5 % off on average.  Llama-7B widths, rank 64, q/k/v, two layers and the plan in a graph, single / shared
+// projections at 1, 2, 4 splits, us: 64 tokens 53, 41, 35 / 110, 67, 50; 1280 tokens 86, 81, 87 / 137, 101, 85; 6000 tokens 211,
+// 211, 229 / 232, 202, 213.
+void shrink_shape(mlora::SgmvArgs &a, int tiles, int max_rank, const SgmvWs &w)
+{
+    static const int tried[] = {1, 2, 3, 4, 6, 8};
+    const int cus = mlora::device_compute_units(), rows = max_rank <= 16 ? 16 : (max_rank <= 32 ? 32 : 64);
+    int hin_min = a.pr[0].hin;
+    for (int p = 1; p < a.n_proj; p++) hin_min = a.pr[p].hin < hin_min ? a.pr[p].hin : hin_min;
+    // up to three consecutive projections that read the same activations form a group
+    a.n_grp = 0;
+    for (int p = 0; p < a.n_proj; p++) {
+        if (p > 0 && a.pr[p].x == a.pr[p - 1].x && a.pr[p].hin == a.pr[p - 1].hin && a.grp_n[a.n_grp - 1] < 3) a.grp_n[a.n_grp - 1]++;
+        else { a.grp_first[a.n_grp] = p; a.grp_n[a.n_grp] = 1; a.n_grp++; }
+    }
+    double best = 0.0;
+    int best_k = 1;
+    for (int share = 0; share <= (a.seg_uniform_len == 0 ? 1 : 0); share++) {
+        // workgroups a unit holds, by their LDS (sh_group_bytes in sgmv_prefill.hip)
+        const long long slots = (long long)cus * (rows == 16 || (share && rows == 32) ? 2 : 1);
+        for (int t = 0; t < 6; t++) {
+            const int k = tried[t];
+            long long count[MLORA_MAX_PROJ];
+            double len[MLORA_MAX_PROJ], lines = 0.0, parts = 0.0;
+            for (int g = 0; g < a.n_grp; g++) {
+                const int hin = a.pr[a.grp_first[g]].hin, nm = a.grp_n[g], stages = (hin + 63) / 64, ks = splits_of(hin, hin_min, k, w);
+                count[g] = (long long)tiles * ks * (share ? 1 : nm);
+                len[g] = (double)((stages + ks - 1) / ks) * (64 + (share ? nm : 1) * rows);
+                lines += (double)tiles * stages * (share ? 64 + nm * rows : nm * (64 + rows));
+                if (ks > 1) parts += (double)ks * nm * a.T;
+            }
+            for (int g = 1; g < a.n_grp; g++)                                   // longest first
+                for (int r = g; r > 0 && len[r] > len[r - 1]; r--) {
+                    const double l = len[r]; len[r] = len[r - 1]; len[r - 1] = l;
+                    const long long c = count[r]; count[r] = count[r - 1]; count[r - 1] = c;
+                }
+            // dealing: slots that are free at the same time are kept together
+            double at[2 * MLORA_MAX_PROJ + 2];
+            long long n[2 * MLORA_MAX_PROJ + 2];
+            int nb = 1;
+            at[0] = 0.0; n[0] = slots;
+            double end = 0.0;
+            for (int g = 0; g < a.n_grp; g++) {
+                long long c = count[g];
+                const long long full = c / slots;                               // whole rounds over all slots
+                if (full > 0) { for (int i = 0; i < nb; i++) at[i] += full * len[g]; c -= full * slots; }
+                while (c > 0) {
+                    int first = 0;
+                    for (int i = 1; i < nb; i++) if (at[i] < at[first]) first = i;
+                    const long long m = n[first] < c ? n[first] : c;
+                    const double till = at[first] + len[g];
+                    n[first] -= m;
+                    c -= m;
+                    int same = -1;
+                    for (int i = 0; i < nb; i++) if (at[i] == till) same = i;
+                    if (same >= 0) n[same] += m;
+                    else if (n[first] == 0) { at[first] = till; n[first] = m; }
+                    else { at[nb] = till; n[nb] = m; nb++; }
+                    if (n[first] == 0 && first < nb) { nb--; at[first] = at[nb]; n[first] = n[nb]; }
+                }
+            }
+            for (int i = 0; i < nb; i++) if (n[i] > 0 && at[i] > end) end = at[i];
+            double us = 0.004 * end;
+            const double all = 2e-5 * lines;
+            us = (us > all ? us : all) + 5e-5 * parts;
+            if ((share == 0 && t == 0) || us < best) { best = us; best_k = k; a.share_x = share; }
+        }
+    }
+    for (int p = 0; p < a.n_proj; p++) a.pr[p].ksplit = splits_of(a.pr[p].hin, hin_min, best_k, w);
+    // longest workgroups first
+    auto length = [&](int g) {
+        const mlora::SgmvProj &pj = a.pr[a.grp_first[g]];
+        return ((pj.hin + 63) / 64 + pj.ksplit - 1) / pj.ksplit * (64 + (a.share_x ? a.grp_n[g] : 1) * rows);
+    };
+    for (int g = 1; g < a.n_grp; g++)
+        for (int r = g; r > 0 && length(r) > length(r - 1); r--) {
+            const int f = a.grp_first[r], n = a.grp_n[r];
+            a.grp_first[r] = a.grp_first[r - 1]; a.grp_n[r] = a.grp_n[r - 1];
+            a.grp_first[r - 1] = f; a.grp_n[r - 1] = n;
+        }
+}
+
+void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w, int max_rank)
 {
     char *base = static_cast<char *>(workspace);
     int32_t *ip = reinterpret_cast<int32_t *>(base);
@@ -744,32 +843,28 @@ void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w)
     a.tok_cover = reinterpret_cast<int32_t *>(base + w.off_cover);
     a.tile_rec = reinterpret_cast<int32_t *>(base + w.off_rec);
     a.max_tiles = w.max_tiles;
-    int hin_min = a.pr[0].hin;
-    for (int p = 1; p < a.n_proj; p++) hin_min = a.pr[p].hin < hin_min ? a.pr[p].hin : hin_min;
+    const int tiles = a.seg_uniform_len > 0 ? a.n_seg * ((a.seg_uniform_len + SG_TM - 1) / SG_TM) : (a.T + SG_TM / 2 * (a.n_seg - 1) + SG_TM - 1) / SG_TM;
+    a.tiles = tiles;
     for (int p = 0; p < a.n_proj; p++) {
         char *pb = base + w.off_proj + w.per_proj * p;
         a.pr[p].v = reinterpret_cast<float *>(pb);
         a.pr[p].vhi = reinterpret_cast<uint16_t *>(pb + w.off_hi);
         a.pr[p].vlo = reinterpret_cast<uint16_t *>(pb + w.off_lo);
-        int ks = (int)(((long long)w.ksplit * a.pr[p].hin + hin_min / 2) / (hin_min > 0 ? hin_min : 1));
-        ks = ks < w.ksplit ? w.ksplit : (ks > w.ks_cap ? w.ks_cap : ks);
-        const int nst = (a.pr[p].hin + 127) / 128;             // stages of the shrink: more splits than that would be empty
-        a.pr[p].ksplit = ks < nst ? ks : nst;
         int ncb = 0;
         const int cols = expand_block_cols(a.n_proj, w.max_tiles, a.pr[p].hout, &ncb);
         a.pr[p].cols = cols;
         a.pr[p].ncb = ncb;
     }
-    // shrink groups: up to three consecutive projections that read the same activations (one workgroup serves a group).
-    // A launch that leaves the chip half empty keeps them apart: x comes from L2 then, and three times as many
-    // workgroups share the work (three projections at rank 64, together / apart: 64 tokens 25.6 / 19.7 us a call, 1024
-    // tokens 41 / 36; four prompts of 512 52 / 52; seven projections, eight prompts of 100 tokens 76 / 83).
-    const bool share_x = (long long)w.max_tiles * a.n_proj * w.ksplit >= 704;
-    a.n_grp = 0;
-    for (int p = 0; p < a.n_proj; p++) {
-        if (p > 0 && share_x && a.pr[p].x == a.pr[p - 1].x && a.pr[p].hin == a.pr[p - 1].hin && a.grp_n[a.n_grp - 1] < 3) a.grp_n[a.n_grp - 1]++;
-        else { a.grp_first[a.n_grp] = p; a.grp_n[a.n_grp] = 1; a.n_grp++; }
-    }
+    shrink_shape(a, tiles, max_rank, w);
+    // Whether x is read with the streaming hint: what a small call leaves in the last-level cache the next call on it finds there
+    // (the reference's q, k, v calls, single projections), what a large call leaves there only pushes other things out.
+    // Rank 64, states of three batches in turn, ordinary / streaming, us: the reference's three calls, x and y of a call
+    // 92 MB 106 / 108, 109 MB 126 / 122, 134 MB 141 / 126; q, k, v, o 197 MB 79 / 86, 295 MB 117 / 115; seven projections
+    // 210 MB 109 / 105, 525 MB 221 / 210.
+    long long bytes = 0;
+    for (int g = 0; g < a.n_grp; g++) bytes += (long long)a.T * a.pr[a.grp_first[g]].hin * 2;
+    for (int p = 0; p < a.n_proj; p++) bytes += (long long)a.T * a.pr[p].hout * 2;
+    a.stream_x = bytes > (a.n_proj == 1 ? 100000000LL : 200000000LL);
 }
 
 }  // namespace
@@ -838,7 +933,7 @@ static int sgmv_common(int n_proj, void *const *y, const void *const *x, const v
         return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)w.total);
     a.seg_start = seg_start; a.seg_len = seg_len; a.seg_adapter = seg_adapter; a.n_seg = n_seg;
     a.T = T; a.accumulate = accumulate ? 1 : 0; a.b_transposed = 0; a.seg_uniform_len = 0; a.tile_aligned = tile_aligned;
-    carve(a, workspace, w);
+    carve(a, workspace, w, max_rank);
     rc = mlora::launch_sgmv(a, dtype, max_rank, phases, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "sgmv launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;
@@ -987,7 +1082,7 @@ int mlora_gemm_lora_split(int n_proj, void *const *y, const void *const *x, cons
             return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)ws.total);
         a.seg_start = seg_start; a.seg_len = seg_len; a.seg_adapter = seg_adapter; a.n_seg = n_seg;
         a.T = T; a.accumulate = 0; a.b_transposed = 0; a.seg_uniform_len = 0;
-        carve(a, workspace, ws);
+        carve(a, workspace, ws, max_rank);
         rc = mlora::launch_sgmv(a, dtype, max_rank, mlora::SGMV_SHRINK, static_cast<hipStream_t>(stream));
         if (rc) return fail(MLORA_ELAUNCH, "shrink launch failed: %s", hipGetErrorString((hipError_t)rc));
         for (int p = 0; p < n_proj; p++) {
@@ -1036,7 +1131,7 @@ int mlora_prefill_reflayout(void *y, const void *x, const void *A_T, const void 
     a.pr[0].b_rows = static_cast<const uint16_t *>(B_T) + (size_t)layer_idx * hout * r;
     a.pr[0].hin = hin; a.pr[0].hout = hout;
     a.n_seg = B; a.T = T; a.accumulate = 0; a.b_transposed = 1; a.seg_uniform_len = Lpad;
-    carve(a, workspace, w);
+    carve(a, workspace, w, r);
     a.max_tiles = B * ((Lpad + SG_TM - 1) / SG_TM);
     rc = mlora::launch_sgmv(a, dtype, r, mlora::SGMV_PLAN | mlora::SGMV_APPLY, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "prefill launch failed: %s", hipGetErrorString((hipError_t)rc));

@@ -71,6 +71,7 @@ __global__ __launch_bounds__(256) void gemm_lora_reduce_kernel(const GemmLoraArg
     const int tile = blockIdx.x;
     if (tile >= p.n_tiles[0]) return;
     const GemmProj &pj = p.pr[blockIdx.y];
+    if (pj.ksplit == 1) return;                    // the shrink stored the halves itself
     const int32_t *__restrict__ rec = p.tile_rec + (size_t)tile * TILE_WORDS;
     const int ntok = rec[0], adapter = rec[1], tok0 = rec[4];
     if (adapter < 0 || ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
@@ -725,7 +726,9 @@ static int launch_gl(const GemmLoraArgs &a, hipStream_t s)
     }
     if (end == 0) return 0;
     int rc = 0;
-    if (g.lora) {
+    bool partial_v = false;
+    for (int q = 0; q < g.n_proj; q++) partial_v = partial_v || g.pr[q].ksplit > 1;
+    if (g.lora && partial_v) {
         hipLaunchKernelGGL((gemm_lora_reduce_kernel<DT, RMAX>), dim3((unsigned)g.max_tiles, (unsigned)g.n_proj), dim3(256), 0, s, g);
         rc = (int)hipGetLastError();
         if (rc) return rc;

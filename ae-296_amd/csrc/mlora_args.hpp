@@ -130,9 +130,10 @@ struct SgmvProj {
 struct SgmvArgs {
     SgmvProj pr[MAX_PROJ];
     int n_proj;
-    // Shrink launch: up to three consecutive projections that read the same x form a group, served by one
-    // workgroup per (tile, K split): x comes from HBM once per group and is multiplied with every member's A.
-    // grp_end[g] = first workgroup id after group g.
+    // Shrink launch: up to three consecutive projections that read the same x form a group, served by one workgroup per
+    // (tile, K split) where share_x is set and by neighbouring ones otherwise.  grp_end[g] = first workgroup id after group g.
+    int share_x;
+    int stream_x;          // x by streaming loads
     int n_grp;
     int grp_first[MAX_PROJ], grp_n[MAX_PROJ];
     unsigned grp_end[MAX_PROJ];
@@ -146,6 +147,7 @@ struct SgmvArgs {
     int accumulate;
     int b_transposed;      // B given as [hout, r] blocks (reference layout)
     int seg_uniform_len;   // > 0: segment s covers [s*len, (s+1)*len), adapter s (reference prefill)
+    int scaled;            // shrink with one K split: store the halves of scaling * sum (set by the launcher)
     int fold;              // expand: sum the K splits itself instead of reading what the reduce launch made (set by the launcher)
     int tile_aligned;      // plan: cut tiles at multiples of 64 tokens (and at segment ends) instead of every 64 tokens of a segment
     // workspace carve-up
@@ -156,6 +158,7 @@ struct SgmvArgs {
     int32_t *tok_cover;    // [T] 1 where a token belongs to a tile (written by the plan): rows of y = delta mode outside are zeroed
     int32_t *tile_rec;     // [max_tiles * TILE_WORDS] per-tile records (layout below)
     int max_tiles;
+    int tiles;             // about how many are in use (the host's estimate: decides launch shapes, never what is computed)
 };
 
 // One projection of a base GEMM + LoRA call.

@@ -162,6 +162,27 @@ __device__ __forceinline__ void sum_splits_any(const float *__restrict__ src, si
     else sum_splits<16>(src, stride, n, v);
 }
 
+// Four neighbouring partial sums over up to eight K splits, in ascending order, the loads of all splits in one batch.
+template <int U>
+__device__ __forceinline__ void sum_splits4_of(const float *__restrict__ src, size_t stride, int n, float (&v)[4])
+{
+    float4_t a[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) a[u] = *reinterpret_cast<const float4_t *>(src + (size_t)(u < n ? u : 0) * stride);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        v[e] = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; u++) v[e] += u < n ? a[u][e] : 0.f;
+    }
+}
+__device__ __forceinline__ void sum_splits4(const float *__restrict__ src, size_t stride, int n, float (&v)[4])
+{
+    if (n <= 2) sum_splits4_of<2>(src, stride, n, v);
+    else if (n <= 4) sum_splits4_of<4>(src, stride, n, v);
+    else sum_splits4_of<8>(src, stride, n, v);
+}
+
 // Sum over each aligned group of 16 lanes (a DPP "row"); every lane of the row gets the sum.
 __device__ __forceinline__ float row16_sum(float v)
 {

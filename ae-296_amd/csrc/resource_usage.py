@@ -13,7 +13,8 @@ the limits below.  The limits say what the kernels were designed around:
   32-row blocks keeps 64 MI of them and may move 320 MI times (the epilogue reads 256 MI; at -O1 400, 704 and 1008);
 * the decode shrink of a one-round launch needs at least four (rank <= 16) or three (rank 32) workgroups per
   compute unit, the expand three;
-* M0 in `gemm_lora_kernel` and `gemm_lora_short_kernel` is written only by the kernel's own LDS-bound loads: one
+* the prefill shrink keeps a workgroup of eight wavefronts, or one of four that shares x, on a compute unit (more up to rank 32);
+* M0 in `gemm_lora_kernel`, `gemm_lora_short_kernel` and `sgmv_shrink_kernel` is written only by the kernel's own LDS-bound loads: one
   `s_mov_b32 m0` per such load and no other instruction that names M0.
 """
 from __future__ import annotations
@@ -41,8 +42,10 @@ LIMITS = [
     ("bgmv_split.hip", r"bgmv_expand_kernel<\d, [124], 32, 128, 128, false>", {"occupancy": (3, 8)}),
     ("bgmv_decode.hip", r".", {"scratch": (0, 0), "vgpr_spill": (0, 0)}),
     ("sgmv_prefill.hip", r".", {"scratch": (0, 0), "vgpr_spill": (0, 0)}),
-    ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, (16|32), \d, (true|false)>", {"occupancy": (3, 8)}),
-    ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, 64, \d, (true|false)>", {"occupancy": (2, 8)}),
+    ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, 16, (true|false), false>", {"occupancy": (4, 8), "lds": (0, 80 * 1024)}),
+    ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, (32|64), (true|false), false>", {"occupancy": (2, 8), "lds": (0, 160 * 1024)}),
+    ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, (16|32), false, true>", {"occupancy": (2, 8), "lds": (0, 80 * 1024)}),
+    ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, 64, false, true>", {"occupancy": (1, 8), "lds": (0, 160 * 1024)}),
 ]
 
 FIELDS = {"TotalSGPRs": "sgprs", "VGPRs": "vgprs", "AGPRs": "agprs", "ScratchSize [bytes/lane]": "scratch",
@@ -84,7 +87,7 @@ def parse_asm(text: str, kernels):
         code = [ln.strip() for ln in body if ln.strip() and not ln.strip().startswith(".")]
         rec["accvgpr_moves"] = sum(1 for ln in code if ln.startswith("v_accvgpr_"))
         rec["scratch_insts"] = sum(1 for ln in code if ln.startswith("scratch_"))
-        rec["lds_loads"] = sum(1 for ln in code if ln.startswith("buffer_load") and ln.endswith(" lds"))
+        rec["lds_loads"] = sum(1 for ln in code if (ln.startswith("buffer_load") and ln.endswith(" lds")) or ln.startswith("global_load_lds"))
         rec["m0_writes"] = sum(1 for ln in code if re.match(r"s_mov_b32 m0, ", ln))
         rec["m0_other"] = sum(1 for ln in code if re.search(r"\bm0\b", ln) and not re.match(r"s_mov_b32 m0, ", ln))
     return kernels
@@ -129,10 +132,11 @@ def violations(source: str, report):
                 for field, lo, hi in (("agprs", 64 * mi, 64 * mi), ("accvgpr_moves", 0, 320 * mi)):
                     if not lo <= rec.get(field, -1) <= hi:
                         bad.append(f"{source}: {name}: {field} = {rec.get(field)}, allowed {lo}..{hi}")
-            if re.search(r"gemm_lora_(short_)?kernel<", name):
-                if rec.get("m0_other", 1) != 0 or rec.get("m0_writes", 0) != rec.get("lds_loads", -1):
-                    bad.append(f"{source}: {name}: M0 is named by {rec.get('m0_other')} instructions besides its "
-                               f"{rec.get('m0_writes')} writes, for {rec.get('lds_loads')} LDS-bound loads")
+    for name, rec in report.items():
+        if re.search(r"gemm_lora_(short_)?kernel<|sgmv_shrink_kernel<", name):
+            if rec.get("m0_other", 1) != 0 or rec.get("m0_writes", 0) != rec.get("lds_loads", -1):
+                bad.append(f"{source}: {name}: M0 is named by {rec.get('m0_other')} instructions besides its "
+                           f"{rec.get('m0_writes')} writes, for {rec.get('lds_loads')} LDS-bound loads")
     return bad
 
 

@@ -2,13 +2,13 @@
 //     y[t] (+)= s_a * (x[t] . A_a) . B_a
 // computed on v_mfma_f32_16x16x32_{f16,bf16} tiles in three or four launches on one stream (the first can be shared by all projections and layers of a batch):
 //   plan   : cuts every segment into tiles of at most 64 tokens (work list in the workspace);
-//   shrink : V[split][t][0..R) = x[t, Kslice] . A_a[:, Kslice]^T   (split-K, fp32 partials);
-//   reduce : sums the K splits and stores the result as a hi + lo pair of 16-bit values, so
-//            the intermediate keeps fp32 accuracy through the second MFMA (up to rank 32 and eight
-//            splits the expand does this itself where y accumulates);
+//   shrink : V[split][t][0..R) = x[t, Kslice] . A_a[:, Kslice]^T   (split-K, fp32 partials), or with one
+//            split the result itself as a hi + lo pair of 16-bit values, so that the intermediate keeps
+//            fp32 accuracy through the second MFMA;
+//   reduce : sums the K splits into such pairs (up to rank 32 the expand does this itself where y accumulates; with one split there is nothing to do);
 //   expand : y[t, cols] (+)= s_a * (Vhi + Vlo) . B_a[:, cols].
-// Both MFMA operands of the shrink are read straight from global memory in operand layout
-// (8 contiguous K values per lane).  The expand parks the B tile in LDS (rank must be the
+// Both MFMA operands of the shrink pass through a ring of LDS stages that global memory fills directly.
+// The expand parks the B tile in LDS (rank must be the
 // in-lane K dimension, the pool stores rank rows), reads it back with the transposing LDS read,
 // and passes the output through a wavefront-private LDS tile so that every y access is a
 // 16-byte, row-contiguous one (8-byte accesses straight from the accumulators were measured slower).
@@ -16,6 +16,7 @@
 // Replaces torch.bmm(torch.bmm(x, A), B) at lightllm/models/lora_gpu.py:127-128,145-146,157-158.
 #include "mlora_args.hpp"
 #include "mlora_dev.hpp"
+#include <type_traits>
 
 namespace mlora {
 
@@ -51,13 +52,15 @@ __device__ __forceinline__ void seg_of(const SgmvArgs &p, int s, int &start, int
 // run that have the same second index read the same slice of A (or B): they are given ids with the same
 // residue mod 8, i.e. one XCD, and the residue rotates with the second index so the XCDs stay balanced.
 constexpr int XRUN = 8;
-__device__ __forceinline__ bool xcd_remap(int w, int n_second, int &tile, int &second)
+// So does `rot`, from one group of projections to the next: tiles are rarely a multiple of 64, and the XCDs with a run more
+// than the others would be the same ones every time.
+__device__ __forceinline__ bool xcd_remap(int w, int n_second, int rot, int &tile, int &second)
 {
     const int r = w & 7, slot = w >> 3;
     const int i = slot % XRUN;
     second = (slot / XRUN) % n_second;
     const int j = slot / (XRUN * n_second);
-    const int run = ((r - second) & 7) + 8 * j;
+    const int run = ((r - second - rot) & 7) + 8 * j;
     tile = run * XRUN + i;
     return true;
 }
@@ -71,10 +74,10 @@ __host__ __device__ inline long long xcd_grid(int max_tiles, int n_second)
 // batch of a tile or two without work (512 workgroups for 8 at one tile and eight splits), and what runs together
 // is everything anyway.
 __host__ __device__ inline bool few_tiles(int max_tiles) { return max_tiles < XRUN * 8; }
-__device__ __forceinline__ void place(int w, int n_second, int max_tiles, int &tile, int &second)
+__device__ __forceinline__ void place(int w, int n_second, int max_tiles, int rot, int &tile, int &second)
 {
     if (few_tiles(max_tiles)) { tile = w / n_second; second = w - tile * n_second; }
-    else xcd_remap(w, n_second, tile, second);
+    else xcd_remap(w, n_second, rot, tile, second);
 }
 __host__ __device__ inline long long place_grid(int max_tiles, int n_second)
 {
@@ -239,158 +242,255 @@ __device__ __forceinline__ float4_t mfma16(const uint4 &a, const uint4 &b, float
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf168_t, a), __builtin_bit_cast(bf168_t, b), c, 0, 0, 0);
 }
 
-constexpr int SG_NM = 3;     // projections of one x that a shrink workgroup serves at most (a larger group is cut by the host)
+constexpr int SG_NM = 3;                    // projections of one x that a shrink workgroup serves at most (a larger group is cut by the host)
+constexpr int SH_CH = 8;                    // 16-byte chunks of a stage row: one 128-byte line
+constexpr int SH_ROWB = SH_CH * 16;
+// How a workgroup is built: SHARE: four wavefronts, up to SG_NM projections; otherwise KG groups of four, one projection,
+// each group with its own half of the K range and its own ring.
+template <bool SHARE> constexpr int SH_KG = SHARE ? 1 : 2;
+// LDS of a group's ring: four stages of the most rows (more of fewer rows)
+template <int RMAX, bool SHARE> constexpr int sh_group_bytes() { return 4 * (TM + (SHARE ? SG_NM : 1) * RMAX) * SH_ROWB; }
 
-// NM: the largest group of the launch (1 or SG_NM), which sizes the LDS: at rank 64 a launch whose groups are single
-// projections fits four workgroups on a unit instead of two.
-template <int DT, int RMAX, int NM, bool UNIFORM>
-__global__ __launch_bounds__(SG_NT) void sgmv_shrink_kernel(const SgmvArgs p)
+// hi + lo 16-bit halves of N values (hi = round16(v), lo = round16(v - hi)), packed in pairs.
+template <int DT, int N>
+__device__ __forceinline__ void split_hi_lo(const float (&v)[N], uint32_t (&hi)[N / 2], uint32_t (&lo)[N / 2])
 {
-    // One workgroup: 64 tokens x RMAX ranks over one K slice, for every projection of its group (up to SG_NM
-    // projections that read the same x: q, k, v; gate, up).  A stage is 128 columns: the X tile (64 rows x 256 B)
-    // and one A tile per projection (RMAX rows x 256 B) are read with 16-byte loads in which every 16-lane row
-    // covers 256 contiguous bytes, parked in LDS, and consumed from there as MFMA operands (8 contiguous K
-    // values per lane); the X operand of a step is read from LDS once and multiplied with every projection's A.
-    // The next stage's loads are in flight while this one computes.  x is fetched once per group (streaming).
-    constexpr int NB = RMAX / 16;            // rank blocks of 16
-    constexpr int KB = 128;                  // columns per stage
-    constexpr int CPR = KB / 8;              // 16-byte chunks per row and stage
-    constexpr int PITCH = KB * 2 + 32;       // LDS row pitch in bytes; the padding spreads the operand reads over the banks
-                                             // (measured: no padding 2x slower, 16 bytes 6 % slower than 32, 48..144 slower again)
-    constexpr int XP = TM * CPR / SG_NT;     // X loads per thread and stage (4)
-    constexpr int AP = (RMAX * CPR + SG_NT - 1) / SG_NT;   // A loads per thread, projection and stage (1, 2 or 4)
-    __shared__ __attribute__((aligned(16))) unsigned char s_x[TM * PITCH];
-    __shared__ __attribute__((aligned(16))) unsigned char s_a[NM][RMAX * PITCH];
+    uint32_t h[N], l[N];
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+        h[e] = cvt16<DT>(v[e]);
+        const float back = lo_f32<DT>(h[e]);
+        l[e] = cvt16<DT>(v[e] - back);
+    }
+#pragma unroll
+    for (int e = 0; e < N / 2; e++) { hi[e] = h[2 * e] | (h[2 * e + 1] << 16); lo[e] = l[2 * e] | (l[2 * e + 1] << 16); }
+}
+
+// One workgroup: 64 tokens x RMAX ranks over one K range, for one projection, or (SHARE) for up to SG_NM projections that
+// read the same x.  A stage is 64 columns of the x rows and of every projection's A rows; global memory fills a ring of stages
+// in LDS directly (global_load_lds, whole lines), so that three or more stages are in flight while one is multiplied.  A
+// wavefront takes half of the tokens and half of the ranks (at rank 16 a quarter of the tokens).
+// What bounds it is the lines a compute unit can have on their way (some hundred, whatever the kernel asks for) times how
+// long they take: 11 million lines of 735 cycles for sixteen ragged prompts of Llama-13B, 9216 tokens, of which the A rows of
+// every tile are more than half.  Staging a stage in registers, with the next one requested only when it had been parked in LDS,
+// and every wavefront reading all of A back (4 KiB of LDS reads a column for three projections; now 2): that batch 189 us
+// (now 176), 16 x 512 tokens of one projection at rank 64 19.5 us (15.3), one prompt of 64 tokens, three projections, 7.0 us
+// (6.0).  Reading operands straight from global memory, 64 bytes a row and load, took 328 and 21 us.
+template <int DT, int RMAX, bool UNIFORM, bool SHARE>
+__global__ __launch_bounds__(SG_NT *SH_KG<SHARE>) void sgmv_shrink_kernel(const SgmvArgs p)
+{
+    constexpr int KG = SH_KG<SHARE>;
+    constexpr int NB = RMAX / 16;                               // rank blocks of 16
+    constexpr int WT = NB >= 2 ? 2 : 4;                         // wavefronts along the tokens, the others along the ranks
+    constexpr int TBW = TM / 16 / WT, NBW = NB * WT / 4;        // 16 x 16 blocks per wavefront and projection
+    constexpr int GROUP_BYTES = sh_group_bytes<RMAX, SHARE>();
+    constexpr int CH = SH_CH, ROWB = SH_ROWB;
+    constexpr int RPL = 1024 / ROWB;                            // rows one load of a wavefront fills
+    __shared__ __attribute__((aligned(16))) unsigned char s_ring[KG * GROUP_BYTES];
     int grp = 0;
     while (grp + 1 < p.n_grp && blockIdx.x >= p.grp_end[grp]) grp++;
+    // SHARE: a workgroup per (tile, split) of a group; otherwise one per projection, the projections of a group being the
+    // fastest index, so that they run side by side on one XCD and find x in its L2
     int tile, split;
-    const int nm = p.grp_n[grp] < NM ? p.grp_n[grp] : NM;       // projections this workgroup serves
-    place((int)(blockIdx.x - (grp ? p.grp_end[grp - 1] : 0u)), p.pr[p.grp_first[grp]].ksplit, p.max_tiles, tile, split);
-    const int p0 = p.grp_first[grp];
+    const int w = (int)(blockIdx.x - (grp ? p.grp_end[grp - 1] : 0u)), ng = SHARE ? 1 : p.grp_n[grp];
+    const bool few = few_tiles(p.max_tiles);
+    const int wq = few ? w / ng : (w >> 3) / ng * 8 + (w & 7);
+    const int p0 = p.grp_first[grp] + (few ? w - wq * ng : (w >> 3) % ng);
+    const int nm = SHARE ? p.grp_n[grp] : 1;
     const SgmvProj &pj = p.pr[p0];
+    place(wq, pj.ksplit, p.max_tiles, grp * 3, tile, split);
     if (tile >= p.max_tiles) return;                            // records beyond the tiles in use hold no tokens
     const Tile<UNIFORM> tl = tile_of<UNIFORM>(p, tile);
     const int ntok = tl.ntok, tok0 = tl.tok0;
     if (tl.adapter < 0 || ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = wave_all >> 2, wave = wave_all & 3;
     const int m = lane & 15, g = lane >> 4;
-
     const int hin = pj.hin;
-    const uint16_t *__restrict__ x = static_cast<const uint16_t *>(pj.x);
-    const int lrow = tid >> 4, lchk = tid & 15;                // this thread's row (per pass of 16) and chunk
-    const uint4 *xp[XP];
-#pragma unroll
-    for (int q = 0; q < XP; q++) {
-        int t = lrow + 16 * q;
-        t = t < ntok ? t : ntok - 1;                            // tail rows repeat the last token; never stored
-        xp[q] = reinterpret_cast<const uint4 *>(x + (size_t)(tok0 + t) * hin);
-    }
-    const uint4 *ap[NM][AP];
-#pragma unroll
-    for (int mm = 0; mm < NM; mm++) {
-        const uint16_t *arows = static_cast<const uint16_t *>(p.pr[p0 + (mm < nm ? mm : 0)].a_rows);
-#pragma unroll
-        for (int q = 0; q < AP; q++) {
-            const int j = lrow + 16 * q;
-            const int row = j < RMAX ? tl.row(j, p.pool.n_rows_a) : -1;
-            ap[mm][q] = reinterpret_cast<const uint4 *>(arows + (size_t)(row >= 0 ? row : 0) * hin);
-        }
-    }
-    float4_t acc[NM][NB];
-#pragma unroll
-    for (int mm = 0; mm < NM; mm++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) acc[mm][nb] = float4_t{0.f, 0.f, 0.f, 0.f};
-
     const int ncc = hin >> 3;                                   // 16-byte chunks per row
-    const int nstage = (ncc + CPR - 1) / CPR;
+    const int whole = ncc / CH, nstage = (ncc + CH - 1) / CH;   // full stages, stages
     const int per = (nstage + pj.ksplit - 1) / pj.ksplit;
-    const int st0 = split * per;
-    const int st1 = st0 + per < nstage ? st0 + per : nstage;
-    uint4 xr[XP], ar[NM][AP];
-    auto load_stage = [&](int st) {
-        const int c = st * CPR + lchk;
-        const bool ok = c < ncc;                                // K tail: both operands become zero
-        const int cs = ok ? c : ncc - 1;
+    const int st0 = split * per < whole ? split * per : whole, st1 = st0 + per < whole ? st0 + per : whole;
+    const int half = (st1 - st0 + KG - 1) / KG;                 // every group walks this many steps, the last one may have fewer stages
+    const int g0 = st0 + kg * half < st1 ? st0 + kg * half : st1;
+    const int n = st1 - g0 < half ? st1 - g0 : half;
+    const bool tail = whole < nstage && split == whole / per;   // this range ends with a stage of fewer columns
+    unsigned char *ring = s_ring + kg * GROUP_BYTES;
+    typedef __attribute__((address_space(3))) unsigned char lds_byte;
+    const unsigned ring_at = (unsigned)(__UINTPTR_TYPE__)(lds_byte *)ring;
+
+    auto run = [&](auto nm_tag) {
+        constexpr int NM = decltype(nm_tag)::value;
+        constexpr int ROWS = TM + NM * RMAX, STAGE = ROWS * ROWB;
+        constexpr int D = GROUP_BYTES / STAGE < 8 ? GROUP_BYTES / STAGE : 8;            // stages of the ring
+        constexpr int XU = TM / RPL / 4, AI = NM * RMAX / RPL, AU = (AI + 3) / 4, NL = XU + AU;
+        static_assert(D >= 3 && NL * (D - 2) < 64, "the ring and the load counter");
+        // One load of a wavefront fills RPL rows of a stage (1 KiB): lane i row i / CH, slot i % CH.  Chunk c of row r is stored
+        // in slot c ^ key(r): 16 operand rows of one chunk column then lie in 16 different bank groups.
+        // Rows past the tile's tokens repeat the last one, absent rank rows read row 0; neither is stored.
+        auto key = [](int r) { return (r >> 1) & 7; };
+        const char *src[NL];
+        unsigned dst[NL];
 #pragma unroll
-        for (int q = 0; q < XP; q++) {
-            xr[q] = ldg16_stream(xp[q] + cs);                   // x passes through once per group
-            if (!ok) xr[q] = zero16();
+        for (int u = 0; u < NL; u++) {
+            const int i = u < XU ? wave + 4 * u : (wave + 4 * (u - XU) < AI ? wave + 4 * (u - XU) : wave + 4 * (u - XU) - AI);
+            const int r = i * RPL + lane / CH;                  // row of the x tile, or of the A tiles one after the other
+            const int c = lane % CH ^ key(r);
+            const char *row;
+            if (u < XU) {
+                row = reinterpret_cast<const char *>(static_cast<const uint16_t *>(pj.x) + (size_t)(tok0 + (r < ntok ? r : ntok - 1)) * hin);
+            } else {
+                const int mm = i * RPL / RMAX, at = tl.row(r - mm * RMAX, p.pool.n_rows_a);
+                row = reinterpret_cast<const char *>(static_cast<const uint16_t *>(p.pr[p0 + mm].a_rows) + (size_t)(at >= 0 ? at : 0) * hin);
+            }
+            src[u] = row + (size_t)g0 * ROWB + c * 16;
+            dst[u] = (unsigned)(i * RPL + (u < XU ? 0 : TM)) * ROWB;
         }
+        auto request = [&](int slot) {                          // the next stage, into a slot of the ring
+            const unsigned at = ring_at + (unsigned)slot * STAGE;
+            if (p.stream_x) {
+#pragma unroll
+                for (int u = 0; u < XU; u++)
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" :: "s"(at + dst[u]), "v"(src[u]) : "memory");
+            } else {
+#pragma unroll
+                for (int u = 0; u < XU; u++)
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(at + dst[u]), "v"(src[u]) : "memory");
+            }
+#pragma unroll
+            for (int u = XU; u < NL; u++)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(at + dst[u]), "v"(src[u]) : "memory");
+#pragma unroll
+            for (int u = 0; u < NL; u++) src[u] += ROWB;
+        };
+        // operands: x rows of this wavefront's token blocks, A rows of its rank blocks; slice k of 32 columns is chunk 4 k + g
+        const int tw = WT == 4 ? wave : wave >> 1, rw = WT == 4 ? 0 : wave & 1;
+        unsigned xat[CH / 4], aat[CH / 4];
+#pragma unroll
+        for (int k = 0; k < CH / 4; k++) {
+            const unsigned slot = (unsigned)(((4 * k + g) ^ key(m)) * 16);
+            xat[k] = (unsigned)(tw * TBW * 16 + m) * ROWB + slot;
+            aat[k] = (unsigned)(TM + rw * NBW * 16 + m) * ROWB + slot;
+        }
+        float4_t acc[NM][TBW][NBW];
 #pragma unroll
         for (int mm = 0; mm < NM; mm++)
-            if (mm < nm) {
 #pragma unroll
-                for (int q = 0; q < AP; q++) { ar[mm][q] = ldg16(ap[mm][q] + cs); if (!ok) ar[mm][q] = zero16(); }
-            }
-    };
-    if (st0 < st1) load_stage(st0);
-#pragma unroll 1
-    for (int st = st0; st < st1; st++) {
-        __syncthreads();                                        // the previous stage has been consumed
+            for (int tb = 0; tb < TBW; tb++)
 #pragma unroll
-        for (int q = 0; q < XP; q++)
-            *reinterpret_cast<uint4 *>(s_x + (lrow + 16 * q) * PITCH + lchk * 16) = xr[q];
+                for (int nb = 0; nb < NBW; nb++) acc[mm][tb][nb] = float4_t{0.f, 0.f, 0.f, 0.f};
+        auto multiply = [&](const unsigned char *st) {
 #pragma unroll
-        for (int mm = 0; mm < NM; mm++)
-            if (mm < nm) {
+            for (int k = 0; k < CH / 4; k++) {
+                uint4 xf[TBW];
 #pragma unroll
-                for (int q = 0; q < AP; q++)
-                    if (lrow + 16 * q < RMAX) *reinterpret_cast<uint4 *>(s_a[mm] + (lrow + 16 * q) * PITCH + lchk * 16) = ar[mm][q];
-            }
-        __syncthreads();
-        if (st + 1 < st1) load_stage(st + 1);
+                for (int tb = 0; tb < TBW; tb++) xf[tb] = *reinterpret_cast<const uint4 *>(st + xat[k] + tb * 16 * ROWB);
 #pragma unroll
-        for (int ks = 0; ks < KB / 32; ks++) {
-            const uint4 xf = *reinterpret_cast<const uint4 *>(s_x + (wave * 16 + m) * PITCH + (ks * 4 + g) * 16);
+                for (int mm = 0; mm < NM; mm++)
 #pragma unroll
-            for (int mm = 0; mm < NM; mm++)
-                if (mm < nm) {
+                    for (int nb = 0; nb < NBW; nb++) {
+                        const uint4 af = *reinterpret_cast<const uint4 *>(st + aat[k] + (mm * RMAX + nb * 16) * ROWB);
 #pragma unroll
-                    for (int nb = 0; nb < NB; nb++) {
-                        const uint4 af = *reinterpret_cast<const uint4 *>(s_a[mm] + (nb * 16 + m) * PITCH + (ks * 4 + g) * 16);
-                        acc[mm][nb] = mfma16<DT>(xf, af, acc[mm][nb]);
+                        for (int tb = 0; tb < TBW; tb++) acc[mm][tb][nb] = mfma16<DT>(af, xf[tb], acc[mm][tb][nb]);
                     }
-                }
+            }
+        };
+        // At the barrier of step i every wavefront's loads of stage i have landed and all reads of stage i - 1 are done,
+        // so its slot takes stage i + D - 1.
+#pragma unroll
+        for (int d = 0; d < D - 1; d++)
+            if (d < n) request(d);
+        int slot = 0;
+#pragma unroll 1
+        for (int i = 0; i < half; i++) {
+            if (i + D - 2 < n) __builtin_amdgcn_s_waitcnt(0x0f70 | ((NL * (D - 2)) & 15) | (((NL * (D - 2)) >> 4) << 14));
+            else __builtin_amdgcn_s_waitcnt(0x0f70);
+            __syncthreads();
+            if (i + D - 1 < n) request(slot == 0 ? D - 1 : slot - 1);
+            if (i < n) multiply(ring + slot * STAGE);
+            slot = slot + 1 < D ? slot + 1 : 0;
         }
-    }
-    // D[token 4g+i][rank m] per 16x16 block; rank columns that do not exist are stored as zero.
+        if (tail) {
+            // chunks past the rows' end are zeros on both sides; the last group of wavefronts does this stage
+            __syncthreads();
+            if (kg == KG - 1) {
 #pragma unroll
-    for (int mm = 0; mm < NM; mm++)
-        if (mm < nm) {
-            float *vout = p.pr[p0 + mm].v + ((size_t)split * p.T + tok0 + wave * 16) * VSTRIDE;
+                for (int u = 0; u < NL; u++) {
+                    const int r = (int)(dst[u] / ROWB) + lane / CH, c = lane % CH ^ key(r);
+                    const bool ok = whole * CH + c < ncc;
+                    const uint4 v = ok ? ldg16(src[u] + (size_t)(whole - g0 - n) * ROWB) : zero16();
+                    *reinterpret_cast<uint4 *>(ring + dst[u] + lane * 16) = v;
+                }
+            }
+            __syncthreads();
+            if (kg == KG - 1) multiply(ring);
+        }
+        if constexpr (KG > 1) {                                 // the groups' sums, in K order
+            __syncthreads();
+            float4_t *s_acc = reinterpret_cast<float4_t *>(s_ring);
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                const int col = nb * 16 + m;
-                const bool col_ok = tl.row(col, p.pool.n_rows_a) >= 0;
+            for (int q = 1; q < KG; q++)
+                if (kg == q)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int trow_o = wave * 16 + 4 * g + i;
-                    if (trow_o < ntok) vout[(size_t)(4 * g + i) * VSTRIDE + col] = col_ok ? acc[mm][nb][i] : 0.f;
+                    for (int tb = 0; tb < TBW; tb++)
+#pragma unroll
+                        for (int nb = 0; nb < NBW; nb++) s_acc[(((q - 1) * 4 + wave) * TBW * NBW + tb * NBW + nb) * 64 + lane] = acc[0][tb][nb];
+            __syncthreads();
+            if (kg > 0) return;
+#pragma unroll
+            for (int q = 1; q < KG; q++)
+#pragma unroll
+                for (int tb = 0; tb < TBW; tb++)
+#pragma unroll
+                    for (int nb = 0; nb < NBW; nb++) acc[0][tb][nb] += s_acc[(((q - 1) * 4 + wave) * TBW * NBW + tb * NBW + nb) * 64 + lane];
+        }
+        // D[rank 4g+i][token m] per 16x16 block: a lane holds four neighbouring ranks of a token; ranks that do not exist
+        // are stored as zero.
+#pragma unroll
+        for (int nb = 0; nb < NBW; nb++) {
+            const int c0 = (rw * NBW + nb) * 16 + 4 * g;
+            bool real[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) real[e] = tl.row(c0 + e, p.pool.n_rows_a) >= 0;
+#pragma unroll
+            for (int mm = 0; mm < NM; mm++) {
+                const SgmvProj &pm = p.pr[p0 + mm];
+#pragma unroll
+                for (int tb = 0; tb < TBW; tb++) {
+                    const int t = (tw * TBW + tb) * 16 + m;
+                    if (t >= ntok) continue;
+                    float o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[e] = real[e] ? acc[mm][tb][nb][e] : 0.f;
+                    if (pm.ksplit > 1) {
+                        *reinterpret_cast<float4_t *>(pm.v + ((size_t)split * p.T + tok0 + t) * VSTRIDE + c0) = float4_t{o[0], o[1], o[2], o[3]};
+                        continue;
+                    }
+                    if (p.scaled) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) o[e] = tl.scale * o[e];
+                    }
+                    uint32_t hi[2], lo[2];
+                    split_hi_lo<DT>(o, hi, lo);
+                    *reinterpret_cast<uint2 *>(pm.vhi + (size_t)(tok0 + t) * VSTRIDE + c0) = make_uint2(hi[0], hi[1]);
+                    *reinterpret_cast<uint2 *>(pm.vlo + (size_t)(tok0 + t) * VSTRIDE + c0) = make_uint2(lo[0], lo[1]);
                 }
             }
         }
+    };
+    if constexpr (SHARE) {
+        if (nm == 3) { run(std::integral_constant<int, 3>{}); return; }
+        if (nm == 2) { run(std::integral_constant<int, 2>{}); return; }
+    }
+    run(std::integral_constant<int, 1>{});
 }
 
 // ------------------------------------------------------------------ reduce
-// vsum[t][c] = sum over K splits of the shrink partials, stored as hi + lo 16-bit halves
-// (hi = round16(v), lo = round16(v - hi)) so that the expand MFMAs see the fp32 value to
-// about 2^-16 relative.  One thread per (token, 8 rank columns).
-template <int DT>
-__device__ __forceinline__ void split_hi_lo(const float (&v)[8], uint4 &hi, uint4 &lo)
-{
-    uint32_t h[8], l[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        h[e] = cvt16<DT>(v[e]);
-        const float back = lo_f32<DT>(h[e]);
-        l[e] = cvt16<DT>(v[e] - back);
-    }
-    hi = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
-    lo = make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16), l[4] | (l[5] << 16), l[6] | (l[7] << 16));
-}
-
+// vsum[t][c] = sum over K splits of the shrink partials, stored as hi + lo 16-bit halves so that the expand MFMAs see the
+// fp32 value to about 2^-16 relative.  One thread per (token, 8 rank columns).  With one split the shrink has stored
+// the halves itself; what is left then is to define the rows outside every segment.
 template <int DT, int RMAX>
 __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
 {
@@ -408,19 +508,19 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
         }
         return;
     }
+    if (pj.ksplit == 1) return;
     float v[8];
     sum_splits_any(pj.v + (size_t)t * VSTRIDE + c0, (size_t)p.T * VSTRIDE, pj.ksplit, v);
-    uint4 hi, lo;
+    uint32_t hi[4], lo[4];
     split_hi_lo<DT>(v, hi, lo);
-    stg16(pj.vhi + (size_t)t * VSTRIDE + c0, hi);
-    stg16(pj.vlo + (size_t)t * VSTRIDE + c0, lo);
+    stg16(pj.vhi + (size_t)t * VSTRIDE + c0, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+    stg16(pj.vlo + (size_t)t * VSTRIDE + c0, make_uint4(lo[0], lo[1], lo[2], lo[3]));
 }
 
 // ------------------------------------------------------------------ expand
-// Up to rank 32 the expand sums up to eight K splits itself and the reduce launch falls away: seven projections at rank
-// 16, 16 tokens 28.8 -> 26.6 us a call, 8 x 512 tokens 184.6 -> 179.4.  At rank 64 the sums are four times as long and
-// every column block of a tile repeats them: 8 x 512 tokens 221 -> 232 us, 16 ragged prompts 375 -> 417 us of expand.
-template <int RMAX> constexpr bool FOLD_RANK = RMAX <= 32;
+// Up to FOLD_SPLITS K splits are summed by the expand itself and the reduce launch falls away.  At rank 64 the sums are
+// four times as long as at 16 and every column block of a tile repeats them, so the reduce launch stays there: 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing, 55.4 and a reduce
+// of 5.2 not; at rank 16 the whole call of 8 x 512 tokens 185 -> 179.
 constexpr int FOLD_SPLITS = 8;
 
 template <int DT, int RMAX, bool BT>
@@ -442,6 +542,8 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     __shared__ __attribute__((aligned(16))) unsigned char s_b[BT ? TN * TPITCH : KP * BPITCH];
     __shared__ __attribute__((aligned(16))) float s_out[SG_NT / 64][16][OPITCH];
     __shared__ int s_brow[BT ? 1 : KP];
+    constexpr int VPITCH = KP + 8;             // 16-bit values per token row of the folded intermediate, which lies in s_out for a while
+    static_assert(2 * TM * VPITCH * 2 <= (int)sizeof(s_out), "the folded intermediate fits the staging tiles");
     typedef __attribute__((address_space(3))) volatile float lds_vfloat;
     typedef __attribute__((address_space(3))) volatile float4_t lds_vfloat4;
 
@@ -458,7 +560,7 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
             colblk = (w - tile * ncb8 + ncb8 - ((tile >> 3) & 7)) % ncb8;
             if (colblk >= pj.ncb) return;
         } else {
-            place(w, pj.ncb, p.max_tiles, tile, colblk);
+            place(w, pj.ncb, p.max_tiles, 0, tile, colblk);
         }
     }
     if (tile >= p.max_tiles) return;
@@ -499,26 +601,45 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     int trow = wave * 16 + m;
     trow = trow < ntok ? trow : ntok - 1;
     uint4 vhi[KS], vlo[KS];
+    const bool fold = p.fold && pj.ksplit > 1;
+    if (fold) {
+        // whole rows of the partial sums, four ranks a thread; the operands are read back from LDS behind the barrier
+        uint16_t *s_v = reinterpret_cast<uint16_t *>(&s_out[0][0][0]);
+        constexpr int RQ = RMAX / 4;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        const int c0 = ks * 32 + 8 * g;
-        vhi[ks] = zero16(); vlo[ks] = zero16();
-        if constexpr (FOLD_RANK<RMAX>) {
-            if (c0 < RMAX && p.fold) {
-                float v[8];
-                sum_splits<8>(pj.v + (size_t)(tok0 + trow) * VSTRIDE + c0, (size_t)p.T * VSTRIDE, pj.ksplit, v);
-                split_hi_lo<DT>(v, vhi[ks], vlo[ks]);
-                continue;
-            }
+        for (int i = 0; i < TM * RQ / SG_NT; i++) {
+            const int e = i * SG_NT + tid, t = e / RQ, c0 = (e - t * RQ) * 4;
+            float v[4];
+            sum_splits4(pj.v + (size_t)(tok0 + (t < ntok ? t : ntok - 1)) * VSTRIDE + c0, (size_t)p.T * VSTRIDE, pj.ksplit, v);
+            uint32_t hi[2], lo[2];
+            split_hi_lo<DT>(v, hi, lo);
+            *reinterpret_cast<uint2 *>(s_v + t * VPITCH + c0) = make_uint2(hi[0], hi[1]);
+            *reinterpret_cast<uint2 *>(s_v + (TM + t) * VPITCH + c0) = make_uint2(lo[0], lo[1]);
         }
-        if (c0 < RMAX) {
-            vhi[ks] = ldg16(pj.vhi + ((size_t)(tok0 + trow) * VSTRIDE + c0));
-            vlo[ks] = ldg16(pj.vlo + ((size_t)(tok0 + trow) * VSTRIDE + c0));
+    } else {
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int c0 = ks * 32 + 8 * g;
+            vhi[ks] = zero16(); vlo[ks] = zero16();
+            if (c0 < RMAX) {
+                vhi[ks] = ldg16(pj.vhi + ((size_t)(tok0 + trow) * VSTRIDE + c0));
+                vlo[ks] = ldg16(pj.vlo + ((size_t)(tok0 + trow) * VSTRIDE + c0));
+            }
         }
     }
     const uint16_t *__restrict__ brows = static_cast<const uint16_t *>(pj.b_rows);
     const uint16_t *__restrict__ bt = brows + (BT ? (size_t)adapter * (size_t)pv.b_dense_stride : 0);
     __syncthreads();
+    if (fold) {
+        const uint16_t *s_v = reinterpret_cast<const uint16_t *>(&s_out[0][0][0]);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int c0 = ks * 32 + 8 * g;
+            const bool real = c0 < RMAX;
+            vhi[ks] = real ? *reinterpret_cast<const uint4 *>(s_v + trow * VPITCH + c0) : zero16();
+            vlo[ks] = real ? *reinterpret_cast<const uint4 *>(s_v + (TM + trow) * VPITCH + c0) : zero16();
+        }
+    }
 
     // Loads of a step (this thread's share of the B tile and of the y rows) are issued one step ahead.
     // y rows of this wavefront: lane handles (token p / 16, 16-byte chunk p % 16), p = lane + 64 q.
@@ -656,7 +777,7 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     SgmvArgs g = a;
     unsigned end = 0;
     for (int q = 0; q < g.n_grp; q++) {
-        end += (unsigned)place_grid(g.max_tiles, g.pr[g.grp_first[q]].ksplit);
+        end += (unsigned)(place_grid(g.max_tiles, g.pr[g.grp_first[q]].ksplit) * (g.share_x ? 1 : g.grp_n[q]));
         g.grp_end[q] = end;
     }
     const unsigned sgrid = end;
@@ -666,18 +787,19 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
         g.ex_end[q] = end;
     }
     const unsigned egrid = end;
-    int nm = 1;
-    for (int q = 0; q < g.n_grp; q++) nm = g.grp_n[q] > nm ? g.grp_n[q] : nm;
-    if ((g.seg_uniform_len > 0) != (g.b_transposed != 0) || (g.b_transposed && nm != 1)) return (int)hipErrorInvalidValue;
-    if (g.seg_uniform_len > 0) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, 1, true>), dim3(sgrid), dim3(SG_NT), 0, s, g);
-    else if (nm == 1) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, 1, false>), dim3(sgrid), dim3(SG_NT), 0, s, g);
-    else hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, SG_NM, false>), dim3(sgrid), dim3(SG_NT), 0, s, g);
+    if ((g.seg_uniform_len > 0) != (g.b_transposed != 0)) return (int)hipErrorInvalidValue;
+    g.scaled = !(phases & SGMV_APPLY);                          // the base GEMM + LoRA kernel takes the scaled intermediate
+    if (g.seg_uniform_len > 0 && g.share_x) return (int)hipErrorInvalidValue;
+    const dim3 threads(SG_NT * (g.share_x ? SH_KG<true> : SH_KG<false>));
+    if (g.seg_uniform_len > 0) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, true, false>), dim3(sgrid), threads, 0, s, g);
+    else if (g.share_x) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, false, true>), dim3(sgrid), threads, 0, s, g);
+    else hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, false, false>), dim3(sgrid), threads, 0, s, g);
     rc = (int)hipGetLastError();
     if (rc || !(phases & SGMV_APPLY)) return rc;
-    // Few K splits are summed by the expand itself (FOLD_RANK); rows outside every segment are zeroed by the reduce launch only.
+    // Few K splits are summed by the expand itself; rows outside every segment are zeroed by the reduce launch only.
     int most = 1;
     for (int q = 0; q < g.n_proj; q++) most = g.pr[q].ksplit > most ? g.pr[q].ksplit : most;
-    g.fold = FOLD_RANK<RMAX> && most <= FOLD_SPLITS && (g.accumulate || g.seg_uniform_len > 0);
+    g.fold = most <= FOLD_SPLITS && RMAX <= 32 && (g.accumulate || g.seg_uniform_len > 0);
     if (!g.fold) {
         const long long n = (long long)g.T * (RMAX / 8);
         hipLaunchKernelGGL((sgmv_reduce_kernel<DT, RMAX>), dim3((unsigned)((n + 255) / 256), (unsigned)g.n_proj), dim3(256), 0, s, g);

@@ -375,3 +375,42 @@ def test_a_workspace_of_a_larger_call_serves_a_smaller_one(long, T, n_seg, n_pro
     for y in outs:
         got = y.double().cpu().numpy()
         assert (np.abs(got - base) <= ATOL + RTOL * np.abs(base)).all()
+
+
+@pytest.mark.parametrize("lens,ranks,hin,inputs", [
+    ([30], [16], 8, [0]),                                    # no whole stage of 64 columns
+    ([64, 1], [8, 16], 72, [0, 1]),                          # one whole stage and a short one; a group of wavefronts without any
+    ([129], [32, 20], 1096, [0, 0]),                         # ranges of unlike length, the last with the short stage
+    ([100, 28], [64], 4160, [0, 0, 0, 0]),                   # eight splits, four projections of one input
+    ([64] * 70 + [17], [64, 40], 200, [0, 0, 0, 1]),         # one workgroup for three projections, and for one beside it
+    ([64] * 70 + [33], [32], 136, [0, 0, 1, 1, 1]),          # for two and for three
+    ([64] * 90, [16, 5], 640, [0, 0, 0, 0]),                 # a fourth projection of the same input starts a new group
+])
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+def test_sgmv_shrink_stages_and_groups(lens, ranks, hin, inputs, dtype):
+    """The ring of stages at its ends (rows shorter than a stage, a last stage of fewer columns, more slots than stages) and
+    every number of projections that a workgroup serves, with one K split and with several."""
+    from mlora import sgmv_multi
+    rng = np.random.default_rng(sum(lens) + hin)
+    hout = 136
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
+    names = [f"p{i}" for i in range(len(inputs))]
+    pool = upload_pool(pp, projections={nm: (hin, hout) for nm in names})
+    for nm in names:
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, dtype))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, dtype))
+    seg = _segments(lens, rng.integers(0, len(ranks), len(lens)))
+    T = sum(lens) + 3
+    tok = _tok_of(*seg, T)
+    plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in seg), T, pool, n_proj=len(inputs))
+    xs = [bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype) for _ in range(max(inputs) + 1)]
+    xt = [bits_to_torch(x, dtype, "cuda") for x in xs]
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
+    for accumulate in (True, False):
+        say(f"sgmv stages lens={lens[:2]}x{len(lens)} hin={hin} inputs={inputs} dtype={dtype} accumulate={accumulate}")
+        ys = [bits_to_torch(y0, dtype, "cuda") for _ in names]
+        sgmv_multi(ys, [xt[i] for i in inputs], pool, 0, names, plan, accumulate=accumulate)
+        torch.cuda.synchronize()
+        want = [oracle_apply(pp, x, tok, y0 if accumulate else None) for x in xs]
+        for i, y in zip(inputs, ys):
+            assert_close_bits(torch_to_bits(y), want[i], dtype, f"input {i}")
