@@ -747,17 +747,17 @@ int splits_of(int hin, int hin_min, int k, const SgmvWs &w)
 
 // Shape of a prefill call's shrink launch: whether a workgroup serves up to three projections of one x (share_x), the groups, and
 // the K splits.  More splits and single projections make more and shorter workgroups; fewer splits mean fewer partial
-// sums, shared x fewer lines from L2.  The rule estimates the launch for both kinds and six numbers of splits, and takes
-// the least: workgroups of known length (4 ns a 128-byte line and compute unit) are dealt, longest first, to the slots of
-// the device, but not below what all lines take together (6.4 TB/s); a split costs 0.05 ns a token and projection (written,
-// and read by the reduce launch or the expand).  Fitted to both kinds at 1, 2 and 4 splits over 46 batches of 16 to 9216
-// tokens (ranks 16 to 64; one, three, four and seven projections): the shape it names is within 5 % of the best of the six
-// everywhere and 0.5 % off on average.  Llama-7B widths, rank 64, q/k/v, two layers and the plan in a graph, single / shared
+// sums, shared x fewer lines from L2.  The rule estimates the launch for both kinds and four numbers of splits, and takes
+// the least: workgroups of known length (4 ns a 128-byte line and compute unit) dealt, longest first, to the slots of the
+// device; what all lines take together (2 us and 6.4 TB/s); the longer of the two and 0.3 of the other; 0.2 ns a split, token
+// and projection (written, and read by the reduce launch or the expand).  Fitted to those eight shapes over 52 batches of 16
+// to 9216 tokens (ranks 16 to 64; one, three, four and seven projections): the shape it names is 0.9 % off the best on
+// average and 9 % at worst.  Llama-7B widths, rank 64, q/k/v, two layers and the plan in a graph, single / shared
 // projections at 1, 2, 4 splits, us: 64 tokens 53, 41, 35 / 110, 67, 50; 1280 tokens 86, 81, 87 / 137, 101, 85; 6000 tokens 211,
 // 211, 229 / 232, 202, 213.
 void shrink_shape(mlora::SgmvArgs &a, int tiles, int max_rank, const SgmvWs &w)
 {
-    static const int tried[] = {1, 2, 3, 4, 6, 8};
+    static const int tried[] = {1, 2, 4, 8};
     const int cus = mlora::device_compute_units(), rows = max_rank <= 16 ? 16 : (max_rank <= 32 ? 32 : 64);
     int hin_min = a.pr[0].hin;
     for (int p = 1; p < a.n_proj; p++) hin_min = a.pr[p].hin < hin_min ? a.pr[p].hin : hin_min;
@@ -772,7 +772,7 @@ void shrink_shape(mlora::SgmvArgs &a, int tiles, int max_rank, const SgmvWs &w)
     for (int share = 0; share <= (a.seg_uniform_len == 0 ? 1 : 0); share++) {
         // workgroups a unit holds, by their LDS (sh_group_bytes in sgmv_prefill.hip)
         const long long slots = (long long)cus * (rows == 16 || (share && rows == 32) ? 2 : 1);
-        for (int t = 0; t < 6; t++) {
+        for (int t = 0; t < 4; t++) {
             const int k = tried[t];
             long long count[MLORA_MAX_PROJ];
             double len[MLORA_MAX_PROJ], lines = 0.0, parts = 0.0;
@@ -814,9 +814,8 @@ void shrink_shape(mlora::SgmvArgs &a, int tiles, int max_rank, const SgmvWs &w)
                 }
             }
             for (int i = 0; i < nb; i++) if (n[i] > 0 && at[i] > end) end = at[i];
-            double us = 0.004 * end;
-            const double all = 2e-5 * lines;
-            us = (us > all ? us : all) + 5e-5 * parts;
+            const double chain = 0.004 * end, all = 2.0 + 2e-5 * lines;
+            const double us = (chain > all ? chain + 0.3 * all : all + 0.3 * chain) + 2e-4 * parts;
             if ((share == 0 && t == 0) || us < best) { best = us; best_k = k; a.share_x = share; }
         }
     }

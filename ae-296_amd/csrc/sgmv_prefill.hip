@@ -5,7 +5,8 @@
 //   shrink : V[split][t][0..R) = x[t, Kslice] . A_a[:, Kslice]^T   (split-K, fp32 partials), or with one
 //            split the result itself as a hi + lo pair of 16-bit values, so that the intermediate keeps
 //            fp32 accuracy through the second MFMA;
-//   reduce : sums the K splits into such pairs (up to rank 32 the expand does this itself where y accumulates; with one split there is nothing to do);
+//   reduce : sums the K splits into such pairs (up to rank 32, and in launches of few tiles, the expand
+//            does this itself where y accumulates; with one split there is nothing to do);
 //   expand : y[t, cols] (+)= s_a * (Vhi + Vlo) . B_a[:, cols].
 // Both MFMA operands of the shrink pass through a ring of LDS stages that global memory fills directly.
 // The expand parks the B tile in LDS (rank must be the
@@ -519,7 +520,8 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
 
 // ------------------------------------------------------------------ expand
 // Up to FOLD_SPLITS K splits are summed by the expand itself and the reduce launch falls away.  At rank 64 the sums are
-// four times as long as at 16 and every column block of a tile repeats them, so the reduce launch stays there: 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing, 55.4 and a reduce
+// four times as long as at 16 and every column block of a tile repeats them, so the reduce launch stays there but for the
+// launches of few tiles below: 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing, 55.4 and a reduce
 // of 5.2 not; at rank 16 the whole call of 8 x 512 tokens 185 -> 179.
 constexpr int FOLD_SPLITS = 8;
 
@@ -763,6 +765,144 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     }
 }
 
+// The expand of a launch of few tiles above rank 32.  The kernel above takes 64 tokens at a time, one 128-column step after the other, so a
+// prompt of a tile or two is a chain of a few long steps on a part of the chip.  Here a workgroup takes 16 tokens and 256
+// columns, 64 per wavefront, in one step, everything requested at once; B is read by four workgroups instead of one.
+// Two layers and the plan in a graph, that kernel -> this one, us: 64 tokens, q/k/v, rank 64 36.8 -> 33.6 (192 workgroups);
+// the reference's call, 64 tokens, 41.1 -> 32.4, 2 x 200 tokens 44.7 -> 37.2 (512); 4 x 300 tokens 60.5 -> 60.0 (1280); 200 tokens,
+// seven projections 64.4 -> 86.0 (2560).  So up to 512 workgroups, and not up to rank 32, where there is little B and less to sum:
+// 64 tokens, rank 16 28.2 -> 27.3, two prompts of 20 and 60, four projections 27.2 -> 29.6.
+constexpr int FEW_COLS = 256;
+constexpr int FEW_EXPAND = 512;             // workgroups up to which it is taken
+template <int DT, bool BT>
+__global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p)
+{
+    constexpr int KP = MAX_RANK, KS = KP / 32;                  // K of the MFMAs (rank padded with zeros)
+    constexpr int CW = FEW_COLS / 4, NBC = CW / 16;             // columns of a wavefront
+    constexpr int BPITCH = CW * 2 + 16, TPITCH = KP * 2 + 16;   // bytes per LDS row of B: a rank row, or (reference layout) an output column
+    constexpr int BQ = KP / 8;                                  // B loads per lane
+    constexpr int VPITCH = KP + 8, OPITCH = CW + 4;
+    constexpr int WBYTES = BT ? CW * TPITCH : KP * BPITCH;
+    __shared__ __attribute__((aligned(16))) unsigned char s_b[4][WBYTES];       // private to a wavefront: B, then its result
+    __shared__ __attribute__((aligned(16))) uint16_t s_v[2][16][VPITCH];
+    static_assert(16 * OPITCH * 4 <= WBYTES, "a wavefront's result fits its B tile");
+
+    int proj = 0;
+    while (proj + 1 < p.n_proj && blockIdx.x >= p.ex_end[proj]) proj++;
+    const SgmvProj &pj = p.pr[proj];
+    const int w = (int)(blockIdx.x - (proj ? p.ex_end[proj - 1] : 0u));
+    const int ncb = (pj.hout + FEW_COLS - 1) / FEW_COLS;
+    const int piece = w / ncb, colblk = w - piece * ncb, tile = piece >> 2, sub = piece & 3;
+    if (tile >= p.max_tiles) return;
+    const Tile<BT> tl = tile_of<BT>(p, tile);
+    const int ntok = tl.ntok - sub * 16 < 16 ? tl.ntok - sub * 16 : 16, tok0 = tl.tok0 + sub * 16;
+    if (ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
+    const int hout = pj.hout, r = tl.rank;
+    uint16_t *__restrict__ y = static_cast<uint16_t *>(pj.y);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = lane & 15, g = lane >> 4;
+    const int col0 = colblk * FEW_COLS + wave * CW;
+    // this lane's pieces of y: token q * 8 + lane / 8, 8 columns
+    const int yc = col0 + (lane & 7) * 8;
+    if (tl.adapter < 0) {
+        if (!p.accumulate && yc < hout)
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+                if (q * 8 + (lane >> 3) < ntok) stg16(y + (size_t)(tok0 + q * 8 + (lane >> 3)) * hout + yc, zero16());
+        return;
+    }
+    const uint16_t *__restrict__ brows = static_cast<const uint16_t *>(pj.b_rows);
+    uint4 bv[BQ];
+#pragma unroll
+    for (int q = 0; q < BQ; q++) {
+        if constexpr (!BT) {
+            const int row = tl.row(q * 8 + (lane >> 3), p.pool.n_rows_a);
+            bv[q] = (row >= 0 && row < p.pool.n_rows_b && yc < hout) ? ldg16(brows + (size_t)row * hout + yc) : zero16();
+        } else {
+            const int e = q * 64 + lane, col = col0 + e / (KP / 8), k0 = (e % (KP / 8)) * 8;
+            bv[q] = (col < hout && k0 < r) ? ldg16(brows + (size_t)tl.adapter * (size_t)p.pool.b_dense_stride + (size_t)col * r + k0) : zero16();
+        }
+    }
+    uint4 yv[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int t = q * 8 + (lane >> 3);
+        yv[q] = (p.accumulate && t < ntok && yc < hout) ? ldg16_stream(y + (size_t)(tok0 + t) * hout + yc) : zero16();
+    }
+    const bool fold = p.fold && pj.ksplit > 1;
+    const int trow = m < ntok ? m : ntok - 1;
+    uint4 vhi[KS], vlo[KS];
+    if (fold) {
+        const int t = tid / (KP / 4), c0 = (tid % (KP / 4)) * 4;        // 16 tokens x 16 quads
+        float v[4];
+        sum_splits4(pj.v + (size_t)(tok0 + (t < ntok ? t : ntok - 1)) * VSTRIDE + c0, (size_t)p.T * VSTRIDE, pj.ksplit, v);
+        uint32_t hi[2], lo[2];
+        split_hi_lo<DT>(v, hi, lo);
+        *reinterpret_cast<uint2 *>(&s_v[0][t][c0]) = make_uint2(hi[0], hi[1]);
+        *reinterpret_cast<uint2 *>(&s_v[1][t][c0]) = make_uint2(lo[0], lo[1]);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+        const int c0 = ks * 32 + 8 * g;
+        vhi[ks] = fold ? *reinterpret_cast<const uint4 *>(&s_v[0][trow][c0]) : ldg16(pj.vhi + (size_t)(tok0 + trow) * VSTRIDE + c0);
+        vlo[ks] = fold ? *reinterpret_cast<const uint4 *>(&s_v[1][trow][c0]) : ldg16(pj.vlo + (size_t)(tok0 + trow) * VSTRIDE + c0);
+    }
+    // the wavefront's B tile through its own LDS, then its result: operations of one wavefront on LDS complete in order
+    unsigned char *sb = s_b[wave];
+#pragma unroll
+    for (int q = 0; q < BQ; q++) {
+        const int e = q * 64 + lane;
+        unsigned char *at = BT ? sb + e / (KP / 8) * TPITCH + e % (KP / 8) * 16 : sb + e / 8 * BPITCH + e % 8 * 16;
+        *reinterpret_cast<uint4 *>(at) = bv[q];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float4_t acc[NBC];
+#pragma unroll
+    for (int nb = 0; nb < NBC; nb++) {
+        acc[nb] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            uint4 bop;
+            if constexpr (!BT) {
+                // lane (column m, ranks ks * 32 + 8 g ..) by the transposing read, see the kernel above
+                const unsigned char *src = sb + (ks * 32 + 8 * g + (m >> 2)) * BPITCH + (nb * 16 + (m & 3) * 4) * 2;
+                const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)src));
+                const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(src + 4 * BPITCH)));
+                bop = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            } else {
+                bop = *reinterpret_cast<const uint4 *>(sb + (nb * 16 + m) * TPITCH + (ks * 4 + g) * 16);
+            }
+            acc[nb] = mfma16<DT>(vhi[ks], bop, acc[nb]);
+            acc[nb] = mfma16<DT>(vlo[ks], bop, acc[nb]);
+        }
+    }
+    // D[token 4g+i][column m of the block]
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float *so = reinterpret_cast<float *>(sb);
+#pragma unroll
+    for (int nb = 0; nb < NBC; nb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) so[(4 * g + i) * OPITCH + nb * 16 + m] = acc[nb][i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int t = q * 8 + (lane >> 3);
+        if (t >= ntok || yc >= hout) continue;
+        const float4_t d0 = *reinterpret_cast<const float4_t *>(so + t * OPITCH + (lane & 7) * 8);
+        const float4_t d1 = *reinterpret_cast<const float4_t *>(so + t * OPITCH + (lane & 7) * 8 + 4);
+        float o[8];
+        unpack8<DT>(yv[q], o);                                  // zeros when not accumulating
+#pragma unroll
+        for (int e = 0; e < 4; e++) { o[e] = fmaf(tl.scale, d0[e], o[e]); o[4 + e] = fmaf(tl.scale, d1[e], o[4 + e]); }
+        stg16_stream(y + (size_t)(tok0 + t) * hout + yc, pack8<DT>(o));
+    }
+}
+
 template <int DT, int RMAX>
 static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
 {
@@ -782,8 +922,11 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     }
     const unsigned sgrid = end;
     end = 0;
+    long long few_wgs = 0;
+    for (int q = 0; q < g.n_proj; q++) few_wgs += (long long)g.tiles * 4 * ((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS);
+    const bool few = RMAX > 32 && few_wgs <= FEW_EXPAND;
     for (int q = 0; q < g.n_proj; q++) {
-        end += (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
+        end += few ? (unsigned)g.max_tiles * 4u * (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
         g.ex_end[q] = end;
     }
     const unsigned egrid = end;
@@ -799,12 +942,19 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     // Few K splits are summed by the expand itself; rows outside every segment are zeroed by the reduce launch only.
     int most = 1;
     for (int q = 0; q < g.n_proj; q++) most = g.pr[q].ksplit > most ? g.pr[q].ksplit : most;
-    g.fold = most <= FOLD_SPLITS && RMAX <= 32 && (g.accumulate || g.seg_uniform_len > 0);
+    g.fold = most <= FOLD_SPLITS && (RMAX <= 32 || few) && (g.accumulate || g.seg_uniform_len > 0);
     if (!g.fold) {
         const long long n = (long long)g.T * (RMAX / 8);
         hipLaunchKernelGGL((sgmv_reduce_kernel<DT, RMAX>), dim3((unsigned)((n + 255) / 256), (unsigned)g.n_proj), dim3(256), 0, s, g);
         rc = (int)hipGetLastError();
         if (rc) return rc;
+    }
+    if constexpr (RMAX > 32) {
+        if (few) {
+            if (g.b_transposed) hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, true>), dim3(egrid), dim3(SG_NT), 0, s, g);
+            else hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, false>), dim3(egrid), dim3(SG_NT), 0, s, g);
+            return (int)hipGetLastError();
+        }
     }
     if (g.b_transposed)
         hipLaunchKernelGGL((sgmv_expand_kernel<DT, RMAX, true>), dim3(egrid), dim3(SG_NT), 0, s, g);

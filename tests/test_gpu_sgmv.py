@@ -414,3 +414,41 @@ def test_sgmv_shrink_stages_and_groups(lens, ranks, hin, inputs, dtype):
         want = [oracle_apply(pp, x, tok, y0 if accumulate else None) for x in xs]
         for i, y in zip(inputs, ys):
             assert_close_bits(torch_to_bits(y), want[i], dtype, f"input {i}")
+
+
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("lens,ranks,hin,hout,n_proj", [
+    ([1], [40], 64, 8, 1),                         # one token, one piece of y
+    ([17, 15, 33], [64, 8], 520, 264, 3),          # pieces of 16 tokens with a remainder; a last column block of 8
+    ([48], [48], 4096, 2568, 2),                   # eight splits
+    ([64, 64], [33], 72, 4096, 4),                 # one split: halves from the shrink; 512 workgroups
+])
+def test_sgmv_few_tiles(lens, ranks, hin, hout, n_proj, dtype):
+    """The expand of 16-token pieces, summing the splits itself, behind the reduce launch (y = delta) and on one split; a
+    segment without an adapter and rows outside every segment."""
+    from mlora import sgmv_multi
+    rng = np.random.default_rng(sum(lens) + hin)
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
+    names = [f"p{i}" for i in range(n_proj)]
+    pool = upload_pool(pp, projections={nm: (hin, hout) for nm in names})
+    for nm in names:
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, dtype))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, dtype))
+    adapters = rng.integers(0, len(ranks), len(lens))
+    if len(lens) > 2:
+        adapters[1] = -1
+    seg = _segments(lens, adapters)
+    T = sum(lens) + 2
+    tok = _tok_of(*seg, T)
+    plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in seg), T, pool, n_proj=n_proj)
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
+    xt = bits_to_torch(x, dtype, "cuda")
+    for accumulate in (True, False):
+        say(f"sgmv few tiles lens={lens} {hin}->{hout} n_proj={n_proj} dtype={dtype} accumulate={accumulate}")
+        ys = [bits_to_torch(y0, dtype, "cuda") for _ in names]
+        sgmv_multi(ys, [xt] * n_proj, pool, 0, names, plan, accumulate=accumulate)
+        torch.cuda.synchronize()
+        want = oracle_apply(pp, x, tok, y0 if accumulate else None)
+        for y in ys:
+            assert_close_bits(torch_to_bits(y), want, dtype)
