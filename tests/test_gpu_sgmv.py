@@ -452,3 +452,37 @@ def test_sgmv_few_tiles(lens, ranks, hin, hout, n_proj, dtype):
         want = oracle_apply(pp, x, tok, y0 if accumulate else None)
         for y in ys:
             assert_close_bits(torch_to_bits(y), want, dtype)
+
+
+@pytest.mark.parametrize("aligned", [False, True])
+@pytest.mark.parametrize("n_seg,longest", [(300, 5), (17, 1100), (1, 1)])
+def test_plan_over_several_workgroups(n_seg, longest, aligned):
+    """More segments than a workgroup looks at together, more tiles and more tokens than one writes: the tile list is the
+    oracle's, and y = delta is zero exactly in the rows outside every segment."""
+    from oracle import oracle as orc
+    rng = np.random.default_rng(n_seg)
+    lens = rng.integers(1, longest + 1, n_seg).astype(np.int32)
+    gaps = rng.integers(0, 3, n_seg).astype(np.int32)
+    ss = (np.cumsum(lens + gaps) - lens).astype(np.int32)
+    T = int(ss[-1] + lens[-1]) + 4
+    pp = PagedPool(rng, [16, 8, 4], 64, 64, page_rows=8, dtype=FP16)
+    pool = upload_pool(pp)
+    sa = rng.integers(0, 3, n_seg).astype(np.int32)
+    say(f"plan of {n_seg} segments, {T} tokens, aligned={aligned}")
+    plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in (ss, lens, sa)), T, pool, aligned=aligned)
+    torch.cuda.synchronize()
+    want = orc.sgmv_plan(ss, lens, 64, aligned=aligned)
+    max_tiles = T // 64 + 2 * n_seg + 1
+    words = plan.workspace[:(3 * max_tiles + 1) * 4].cpu().numpy().view(np.int32)
+    n = int(words[3 * max_tiles])
+    assert n == len(want[0])
+    for i in range(3):
+        assert np.array_equal(words[i * max_tiles:i * max_tiles + n], want[i])
+    x = torch.ones(T, 64, device="cuda", dtype=torch.float16)
+    y = torch.full((T, 64), float("nan"), device="cuda", dtype=torch.float16)
+    sgmv(y, x, pool, 0, "p", plan=plan, accumulate=False)
+    torch.cuda.synchronize()
+    covered = np.zeros(T, bool)
+    for s, ln in zip(ss, lens):
+        covered[s:s + ln] = True
+    assert np.array_equal((y != 0).any(1).cpu().numpy(), covered) and bool(torch.isfinite(y).all())
