@@ -6,6 +6,8 @@
 // small batch run.  Host time per call, launches included, in Python -> here: plan_decode 9.2 -> 4.5 us, bgmv over seven
 // projections in two launches 19.4 -> 9.1 us (0.5 of it the allocation of its intermediate), sgmv_multi over seven (three
 // launches) 34.5 -> 10.7 us.
+// The reference's q, k and v calls of a layer, outputs included (deltas_ref and Lora_GPU._invoke): 21 -> 16 us, a step of four layers
+// that the host bounds 86 -> 65 us.
 // Nothing is kept from one call for the next: every tensor is checked and every slab looked up on every call.  A negative
 // code of the C ABI is returned, and raised by the caller.
 #include <Python.h>
@@ -46,7 +48,7 @@ struct Ref {        // an owned reference
 
 PyObject *s_page_tbl, *s_rank, *s_scaling, *s_work, *s_group, *s_vws, *s_perm, *s_seg_start, *s_seg_len, *s_seg_adapter,
     *s_chunk_start, *s_chunk_len, *s_chunk_adapter, *s_counters, *s_row_off, *s_tok_rank, *s_tok_scale, *s_T, *s_workspace,
-    *s_n_slots, *s_max_pages, *s_page_rows, *s_n_pages, *s_max_rank, *s_tok_adapter, *s_dtype_code, *s_projections, *s_a_rows, *s_b_rows;
+    *s_n_slots, *s_max_pages, *s_page_rows, *s_n_pages, *s_max_rank, *s_tok_adapter, *s_dtype_code, *s_projections, *s_a_rows, *s_b_rows, *s_buf;
 
 void *attr_ptr(PyObject *o, PyObject *name)          // data pointer of a tensor attribute, null for None
 {
@@ -269,28 +271,19 @@ at::Tensor intermediate(PyObject *plan, int64_t bytes, const at::Tensor &like)
     return t;
 }
 
-// bgmv_ref(plan, ys, xs, was, wbs, layer, scale, accumulate, T, N, L, r)
-PyObject *bgmv_ref(PyObject *const *v, Py_ssize_t nargs)
+// A reference-layout decode call over n projections: every check, then the launch.  y, x, a, b give the tensors of a projection.
+template <typename Y, typename X, typename A, typename B>
+int ref_call(PyObject *plan, int n, Y y_of, X x_of, A a_of, B b_of, int layer, float scale, bool accumulate, int64_t T, int64_t N, int64_t L, int64_t r)
 {
-    if (nargs != 12) raise(PyExc_TypeError, "bgmv_ref takes 12 arguments");
-    PyObject *plan = v[0];
-    const List ys(v[1]), xs(v[2]), was(v[3]), wbs(v[4]);
-    const int64_t T = as_int(v[8]), N = as_int(v[9]), L = as_int(v[10]), r = as_int(v[11]);
-    const int n = (int)ys.size();
-    if (n < 1 || n > MLORA_MAX_PROJ || xs.size() != n || was.size() != n || wbs.size() != n)
-        raise(PyExc_ValueError, "need 1..%d projections with one y, x, wa and wb each", MLORA_MAX_PROJ);
-    const List *all[4] = {&ys, &xs, &was, &wbs};
-    for (const List *l : all)
-        for (int i = 0; i < n; i++) need_device((*l)[i]);
-    for (const List *l : all)
-        for (int i = 0; i < n; i++) need_contiguous((*l)[i]);
+    for (int i = 0; i < n; i++) { need_device(y_of(i)); need_device(x_of(i)); need_device(a_of(i)); need_device(b_of(i)); }
+    for (int i = 0; i < n; i++) { need_contiguous(y_of(i)); need_contiguous(x_of(i)); need_contiguous(a_of(i)); need_contiguous(b_of(i)); }
     void *y[MLORA_MAX_PROJ];
     const void *x[MLORA_MAX_PROJ], *a[MLORA_MAX_PROJ], *b[MLORA_MAX_PROJ];
     int32_t hin[MLORA_MAX_PROJ], hout[MLORA_MAX_PROJ];
-    const at::ScalarType type = ys[0].scalar_type();
+    const at::ScalarType type = y_of(0).scalar_type();
     int max_hin = 0;
     for (int i = 0; i < n; i++) {
-        const at::Tensor &yt = ys[i], &xt = xs[i], &at = was[i], &bt = wbs[i];
+        const at::Tensor &yt = y_of(i), &xt = x_of(i), &at = a_of(i), &bt = b_of(i);
         if (at.dim() != 4 || bt.dim() != 4) raise(PyExc_ValueError, "wa_T_all must be [N, L, r, Hin] and wb_T_all [N, L, Hout, r]");
         if (at.size(0) != N || at.size(1) != L || at.size(2) != r || bt.size(0) != N || bt.size(1) != L || bt.size(3) != r)
             raise(PyExc_ValueError, "pool tensors disagree with each other or with the plan on N, L or r");
@@ -303,14 +296,54 @@ PyObject *bgmv_ref(PyObject *const *v, Py_ssize_t nargs)
         max_hin = hin[i] > max_hin ? hin[i] : max_hin;
     }
     if (type != at::kHalf && type != at::kBFloat16) raise(PyExc_TypeError, "mlora kernels take float16 or bfloat16 tensors");
-    static PyObject *s_buf = PyUnicode_InternFromString("buf");
     const int64_t bytes = mlora_bgmv_workspace_bytes(n, (int)T, max_hin, (int)r);
-    const at::Tensor room = bytes > 0 ? intermediate(plan, bytes, ys[0]) : at::Tensor();
+    const at::Tensor room = bytes > 0 ? intermediate(plan, bytes, y_of(0)) : at::Tensor();
     void *ws = room.defined() ? room.data_ptr() : nullptr;
-    const int rc = launch(mlora_bgmv_reflayout_multi, n, y, x, a, b, hin, hout, attr_ptr(plan, s_buf), (int)T, (int)N, (int)L, (int)r,
-                                              (int)as_int(v[5]), (float)PyFloat_AsDouble(v[6]), (int)attr_int(plan, s_group),
-                                              type == at::kHalf ? MLORA_F16 : MLORA_BF16, v[7] == Py_True, ws, bytes, stream());
-    return PyLong_FromLong(rc);
+    return launch(mlora_bgmv_reflayout_multi, n, y, x, a, b, hin, hout, attr_ptr(plan, s_buf), (int)T, (int)N, (int)L, (int)r,
+                  layer, scale, (int)attr_int(plan, s_group), type == at::kHalf ? MLORA_F16 : MLORA_BF16, accumulate, ws, bytes, stream());
+}
+
+// bgmv_ref(plan, ys, xs, was, wbs, layer, scale, accumulate, T, N, L, r)
+PyObject *bgmv_ref(PyObject *const *v, Py_ssize_t nargs)
+{
+    if (nargs != 12) raise(PyExc_TypeError, "bgmv_ref takes 12 arguments");
+    const List ys(v[1]), xs(v[2]), was(v[3]), wbs(v[4]);
+    const int n = (int)ys.size();
+    if (n < 1 || n > MLORA_MAX_PROJ || xs.size() != n || was.size() != n || wbs.size() != n)
+        raise(PyExc_ValueError, "need 1..%d projections with one y, x, wa and wb each", MLORA_MAX_PROJ);
+    return PyLong_FromLong(ref_call(v[0], n, [&](int i) -> const at::Tensor & { return ys[i]; }, [&](int i) -> const at::Tensor & { return xs[i]; },
+                                    [&](int i) -> const at::Tensor & { return was[i]; }, [&](int i) -> const at::Tensor & { return wbs[i]; },
+                                    (int)as_int(v[5]), (float)PyFloat_AsDouble(v[6]), v[7] == Py_True, as_int(v[8]), as_int(v[9]),
+                                    as_int(v[10]), as_int(v[11])));
+}
+
+// deltas_ref(plan, x, weights (wa, wb of every projection in turn), layer, T, N, L, r): the deltas alone, in new tensors of x's
+// type; a tuple of them, or the C ABI's negative code
+PyObject *deltas_ref(PyObject *const *v, Py_ssize_t nargs)
+{
+    if (nargs != 8) raise(PyExc_TypeError, "deltas_ref takes 8 arguments");
+    const at::Tensor &x = tensor(v[1]);
+    const List w(v[2]);
+    const int n = (int)w.size() / 2;
+    if (n < 1 || n > MLORA_MAX_PROJ || w.size() != 2 * n) raise(PyExc_ValueError, "need 1..%d projections with one wa and wb each", MLORA_MAX_PROJ);
+    need_device(x);
+    at::Tensor y[MLORA_MAX_PROJ];
+    for (int i = 0; i < n; i++) {
+        if (w[2 * i + 1].dim() != 4) raise(PyExc_ValueError, "wa_T_all must be [N, L, r, Hin] and wb_T_all [N, L, Hout, r]");
+        y[i] = at::empty({x.size(0), w[2 * i + 1].size(2)}, x.options());
+    }
+    const int rc = ref_call(v[0], n, [&](int i) -> const at::Tensor & { return y[i]; }, [&](int) -> const at::Tensor & { return x; },
+                            [&](int i) -> const at::Tensor & { return w[2 * i]; }, [&](int i) -> const at::Tensor & { return w[2 * i + 1]; },
+                            (int)as_int(v[3]), 1.0f, false, as_int(v[4]), as_int(v[5]), as_int(v[6]), as_int(v[7]));
+    if (rc) return PyLong_FromLong(rc);
+    Ref out(PyTuple_New(n));
+    for (int i = 0; i < n; i++) {
+        PyObject *t = THPVariable_Wrap(y[i]);
+        if (!t) throw PyFail();
+        PyTuple_SET_ITEM(out.o, i, t);
+    }
+    Py_INCREF(out.o);
+    return out.o;
 }
 
 // ---------------------------------------------------------------- prefill
@@ -381,7 +414,7 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 }
 
 #define MLORA_FN(name) {#name, (PyCFunction)(void (*)())entry<name>, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {MLORA_FN(gather), MLORA_FN(bgmv), MLORA_FN(bgmv_ref), MLORA_FN(prefill_plan),
+PyMethodDef methods[] = {MLORA_FN(gather), MLORA_FN(bgmv), MLORA_FN(bgmv_ref), MLORA_FN(deltas_ref), MLORA_FN(prefill_plan),
                          MLORA_FN(sgmv_multi), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native launch path of mlora's eager calls.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
@@ -396,7 +429,7 @@ PyMODINIT_FUNC PyInit__host()
         {&s_row_off, "row_off"}, {&s_tok_rank, "tok_rank"}, {&s_tok_scale, "tok_scale"}, {&s_T, "T"}, {&s_workspace, "workspace"},
         {&s_n_slots, "n_slots"}, {&s_max_pages, "max_pages"}, {&s_page_rows, "page_rows"}, {&s_n_pages, "n_pages"},
         {&s_max_rank, "max_rank"}, {&s_tok_adapter, "tok_adapter"}, {&s_dtype_code, "dtype_code"}, {&s_projections, "projections"},
-        {&s_a_rows, "a_rows"}, {&s_b_rows, "b_rows"}};
+        {&s_a_rows, "a_rows"}, {&s_b_rows, "b_rows"}, {&s_buf, "buf"}};
     for (const auto &p : names)
         if (!(*p.first = PyUnicode_InternFromString(p.second))) return nullptr;
     return PyModule_Create(&module);

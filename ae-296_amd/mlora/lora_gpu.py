@@ -12,10 +12,14 @@ swapper process (``lora_gpu.py:76-118,246-296``) and the progress polling (``:29
 """
 from __future__ import annotations
 
+from operator import attrgetter
+
 import numpy as np
 import torch
 
-from . import ops
+from . import _ext, ops
+
+_QKV_WEIGHTS = attrgetter("q_down", "q_up", "k_down", "k_up", "v_down", "v_up")
 
 
 class Lora_GPU:
@@ -113,13 +117,17 @@ class Lora_GPU:
         bsz = x.shape[0]
         if not ops.ref_rank_supported(self.lora_rank):
             return tuple(self._invoke_single(n, x, layer_id, lora_ids) for n in "qkv")
-        plan = self._plan_for(bsz, lora_ids)
+        return self._deltas(x, layer_id, self._plan_for(bsz, lora_ids), _QKV_WEIGHTS(self))
+
+    @staticmethod
+    def _deltas(x, layer_id, plan, weights):
+        """The deltas of one input and the projections whose down and up tensors `weights` lists, in new tensors."""
         if not x.is_contiguous():
             x = x.contiguous()
-        ys = [torch.empty(bsz, self.output_size, device=x.device, dtype=x.dtype) for _ in range(3)]
-        ops.add_lora_bgmv_multi(ys, [x, x, x], [self.q_down, self.k_down, self.v_down], [self.q_up, self.k_up, self.v_up],
-                                plan, layer_id, 1.0, accumulate=False)
-        return tuple(ys)
+        ys = _ext.host().deltas_ref(plan, x, weights, layer_id, plan.T, plan.N, plan.L, plan.r)
+        if ys.__class__ is int:
+            _ext.check(ys)
+        return ys
 
     def _invoke_single(self, name, x, layer_id, lora_ids):
         bsz = x.shape[0]
@@ -146,13 +154,15 @@ class Lora_GPU:
         # (transformer_layer_infer.py:109-111): the first of the three calls computes all of them in one call pair,
         # the other two are answered from that result as long as it is the same input tensor object at the same
         # torch version, the same layer, the same plan and the same weight tensors at the same versions.
-        self._plan_for(bsz, lora_ids)
-        weights = [getattr(self, f"{n}_{side}") for n in "qkv" for side in ("down", "up")]
-        key = (x._version, tuple(x.shape), layer_id, self._plan_gen, tuple(w._version for w in weights))
-        fresh = (self._qkv_key != key or self._qkv_x is not x or name not in self._qkv
-                 or any(a is not b for a, b in zip(self._qkv_w, weights)))
+        plan = self._plan_for(bsz, lora_ids)
+        weights = _QKV_WEIGHTS(self)
+        a, b, c, d, e, f = weights
+        key = (x._version, x.shape, layer_id, self._plan_gen, a._version, b._version, c._version, d._version, e._version, f._version)
+        kept = self._qkv_w
+        fresh = (self._qkv_key != key or self._qkv_x is not x or name not in self._qkv or a is not kept[0] or b is not kept[1]
+                 or c is not kept[2] or d is not kept[3] or e is not kept[4] or f is not kept[5])
         if fresh:
-            q, k, v = self.invoke_one_layer_qkv(x, layer_id, lora_ids)
+            q, k, v = self._deltas(x, layer_id, plan, weights)
             self._qkv, self._qkv_x, self._qkv_w, self._qkv_key = {"q": q, "k": k, "v": v}, x, weights, key
         return self._qkv.pop(name)
 

@@ -48,3 +48,14 @@ def test_gather_refuses_a_larger_pool_and_other_buffers():
             _ext.host().gather(_pool(), dataclasses.replace(_plan(9, _pool()), **{name: other}), torch.zeros(9, dtype=torch.int32), 1)
     with pytest.raises(ValueError, match="device tensors"):      # the buffers fit: what is left to refuse is host memory
         _ext.host().gather(_pool(), _plan(9, _pool()), torch.zeros(9, dtype=torch.int32), 1)
+
+
+@pytest.mark.parametrize("weights, error", [
+    ([torch.zeros(2, 1, 8, 16), torch.zeros(2, 1, 24, 8)], "device tensors"),          # the input and the pool are in host memory
+    ([torch.zeros(2, 1, 8, 16)], "one wa and wb each"),
+    ([], "one wa and wb each"),
+])
+def test_reference_layout_deltas_check_their_tensors(weights, error):
+    plan = ops.RefDecodePlan(torch.zeros(3, dtype=torch.int64), 1, 2, 1, 8, torch.zeros(16, dtype=torch.uint8))
+    with pytest.raises(ValueError, match=error):
+        _ext.host().deltas_ref(plan, torch.zeros(3, 16), weights, 0, 3, 2, 1, 8)
