@@ -46,7 +46,7 @@ struct Ref {        // an owned reference
     Ref &operator=(const Ref &) = delete;
 };
 
-PyObject *s_page_tbl, *s_rank, *s_scaling, *s_work, *s_group, *s_vws, *s_perm, *s_seg_start, *s_seg_len, *s_seg_adapter,
+PyObject *s_page_tbl, *s_rank, *s_scaling, *s_work, *s_group, *s_perm, *s_seg_start, *s_seg_len, *s_seg_adapter,
     *s_chunk_start, *s_chunk_len, *s_chunk_adapter, *s_counters, *s_row_off, *s_tok_rank, *s_tok_scale, *s_T, *s_workspace,
     *s_n_slots, *s_max_pages, *s_page_rows, *s_n_pages, *s_max_rank, *s_tok_adapter, *s_dtype_code, *s_projections, *s_a_rows, *s_b_rows, *s_buf;
 
@@ -258,19 +258,6 @@ PyObject *bgmv(PyObject *const *v, Py_ssize_t nargs)
     return PyLong_FromLong(rc);
 }
 
-// The reference-layout plan's intermediate: at least `bytes` on the device of `like`, allocated when it is missing or too small.
-at::Tensor intermediate(PyObject *plan, int64_t bytes, const at::Tensor &like)
-{
-    {
-        Ref have(PyObject_GetAttr(plan, s_vws));
-        if (have.o != Py_None && tensor(have.o).numel() >= bytes) return tensor(have.o);
-    }
-    at::Tensor t = at::empty({bytes}, like.options().dtype(at::kByte));
-    Ref made(THPVariable_Wrap(t));
-    if (PyObject_SetAttr(plan, s_vws, made.o)) throw PyFail();
-    return t;
-}
-
 // A reference-layout decode call over n projections: every check, then the launch.  y, x, a, b give the tensors of a projection.
 template <typename Y, typename X, typename A, typename B>
 int ref_call(PyObject *plan, int n, Y y_of, X x_of, A a_of, B b_of, int layer, float scale, bool accumulate, int64_t T, int64_t N, int64_t L, int64_t r)
@@ -297,7 +284,8 @@ int ref_call(PyObject *plan, int n, Y y_of, X x_of, A a_of, B b_of, int layer, f
     }
     if (type != at::kHalf && type != at::kBFloat16) raise(PyExc_TypeError, "mlora kernels take float16 or bfloat16 tensors");
     const int64_t bytes = mlora_bgmv_workspace_bytes(n, (int)T, max_hin, (int)r);
-    const at::Tensor room = bytes > 0 ? intermediate(plan, bytes, y_of(0)) : at::Tensor();
+    // this call's own, as in bgmv
+    const at::Tensor room = bytes > 0 ? at::empty({bytes}, y_of(0).options().dtype(at::kByte)) : at::Tensor();
     void *ws = room.defined() ? room.data_ptr() : nullptr;
     return launch(mlora_bgmv_reflayout_multi, n, y, x, a, b, hin, hout, attr_ptr(plan, s_buf), (int)T, (int)N, (int)L, (int)r,
                   layer, scale, (int)attr_int(plan, s_group), type == at::kHalf ? MLORA_F16 : MLORA_BF16, accumulate, ws, bytes, stream());
@@ -423,7 +411,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native launch path of mlo
 PyMODINIT_FUNC PyInit__host()
 {
     const std::pair<PyObject **, const char *> names[] = {
-        {&s_page_tbl, "page_tbl"}, {&s_rank, "rank"}, {&s_scaling, "scaling"}, {&s_work, "work"}, {&s_group, "group"}, {&s_vws, "vws"},
+        {&s_page_tbl, "page_tbl"}, {&s_rank, "rank"}, {&s_scaling, "scaling"}, {&s_work, "work"}, {&s_group, "group"},
         {&s_perm, "perm"}, {&s_seg_start, "seg_start"}, {&s_seg_len, "seg_len"}, {&s_seg_adapter, "seg_adapter"},
         {&s_chunk_start, "chunk_start"}, {&s_chunk_len, "chunk_len"}, {&s_chunk_adapter, "chunk_adapter"}, {&s_counters, "counters"},
         {&s_row_off, "row_off"}, {&s_tok_rank, "tok_rank"}, {&s_tok_scale, "tok_scale"}, {&s_T, "T"}, {&s_workspace, "workspace"},

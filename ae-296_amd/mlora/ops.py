@@ -237,7 +237,6 @@ class RefDecodePlan:
     L: int
     r: int
     buf: torch.Tensor              # uint8: perm, segments, chunks, counters, work records
-    vws: Optional[torch.Tensor] = None
 
     @property
     def T(self) -> int:

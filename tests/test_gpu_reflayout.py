@@ -257,3 +257,34 @@ def test_lora_gpu_keeps_its_workspace_for_a_shorter_prefill():
         assert torch.allclose(y.float(), want, rtol=RTOL, atol=ATOL)
         seen.append(g._workspace)
     assert seen[0] is seen[1]
+
+
+def test_reference_calls_that_share_a_plan_on_two_streams():
+    """A call leaves its plan as it was (its intermediate is its own), so calls of one plan may overlap."""
+    from mlora import add_lora_bgmv_multi, plan_decode_ref
+    N, L, r, H, T = 7, 2, 32, 1024, 40
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    rand = lambda *shape: torch.randn(*shape, device="cuda", generator=gen).half()  # noqa: E731
+    wa, wb, ids = rand(N, L, r, H) * 0.05, rand(N, L, H, r) * 0.05, torch.arange(T, device="cuda") % N
+    plan = plan_decode_ref(ids, N, L, r)
+    before = dict(vars(plan))
+    xs = [rand(T, H) for _ in range(6)]
+    out = lambda: [torch.full((T, H), float("nan"), device="cuda").half() for _ in range(2)]  # noqa: E731
+    call = lambda ys, x: add_lora_bgmv_multi(ys, [x, x], [wa, wa], [wb, wb], plan, 1, 1.0, accumulate=False)  # noqa: E731
+    say("reference-layout calls on two streams and one plan")
+    want = []
+    for x in xs:
+        want.append(out())
+        call(want[-1], x)
+    assert vars(plan).keys() == before.keys() and all(v is before[k] for k, v in vars(plan).items())
+    got = [[out() for _ in range(30)] for _ in range(2)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for i in range(30):
+        for j in range(2):
+            with torch.cuda.stream(streams[j]):
+                call(got[j][i], xs[(j + i) % 6])
+    torch.cuda.synchronize()
+    for j in range(2):
+        for i in range(30):
+            assert all(torch.equal(a, b) for a, b in zip(got[j][i], want[(j + i) % 6])), (j, i)
