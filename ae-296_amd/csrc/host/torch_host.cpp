@@ -14,6 +14,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../../include/mlora.h"
@@ -334,6 +335,22 @@ PyObject *deltas_ref(PyObject *const *v, Py_ssize_t nargs)
     return out.o;
 }
 
+// order(): (thread, device, stream, capture number or 0): what a program queues under equal values runs in the order it is queued.
+PyObject *order(PyObject *const *, Py_ssize_t nargs)
+{
+    if (nargs != 0) raise(PyExc_TypeError, "order takes no arguments");
+    const c10::hip::HIPStream s = c10::hip::getCurrentHIPStream();
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    // the null stream cannot be captured, and asking it during another stream's capture is an error
+    if (s.stream() && hipStreamGetCaptureInfo(s.stream(), &status, &id) != hipSuccess)
+        raise(PyExc_RuntimeError, "the capture state of the current stream is not known: %s", hipGetErrorString(hipGetLastError()));
+    Ref t(Py_BuildValue("(kiKK)", PyThread_get_thread_ident(), (int)s.device_index(), (unsigned long long)(uintptr_t)s.stream(),
+                        status == hipStreamCaptureStatusNone ? 0ULL : id));
+    Py_INCREF(t.o);
+    return t.o;
+}
+
 // ---------------------------------------------------------------- prefill
 struct Segments { const int32_t *start, *len, *adapter; int64_t n; };
 
@@ -402,7 +419,7 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 }
 
 #define MLORA_FN(name) {#name, (PyCFunction)(void (*)())entry<name>, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {MLORA_FN(gather), MLORA_FN(bgmv), MLORA_FN(bgmv_ref), MLORA_FN(deltas_ref), MLORA_FN(prefill_plan),
+PyMethodDef methods[] = {MLORA_FN(gather), MLORA_FN(bgmv), MLORA_FN(bgmv_ref), MLORA_FN(deltas_ref), MLORA_FN(order), MLORA_FN(prefill_plan),
                          MLORA_FN(sgmv_multi), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native launch path of mlora's eager calls.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

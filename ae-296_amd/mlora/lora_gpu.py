@@ -12,6 +12,7 @@ swapper process (``lora_gpu.py:76-118,246-296``) and the progress polling (``:29
 """
 from __future__ import annotations
 
+import itertools
 from operator import attrgetter
 
 import numpy as np
@@ -54,18 +55,19 @@ class Lora_GPU:
                             for i in range(self.batch_size)]
         self._workspace = None
         self._workspace_for = (0, 0)                   # rows and requests it was sized for
-        # Grouping of the current decode batch by adapter.  It is served again only for the very tensor object it was
-        # made from (`_plan_src`, kept alive here so that neither its address nor its Python identity can pass to
-        # another tensor) at the same torch version counter: a serving loop builds `lora_ids` afresh every step
-        # (pre_process.py:50,100), and a new tensor of the same size often gets the freed one's address.
-        self._plan = None
-        self._plan_src = None
-        self._plan_ver = None
-        self._plan_gen = 0
-        self._qkv = None           # q, k, v deltas of the last decode input ...
-        self._qkv_x = None         # ... the input tensor itself (kept alive for the same reason) ...
-        self._qkv_w = []           # ... the six weight tensors ...
-        self._qkv_key = None       # ... and what else they were computed from
+        # Grouping of the current decode batch by adapter: (plan, the index tensor it was made from, its torch version, the
+        # order it belongs to, its number).  It is served again only for the very tensor object it was made from (kept
+        # alive here so that neither its address nor its Python identity can pass to another tensor) at the same version
+        # counter: a serving loop builds `lora_ids` afresh every step (pre_process.py:50,100), and a new tensor of the same
+        # size often gets the freed one's address.  A plan that an invoke call made by itself belongs to that call's thread,
+        # stream and graph capture (mlora._host.order): a call elsewhere is not ordered behind the launch that writes it, and
+        # makes its own.  One that plan_decode made (order None) serves wherever the program has ordered its calls behind that.
+        self._plan_state = (None, None, None, None, 0)
+        self._plan_gen = 0                             # number of the newest plan
+        self._plan_numbers = itertools.count(1)
+        # q, k, v deltas of the last decode input that were not asked for yet: (what they were computed from, the input
+        # tensor itself and the six weight tensors (kept alive for the same reason), the deltas)
+        self._qkv = None
 
     def _rand(self, n, rows, cols):
         """[n, L, rows, cols] * 0.001, stored transposed and contiguous as the reference does."""
@@ -95,20 +97,27 @@ class Lora_GPU:
         per step; ``invoke_one_layer_*`` call it themselves when they are handed another index tensor than the one
         the current plan was made from, or the same one after torch has written to it.  A tensor whose contents
         were changed behind torch's back (a raw kernel writing through its pointer) needs this call."""
+        return self._group(bsz, lora_ids, None)[0]
+
+    def _group(self, bsz, lora_ids, order):
+        """A new plan and its number.  It takes the buffers of the plan before it only where no call elsewhere may read them."""
         src = self._index_source(bsz, lora_ids)
         cur_inds = self._indices(bsz, lora_ids, self.q_down.device)
-        reuse = self._plan if (self._plan is not None and self._plan.T == bsz) else None
-        self._plan = ops.plan_decode_ref(cur_inds, self.batch_size, self.n_layers, self.lora_rank, out=reuse)
-        self._plan_src, self._plan_ver = src, src._version
-        self._plan_gen += 1
-        self._qkv_key = None
-        return self._plan
+        last, _, _, belongs, _ = self._plan_state
+        mine = belongs == order or (order is None and belongs == _ext.host().order())
+        reuse = last if (last is not None and mine and last.T == bsz) else None
+        plan = ops.plan_decode_ref(cur_inds, self.batch_size, self.n_layers, self.lora_rank, out=reuse)
+        self._plan_gen = number = next(self._plan_numbers)
+        self._plan_state = (plan, src, src._version, order, number)
+        self._qkv = None
+        return plan, number
 
-    def _plan_for(self, bsz, lora_ids):
+    def _plan_for(self, bsz, lora_ids, order):
         src = self._index_source(bsz, lora_ids)
-        if self._plan is None or self._plan_src is not src or self._plan_ver != src._version or self._plan.T != bsz:
-            self.plan_decode(bsz, lora_ids)
-        return self._plan
+        plan, made_from, version, belongs, number = self._plan_state
+        if plan is None or made_from is not src or version != src._version or plan.T != bsz or (belongs is not None and belongs != order):
+            return self._group(bsz, lora_ids, order)
+        return plan, number
 
     def invoke_one_layer_qkv(self, x, layer_id, lora_ids=None):
         """The q, k and v deltas of one decode layer in one call pair (the reference makes three
@@ -117,7 +126,7 @@ class Lora_GPU:
         bsz = x.shape[0]
         if not ops.ref_rank_supported(self.lora_rank):
             return tuple(self._invoke_single(n, x, layer_id, lora_ids) for n in "qkv")
-        return self._deltas(x, layer_id, self._plan_for(bsz, lora_ids), _QKV_WEIGHTS(self))
+        return self._deltas(x, layer_id, self._plan_for(bsz, lora_ids, _ext.host().order())[0], _QKV_WEIGHTS(self))
 
     @staticmethod
     def _deltas(x, layer_id, plan, weights):
@@ -153,18 +162,23 @@ class Lora_GPU:
         # ``_get_qkv`` asks for q, k and v of the same input one after the other
         # (transformer_layer_infer.py:109-111): the first of the three calls computes all of them in one call pair,
         # the other two are answered from that result as long as it is the same input tensor object at the same
-        # torch version, the same layer, the same plan and the same weight tensors at the same versions.
-        plan = self._plan_for(bsz, lora_ids)
+        # torch version, the same layer, the same plan, the same weight tensors at the same versions, and the same thread,
+        # stream and graph capture: a call elsewhere is not ordered behind the launches that write the result.
+        order = _ext.host().order()
+        plan, number = self._plan_for(bsz, lora_ids, order)
         weights = _QKV_WEIGHTS(self)
         a, b, c, d, e, f = weights
-        key = (x._version, x.shape, layer_id, self._plan_gen, a._version, b._version, c._version, d._version, e._version, f._version)
-        kept = self._qkv_w
-        fresh = (self._qkv_key != key or self._qkv_x is not x or name not in self._qkv or a is not kept[0] or b is not kept[1]
-                 or c is not kept[2] or d is not kept[3] or e is not kept[4] or f is not kept[5])
-        if fresh:
-            q, k, v = self._deltas(x, layer_id, plan, weights)
-            self._qkv, self._qkv_x, self._qkv_w, self._qkv_key = {"q": q, "k": k, "v": v}, x, weights, key
-        return self._qkv.pop(name)
+        key = (x._version, x.shape, layer_id, number, order, a._version, b._version, c._version, d._version, e._version, f._version)
+        if (kept := self._qkv) is not None:
+            made_from, of, (ka, kb, kc, kd, ke, kf), left = kept
+            if of is x and made_from == key and a is ka and b is kb and c is kc and d is kd and e is ke and f is kf:
+                y = left.pop(name, None)
+                if y is not None:
+                    return y
+        left = dict(zip("qkv", self._deltas(x, layer_id, plan, weights)))
+        y = left.pop(name)
+        self._qkv = (key, x, weights, left)
+        return y
 
     def invoke_one_layer_q(self, x, layer_id, prefill=False, lora_ids=None):
         return self._invoke("q", x, layer_id, prefill, lora_ids)
@@ -178,7 +192,7 @@ class Lora_GPU:
     # ------------------------------------------------------------------ slot management
     def prepare_lora_prefill(self, batch_size):
         """lora_gpu.py:190-200: fresh random prefill adapters, one slot per request."""
-        self._qkv_key = None
+        self._qkv = None
         for name in ("q", "k", "v"):
             setattr(self, f"{name}_down_prefill", self._rand(batch_size, self.in_size, self.lora_rank))
             setattr(self, f"{name}_up_prefill", self._rand(batch_size, self.lora_rank, self.output_size))
@@ -186,7 +200,7 @@ class Lora_GPU:
     def merge_lora_prefill(self, bsz, re_inds=None):
         """lora_gpu.py:202-217: copy the first bsz prefill slots into decode slots (random targets
         in the reference; pass re_inds to choose them)."""
-        self._qkv_key = None                    # weights change: results computed from the old ones are not served again
+        self._qkv = None                        # weights change: results computed from the old ones are not served again
         if re_inds is None:
             re_inds = np.random.randint(0, self.batch_size, size=bsz)
         for idx, re_ind in enumerate(re_inds):
@@ -201,7 +215,7 @@ class Lora_GPU:
         is applied to the adapter axis here."""
         if running_bsz <= 0:
             return
-        self._qkv_key = None
+        self._qkv = None
         if chosen is None:
             chosen = np.random.randint(0, running_bsz, size=len(rm_ids))
         for rm_id in chosen:

@@ -288,3 +288,57 @@ def test_reference_calls_that_share_a_plan_on_two_streams():
     for j in range(2):
         for i in range(30):
             assert all(torch.equal(a, b) for a, b in zip(got[j][i], want[(j + i) % 6])), (j, i)
+
+
+@pytest.mark.parametrize("planned", [False, True])
+def test_lora_gpu_calls_of_a_layer_on_other_streams_and_in_captures(planned):
+    """q on one stream, k on another while the first is still busy, v in a graph capture: each is computed where it is
+    called, from what the input holds there."""
+    cfg = dict(n_layers=2, batch_size=8, lora_rank=16, hidden_dim=1024, tp_degree=1, max_prefill_batch_size=1)
+    g = Lora_GPU(cfg, seed=3)
+    for name in "qkv":
+        getattr(g, f"{name}_down").mul_(100.0)
+        getattr(g, f"{name}_up").mul_(100.0)
+    x = torch.randn(19, 1024, device="cuda", dtype=torch.float16)
+    ids = torch.randint(0, 8, (19,), device="cuda")
+
+    def want_of(name, x):
+        down, up = getattr(g, f"{name}_down"), getattr(g, f"{name}_up")
+        return torch.stack([x[i].float() @ down[ids[i], 1].float().t() @ up[ids[i], 1].float().t() for i in range(19)])
+
+    want = {n: want_of(n, x) for n in "qkv"}
+    close = lambda got, ref: torch.allclose(got.float(), ref, rtol=RTOL, atol=ATOL)  # noqa: E731
+    busy = torch.randn(4096, 4096, device="cuda")
+    if planned:
+        g.plan_decode(19, ids)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    say(f"Lora_GPU: q on a busy stream, k on another, planned={planned}")
+    with torch.cuda.stream(streams[0]):
+        for _ in range(40):
+            busy = torch.mm(busy, busy).mul_(1e-3)
+        q = g.invoke_one_layer_q(x, 1, False, lora_ids=ids)
+    with torch.cuda.stream(streams[1]):
+        k = g.invoke_one_layer_k(x, 1, False, lora_ids=ids)
+    streams[1].synchronize()
+    assert close(k, want["k"])
+    torch.cuda.synchronize()
+    assert close(q, want["q"])
+
+    say("Lora_GPU: q before a capture, k and v in it, q after it")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(streams[0]):
+        g.invoke_one_layer_q(x, 1, False, lora_ids=ids)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=streams[0]):
+            k = g.invoke_one_layer_k(x, 1, False, lora_ids=ids)
+            v = g.invoke_one_layer_v(x, 1, False, lora_ids=ids)
+        q = g.invoke_one_layer_q(x, 1, False, lora_ids=ids)
+    torch.cuda.synchronize()
+    assert close(q, want["q"])
+    for rep in range(3):
+        x.copy_(torch.randn(19, 1024, device="cuda"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert close(k, want_of("k", x)) and close(v, want_of("v", x)), rep
