@@ -833,7 +833,7 @@ void shrink_shape(mlora::SgmvArgs &a, int tiles, int max_rank, const SgmvWs &w)
         }
 }
 
-void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w, int max_rank)
+void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w)
 {
     char *base = static_cast<char *>(workspace);
     int32_t *ip = reinterpret_cast<int32_t *>(base);
@@ -841,14 +841,21 @@ void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w, int max_rank)
     a.n_tiles = ip + 3 * (size_t)w.max_tiles;
     a.tok_cover = reinterpret_cast<int32_t *>(base + w.off_cover);
     a.tile_rec = reinterpret_cast<int32_t *>(base + w.off_rec);
-    a.max_tiles = w.max_tiles;
-    const int tiles = a.seg_uniform_len > 0 ? a.n_seg * ((a.seg_uniform_len + SG_TM - 1) / SG_TM) : (a.T + SG_TM / 2 * (a.n_seg - 1) + SG_TM - 1) / SG_TM;
-    a.tiles = tiles;
     for (int p = 0; p < a.n_proj; p++) {
         char *pb = base + w.off_proj + w.per_proj * p;
         a.pr[p].v = reinterpret_cast<float *>(pb);
         a.pr[p].vhi = reinterpret_cast<uint16_t *>(pb + w.off_hi);
         a.pr[p].vlo = reinterpret_cast<uint16_t *>(pb + w.off_lo);
+    }
+}
+
+// The shape of a call's launches, but for what sgmv_launch_shape adds.
+void apply_shape(mlora::SgmvArgs &a, int max_rank, const SgmvWs &w)
+{
+    const int tiles = a.seg_uniform_len > 0 ? a.n_seg * ((a.seg_uniform_len + SG_TM - 1) / SG_TM) : (a.T + SG_TM / 2 * (a.n_seg - 1) + SG_TM - 1) / SG_TM;
+    a.tiles = tiles;
+    a.max_tiles = a.seg_uniform_len > 0 ? tiles : w.max_tiles;
+    for (int p = 0; p < a.n_proj; p++) {
         int ncb = 0;
         const int cols = expand_block_cols(a.n_proj, w.max_tiles, a.pr[p].hout, &ncb);
         a.pr[p].cols = cols;
@@ -887,6 +894,33 @@ int mlora_sgmv_splits(int T, int n_seg, int n_proj, int64_t workspace_bytes)
     if (T <= 0 || n_seg <= 0 || n_proj < 1 || n_proj > MLORA_MAX_PROJ || workspace_bytes < 0) return 0;
     const SgmvWs w = sgmv_layout(T, n_seg, n_proj, workspace_bytes);
     return (int64_t)w.total <= workspace_bytes ? w.ks_cap : 0;
+}
+
+int mlora_sgmv_shape(int n_proj, const void *const *x, const int32_t *hin, const int32_t *hout, int T, int n_seg, int seg_len,
+                     int max_rank, int accumulate, int64_t workspace_bytes, int32_t *shape)
+{
+    if (n_proj < 1 || n_proj > MLORA_MAX_PROJ) return fail(MLORA_ERANGE, "n_proj must be in 1..%d (got %d)", MLORA_MAX_PROJ, n_proj);
+    if (!x || !hin || !hout || !shape) return fail(MLORA_EINVAL, "NULL pointer");
+    if (T <= 0 || n_seg <= 0 || seg_len < 0) return fail(MLORA_EINVAL, "T and n_seg must be positive (got %d, %d), seg_len >= 0", T, n_seg);
+    if (seg_len > 0 && ((int64_t)n_seg * seg_len != T || n_proj != 1 || accumulate))
+        return fail(MLORA_EINVAL, "equally long segments: T = n_seg * seg_len, one projection, y = delta");
+    if (max_rank < 1 || max_rank > MLORA_MAX_RANK) return fail(MLORA_ERANGE, "max_rank must be in 1..%d (got %d)", MLORA_MAX_RANK, max_rank);
+    mlora::SgmvArgs a;
+    memset(&a, 0, sizeof(a));
+    a.n_proj = n_proj; a.T = T; a.n_seg = n_seg; a.seg_uniform_len = seg_len; a.accumulate = accumulate ? 1 : 0;
+    for (int p = 0; p < n_proj; p++) {
+        const int rc = check_dims(hin[p], hout[p]);
+        if (rc) return rc;
+        a.pr[p].x = x[p]; a.pr[p].hin = hin[p]; a.pr[p].hout = hout[p];
+    }
+    const SgmvWs w = sgmv_layout(T, n_seg, n_proj, workspace_bytes < 0 ? 0 : workspace_bytes);
+    if (workspace_bytes < (int64_t)w.total)
+        return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)w.total);
+    apply_shape(a, max_rank, w);
+    mlora::sgmv_launch_shape(a, max_rank, mlora::SGMV_APPLY);
+    shape[0] = a.share_x; shape[1] = a.stream_x; shape[2] = a.reduce; shape[3] = a.few;
+    for (int p = 0; p < n_proj; p++) shape[4 + p] = a.pr[p].ksplit;
+    return MLORA_OK;
 }
 
 int64_t mlora_sgmv_multi_workspace_bytes(int T, int n_seg, int n_proj)
@@ -932,7 +966,8 @@ static int sgmv_common(int n_proj, void *const *y, const void *const *x, const v
         return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)w.total);
     a.seg_start = seg_start; a.seg_len = seg_len; a.seg_adapter = seg_adapter; a.n_seg = n_seg;
     a.T = T; a.accumulate = accumulate ? 1 : 0; a.b_transposed = 0; a.seg_uniform_len = 0; a.tile_aligned = tile_aligned;
-    carve(a, workspace, w, max_rank);
+    carve(a, workspace, w);
+    apply_shape(a, max_rank, w);
     rc = mlora::launch_sgmv(a, dtype, max_rank, phases, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "sgmv launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;
@@ -1081,7 +1116,8 @@ int mlora_gemm_lora_split(int n_proj, void *const *y, const void *const *x, cons
             return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)ws.total);
         a.seg_start = seg_start; a.seg_len = seg_len; a.seg_adapter = seg_adapter; a.n_seg = n_seg;
         a.T = T; a.accumulate = 0; a.b_transposed = 0; a.seg_uniform_len = 0;
-        carve(a, workspace, ws, max_rank);
+        carve(a, workspace, ws);
+        apply_shape(a, max_rank, ws);
         rc = mlora::launch_sgmv(a, dtype, max_rank, mlora::SGMV_SHRINK, static_cast<hipStream_t>(stream));
         if (rc) return fail(MLORA_ELAUNCH, "shrink launch failed: %s", hipGetErrorString((hipError_t)rc));
         for (int p = 0; p < n_proj; p++) {
@@ -1130,8 +1166,8 @@ int mlora_prefill_reflayout(void *y, const void *x, const void *A_T, const void 
     a.pr[0].b_rows = static_cast<const uint16_t *>(B_T) + (size_t)layer_idx * hout * r;
     a.pr[0].hin = hin; a.pr[0].hout = hout;
     a.n_seg = B; a.T = T; a.accumulate = 0; a.b_transposed = 1; a.seg_uniform_len = Lpad;
-    carve(a, workspace, w, r);
-    a.max_tiles = B * ((Lpad + SG_TM - 1) / SG_TM);
+    carve(a, workspace, w);
+    apply_shape(a, r, w);
     rc = mlora::launch_sgmv(a, dtype, r, mlora::SGMV_PLAN | mlora::SGMV_APPLY, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "prefill launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;

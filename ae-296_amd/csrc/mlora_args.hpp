@@ -147,8 +147,11 @@ struct SgmvArgs {
     int accumulate;
     int b_transposed;      // B given as [hout, r] blocks (reference layout)
     int seg_uniform_len;   // > 0: segment s covers [s*len, (s+1)*len), adapter s (reference prefill)
-    int scaled;            // shrink with one K split: store the halves of scaling * sum (set by the launcher)
-    int fold;              // expand: sum the K splits itself instead of reading what the reduce launch made (set by the launcher)
+    // set by sgmv_launch_shape
+    int scaled;            // shrink with one K split: store the halves of scaling * sum
+    int few;               // expand by pieces of 16 tokens and 256 columns
+    int fold;              // expand: sum the K splits itself instead of reading what the reduce launch made
+    int reduce;            // there is a reduce launch
     int tile_aligned;      // plan: cut tiles at multiples of 64 tokens (and at segment ends) instead of every 64 tokens of a segment
     // workspace carve-up
     int32_t *tile_seg;     // [max_tiles]
@@ -208,6 +211,7 @@ int launch_assist_import(const AssistArgs &a, hipStream_t s);
 constexpr int SGMV_PLAN = 1;    // write the tile list and records into the workspace
 constexpr int SGMV_APPLY = 2;   // shrink, reduce, expand (the workspace already holds the plan unless SGMV_PLAN is set too)
 constexpr int SGMV_SHRINK = 4;  // the shrink launch alone: its partial sums feed the base GEMM + LoRA kernel
+void sgmv_launch_shape(SgmvArgs &a, int max_rank, int phases);   // what follows from the fields the caller has filled
 int launch_sgmv(const SgmvArgs &a, int dtype, int max_rank, int phases, hipStream_t s);
 int launch_gemm_lora(const GemmLoraArgs &a, int dtype, int max_rank, hipStream_t s);
 // the shape for a.T, a.n_proj and the projections' hin and hout; returns the bytes of partial sums it takes

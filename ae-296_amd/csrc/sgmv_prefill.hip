@@ -916,6 +916,22 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p
     }
 }
 
+void sgmv_launch_shape(SgmvArgs &a, int max_rank, int phases)
+{
+    a.scaled = !(phases & SGMV_APPLY);                          // the base GEMM + LoRA kernel takes the scaled intermediate
+    if (a.scaled) return;
+    long long few_wgs = 0;
+    int most = 1;
+    for (int q = 0; q < a.n_proj; q++) {
+        few_wgs += (long long)a.tiles * 4 * ((a.pr[q].hout + FEW_COLS - 1) / FEW_COLS);
+        most = a.pr[q].ksplit > most ? a.pr[q].ksplit : most;
+    }
+    a.few = max_rank > 32 && few_wgs <= FEW_EXPAND;
+    // Few K splits are summed by the expand itself; rows outside every segment are zeroed by the reduce launch only.
+    a.fold = most <= FOLD_SPLITS && (max_rank <= 32 || a.few) && (a.accumulate || a.seg_uniform_len > 0);
+    a.reduce = !a.fold;
+}
+
 template <int DT, int RMAX>
 static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
 {
@@ -927,8 +943,9 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
         if (rc) return rc;
     }
     if (!(phases & (SGMV_APPLY | SGMV_SHRINK))) return 0;
-    // The caller has filled pr[], the shrink groups, ksplit, cols and ncb; the grid ends are set here.
+    // The caller has filled pr[], the shrink groups, ksplit, cols and ncb; the rest of the shape and the grid ends are set here.
     SgmvArgs g = a;
+    sgmv_launch_shape(g, RMAX, phases);
     unsigned end = 0;
     for (int q = 0; q < g.n_grp; q++) {
         end += (unsigned)(place_grid(g.max_tiles, g.pr[g.grp_first[q]].ksplit) * (g.share_x ? 1 : g.grp_n[q]));
@@ -936,16 +953,12 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     }
     const unsigned sgrid = end;
     end = 0;
-    long long few_wgs = 0;
-    for (int q = 0; q < g.n_proj; q++) few_wgs += (long long)g.tiles * 4 * ((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS);
-    const bool few = RMAX > 32 && few_wgs <= FEW_EXPAND;
     for (int q = 0; q < g.n_proj; q++) {
-        end += few ? (unsigned)g.max_tiles * 4u * (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
+        end += g.few ? (unsigned)g.max_tiles * 4u * (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
         g.ex_end[q] = end;
     }
     const unsigned egrid = end;
     if ((g.seg_uniform_len > 0) != (g.b_transposed != 0)) return (int)hipErrorInvalidValue;
-    g.scaled = !(phases & SGMV_APPLY);                          // the base GEMM + LoRA kernel takes the scaled intermediate
     if (g.seg_uniform_len > 0 && g.share_x) return (int)hipErrorInvalidValue;
     const dim3 threads(SG_NT * (g.share_x ? SH_KG<true> : SH_KG<false>));
     if (g.seg_uniform_len > 0) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, true, false>), dim3(sgrid), threads, 0, s, g);
@@ -953,18 +966,14 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     else hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, false, false>), dim3(sgrid), threads, 0, s, g);
     rc = (int)hipGetLastError();
     if (rc || !(phases & SGMV_APPLY)) return rc;
-    // Few K splits are summed by the expand itself; rows outside every segment are zeroed by the reduce launch only.
-    int most = 1;
-    for (int q = 0; q < g.n_proj; q++) most = g.pr[q].ksplit > most ? g.pr[q].ksplit : most;
-    g.fold = most <= FOLD_SPLITS && (RMAX <= 32 || few) && (g.accumulate || g.seg_uniform_len > 0);
-    if (!g.fold) {
+    if (g.reduce) {
         const long long n = (long long)g.T * (RMAX / 8);
         hipLaunchKernelGGL((sgmv_reduce_kernel<DT, RMAX>), dim3((unsigned)((n + 255) / 256), (unsigned)g.n_proj), dim3(256), 0, s, g);
         rc = (int)hipGetLastError();
         if (rc) return rc;
     }
     if constexpr (RMAX > 32) {
-        if (few) {
+        if (g.few) {
             if (g.b_transposed) hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, true>), dim3(egrid), dim3(SG_NT), 0, s, g);
             else hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, false>), dim3(egrid), dim3(SG_NT), 0, s, g);
             return (int)hipGetLastError();

@@ -70,6 +70,7 @@ SIGNATURES = {
                                   _i32, _i64, _i32, _i32, _i32, _vp, _i64, _vp]),
     "mlora_sgmv_multi_workspace_bytes": (_i64, [_i32, _i32, _i32]),
     "mlora_sgmv_expand_cols": (_i32, [_i32, _i32, _i32, _i32]),
+    "mlora_sgmv_shape": (_i32, [_i32, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i64, _vp]),
     "mlora_sgmv_multi_planned": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32,
                                         _i32, _i32, _i64, _i32, _i32, _i32, _vp, _i64, _vp]),
     "mlora_gemm_lora_planned": (_i32, [_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _i32,

@@ -356,6 +356,16 @@ int64_t mlora_sgmv_multi_workspace_bytes(int T, int n_seg, int n_proj);
  * counterpart in the reference (its prefill is two library GEMMs, lora_gpu.py:127-128).
  */
 int mlora_sgmv_expand_cols(int T, int n_seg, int n_proj, int hout);
+/*
+ * The shape of such a call's launches with a workspace of that many bytes (seg_len > 0: of mlora_prefill_reflayout over
+ * n_seg equal segments): shape[0] 1 where one shrink workgroup serves up to three projections of one x, [1] where x is read
+ * by streaming loads, [2] where there is a reduce launch, [3] where the expand works by pieces of 16 tokens and 256 columns,
+ * [4 + p] K splits of projection p.  x, hin, hout are HOST arrays of n_proj entries; x[p] is only compared, never read.
+ * Informational, like the workspace sizes; MLORA_ENOSPACE where the call would not fit.  No counterpart in the reference.
+ */
+#define MLORA_SGMV_SHAPE_WORDS (4 + MLORA_MAX_PROJ)
+int mlora_sgmv_shape(int n_proj, const void *const *x, const int32_t *hin, const int32_t *hout, int T, int n_seg, int seg_len,
+                     int max_rank, int accumulate, int64_t workspace_bytes, int32_t *shape);
 int mlora_sgmv_multi_planned(int n_proj, void *const *y, const void *const *x,
                              const void *const *a_rows, const void *const *b_rows,
                              const int32_t *hin, const int32_t *hout,

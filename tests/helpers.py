@@ -108,3 +108,16 @@ def exact_round16(fr: Fraction, dtype: int) -> int:
     if n < (1 << mant):                          # subnormal
         return sign | n
     return sign | ((e + bias) << mant) | (n - (1 << mant))
+
+
+def sgmv_shape(widths, inputs, T, n_seg, max_rank, accumulate=True, seg_len=0, workspace_bytes=1 << 50):
+    """The shape the library takes for a prefill call over projections of widths (hin, hout), projection p reading the input
+    numbered inputs[p] (mlora_sgmv_shape)."""
+    import ctypes as C
+    from mlora import _ext
+    n = len(widths)
+    x = (C.c_void_p * n)(*(4096 * (i + 1) for i in inputs))
+    hin, hout = ((C.c_int32 * n)(*(w[i] for w in widths)) for i in (0, 1))
+    shape = (C.c_int32 * (4 + _ext.MAX_PROJ))()
+    _ext.check(_ext.lib().mlora_sgmv_shape(n, x, hin, hout, T, n_seg, seg_len, max_rank, int(accumulate), workspace_bytes, shape))
+    return dict(share=shape[0], stream=shape[1], reduce=shape[2], few=shape[3], splits=list(shape[4:4 + n]))

@@ -6,6 +6,7 @@ import re
 
 import pytest
 
+from helpers import sgmv_shape
 from mlora import _ext
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -152,6 +153,24 @@ def test_a_prefill_workspace_serves_every_smaller_call(T):
                         grew += got < full
     assert grew > 0 or T <= 64                   # the sweep meets calls that would take more than they are given
     assert lib.mlora_sgmv_splits(T, 1, 1, 256) == 0
+
+
+def test_prefill_shape_query():
+    """The shape query refuses what a call would refuse, and names shapes within their limits."""
+    q = dict(widths=[(4096, 4096)], inputs=[0], T=512, n_seg=1, max_rank=64)
+    for wrong, code in [(dict(T=0), _ext.MLORA_EINVAL), (dict(n_seg=0), _ext.MLORA_EINVAL), (dict(max_rank=65), _ext.MLORA_ERANGE),
+                        (dict(widths=[(4100, 4096)]), _ext.MLORA_EALIGN), (dict(workspace_bytes=256), _ext.MLORA_ENOSPACE),
+                        (dict(seg_len=100), _ext.MLORA_EINVAL), (dict(seg_len=512), _ext.MLORA_EINVAL)]:   # 512 accumulating
+        with pytest.raises(_ext.MloraError) as e:
+            sgmv_shape(**{**q, **wrong})
+        assert e.value.code == code, wrong
+    need = _ext.lib().mlora_sgmv_workspace_bytes(512, 1)
+    assert sgmv_shape(**q, workspace_bytes=need) == sgmv_shape(**q)
+    for n in (1, 2, 3, 7, 8):
+        for T in (1, 64, 700, 9216):
+            for hin in (8, 520, 4096, 13824):
+                s = sgmv_shape([(hin, 4096)] * n, [0] * n, T, 4, 64)
+                assert all(1 <= k <= max(1, min(8, (hin + 511) // 512)) for k in s["splits"]), (n, T, hin, s)
 
 
 def test_one_make_builds_what_the_package_imports():
