@@ -371,7 +371,8 @@ def sgmv(y: torch.Tensor, x: torch.Tensor, pool: AdapterPool, layer: int, proj: 
 def sgmv_multi(ys: Sequence[torch.Tensor], xs: Sequence[torch.Tensor], pool: AdapterPool, layer: int,
                projs: Sequence[str], plan: PrefillPlan, accumulate: bool = True) -> None:
     """Prefill LoRA apply for up to 8 projections of one layer against one plan, three launches in all
-    (two up to rank 32 where y accumulates: the expand then sums the K splits).
+    (two where y accumulates and there are no K splits, or few enough at up to rank 32 or in a short batch: the expand then
+    sums them).
     Projections listed next to each other with the same x tensor (q, k, v; gate, up) share its reads.
     The plan's workspace must have been sized for this many projections (``plan_prefill(..., n_proj=)``)."""
     pool.sync()

@@ -340,8 +340,10 @@ int mlora_sgmv_planned(void *y, const void *x, const void *a_rows, const void *b
                        int dtype, int accumulate, void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
- * Several projections of one layer against one plan, in three launches in all (shrink, reduce, expand; an
- * accumulating call of max_rank <= 32 and at most eight K splits needs no reduce) instead of three per projection.  y, x, a_rows, b_rows, hin, hout are HOST arrays of n_proj entries as
+ * Several projections of one layer against one plan, in two or three launches in all (shrink, reduce, expand) instead of
+ * three per projection.  A call that writes y = delta always has the reduce, which zeroes the rows outside every segment; an
+ * accumulating one has it only where there are K splits and the expand does not sum them: above max_rank 32, but for batches of
+ * few tiles (mlora_sgmv_shape tells).  y, x, a_rows, b_rows, hin, hout are HOST arrays of n_proj entries as
  * in mlora_bgmv_multi.  Consecutive projections that are given the same x pointer (q, k, v; gate, up)
  * share its reads in the shrink launch: their workgroups for the same tokens run back to back on one
  * XCD, so x comes from HBM once.  The workspace: mlora_sgmv_multi_workspace_bytes(T, n_seg,

@@ -173,6 +173,20 @@ def test_prefill_shape_query():
                 assert all(1 <= k <= max(1, min(8, (hin + 511) // 512)) for k in s["splits"]), (n, T, hin, s)
 
 
+@pytest.mark.parametrize("hin,T,n_seg,rank,splits", [(512, 1600, 25, 64, False), (200, 70 * 64, 70, 64, False), (4096, 6000, 1, 64, None),
+                                                     (512, 1600, 25, 32, False), (4096, 64, 1, 16, True), (4096, 2000, 4, 64, True)])
+def test_the_reduce_launch_is_made_where_it_has_something_to_do(hin, T, n_seg, rank, splits):
+    """Splits to sum that the expand does not sum, or rows outside every segment to zero (y = delta)."""
+    for n in (1, 2, 4):
+        for accumulate in (True, False):
+            s = sgmv_shape([(hin, 512)] * n, [0] * n, T, n_seg, rank, accumulate)
+            many = max(s["splits"]) > 1
+            assert splits is None or many == splits
+            assert s["reduce"] == (not accumulate or (many and rank > 32 and not s["few"])), s
+    s = sgmv_shape([(hin, 4096)], [0], T // n_seg * n_seg, n_seg, rank, False, seg_len=T // n_seg)     # all rows are covered
+    assert s["reduce"] == (max(s["splits"]) > 1 and rank > 32 and not s["few"]), s
+
+
 def test_one_make_builds_what_the_package_imports():
     """`make -C csrc` alone builds the library and the launch path that loads with it, and the launch path by itself the
     library it links (make's dry run)."""
