@@ -659,27 +659,22 @@ namespace {
 
 constexpr int SG_TM = 64;   // tokens per tile, as in sgmv_prefill.hip
 
-struct SgmvWs { int max_tiles; int ksplit; int ks_cap; size_t off_cover, off_rec, off_proj, per_proj, off_hi, off_lo, total; };
+struct SgmvWs { int max_tiles; int ks_cap; size_t off_cover, off_rec, off_proj, per_proj, off_hi, off_lo, total; };
 
 // Workspace: the plan (tile list, tile records: depends on T and n_seg only), then per projection the
-// K-split partial sums and the hi / lo halves of their sum.  `most`: splits of a projection, `cap`: of one with a longer K.
-SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int most, int cap)
+// K-split partial sums and the hi / lo halves of their sum.  `cap`: splits that there is room for at most.
+SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int cap)
 {
     SgmvWs w;
     w.max_tiles = T / SG_TM + 2 * n_seg + 1;       // aligned cuts can add one partial tile at either end of a segment
-    // shrink workgroups: about three per CU for a single projection; a call over several projections has about
-    // that many with one or two splits already (one workgroup serves the projections that share x), and fewer
-    // splits mean less partial-sum traffic (swept 512 .. 4096 on configs 4 and 5: 768 - 1024 is the flat optimum)
+    // Room for the splits that a call of this size has a use for (shrink_shape chooses among those): all eight for a short
+    // batch; for longer ones as many as make about 1024 workgroups of a tile, projection and split each (768 for a single
+    // projection), and up to three times as many for a projection with a longer K than the others of its call.
     const long long per_split = (long long)w.max_tiles * n_proj;
     const long long target = n_proj > 1 ? 1024 : 768;
     long long ks = (target + per_split - 1) / per_split;
-    w.ksplit = ks < 1 ? 1 : (ks > most ? most : (int)ks);
-    // a projection with a longer K than the others of its call gets proportionally more splits (up to three
-    // times as many, at most 8 or as many as the others have), so that every shrink workgroup walks about the same
-    // number of columns
-    w.ks_cap = n_proj > 1 && w.ksplit < 8 ? (3 * w.ksplit < 8 ? 3 * w.ksplit : 8) : w.ksplit;
-    w.ks_cap = w.ks_cap < cap ? w.ks_cap : cap;
-    w.ksplit = w.ksplit < w.ks_cap ? w.ksplit : w.ks_cap;
+    ks = n_proj > 1 ? 3 * ks : ks;
+    w.ks_cap = ks < cap ? (int)ks : cap;
     size_t off = ((size_t)w.max_tiles * 3 + 4) * sizeof(int32_t);
     off = (off + 255) & ~(size_t)255;
     w.off_cover = off;                              // int32 [T]: 1 where a token belongs to some segment
@@ -697,24 +692,17 @@ SgmvWs sgmv_layout_splits(int T, int n_seg, int n_proj, int most, int cap)
 }
 
 // The layout for a workspace of `have` bytes (negative: as large as the call can use).
-// A prompt of a tile or two takes up to sixteen splits, two stages of 128 columns each at hidden 4096: the launch
-// is a chain of loads and more workgroups shorten it (one prompt of 64 tokens, three projections at rank 64: 20.0 us a
-// call with eight splits, 18.6 with sixteen, 21.0 with thirty-two; 512 tokens 24.9, 26.9, 30.9: partial sums).
 // The number of splits steps up as a batch gets shorter, so a shorter batch can have a use for more workspace than a longer
-// one, and fewer projections for more than many; where `have` does not hold what the call would take, it takes the
-// splits that fit (eight of the sixteen first), down to one: with one split the size only grows with tokens, segments and
+// one, and fewer projections for more than many; where `have` does not hold the room for all of them, it holds as
+// many as fit, down to one: with one split the size only grows with tokens, segments and
 // projections, so a workspace sized for a larger call always serves a smaller one.
 SgmvWs sgmv_layout(int T, int n_seg, int n_proj, int64_t have = -1)
 {
-    if (T / SG_TM + 2 * n_seg + 1 <= 6) {
-        const SgmvWs w = sgmv_layout_splits(T, n_seg, n_proj, 16, 16);
-        if (have < 0 || (int64_t)w.total <= have) return w;
-    }
-    const SgmvWs w = sgmv_layout_splits(T, n_seg, n_proj, 8, 8);
+    const SgmvWs w = sgmv_layout_splits(T, n_seg, n_proj, mlora::SGMV_SPLITS);
     if (have < 0 || (int64_t)w.total <= have) return w;
     const int64_t split = (int64_t)T * MLORA_MAX_RANK * (int64_t)sizeof(float);        // as large as the hi / lo halves together
     const int64_t fit = (have - (int64_t)w.off_proj) / n_proj / split - 1;
-    return sgmv_layout_splits(T, n_seg, n_proj, 8, fit < 1 ? 1 : (int)fit);
+    return sgmv_layout_splits(T, n_seg, n_proj, fit < 1 ? 1 : (int)fit);
 }
 
 // Columns of y one expand workgroup covers, and the column blocks per tile that follow from it.
@@ -739,7 +727,7 @@ int expand_block_cols(int n_proj, int max_tiles, int hout, int *ncb_out)
 // stages of 64 columns a split, and what the workspace holds.
 int splits_of(int hin, int hin_min, int k, const SgmvWs &w)
 {
-    const int most = (hin + 511) / 512 < 8 ? (hin + 511) / 512 : 8;
+    const int most = (hin + 511) / 512 < mlora::SGMV_SPLITS ? (hin + 511) / 512 : mlora::SGMV_SPLITS;
     int ks = (int)(((long long)k * hin + hin_min / 2) / hin_min);
     ks = ks < 1 ? 1 : (ks > most ? most : ks);
     return ks < w.ks_cap ? ks : w.ks_cap;
@@ -757,7 +745,7 @@ int splits_of(int hin, int hin_min, int k, const SgmvWs &w)
 // 211, 229 / 232, 202, 213.
 void shrink_shape(mlora::SgmvArgs &a, int tiles, int max_rank, const SgmvWs &w)
 {
-    static const int tried[] = {1, 2, 4, 8};
+    static const int tried[] = {1, 2, 4, mlora::SGMV_SPLITS};
     const int cus = mlora::device_compute_units(), rows = max_rank <= 16 ? 16 : (max_rank <= 32 ? 32 : 64);
     int hin_min = a.pr[0].hin;
     for (int p = 1; p < a.n_proj; p++) hin_min = a.pr[p].hin < hin_min ? a.pr[p].hin : hin_min;

@@ -208,6 +208,7 @@ int launch_gather(const GatherArgs &a, hipStream_t s);
 int launch_scatter(const ScatterArgs &a, hipStream_t s);
 int launch_assist_export(const AssistArgs &a, hipStream_t s);
 int launch_assist_import(const AssistArgs &a, hipStream_t s);
+constexpr int SGMV_SPLITS = 8;  // K splits of a projection of a prefill call at most (sum_splits4 takes as many)
 constexpr int SGMV_PLAN = 1;    // write the tile list and records into the workspace
 constexpr int SGMV_APPLY = 2;   // shrink, reduce, expand (the workspace already holds the plan unless SGMV_PLAN is set too)
 constexpr int SGMV_SHRINK = 4;  // the shrink launch alone: its partial sums feed the base GEMM + LoRA kernel

@@ -154,12 +154,11 @@ __device__ __forceinline__ void sum_splits(const float *__restrict__ src, size_t
     }
 }
 
-// The same with the loads of all splits in one batch, up to sixteen of them (n is uniform over the launch).
+// The same with the loads of all splits in one batch, up to eight of them (n is uniform over the launch).
 __device__ __forceinline__ void sum_splits_any(const float *__restrict__ src, size_t stride, int n, float (&v)[8])
 {
     if (n <= 2) sum_splits<2>(src, stride, n, v);
-    else if (n <= 8) sum_splits<8>(src, stride, n, v);
-    else sum_splits<16>(src, stride, n, v);
+    else sum_splits<8>(src, stride, n, v);
 }
 
 // Four neighbouring partial sums over up to eight K splits, in ascending order, the loads of all splits in one batch.

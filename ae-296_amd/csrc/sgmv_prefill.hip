@@ -533,11 +533,10 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
 }
 
 // ------------------------------------------------------------------ expand
-// Up to FOLD_SPLITS K splits are summed by the expand itself and the reduce launch falls away.  At rank 64 the sums are
+// Up to rank 32 the K splits are summed by the expand itself and the reduce launch falls away.  At rank 64 the sums are
 // four times as long as at 16 and every column block of a tile repeats them, so the reduce launch stays there but for the
-// launches of few tiles below: 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing, 55.4 and a reduce
+// launches of few tiles below (sgmv_launch_shape): 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing, 55.4 and a reduce
 // of 5.2 not; at rank 16 the whole call of 8 x 512 tokens 185 -> 179.
-constexpr int FOLD_SPLITS = 8;
 
 template <int DT, int RMAX, bool BT>
 __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
@@ -928,8 +927,8 @@ void sgmv_launch_shape(SgmvArgs &a, int max_rank, int phases)
         most = a.pr[q].ksplit > most ? a.pr[q].ksplit : most;
     }
     a.few = max_rank > 32 && few_wgs <= FEW_EXPAND;
-    // Few K splits are summed by the expand itself; rows outside every segment are zeroed by the reduce launch only.
-    a.fold = most <= FOLD_SPLITS && (max_rank <= 32 || a.few) && (a.accumulate || a.seg_uniform_len > 0);
+    // The expand sums the splits itself up to rank 32 and in launches of few tiles; rows outside every segment are zeroed by the reduce launch only.
+    a.fold = (max_rank <= 32 || a.few) && (a.accumulate || a.seg_uniform_len > 0);
     // Without splits the shrink has stored the halves itself, and the launch would only read the cover flags: two projections
     // of 25 x 64 tokens, rank 64, hin 512 15.6 -> 14.0 us a call, q/k/v/o of 16 x 500 tokens at hidden 4096 153.4 -> 151.7.
     a.reduce = !a.fold && (most > 1 || !(a.accumulate || a.seg_uniform_len > 0));

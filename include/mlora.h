@@ -295,11 +295,12 @@ int mlora_bgmv_reflayout_multi(int n_proj, void *const *y, const void *const *x,
  * seg_* are device arrays of n_seg entries.  Segments must not overlap; tokens covered by no
  * segment keep y (accumulate) or get zeros.  workspace: mlora_sgmv_workspace_bytes(T, n_seg).
  *
- * The workspace holds the fp32 partial sums of the call's K splits.  One that was sized for more tokens, segments or
- * projections serves every smaller call; where that holds fewer splits than the call would take by itself (a shorter
- * batch takes more), it takes those that fit, which is slower and another order of the same fp32 sums: a result's
- * last rounding can depend on the workspace's size, for every prefill call below.  mlora_sgmv_splits says how many
- * splits a projection of a call can get in a workspace (the one with the longest K; 0: the call does not fit).
+ * The workspace holds the fp32 partial sums of the call's K splits.  A projection is cut into at most eight, and one for
+ * every 512 columns of its K.  A workspace that was sized for more tokens, segments or projections serves every smaller
+ * call; where it holds fewer splits than the call would take by itself (a shorter batch takes more), the call takes those
+ * that fit, which is slower and another order of the same fp32 sums: a result's last rounding can depend on the
+ * workspace's size, for every prefill call below.  mlora_sgmv_splits says how many splits of a projection a workspace has
+ * room for in such a call (at most eight; 0: the call does not fit), mlora_sgmv_shape how many a call takes.
  */
 int64_t mlora_sgmv_workspace_bytes(int T, int n_seg);
 int mlora_sgmv_splits(int T, int n_seg, int n_proj, int64_t workspace_bytes);

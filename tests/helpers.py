@@ -121,3 +121,11 @@ def sgmv_shape(widths, inputs, T, n_seg, max_rank, accumulate=True, seg_len=0, w
     shape = (C.c_int32 * (4 + _ext.MAX_PROJ))()
     _ext.check(_ext.lib().mlora_sgmv_shape(n, x, hin, hout, T, n_seg, seg_len, max_rank, int(accumulate), workspace_bytes, shape))
     return dict(share=shape[0], stream=shape[1], reduce=shape[2], few=shape[3], splits=list(shape[4:4 + n]))
+
+
+def workspace_for_splits(T, n_seg, n_proj, splits):
+    """Bytes of a prefill workspace that has room for that many K splits of every projection: each takes T x 64 floats."""
+    from mlora import _ext
+    lib = _ext.lib()
+    full = lib.mlora_sgmv_multi_workspace_bytes(T, n_seg, n_proj)
+    return full - (lib.mlora_sgmv_splits(T, n_seg, n_proj, full) - splits) * n_proj * T * 64 * 4

@@ -6,7 +6,7 @@ import re
 
 import pytest
 
-from helpers import sgmv_shape
+from helpers import sgmv_shape, workspace_for_splits
 from mlora import _ext
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -151,8 +151,28 @@ def test_a_prefill_workspace_serves_every_smaller_call(T):
                         got, full = lib.mlora_sgmv_splits(t, s, p, have), lib.mlora_sgmv_splits(t, s, p, 1 << 50)
                         assert 1 <= got <= full, (t, s, p, have)
                         grew += got < full
-    assert grew > 0 or T <= 64                   # the sweep meets calls that would take more than they are given
+    assert grew > 0 or T <= 400                  # the sweep meets calls that would take more than they are given; up to
+                                                 # here every call has room for all eight splits
     assert lib.mlora_sgmv_splits(T, 1, 1, 256) == 0
+
+
+@pytest.mark.parametrize("T,n_seg,n_proj", [(1, 1, 1), (255, 1, 1), (640, 4, 3), (2880, 8, 7), (9216, 16, 7), (16000, 16, 1)])
+def test_the_splits_taken_fit_the_workspace(T, n_seg, n_proj):
+    """Whatever room a workspace has, the partial sums of every projection lie inside its part of it."""
+    lib = _ext.lib()
+    full = lib.mlora_sgmv_multi_workspace_bytes(T, n_seg, n_proj)
+    most, widths = lib.mlora_sgmv_splits(T, n_seg, n_proj, full), [(4096, 64)] * (n_proj - 1) + [(11008, 64)]
+    assert 1 <= most <= 8
+    limited = 0
+    for room in range(1, most + 1):
+        need = workspace_for_splits(T, n_seg, n_proj, room)
+        assert lib.mlora_sgmv_splits(T, n_seg, n_proj, need) == room
+        assert lib.mlora_sgmv_splits(T, n_seg, n_proj, need - 1) == room - 1
+        for rank in (16, 64):
+            taken = sgmv_shape(widths, [0] * n_proj, T, n_seg, rank, workspace_bytes=need)["splits"]
+            assert 1 <= min(taken) and max(taken) <= room
+            limited += max(taken) < max(sgmv_shape(widths, [0] * n_proj, T, n_seg, rank)["splits"])
+    assert limited > 0
 
 
 def test_prefill_shape_query():

@@ -5,7 +5,8 @@ import pytest
 import torch
 
 from gpu_common import ATOL, RTOL, assert_close_bits, oracle_apply, say, tdtype, upload_pool
-from helpers import BF16, FP16, PagedPool, bits_of, bits_to_torch, f32_of, torch_to_bits
+from helpers import (BF16, FP16, PagedPool, bits_of, bits_to_torch, f32_of, sgmv_shape, torch_to_bits,
+                     workspace_for_splits)
 from mlora import bgmv, plan_prefill, sgmv
 
 pytestmark = pytest.mark.gpu
@@ -272,7 +273,7 @@ def test_sgmv_multi_projection_call():
 
 @pytest.mark.parametrize("dtype", [FP16, BF16])
 @pytest.mark.parametrize("lens,ranks,hin,hout,n_proj", [
-    ([1], [64], 4096, 640, 3),                     # one tile, sixteen K splits, projections kept apart
+    ([1], [64], 4096, 640, 3),                     # one tile, eight K splits, projections kept apart
     ([65, 3], [16, 32], 264, 1032, 3),             # fewer stages than splits; a width that ends inside a column block
     ([64] * 20 + [17], [33, 8], 4096, 128, 1),     # eight splits, one column block
     ([300, 150], [32, 24, 8], 1024, 2048, 7),      # the expand sums the splits
@@ -308,44 +309,49 @@ def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj, dtype):
             assert_close_bits(torch_to_bits(y), want, dtype, nm)
 
 
-def test_sgmv_workspace_of_a_longer_batch():
-    """A workspace sized for one prompt of 400 tokens takes a shorter prompt, though that one has a use for more."""
-    from mlora import _ext, sgmv_multi
-    from mlora.ops import sgmv_workspace
+@pytest.mark.parametrize("splits", [1, 3])
+def test_sgmv_workspace_of_a_longer_batch(splits):
+    """A workspace with room for fewer splits than a short prompt takes by itself, as a longer batch can leave."""
+    from mlora import sgmv_multi
     rng = np.random.default_rng(5)
     T, hin, hout = 255, 4096, 264
     pp = PagedPool(rng, [64], hin, hout, page_rows=8, dtype=FP16)
     pool = upload_pool(pp)
     seg = _segments([T], [0])
     dev = [torch.from_numpy(a).cuda() for a in seg]
-    ws = sgmv_workspace(400, 1, "cuda", 1)
-    assert ws.numel() < _ext.lib().mlora_sgmv_workspace_bytes(T, 1)
+    ws = torch.empty(workspace_for_splits(T, 1, 1, splits), dtype=torch.uint8, device="cuda")
+    assert sgmv_shape([(hin, hout)], [0], T, 1, 64)["splits"] == [8]
+    assert sgmv_shape([(hin, hout)], [0], T, 1, 64, workspace_bytes=ws.numel())["splits"] == [splits]
     x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), FP16)
     y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), FP16)
     y = bits_to_torch(y0, FP16, "cuda")
-    say(f"sgmv workspace of a longer batch T={T} {hin}->{hout}")
+    say(f"sgmv workspace of a longer batch T={T} {hin}->{hout} splits={splits}")
     plan = plan_prefill(*dev, T, pool, workspace=ws)
     sgmv_multi([y], [bits_to_torch(x, FP16, "cuda")], pool, 0, ["p"], plan)
     torch.cuda.synchronize()
     assert_close_bits(torch_to_bits(y), oracle_apply(pp, x, _tok_of(*seg, T), y0), FP16, "short prompt")
 
 
+@pytest.mark.parametrize("splits", [None, 1])
 @pytest.mark.parametrize("long,T,n_seg,n_proj", [(6848, 6144, 1, 1), (3648, 2880, 8, 7), (3648, 3648, 8, 6), (300, 250, 1, 1)])
-def test_a_workspace_of_a_larger_call_serves_a_smaller_one(long, T, n_seg, n_proj):
-    """Batches that would take more workspace than the larger call's holds (more K splits), through the LoRA call and the
-    one-pass base product; (3648, 3648): fewer projections than it was sized for."""
-    from mlora import _ext, gemm_lora, sgmv_multi, sgmv_workspace
+def test_a_workspace_of_a_larger_call_serves_a_smaller_one(long, T, n_seg, n_proj, splits):
+    """A batch in the workspace of a larger call, and in one that is cut to fewer splits than the batch takes by itself, through
+    the LoRA call and the one-pass base product; (3648, 3648): fewer projections than it was sized for."""
+    from mlora import gemm_lora, sgmv_multi, sgmv_workspace
     rng = np.random.default_rng(long + T)
-    hin, hout = 1032, 72
+    hin, hout = 4104, 72
     names = [f"p{i}" for i in range(n_proj)]
     pp = PagedPool(rng, [64, 16, 40], hin, hout, page_rows=8, dtype=FP16)
     pool = upload_pool(pp, projections={nm: (hin, hout) for nm in names})
     for nm in names:
         pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, FP16))
         pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, FP16))
-    ws = sgmv_workspace(long, n_seg, "cuda", 7 if n_seg == 8 else n_proj)
-    lib = _ext.lib()
-    assert lib.mlora_sgmv_splits(T, n_seg, n_proj, ws.numel()) < lib.mlora_sgmv_splits(T, n_seg, n_proj, 1 << 50)
+    taken = lambda size: sgmv_shape([(hin, hout)] * n_proj, [0] * n_proj, T, n_seg, 64, workspace_bytes=size)["splits"]  # noqa: E731
+    if splits is None:
+        ws = sgmv_workspace(long, n_seg, "cuda", 7 if n_seg == 8 else n_proj)
+    else:
+        ws = torch.empty(workspace_for_splits(T, n_seg, n_proj, splits), dtype=torch.uint8, device="cuda")
+        assert taken(ws.numel()) == [splits] * n_proj and min(taken(1 << 50)) > splits
     cuts = np.sort(rng.choice(np.arange(1, T), n_seg - 1, replace=False)) if n_seg > 1 else np.empty(0, np.int64)
     lens = np.diff(np.concatenate([[0], cuts, [T]])).astype(int)
     seg = _segments(lens, rng.integers(0, 3, n_seg))
@@ -354,7 +360,7 @@ def test_a_workspace_of_a_larger_call_serves_a_smaller_one(long, T, n_seg, n_pro
     y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), FP16)
     xt = bits_to_torch(x, FP16, "cuda")
     ys = [bits_to_torch(y0, FP16, "cuda") for _ in names]
-    say(f"sgmv_multi T={T} in a workspace for {long}")
+    say(f"sgmv_multi T={T} in a workspace for {long}, splits={splits}")
     plan = plan_prefill(*dev, T, pool, workspace=ws)
     sgmv_multi(ys, [xt] * n_proj, pool, 0, names, plan)
     torch.cuda.synchronize()
@@ -364,7 +370,7 @@ def test_a_workspace_of_a_larger_call_serves_a_smaller_one(long, T, n_seg, n_pro
         assert_close_bits(torch_to_bits(y), want, FP16, "sgmv_multi")
     w = (torch.randn(hin, hout, device="cuda") / hin ** 0.5).half()
     outs = [torch.zeros(T, hout, device="cuda").half() for _ in names]
-    say(f"gemm_lora T={T} in a workspace for {long}")
+    say(f"gemm_lora T={T} in a workspace for {long}, splits={splits}")
     plan = plan_prefill(*dev, T, pool, workspace=ws, aligned=True)
     gemm_lora(outs, [xt] * n_proj, [w] * n_proj, pool, 0, names, plan)
     torch.cuda.synchronize()
