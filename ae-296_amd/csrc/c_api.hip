@@ -742,7 +742,7 @@ int splits_of(int hin, int hin_min, int k, const SgmvWs &w)
 // to 9216 tokens (ranks 16 to 64; one, three, four and seven projections): the shape it names is 0.9 % off the best on
 // average and 9 % at worst.  Llama-7B widths, rank 64, q/k/v, two layers and the plan in a graph, single / shared
 // projections at 1, 2, 4 splits, us: 64 tokens 53, 41, 35 / 110, 67, 50; 1280 tokens 86, 81, 87 / 137, 101, 85; 6000 tokens 211,
-// 211, 229 / 232, 202, 213.
+// 211, 229 / 232, 202, 213.  The rule takes the host 0.2 us (q, k, v) to 1.0 us (seven projections) a call.
 void shrink_shape(mlora::SgmvArgs &a, int tiles, int max_rank, const SgmvWs &w)
 {
     static const int tried[] = {1, 2, 4, mlora::SGMV_SPLITS};
@@ -829,6 +829,7 @@ void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w)
     a.n_tiles = ip + 3 * (size_t)w.max_tiles;
     a.tok_cover = reinterpret_cast<int32_t *>(base + w.off_cover);
     a.tile_rec = reinterpret_cast<int32_t *>(base + w.off_rec);
+    a.max_tiles = w.max_tiles;
     for (int p = 0; p < a.n_proj; p++) {
         char *pb = base + w.off_proj + w.per_proj * p;
         a.pr[p].v = reinterpret_cast<float *>(pb);
@@ -945,8 +946,6 @@ static int sgmv_common(int n_proj, void *const *y, const void *const *x, const v
             a.pr[p].y = y[p]; a.pr[p].x = x[p]; a.pr[p].a_rows = a_rows[p]; a.pr[p].b_rows = b_rows[p];
             a.pr[p].hin = hin[p]; a.pr[p].hout = hout[p];
         }
-    } else {
-        a.pr[0].hin = 8; a.pr[0].hout = 8;
     }
     const SgmvWs w = sgmv_layout(T, n_seg, n_proj, workspace_bytes < 0 ? 0 : workspace_bytes);
     if (!workspace || !aligned16(workspace)) return fail(MLORA_EALIGN, "workspace must be a 16-byte aligned device pointer");
@@ -955,7 +954,7 @@ static int sgmv_common(int n_proj, void *const *y, const void *const *x, const v
     a.seg_start = seg_start; a.seg_len = seg_len; a.seg_adapter = seg_adapter; a.n_seg = n_seg;
     a.T = T; a.accumulate = accumulate ? 1 : 0; a.b_transposed = 0; a.seg_uniform_len = 0; a.tile_aligned = tile_aligned;
     carve(a, workspace, w);
-    apply_shape(a, max_rank, w);
+    if (phases & mlora::SGMV_APPLY) apply_shape(a, max_rank, w);                 // the plan itself has no use for one
     rc = mlora::launch_sgmv(a, dtype, max_rank, phases, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "sgmv launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;
