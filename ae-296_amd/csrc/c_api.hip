@@ -839,7 +839,7 @@ void carve(mlora::SgmvArgs &a, void *workspace, const SgmvWs &w)
 }
 
 // The shape of a call's launches, but for what sgmv_launch_shape adds.
-void apply_shape(mlora::SgmvArgs &a, int max_rank, const SgmvWs &w)
+void apply_shape(mlora::SgmvArgs &a, int max_rank, const SgmvWs &w, int phases)
 {
     const int tiles = a.seg_uniform_len > 0 ? a.n_seg * ((a.seg_uniform_len + SG_TM - 1) / SG_TM) : (a.T + SG_TM / 2 * (a.n_seg - 1) + SG_TM - 1) / SG_TM;
     a.tiles = tiles;
@@ -852,14 +852,17 @@ void apply_shape(mlora::SgmvArgs &a, int max_rank, const SgmvWs &w)
     }
     shrink_shape(a, tiles, max_rank, w);
     // Whether x is read with the streaming hint: what a small call leaves in the last-level cache the next call on it finds there
-    // (the reference's q, k, v calls, single projections), what a large call leaves there only pushes other things out.
-    // Rank 64, states of three batches in turn, ordinary / streaming, us: the reference's three calls, x and y of a call
-    // 92 MB 106 / 108, 109 MB 126 / 122, 134 MB 141 / 126; q, k, v, o 197 MB 79 / 86, 295 MB 117 / 115; seven projections
-    // 210 MB 109 / 105, 525 MB 221 / 210.
+    // (calls of one projection each on one x, the base GEMM behind its shrink), what a large call leaves there only
+    // pushes other things out.  States of three batches in turn, ordinary / streaming, us.  Rank 64, by x and y of a call: the
+    // reference's three calls (y written only) 92 MB 106 / 108, 109 MB 126 / 122, 134 MB 141 / 126; one paged projection,
+    // 4096 to 4096, alone 109 MB 50 / 51, 170 MB 65 / 66, 230 MB 85 / 82, and three of them on one x 109 MB 149 / 154, 170 MB
+    // 185 / 198, 230 MB 240 / 247 (11008 to 4096 alone 134 MB 62 / 60, 230 MB 78 / 74; 4096 to 11008 230 MB 89 / 91); q, k, v, o
+    // 197 MB 79 / 86, 295 MB 117 / 115; seven projections 210 MB 109 / 105, 525 MB 221 / 210.  Base + LoRA in one pass, seven
+    // projections: 700 tokens 354 / 355, 2000 tokens (263 MB) 733 / 740, 9216 tokens (1.2 GB) 3064 / 3066; rank 16, 2000 tokens 691 / 700.
     long long bytes = 0;
     for (int g = 0; g < a.n_grp; g++) bytes += (long long)a.T * a.pr[a.grp_first[g]].hin * 2;
     for (int p = 0; p < a.n_proj; p++) bytes += (long long)a.T * a.pr[p].hout * 2;
-    a.stream_x = bytes > (a.n_proj == 1 ? 100000000LL : 200000000LL);
+    a.stream_x = (phases & mlora::SGMV_APPLY) && bytes > (a.seg_uniform_len > 0 ? 100000000LL : 200000000LL);
 }
 
 }  // namespace
@@ -905,7 +908,7 @@ int mlora_sgmv_shape(int n_proj, const void *const *x, const int32_t *hin, const
     const SgmvWs w = sgmv_layout(T, n_seg, n_proj, workspace_bytes < 0 ? 0 : workspace_bytes);
     if (workspace_bytes < (int64_t)w.total)
         return fail(MLORA_ENOSPACE, "workspace has %lld bytes, %lld needed", (long long)workspace_bytes, (long long)w.total);
-    apply_shape(a, max_rank, w);
+    apply_shape(a, max_rank, w, mlora::SGMV_APPLY);
     mlora::sgmv_launch_shape(a, max_rank, mlora::SGMV_APPLY);
     shape[0] = a.share_x; shape[1] = a.stream_x; shape[2] = a.reduce; shape[3] = a.few;
     for (int p = 0; p < n_proj; p++) shape[4 + p] = a.pr[p].ksplit;
@@ -954,7 +957,7 @@ static int sgmv_common(int n_proj, void *const *y, const void *const *x, const v
     a.seg_start = seg_start; a.seg_len = seg_len; a.seg_adapter = seg_adapter; a.n_seg = n_seg;
     a.T = T; a.accumulate = accumulate ? 1 : 0; a.b_transposed = 0; a.seg_uniform_len = 0; a.tile_aligned = tile_aligned;
     carve(a, workspace, w);
-    if (phases & mlora::SGMV_APPLY) apply_shape(a, max_rank, w);                 // the plan itself has no use for one
+    if (phases & mlora::SGMV_APPLY) apply_shape(a, max_rank, w, phases);                 // the plan itself has no use for one
     rc = mlora::launch_sgmv(a, dtype, max_rank, phases, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "sgmv launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;
@@ -1104,7 +1107,7 @@ int mlora_gemm_lora_split(int n_proj, void *const *y, const void *const *x, cons
         a.seg_start = seg_start; a.seg_len = seg_len; a.seg_adapter = seg_adapter; a.n_seg = n_seg;
         a.T = T; a.accumulate = 0; a.b_transposed = 0; a.seg_uniform_len = 0;
         carve(a, workspace, ws);
-        apply_shape(a, max_rank, ws);
+        apply_shape(a, max_rank, ws, mlora::SGMV_SHRINK);
         rc = mlora::launch_sgmv(a, dtype, max_rank, mlora::SGMV_SHRINK, static_cast<hipStream_t>(stream));
         if (rc) return fail(MLORA_ELAUNCH, "shrink launch failed: %s", hipGetErrorString((hipError_t)rc));
         for (int p = 0; p < n_proj; p++) {
@@ -1154,7 +1157,7 @@ int mlora_prefill_reflayout(void *y, const void *x, const void *A_T, const void 
     a.pr[0].hin = hin; a.pr[0].hout = hout;
     a.n_seg = B; a.T = T; a.accumulate = 0; a.b_transposed = 1; a.seg_uniform_len = Lpad;
     carve(a, workspace, w);
-    apply_shape(a, r, w);
+    apply_shape(a, r, w, mlora::SGMV_APPLY);
     rc = mlora::launch_sgmv(a, dtype, r, mlora::SGMV_PLAN | mlora::SGMV_APPLY, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "prefill launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;

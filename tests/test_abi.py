@@ -207,6 +207,15 @@ def test_the_reduce_launch_is_made_where_it_has_something_to_do(hin, T, n_seg, r
     assert s["reduce"] == (max(s["splits"]) > 1 and rank > 32 and not s["few"]), s
 
 
+def test_x_is_streamed_by_large_calls_only():
+    """From 100 MB of x and y on for the reference's call, whose three are measured so, and from 200 MB on for paged ones."""
+    for T, paged, ref in ((5920, 0, 0), (6400, 0, 1), (12000, 0, 1), (12800, 1, 1)):        # 4096 + 4096 columns: 16 KiB a token
+        assert sgmv_shape([(4096, 4096)], [0], T, 16, 64)["stream"] == paged
+        assert sgmv_shape([(4096, 4096)], [0], T, 16, 64, False, seg_len=T // 16)["stream"] == ref
+    assert sgmv_shape([(4096, 4096)] * 3, [0] * 3, 6000, 1, 64)["stream"] == 0              # x once, y three times: 197 MB
+    assert sgmv_shape([(4096, 4096)] * 3, [0] * 3, 6200, 1, 64)["stream"] == 1
+
+
 def test_one_make_builds_what_the_package_imports():
     """`make -C csrc` alone builds the library and the launch path that loads with it, and the launch path by itself the
     library it links (make's dry run)."""
