@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from gpu_common import ATOL, RTOL, assert_close_bits, say
-from helpers import BF16, FP16, bits_of, bits_to_torch, f32_of, torch_to_bits
+from helpers import BF16, FP16, bits_of, bits_to_torch, f32_of, sgmv_shape, torch_to_bits
 from mlora import Lora_GPU, add_lora_bgmv, lora_prefill_ref
 from oracle import oracle as orc
 
@@ -228,10 +228,12 @@ def test_lora_gpu_mirror_calls():
 
 
 @pytest.mark.parametrize("dtype", [FP16, BF16])
-@pytest.mark.parametrize("B,Lpad,r,hin,hout", [(2, 1, 8, 4096, 264), (5, 65, 24, 392, 1032), (22, 130, 64, 128, 136), (40, 128, 16, 640, 128)])
+@pytest.mark.parametrize("B,Lpad,r,hin,hout", [(2, 1, 8, 4096, 264), (5, 65, 24, 392, 1032), (22, 130, 64, 128, 136), (40, 128, 16, 640, 128),
+                                                 (12, 1000, 8, 4104, 264)])
 def test_prefill_ref_tiles_without_a_plan(B, Lpad, r, hin, hout, dtype):
-    """Equal prompts need no plan launch: one and several tiles per prompt, last tiles of one and two tokens, and both
-    numberings of the workgroups (fewer than 64 tiles, and more)."""
+    """Equal prompts need no plan launch: one and several tiles per prompt, last tiles of one and two tokens, both
+    numberings of the workgroups (fewer than 64 tiles, and more), and a call large enough to stream x (105 MB of x and y)."""
+    assert sgmv_shape([(hin, hout)], [0], B * Lpad, B, r, False, seg_len=Lpad)["stream"] == (B * Lpad == 12000)
     rng = np.random.default_rng(B + Lpad)
     A_T = bits_of((rng.standard_normal((B, 2, r, hin)) * 0.02).astype(np.float32), dtype)
     B_T = bits_of((rng.standard_normal((B, 2, hout, r)) * 0.02).astype(np.float32), dtype)
@@ -243,8 +245,8 @@ def test_prefill_ref_tiles_without_a_plan(B, Lpad, r, hin, hout, dtype):
 
 
 def test_lora_gpu_keeps_its_workspace_for_a_shorter_prefill():
-    """One prompt of 300 tokens, then one of 250, which would take more K splits: the workspace that a captured call
-    may still use is not replaced, and both results meet the reference."""
+    """One prompt of 300 tokens, then one of 250: the workspace that a captured call may still use is not replaced, and both
+    results meet the reference."""
     cfg = dict(n_layers=1, batch_size=4, lora_rank=64, hidden_dim=1024, tp_degree=1, max_prefill_batch_size=1)
     g = Lora_GPU(cfg, shared=True, device="cuda", seed=5)
     say("Lora_GPU: a shorter prefill after a longer one")

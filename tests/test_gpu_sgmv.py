@@ -12,6 +12,13 @@ from mlora import bgmv, plan_prefill, sgmv
 pytestmark = pytest.mark.gpu
 
 
+def _assert_shape(want, widths, inputs, T, n_seg, max_rank):
+    """The case is the one it is meant to be: the accumulating call takes the launches that `want` names."""
+    got = sgmv_shape(widths, inputs, T, n_seg, max_rank)
+    got["most"] = max(got["splits"])
+    assert {k: got[k] for k in want} == want, got
+
+
 def _segments(lens, adapters):
     lens = np.asarray(lens, np.int32)
     start = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
@@ -272,15 +279,15 @@ def test_sgmv_multi_projection_call():
 
 
 @pytest.mark.parametrize("dtype", [FP16, BF16])
-@pytest.mark.parametrize("lens,ranks,hin,hout,n_proj", [
-    ([1], [64], 4096, 640, 3),                     # one tile, eight K splits, projections kept apart
-    ([65, 3], [16, 32], 264, 1032, 3),             # fewer stages than splits; a width that ends inside a column block
-    ([64] * 20 + [17], [33, 8], 4096, 128, 1),     # eight splits, one column block
-    ([300, 150], [32, 24, 8], 1024, 2048, 7),      # the expand sums the splits
-    ([64] * 25, [64], 512, 512, 2),                # 76 tiles at most: the numbering in runs
-    ([64] * 30, [16], 384, 256, 3),                # projections that share x in one workgroup
+@pytest.mark.parametrize("lens,ranks,hin,hout,n_proj,shape", [
+    ([1], [64], 4096, 640, 3, dict(share=0, few=1, most=8)),                # one tile, eight K splits, projections kept apart
+    ([65, 3], [16, 32], 264, 1032, 3, dict(most=1)),                        # a short K; a width that ends inside a column block
+    ([64] * 20 + [17], [33, 8], 4096, 128, 1, dict(few=1, most=8)),         # eight splits, one column block
+    ([300, 150], [32, 24, 8], 1024, 2048, 7, dict(reduce=0, most=2)),       # the expand sums the splits
+    ([64] * 25, [64], 512, 512, 2, dict(few=0, reduce=0, most=1)),          # 76 tiles at most: the numbering in runs
+    ([64] * 30, [16], 384, 256, 3, dict(share=1)),                          # projections that share x in one workgroup
 ])
-def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj, dtype):
+def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj, shape, dtype):
     """Both sides of the size rules of the prefill launches: K splits, column blocks, numbering of the workgroups,
     shared x, and who sums the splits, with and without accumulation; a gap of rows no segment covers at the end."""
     from mlora import sgmv_multi
@@ -298,6 +305,7 @@ def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj, dtype):
     x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
     y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
     xt = bits_to_torch(x, dtype, "cuda")
+    _assert_shape(shape, [(hin, hout)] * n_proj, [0] * n_proj, T, len(lens), pool.max_rank)
     plan = plan_prefill(*dev, T, pool, n_proj=n_proj)
     for accumulate in (True, False):
         say(f"sgmv launch shapes lens={lens[:4]}x{len(lens)} {hin}->{hout} n_proj={n_proj} dtype={dtype} accumulate={accumulate}")
@@ -383,17 +391,19 @@ def test_a_workspace_of_a_larger_call_serves_a_smaller_one(long, T, n_seg, n_pro
         assert (np.abs(got - base) <= ATOL + RTOL * np.abs(base)).all()
 
 
-@pytest.mark.parametrize("lens,ranks,hin,inputs", [
-    ([30], [16], 8, [0]),                                    # no whole stage of 64 columns
-    ([64, 1], [8, 16], 72, [0, 1]),                          # one whole stage and a short one; a group of wavefronts without any
-    ([129], [32, 20], 1096, [0, 0]),                         # ranges of unlike length, the last with the short stage
-    ([100, 28], [64], 4160, [0, 0, 0, 0]),                   # eight splits, four projections of one input
-    ([64] * 70 + [17], [64, 40], 200, [0, 0, 0, 1]),         # one workgroup for three projections, and for one beside it
-    ([64] * 70 + [33], [32], 136, [0, 0, 1, 1, 1]),          # for two and for three
-    ([64] * 90, [16, 5], 640, [0, 0, 0, 0]),                 # a fourth projection of the same input starts a new group
+@pytest.mark.parametrize("lens,ranks,hin,inputs,share,most", [
+    ([30], [16], 8, [0], 0, 1),                              # no whole stage of 64 columns
+    ([64, 1], [8, 16], 72, [0, 1], 0, 1),                    # one whole stage and a short one; a group of wavefronts without any
+    ([129], [32, 20], 1096, [0, 0], 0, 3),                   # ranges of unlike length, the last with the short stage
+    ([100, 28], [64], 4160, [0, 0, 0, 0], 0, 8),             # eight splits, four projections of one input
+    ([64] * 70 + [17], [64, 40], 200, [0, 0, 0, 1], 1, 1),   # one workgroup for three projections, and for one beside it
+    ([64] * 70 + [33], [32], 136, [0, 0, 1, 1, 1], 1, 1),    # for two and for three
+    ([64] * 90, [16, 5], 640, [0, 0, 0, 0], 1, 1),           # a fourth projection of the same input starts a new group
+    ([64] * 40 + [30], [64, 24], 1032, [0, 0, 0, 1, 1], 1, 2),   # three and two of them in two ranges, the last with a short stage
+    ([64] * 41, [32, 8], 2056, [0, 0], 1, 4),                # two in four ranges
 ])
 @pytest.mark.parametrize("dtype", [FP16, BF16])
-def test_sgmv_shrink_stages_and_groups(lens, ranks, hin, inputs, dtype):
+def test_sgmv_shrink_stages_and_groups(lens, ranks, hin, inputs, share, most, dtype):
     """The ring of stages at its ends (rows shorter than a stage, a last stage of fewer columns, more slots than stages) and
     every number of projections that a workgroup serves, with one K split and with several."""
     from mlora import sgmv_multi
@@ -408,6 +418,7 @@ def test_sgmv_shrink_stages_and_groups(lens, ranks, hin, inputs, dtype):
     seg = _segments(lens, rng.integers(0, len(ranks), len(lens)))
     T = sum(lens) + 3
     tok = _tok_of(*seg, T)
+    _assert_shape(dict(share=share, most=most), [(hin, hout)] * len(inputs), inputs, T, len(lens), pool.max_rank)
     plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in seg), T, pool, n_proj=len(inputs))
     xs = [bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype) for _ in range(max(inputs) + 1)]
     xt = [bits_to_torch(x, dtype, "cuda") for x in xs]
@@ -422,16 +433,18 @@ def test_sgmv_shrink_stages_and_groups(lens, ranks, hin, inputs, dtype):
             assert_close_bits(torch_to_bits(y), want[i], dtype, f"input {i}")
 
 
-@pytest.mark.parametrize("dtype", [FP16, BF16])
-@pytest.mark.parametrize("lens,ranks,hin,hout,n_proj", [
-    ([1], [40], 64, 8, 1),                         # one token, one piece of y
-    ([17, 15, 33], [64, 8], 520, 264, 3),          # pieces of 16 tokens with a remainder; a last column block of 8
-    ([48], [48], 4096, 2568, 2),                   # eight splits
-    ([64, 64], [33], 72, 4096, 4),                 # one split: halves from the shrink; 512 workgroups
+@pytest.mark.parametrize("lens,gap,ranks,hin,hout,n_proj,shape", [
+    ([1], 2, [40], 64, 8, 1, dict(few=1, most=1)),                     # one token, one piece of y
+    ([17, 15, 33], 2, [64, 8], 520, 264, 3, dict(few=1, most=2)),      # pieces of 16 tokens with a remainder; a last column block of 8
+    ([48], 2, [48], 4096, 2568, 2, dict(few=1, most=8)),               # eight splits
+    ([128], 0, [33], 72, 4096, 4, dict(few=1, most=1)),                # one split: halves from the shrink; 512 workgroups
+    ([128], 0, [33], 72, 4104, 4, dict(few=0, most=1)),                # 544 workgroups: the expand of 64 tokens
+    ([64, 64], 2, [33], 72, 4096, 4, dict(few=0, most=1)),             # 768 by the estimate of two segments in 130 tokens
 ])
-def test_sgmv_few_tiles(lens, ranks, hin, hout, n_proj, dtype):
-    """The expand of 16-token pieces, summing the splits itself, behind the reduce launch (y = delta) and on one split; a
-    segment without an adapter and rows outside every segment."""
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+def test_sgmv_few_tiles(lens, gap, ranks, hin, hout, n_proj, shape, dtype):
+    """The expand of 16-token pieces on both sides of its limit, summing the splits itself, behind the reduce launch (y = delta) and
+    on one split; a segment without an adapter and rows outside every segment."""
     from mlora import sgmv_multi
     rng = np.random.default_rng(sum(lens) + hin)
     pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
@@ -444,8 +457,9 @@ def test_sgmv_few_tiles(lens, ranks, hin, hout, n_proj, dtype):
     if len(lens) > 2:
         adapters[1] = -1
     seg = _segments(lens, adapters)
-    T = sum(lens) + 2
+    T = sum(lens) + gap
     tok = _tok_of(*seg, T)
+    _assert_shape(shape, [(hin, hout)] * n_proj, [0] * n_proj, T, len(lens), pool.max_rank)
     plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in seg), T, pool, n_proj=n_proj)
     x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
     y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
