@@ -53,8 +53,8 @@ class Lora_GPU:
         hi = min(32, self.batch_size)
         self.select_inds = [torch.randint(0, hi, (i + 1,), device=self.device, generator=self._gen)
                             for i in range(self.batch_size)]
-        self._workspace = None
-        self._workspace_for = (0, 0)                   # rows and requests it was sized for
+        self._workspace = None                         # of the newest prefill call ...
+        self._workspace_for = (0, 0, None, None)       # ... the rows and requests it was sized for, the order it belongs to, itself
         # Grouping of the current decode batch by adapter: (plan, the index tensor it was made from, its torch version, the
         # order it belongs to, its number).  It is served again only for the very tensor object it was made from (kept
         # alive here so that neither its address nor its Python identity can pass to another tensor) at the same version
@@ -153,10 +153,17 @@ class Lora_GPU:
                 raise RuntimeError("prefill adapters are not loaded (call prepare_lora_prefill)")
             if not x.is_contiguous():
                 x = x.contiguous()
-            rows, reqs = max(bsz * x.shape[1], self._workspace_for[0]), max(bsz, self._workspace_for[1])
-            if (rows, reqs) != self._workspace_for:    # a shorter batch than it was sized for keeps it
-                self._workspace, self._workspace_for = ops.sgmv_workspace(rows, reqs, x.device), (rows, reqs)
-            return ops.lora_prefill_ref(x, down, up, layer_id, workspace=self._workspace)
+            # A shorter batch than it was sized for keeps the workspace.  It serves one thread, stream and capture
+            # (mlora._host.order): calls elsewhere may overlap, and a captured call goes on using the one it was given.
+            order = _ext.host().order()
+            had_rows, had_reqs, belongs, ws = self._workspace_for
+            if belongs != order:
+                had_rows = had_reqs = 0
+            rows, reqs = max(bsz * x.shape[1], had_rows), max(bsz, had_reqs)
+            if (rows, reqs) != (had_rows, had_reqs):
+                ws = ops.sgmv_workspace(rows, reqs, x.device)
+                self._workspace, self._workspace_for = ws, (rows, reqs, order, ws)
+            return ops.lora_prefill_ref(x, down, up, layer_id, workspace=ws)
         if not ops.ref_rank_supported(self.lora_rank):
             return self._invoke_single(name, x, layer_id, lora_ids)
         # ``_get_qkv`` asks for q, k and v of the same input one after the other

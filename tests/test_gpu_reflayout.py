@@ -344,3 +344,26 @@ def test_lora_gpu_calls_of_a_layer_on_other_streams_and_in_captures(planned):
         graph.replay()
         torch.cuda.synchronize()
         assert close(k, want_of("k", x)) and close(v, want_of("v", x)), rep
+
+
+def test_lora_gpu_prefill_on_two_streams():
+    """Prefill calls of one object that overlap on two streams, each against its own result alone."""
+    cfg = dict(n_layers=1, batch_size=2, lora_rank=64, hidden_dim=2048, tp_degree=1, max_prefill_batch_size=2)
+    g = Lora_GPU(cfg, shared=True, seed=7)
+    for name in "qkv":
+        getattr(g, f"{name}_down_prefill").mul_(100.0)
+        getattr(g, f"{name}_up_prefill").mul_(100.0)
+    xs = [torch.randn(2, 200, 2048, device="cuda").half() for _ in range(4)]
+    want = [g.invoke_one_layer_v(x, 0, True) for x in xs]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    say("Lora_GPU: prefill on two streams")
+    got = [[], []]
+    for i in range(30):
+        for j in range(2):
+            with torch.cuda.stream(streams[j]):
+                got[j].append(g.invoke_one_layer_v(xs[(i + j) % 4], 0, True))
+    torch.cuda.synchronize()
+    for j in range(2):
+        for i in range(30):
+            assert torch.equal(got[j][i], want[(i + j) % 4]), (i, j)

@@ -89,3 +89,18 @@ def test_threads_get_results_of_their_own_input(gpu):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_a_prefill_workspace_serves_one_stream_and_one_capture(gpu, monkeypatch):
+    g, host = gpu
+    g.prepare_lora_prefill(2)
+    used = []
+    monkeypatch.setattr(ops, "sgmv_workspace", lambda rows, reqs, device: torch.empty(rows * 10 + reqs))
+    monkeypatch.setattr(ops, "lora_prefill_ref", lambda x, down, up, layer, workspace: used.append(workspace))
+    call = lambda n, length: g.invoke_one_layer_q(torch.zeros(n, length, 16).half(), 0, True)  # noqa: E731
+    call(1, 300), call(1, 250), call(2, 100)
+    assert used[0] is used[1] and used[2] is not used[1] and used[2].numel() == 3002     # grows, and covers what it covered before
+    for elsewhere in ((0, 0, 7, 0), (0, 0, 7, 2), (0, 0, 7, 0)):
+        host.at = elsewhere
+        call(1, 50), call(1, 40)
+        assert used[-1] is used[-2] and all(used[-1] is not w for w in used[:-2]) and used[-1].numel() == 501
