@@ -7,12 +7,14 @@
 // projections in two launches 19.4 -> 9.1 us (0.5 of it the allocation of its intermediate), sgmv_multi over seven (three
 // launches) 34.5 -> 10.7 us.
 // The reference's q, k and v calls of a layer, outputs included (deltas_ref and Lora_GPU._invoke): 21 -> 16 us, a step of four layers
-// that the host bounds 86 -> 65 us.
+// that the host bounds 86 -> 65 us (66 since results are kept for one thread, stream and capture).
 // Nothing is kept from one call for the next: every tensor is checked and every slab looked up on every call.  A negative
 // code of the C ABI is returned, and raised by the caller.
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/Allocator.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -285,9 +287,13 @@ int ref_call(PyObject *plan, int n, Y y_of, X x_of, A a_of, B b_of, int layer, f
     }
     if (type != at::kHalf && type != at::kBFloat16) raise(PyExc_TypeError, "mlora kernels take float16 or bfloat16 tensors");
     const int64_t bytes = mlora_bgmv_workspace_bytes(n, (int)T, max_hin, (int)r);
-    // this call's own, as in bgmv
-    const at::Tensor room = bytes > 0 ? at::empty({bytes}, y_of(0).options().dtype(at::kByte)) : at::Tensor();
-    void *ws = room.defined() ? room.data_ptr() : nullptr;
+    // this call's own, as in bgmv; straight from torch's allocator, a tensor takes longer to make
+    at::DataPtr room;
+    if (bytes > 0) {
+        const c10::DeviceGuard device(y_of(0).device());
+        room = c10::GetAllocator(at::kCUDA)->allocate((size_t)bytes);
+    }
+    void *ws = room.get();
     return launch(mlora_bgmv_reflayout_multi, n, y, x, a, b, hin, hout, attr_ptr(plan, s_buf), (int)T, (int)N, (int)L, (int)r,
                   layer, scale, (int)attr_int(plan, s_group), type == at::kHalf ? MLORA_F16 : MLORA_BF16, accumulate, ws, bytes, stream());
 }
@@ -335,20 +341,50 @@ PyObject *deltas_ref(PyObject *const *v, Py_ssize_t nargs)
     return out.o;
 }
 
-// order(): (thread, device, stream, capture number or 0): what a program queues under equal values runs in the order it is queued.
+// What orders a program's work: thread, device, stream and capture number (0 outside a capture).  What is queued under equal values
+// runs in the order it is queued.
+struct Order {
+    int64_t v[4];
+    Order()
+    {
+        const c10::hip::HIPStream s = c10::hip::getCurrentHIPStream();
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        unsigned long long id = 0;
+        // the null stream cannot be captured, and asking it during another stream's capture is an error
+        if (s.stream() && hipStreamGetCaptureInfo(s.stream(), &status, &id) != hipSuccess)
+            raise(PyExc_RuntimeError, "the capture state of the current stream is not known: %s", hipGetErrorString(hipGetLastError()));
+        v[0] = (int64_t)PyThread_get_thread_ident();
+        v[1] = s.device_index();
+        v[2] = (int64_t)(uintptr_t)s.stream();
+        v[3] = status == hipStreamCaptureStatusNone ? 0 : (int64_t)id;
+    }
+};
+
+PyObject *bytes_of(const int64_t *v, Py_ssize_t n) { return PyBytes_FromStringAndSize(reinterpret_cast<const char *>(v), n * (Py_ssize_t)sizeof(int64_t)); }
+
+// order(): it, as bytes to compare
 PyObject *order(PyObject *const *, Py_ssize_t nargs)
 {
     if (nargs != 0) raise(PyExc_TypeError, "order takes no arguments");
-    const c10::hip::HIPStream s = c10::hip::getCurrentHIPStream();
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    unsigned long long id = 0;
-    // the null stream cannot be captured, and asking it during another stream's capture is an error
-    if (s.stream() && hipStreamGetCaptureInfo(s.stream(), &status, &id) != hipSuccess)
-        raise(PyExc_RuntimeError, "the capture state of the current stream is not known: %s", hipGetErrorString(hipGetLastError()));
-    Ref t(Py_BuildValue("(kiKK)", PyThread_get_thread_ident(), (int)s.device_index(), (unsigned long long)(uintptr_t)s.stream(),
-                        status == hipStreamCaptureStatusNone ? 0ULL : id));
-    Py_INCREF(t.o);
-    return t.o;
+    const Order o;
+    return bytes_of(o.v, 4);
+}
+
+// state(x, weights): the order, and which objects x and the weights are at which torch versions, as bytes to compare while the
+// objects are alive.  One call for all of it: the q, k and v calls of a layer ask for it every time.
+PyObject *state(PyObject *const *v, Py_ssize_t nargs)
+{
+    if (nargs != 2) raise(PyExc_TypeError, "state takes 2 arguments");
+    const List w(v[1]);
+    if (w.size() > 2 * MLORA_MAX_PROJ) raise(PyExc_ValueError, "at most %d weights", 2 * MLORA_MAX_PROJ);
+    int64_t out[4 + 2 * (1 + 2 * MLORA_MAX_PROJ)];
+    const Order o;
+    for (int i = 0; i < 4; i++) out[i] = o.v[i];
+    Py_ssize_t n = 4;
+    auto add = [&](PyObject *t) { out[n++] = (int64_t)(uintptr_t)t; out[n++] = tensor(t)._version(); };
+    add(v[0]);
+    for (Py_ssize_t i = 0; i < w.size(); i++) add(PySequence_Fast_GET_ITEM(w.o, i));
+    return bytes_of(out, n);
 }
 
 // ---------------------------------------------------------------- prefill
@@ -419,7 +455,7 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t nargs)
 }
 
 #define MLORA_FN(name) {#name, (PyCFunction)(void (*)())entry<name>, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {MLORA_FN(gather), MLORA_FN(bgmv), MLORA_FN(bgmv_ref), MLORA_FN(deltas_ref), MLORA_FN(order), MLORA_FN(prefill_plan),
+PyMethodDef methods[] = {MLORA_FN(gather), MLORA_FN(bgmv), MLORA_FN(bgmv_ref), MLORA_FN(deltas_ref), MLORA_FN(order), MLORA_FN(state), MLORA_FN(prefill_plan),
                          MLORA_FN(sgmv_multi), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Native launch path of mlora's eager calls.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

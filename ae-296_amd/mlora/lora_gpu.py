@@ -65,8 +65,8 @@ class Lora_GPU:
         self._plan_state = (None, None, None, None, 0)
         self._plan_gen = 0                             # number of the newest plan
         self._plan_numbers = itertools.count(1)
-        # q, k, v deltas of the last decode input that were not asked for yet: (what they were computed from, the input
-        # tensor itself and the six weight tensors (kept alive for the same reason), the deltas)
+        # q, k, v deltas of the last decode input that were not asked for yet: (what they were computed from, the deltas, the
+        # input tensor itself and the six weight tensors (kept alive for the same reason))
         self._qkv = None
 
     def _rand(self, n, rows, cols):
@@ -112,11 +112,12 @@ class Lora_GPU:
         self._qkv = None
         return plan, number
 
-    def _plan_for(self, bsz, lora_ids, order):
+    def _plan_for(self, bsz, lora_ids):
         src = self._index_source(bsz, lora_ids)
         plan, made_from, version, belongs, number = self._plan_state
-        if plan is None or made_from is not src or version != src._version or plan.T != bsz or (belongs is not None and belongs != order):
-            return self._group(bsz, lora_ids, order)
+        if plan is None or made_from is not src or version != src._version or plan.T != bsz or (
+                belongs is not None and belongs != _ext.host().order()):
+            return self._group(bsz, lora_ids, _ext.host().order())
         return plan, number
 
     def invoke_one_layer_qkv(self, x, layer_id, lora_ids=None):
@@ -126,7 +127,7 @@ class Lora_GPU:
         bsz = x.shape[0]
         if not ops.ref_rank_supported(self.lora_rank):
             return tuple(self._invoke_single(n, x, layer_id, lora_ids) for n in "qkv")
-        return self._deltas(x, layer_id, self._plan_for(bsz, lora_ids, _ext.host().order())[0], _QKV_WEIGHTS(self))
+        return self._deltas(x, layer_id, self._plan_for(bsz, lora_ids)[0], _QKV_WEIGHTS(self))
 
     @staticmethod
     def _deltas(x, layer_id, plan, weights):
@@ -171,20 +172,18 @@ class Lora_GPU:
         # the other two are answered from that result as long as it is the same input tensor object at the same
         # torch version, the same layer, the same plan, the same weight tensors at the same versions, and the same thread,
         # stream and graph capture: a call elsewhere is not ordered behind the launches that write the result.
-        order = _ext.host().order()
-        plan, number = self._plan_for(bsz, lora_ids, order)
+        plan, number = self._plan_for(bsz, lora_ids)
         weights = _QKV_WEIGHTS(self)
-        a, b, c, d, e, f = weights
-        key = (x._version, x.shape, layer_id, number, order, a._version, b._version, c._version, d._version, e._version, f._version)
-        if (kept := self._qkv) is not None:
-            made_from, of, (ka, kb, kc, kd, ke, kf), left = kept
-            if of is x and made_from == key and a is ka and b is kb and c is kc and d is kd and e is ke and f is kf:
-                y = left.pop(name, None)
-                if y is not None:
-                    return y
-        left = dict(zip("qkv", self._deltas(x, layer_id, plan, weights)))
+        key = (_ext.host().state(x, weights), x.shape, layer_id, number)
+        kept = self._qkv
+        if kept is not None and kept[0] == key:
+            y = kept[1].pop(name, None)
+            if y is not None:
+                return y
+        q, k, v = self._deltas(x, layer_id, plan, weights)
+        left = {"q": q, "k": k, "v": v}
         y = left.pop(name)
-        self._qkv = (key, x, weights, left)
+        self._qkv = (key, left, x, weights)
         return y
 
     def invoke_one_layer_q(self, x, layer_id, prefill=False, lora_ids=None):

@@ -16,6 +16,9 @@ class _Host:
     def order(self):
         return (threading.get_ident(),) + self.at[1:]
 
+    def state(self, x, weights):
+        return self.order() + tuple((id(t), t._version) for t in (x, *weights))
+
     def deltas_ref(self, plan, x, weights, layer, T, N, L, r):
         with self.lock:
             made = len(self.calls)
