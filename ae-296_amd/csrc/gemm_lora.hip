@@ -640,13 +640,17 @@ __global__ __launch_bounds__(256) void gemm_lora_sum_kernel(const GemmLoraArgs p
 // hundred tiles or fewer: most units idle, the longest K (the MLP's second product) is a chain several times as long as
 // the rest, and rows past T are multiplied for nothing.  The rule estimates, for every tile height and number of
 // ranges, rounds of workgroups x mean time of one (or the longest chain) plus the cost of the partial sums, and takes
-// the least; the plain shape stays within 5 % of it, where the estimate does not tell them apart.  Step times are those
-// measured with one workgroup on each unit.  Base products at Llama-7B widths, fp16, us, plain -> chosen (best of the 28
-// shapes tried): q/k/v 16 tokens 77 -> 30 (28), 120 tokens 83 -> 41 (40), 351 tokens 85 -> 64 (63), 700 tokens 95 -> 84 (84);
-// all seven 16 tokens 196 -> 78 (78; 5.2 TB/s of weights), 192 tokens 249 -> 111 (111), 351 tokens 268 -> 199 (191), 500
-// tokens 292 -> 265 (258).  K is cut up to 384 tokens; the plain shape is chosen for the seven from 577 tokens on, but for
-// 1025..1152 and 1793..1920, and for q/k/v at 961..1280, at 1921..2560 and from 3073 on: in between, 256 rows would leave a
-// last round nearly empty (1500 tokens 203 -> 170 with 192 rows).
+// the least; the plain shape is kept where it comes within 5 %, which the estimate does not tell apart.  Base products at Llama-7B
+// widths, fp16, weights of two layers in turn, us, plain -> chosen (best of the 25 shapes): q/k/v 16 tokens 76 -> 24 (24),
+// 120 tokens 74 -> 33 (30), 192 tokens 73 -> 41 (33), 351 tokens 74 -> 53 (45), 700 tokens 79 -> 72 (71), 1500 tokens 182 -> 148
+// (145), 2000 tokens 185 -> 193 (179); all seven 16 tokens 191 -> 77 (77; 5.3 TB/s of weights), 192 tokens 205 -> 100 (100), 351
+// tokens 239 -> 166 (166), 500 tokens 242 -> 229 (217), 900 tokens 368 -> 371 (345), 1500 tokens 529 (529).
+// Step times are those of one workgroup on each unit when x came in stages of 32 columns; x in whole lines shortened every step,
+// and the estimate now cuts K too early: where it is 10 to 25 % off (q/k/v at 120 to 384 tokens), 64 or 128 rows with K whole
+// are the best shape.
+// K is cut up to 384 tokens; the plain shape is chosen for the seven from 577 tokens on, but for
+// 1025..1152 and 1793..1920, and for q/k/v at 961..1280, at 1921..2560 and from 3073 on but for 6657..7104: in between, the
+// estimate has 256 rows leave a last round nearly empty (1500 tokens above, 192 rows).
 // Tiles of 256 rows are never cut: with the ranges the compiler spills accumulators.
 int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out)
 {

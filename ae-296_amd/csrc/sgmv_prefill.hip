@@ -1,6 +1,6 @@
 // SGMV prefill kernels for gfx950: tokens are packed per segment (one adapter per segment)
 //     y[t] (+)= s_a * (x[t] . A_a) . B_a
-// computed on v_mfma_f32_16x16x32_{f16,bf16} tiles in three or four launches on one stream (the first can be shared by all projections and layers of a batch):
+// computed on v_mfma_f32_16x16x32_{f16,bf16} tiles in two to four launches on one stream (the first can be shared by all projections and layers of a batch):
 //   plan   : cuts every segment into tiles of at most 64 tokens (work list in the workspace);
 //   shrink : V[split][t][0..R) = x[t, Kslice] . A_a[:, Kslice]^T   (split-K, fp32 partials), or with one
 //            split the result itself as a hi + lo pair of 16-bit values, so that the intermediate keeps

@@ -353,9 +353,10 @@ int mlora_sgmv_planned(void *y, const void *x, const void *a_rows, const void *b
  */
 int64_t mlora_sgmv_multi_workspace_bytes(int T, int n_seg, int n_proj);
 /*
- * Columns of y that one expand workgroup of such a call covers for a projection of width hout (the library
- * picks 512, or the width whose block count per 64-token tile suits the order its workgroups run in: 640 for
- * hout 5120, 576 for 13824).  Informational, like the workspace sizes; 0 for arguments out of range.  No
+ * Columns of y that one expand workgroup of such a call covers for a projection of width hout where it takes 64 tokens
+ * (the library picks 512, fewer for a short batch, or the width whose block count per 64-token tile suits the order its
+ * workgroups run in: 640 for hout 5120, 576 for 13824); the expand of 16-token pieces (mlora_sgmv_shape) always takes
+ * 256.  Informational, like the workspace sizes; 0 for arguments out of range.  No
  * counterpart in the reference (its prefill is two library GEMMs, lora_gpu.py:127-128).
  */
 int mlora_sgmv_expand_cols(int T, int n_seg, int n_proj, int hout);
@@ -385,7 +386,7 @@ int mlora_sgmv_multi_planned(int n_proj, void *const *y, const void *const *x,
  * or in a segment without adapter, getting the base product alone.  Replaces torch.mm(x, W) followed by
  * `q += q_lora` (layer_infer/transformer_layer_infer.py:145-147 and :160-171), for which the reference
  * writes y, reads it back and writes it again: here y is written once.  Launches: the SGMV shrink, a scaled
- * reduce, and one GEMM launch for all projections in which the expand rides along as rank / 16 extra MFMA
+ * reduce where a projection has K splits, and one GEMM launch for all projections in which the expand rides along as rank / 16 extra MFMA
  * steps per output tile.  The sum is rounded to 16 bits once (the reference rounds the base product, the
  * delta and their sum).  Arrays are HOST arrays of n_proj entries as in mlora_sgmv_multi_planned; the
  * workspace must hold mlora_sgmv_multi_workspace_bytes(T, n_seg, n_proj) bytes and a plan written by
