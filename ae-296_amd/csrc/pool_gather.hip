@@ -2,8 +2,9 @@
 //
 // Groups the tokens of a batch by adapter (stable: ordered by adapter id, then by token id) and derives
 // segments, the decode work list (chunks of at most `group` tokens of one adapter) and the work records.
-// Two forms: counting with one LDS counter per adapter (gather_count_kernel, pools of fewer than 8192 slots)
-// and a bitonic sort of 32-bit keys (gather_kernel, larger pools, whose counters do not fit LDS).
+// Three forms: counting with one LDS counter per adapter, for up to 512 tokens of fewer than 2048 adapters
+// (gather_few_kernel) and for more of either (gather_count_kernel, pools of fewer than 8192 slots), and a bitonic sort
+// of 32-bit keys (gather_kernel, larger pools, whose counters do not fit LDS).
 // Further blocks write the per-token view: page base rows, rank and scaling of each token's
 // adapter.  All outputs are integers or copied floats, so they are bit-exact by construction.
 //
@@ -12,6 +13,7 @@
 // (lightllm/server/router/model_infer/pre_process.py:50,100).
 #include "mlora_args.hpp"
 #include "mlora_dev.hpp"
+#include <type_traits>
 
 namespace mlora {
 
@@ -134,9 +136,8 @@ __device__ __forceinline__ unsigned long long block_scan_inclusive64(unsigned lo
 //   3. every token drops itself at its place, every head of a chunk its chunk header, in LDS;
 //   4. records are written from those headers.
 // Block 0 also writes the grouped view (perm, segments, chunks, counters).  Measured (graph replay of launch after
-// launch, sorting form -> this one): 10.7 -> 6.4 us for 32 tokens of 8 adapters, 16.4 -> 7.2 us for 256 of 64,
-// 30.3 -> 9.0 us for 512 of 1000 with mixed ranks, 358 -> 29 us for 8192 of 1000; about 6 us are the launch and the
-// chain token -> adapter -> page table -> record.
+// launch, sorting form -> this one): 16.4 -> 7.2 us for 256 tokens of 64 adapters, 30.3 -> 9.0 us for 512 of 1000 with mixed
+// ranks (both served by gather_few_kernel now), 358 -> 29 us for 8192 of 1000.
 // T <= 2048 keeps the order by falling rank inside each eighth of the records, beyond that plain chunk order (as
 // the sorting form does).
 template <int MAXT, int MAXN>
@@ -343,6 +344,228 @@ __global__ __launch_bounds__(1024) void gather_count_kernel(const GatherArgs g, 
             }
         }
         out[q] = v;
+    }
+}
+
+// Inclusive sum over the lanes of a wavefront, all of which are active.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v)
+{
+    auto take = [](uint32_t x, auto ctrl, auto rows) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    };
+    using std::integral_constant;
+    v += take(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});       // row_shr:1, 2, 4, 8
+    v += take(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
+    v += take(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
+    v += take(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
+    v += take(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});       // row_bcast:15, 31
+    v += take(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});
+    return v;
+}
+
+// The counting form of an ordinary decode batch: up to 512 tokens over fewer than 2048 adapters.
+//
+// What bounds it is the chain of steps between barriers, so it has fewer and shorter ones than the kernel above: a token's
+// 64-token run (the lanes of one wavefront) adds its count to one byte of the adapter's eight, all runs at once, instead of in
+// turn; the bytes below a run's own give its place and all eight the adapter's tokens (v_sad_u8 adds four).  The scan over
+// the adapters moves between lanes by DPP and takes one barrier, the order by rank is one comparison with each other chunk of
+// the same eighth, and four wavefronts have shorter barriers than sixteen (the records are written by four times as many
+// workgroups).  Time stamps of the kernel above: of 5 to 7 us 1.8 were the scan, 0.6 to 1.0 the counting, 0.5 to 1.6 the order
+// by rank and 1.2 the records.  Whole steps, that kernel -> this one: 32 tokens of 8 adapters and one projection 12.7 -> 11.2 us, a
+// graph of 7 tokens of mixed ranks, four layers 62.0 -> 59.4, 256 tokens of 64 adapters, four layers 93.6 -> 91.8.
+constexpr int FEW_NT = 256;
+constexpr int FEW_MAX_T = 512;               // eight runs of 64
+constexpr int FEW_MAX_N = 2048;              // adapters and one for "none"
+__global__ __launch_bounds__(FEW_NT) void gather_few_kernel(const GatherArgs g, const int n_rec_blocks)
+{
+    constexpr int NT = FEW_NT, EPT = FEW_MAX_T / NT, NW = NT / 64;
+    constexpr int PER_EIGHTH = FEW_MAX_T / 8;                          // chunks of an eighth at most
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int)blockIdx.x >= n_rec_blocks) { per_token_view(g, (int)blockIdx.x - n_rec_blocks, NT); return; }
+    const bool first_block = blockIdx.x == 0;
+
+    __shared__ __attribute__((aligned(8))) uint32_t s_cnt[FEW_MAX_N][2];        // byte w: tokens of run w; [n_adapters] = without one
+    __shared__ uint32_t s_base[FEW_MAX_N];                                      // first position | first chunk << 14
+    __shared__ uint16_t s_perm[FEW_MAX_T];
+    __shared__ int4 s_chunk[FEW_MAX_T];                                         // start | len << 13, adapter (n = none), rank, scaling
+    __shared__ int4 s_rec[FEW_MAX_T];                                           // the same in the order of the records
+    __shared__ __attribute__((aligned(16))) uint16_t s_key[8][PER_EIGHTH];      // rank << 6 | 63 - place, of the chunks of an eighth
+    __shared__ uint32_t s_tot[NW][2];
+    __shared__ int s_bad;
+    const int T = g.T, n = g.n_adapters;
+    for (int i = tid; i <= n; i += NT) *reinterpret_cast<uint2 *>(s_cnt[i]) = make_uint2(0u, 0u);
+    if (tid < 8 * PER_EIGHTH * 2 / 16) reinterpret_cast<int4 *>(s_key)[tid] = make_int4(0, 0, 0, 0);
+    if (tid == 0) s_bad = 0;
+    // adapter (n = none), and what its record will need, of this thread's tokens e * NT + tid
+    int key[EPT], rk[EPT], pg[EPT];
+    float sc[EPT];
+    bool bad[EPT];
+#pragma unroll
+    for (int e = 0; e < EPT; e++) {
+        const int i = e * NT + tid;
+        key[e] = n; rk[e] = 0; sc[e] = 0.f; pg[e] = 0; bad[e] = false;
+        if (i < T) {
+            const int a = gather_adapter(g, i);
+            bad[e] = a >= n;
+            if (a >= 0 && !bad[e]) key[e] = a;
+        }
+    }
+    if (g.work) {
+#pragma unroll
+        for (int e = 0; e < EPT; e++)
+            if (key[e] < n) {                  // requested now, used after the counting; the page table's line for the records
+                const int r = gather_rank(g, key[e]);
+                rk[e] = r < 0 ? 0 : (r > MAX_RANK ? MAX_RANK : r);
+                sc[e] = gather_scale(g, key[e]);
+                if (g.page_tbl) pg[e] = g.page_tbl[(long long)key[e] * g.max_pages];
+            }
+    }
+    int nbits = 1;
+    while ((n >> nbits) != 0) nbits++;
+    __syncthreads();
+    int in_wave[EPT];
+#pragma unroll
+    for (int e = 0; e < EPT; e++) {
+        in_wave[e] = 0;
+        if (e * NT < T) {
+            const bool act = e * NT + tid < T;
+            const unsigned long long same = same_key((unsigned)key[e], nbits, __ballot(act));
+            in_wave[e] = __popcll(same & ((1ull << lane) - 1ull));
+            const int w = e * NW + wave;
+            if (act && in_wave[e] == 0) atomicAdd(&s_cnt[key[e]][w >> 2], (uint32_t)__popcll(same) << (8 * (w & 3)));
+            if (first_block) {
+                const unsigned long long mb = __ballot(bad[e]);
+                if (lane == 0 && mb) atomicAdd(&s_bad, __popcll(mb));
+            }
+        }
+    }
+    __syncthreads();
+    // start, segment index and first chunk of every adapter, in adapter order (tokens without one come last)
+    const int gmask = g.group - 1, gshift = __builtin_ctz((unsigned)g.group);
+    const int per = (n + NT) / NT, a0 = tid * per;                     // adapters a0 .. a0 + per of 0 .. n
+    auto tokens_of = [&](int a) {
+        const uint2 v = *reinterpret_cast<const uint2 *>(s_cnt[a]);
+        return __builtin_amdgcn_sad_u8(v.x, 0u, __builtin_amdgcn_sad_u8(v.y, 0u, 0u));
+    };
+    uint32_t own_ts = 0, own_ch = 0;                                   // tokens | segments << 16, chunks
+    for (int q = 0; q < per; q++) {
+        const int a = a0 + q;
+        const uint32_t c = a <= n ? tokens_of(a) : 0u;
+        own_ts += c | (uint32_t)(c > 0 && a < n) << 16;
+        own_ch += (c + gmask) >> gshift;
+    }
+    const uint32_t in_ts = wave_scan(own_ts), in_ch = wave_scan(own_ch);
+    if (lane == 63) { s_tot[wave][0] = in_ts; s_tot[wave][1] = in_ch; }
+    __syncthreads();
+    uint32_t ts = in_ts - own_ts, ch = in_ch - own_ch, all_ts = 0, all_ch = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        const uint32_t t = s_tot[w][0], c = s_tot[w][1];
+        ts += w < wave ? t : 0u; ch += w < wave ? c : 0u;
+        all_ts += t; all_ch += c;
+    }
+    for (int q = 0; q < per; q++) {
+        const int a = a0 + q;
+        if (a > n) break;
+        const uint32_t c = tokens_of(a), start = ts & 0xffffu, seg = ts >> 16;
+        s_base[a] = start | ch << 14;
+        if (first_block && c > 0 && a < n) { g.seg_start[seg] = (int)start; g.seg_len[seg] = (int)c; g.seg_adapter[seg] = a; }
+        ts += c | (uint32_t)(c > 0 && a < n) << 16;
+        ch += (c + gmask) >> gshift;
+    }
+    const int n_chunks = (int)all_ch, per_xcd = (n_chunks + 7) >> 3;
+    __syncthreads();
+    // Records b, b + 8, ... hold one eighth of the chunks, by falling rank inside it (ties keep chunk order: the chunks of one
+    // adapter stay next to each other).  Where all ranks are equal that is the order of the chunks.
+    const bool by_rank = g.rank != nullptr;
+#pragma unroll
+    for (int e = 0; e < EPT; e++) {
+        const int i = e * NT + tid;
+        if (i < T) {
+            const uint32_t b = s_base[key[e]];
+            const uint2 v = *reinterpret_cast<const uint2 *>(s_cnt[key[e]]);
+            const int w = e * NW + wave;
+            const uint32_t below = (1u << (8 * (w & 3))) - 1u;
+            const int idx = (int)__builtin_amdgcn_sad_u8(v.x & (w < 4 ? below : ~0u), 0u, __builtin_amdgcn_sad_u8(v.y & (w < 4 ? 0u : below), 0u, (uint32_t)in_wave[e]));
+            const int total = (int)__builtin_amdgcn_sad_u8(v.x, 0u, __builtin_amdgcn_sad_u8(v.y, 0u, 0u));
+            const int at = (int)(b & 0x3fffu) + idx;
+            s_perm[at] = (uint16_t)i;
+            if ((idx & gmask) == 0) {
+                const int c = (int)(b >> 14) + (idx >> gshift), left = total - idx;
+                int eighth = 0;
+#pragma unroll
+                for (int k = 1; k < 8; k++) eighth += c >= k * per_xcd;
+                const int4 h = make_int4(at | (left < g.group ? left : g.group) << TOK_BITS, key[e], rk[e], __builtin_bit_cast(int, sc[e]));
+                s_chunk[c] = h;
+                if (by_rank) s_key[eighth][c - eighth * per_xcd] = (uint16_t)(rk[e] << 6 | (63 - (c - eighth * per_xcd)));
+                else s_rec[c] = h;
+            }
+        }
+        asm volatile("" :: "v"(pg[e]));        // the page table's line has arrived
+    }
+    __syncthreads();
+    if (by_rank && g.work) {
+        for (int c = tid; c < n_chunks; c += NT) {
+            int eighth = 0;
+#pragma unroll
+            for (int k = 1; k < 8; k++) eighth += c >= k * per_xcd;
+            const int first = eighth * per_xcd;
+            const uint32_t own = s_key[eighth][c - first];
+            int at = first;
+            for (int j = 0; j < per_xcd; j += 8) {                      // keys past the chunks are 0: never greater
+                const uint4 k8 = *reinterpret_cast<const uint4 *>(&s_key[eighth][j]);
+                at += ((k8.x & 0xffffu) > own) + ((k8.x >> 16) > own) + ((k8.y & 0xffffu) > own) + ((k8.y >> 16) > own) +
+                      ((k8.z & 0xffffu) > own) + ((k8.z >> 16) > own) + ((k8.w & 0xffffu) > own) + ((k8.w >> 16) > own);
+            }
+            s_rec[at] = s_chunk[c];
+        }
+        __syncthreads();
+    }
+    const int tmask = (1 << TOK_BITS) - 1;
+    if (g.work) {
+        // 16 bytes per step: header quad, two token quads, a zero quad, then 16 quads of row indices.
+        constexpr int QPR = WORK_WORDS / 4;
+        int4 *out = reinterpret_cast<int4 *>(g.work);
+        const int quads = g.work_cap * QPR;
+        for (int q = (int)blockIdx.x * NT + tid; q < quads; q += n_rec_blocks * NT) {
+            const int b = q / QPR, w4 = q - b * QPR;
+            const int pos = (b & 7) * per_xcd + (b >> 3);
+            int4 v = make_int4(0, w4 == 0 ? -1 : 0, 0, 0);
+            if ((b >> 3) < per_xcd && pos < n_chunks) {
+                const int4 h = s_rec[pos];
+                const int start = h.x & tmask, len = h.x >> TOK_BITS, a = h.y < n ? h.y : -1, r = h.z;
+                if (w4 == 0) v = make_int4(len, a, r, h.w);
+                else if (w4 <= 2) {
+                    const int k0 = (w4 - 1) * 4;
+                    v.x = k0 + 0 < len ? (int)s_perm[start + k0 + 0] : -1;
+                    v.y = k0 + 1 < len ? (int)s_perm[start + k0 + 1] : -1;
+                    v.z = k0 + 2 < len ? (int)s_perm[start + k0 + 2] : -1;
+                    v.w = k0 + 3 < len ? (int)s_perm[start + k0 + 3] : -1;
+                } else if (w4 >= WORK_ROWS_AT / 4) {
+                    const int j0 = (w4 - WORK_ROWS_AT / 4) * 4;
+                    int rr[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int j = j0 + e;
+                        rr[e] = (a >= 0 && j < r) ? gather_row(g, a, j) : -1;
+                    }
+                    v = make_int4(rr[0], rr[1], rr[2], rr[3]);
+                }
+            }
+            out[q] = v;
+        }
+    }
+    if (first_block) {
+        for (int i = tid; i < T; i += NT) g.perm[i] = s_perm[i];
+        for (int c = tid; c < n_chunks; c += NT) {
+            const int4 h = s_chunk[c];
+            g.chunk_start[c] = h.x & tmask;
+            g.chunk_len[c] = h.x >> TOK_BITS;
+            g.chunk_adapter[c] = h.y < n ? h.y : -1;
+        }
+        if (tid < 8)
+            g.counters[tid] = tid == 0 ? (int)(all_ts >> 16) : tid == 1 ? T - (int)tokens_of(n) : tid == 2 ? n_chunks : tid == 3 ? s_bad : 0;
     }
 }
 
@@ -602,6 +825,15 @@ __global__ __launch_bounds__(GATHER_NT) void gather_kernel(const GatherArgs g)
 int launch_gather(const GatherArgs &a, hipStream_t s)
 {
     const long long per_tok = (a.out_row_off || a.out_rank || a.out_scale) ? (long long)a.T * a.max_pages : 0;
+    // Beyond 512 tokens the runs no longer fit the eight bytes of a counter, beyond 2047 adapters a thread scans more than eight.
+    if (a.perm && a.T <= FEW_MAX_T && a.n_adapters < FEW_MAX_N) {
+        // a workgroup per 256 16-byte pieces of the records, up to a quarter of the chip
+        const long long quads = a.work ? (long long)a.work_cap * (WORK_WORDS / 4) : 0;
+        int nb = (int)((quads + FEW_NT - 1) / FEW_NT);
+        nb = nb < 1 ? 1 : (nb > 64 ? 64 : nb);
+        hipLaunchKernelGGL(gather_few_kernel, dim3((unsigned)(nb + (per_tok + FEW_NT - 1) / FEW_NT)), dim3(FEW_NT), 0, s, a, nb);
+        return (int)hipGetLastError();
+    }
     const unsigned view = (unsigned)((per_tok + GATHER_NT_MAX - 1) / GATHER_NT_MAX);
     // The counting form needs one LDS counter per adapter (and one for "none"); larger pools sort.  512 tokens of 6000
     // adapters, where the counters are cleared and scanned in six rounds: 17 us counting, 31 sorting.

@@ -115,3 +115,15 @@ def test_gather_order_by_rank_over_many_chunks(ranks):
     pool = _pool(1500, rng.choice(ranks, 1500), 8, rng)
     say(f"gather order by rank, ranks {ranks}")
     _check(rng.integers(-1, 1500, 2048).astype(np.int32), pool, 1)
+
+
+@pytest.mark.parametrize("T,N,group", [(1, 2047, 1), (64, 255, 1), (65, 256, 2), (255, 257, 4), (256, 1023, 8), (257, 1024, 1),
+                                       (449, 3, 8), (511, 2047, 1), (512, 511, 1), (512, 2047, 2), (513, 2047, 1)])
+def test_gather_of_an_ordinary_batch(T, N, group):
+    """Runs of 64 tokens, one to eight adapters a thread, up to 64 chunks an eighth: the remainders of each, and one token
+    more than the form takes."""
+    rng = np.random.default_rng(T * 3 + N)
+    pool = _pool(N, rng.choice([8, 16, 24, 40, 64], N), 8, rng)
+    say(f"gather ordinary batch T={T} N={N} group={group}")
+    _check(rng.integers(-1, N, T).astype(np.int32), pool, group)
+    _check(np.minimum(rng.integers(-1, N + 40, T), 7).astype(np.int32) % N, pool, group)     # a few much-used adapters
