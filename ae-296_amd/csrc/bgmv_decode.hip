@@ -18,9 +18,10 @@
 // and across wavefronts through LDS.
 // Expand: every lane owns 8 contiguous output columns, so a wavefront reads 1 KiB
 // contiguous from each B rank row and writes y with 16-byte stores.  With PF the first B rows
-// and the y rows of a lane's first output chunk are requested before the reduction, into the
-// registers the A rows have just vacated, so the expand does not start on a cold pipe (measured:
-// up to 20 % at four tokens per item and rank 64, nothing or a small loss at one or two tokens).
+// and the y rows of a lane's first output chunk are requested ahead of the expand: with one or two tokens
+// an item behind the first A rows (one round trip to memory less: 32 tokens of rank 16 9.0 -> 8.6 us a call,
+// 64 tokens x 3 projections 10.4 -> 10.2), with more into the registers the A rows have just vacated
+// (up to 20 % at four tokens per item and rank 64).
 //
 // Replaces punica.ops.add_lora_bgmv as called from lightllm/models/lora_gpu.py:138,150,162.
 #include "mlora_args.hpp"
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
     const int cl = lane & 15, rg = lane >> 4;
     const PoolView &pv = p.pool;
 
-    int proj, ntok = 1, adapter, r;
+    int proj, part = 0, ntok = 1, adapter, r;
     float scale;
     int tok[G];
     const int32_t *__restrict__ rows = nullptr;                 // WORK: row index of rank row j at rows[j]
@@ -67,8 +68,9 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
         // Records are stored in launch order: record b belongs to workgroup b of every projection.
         // The gather interleaves consecutive chunks over the 8 XCDs (workgroups are dealt to XCDs
         // round-robin by id), so the chunks of one hot adapter share one XCD's L2.
-        const int b = blockIdx.x % p.items_cap;
-        proj = blockIdx.x / p.items_cap;
+        const int b = blockIdx.x % p.items_cap, rest = blockIdx.x / p.items_cap;
+        proj = rest % p.n_proj;
+        part = rest / p.n_proj;
         const int32_t *__restrict__ rec = p.work + (size_t)b * WORK_WORDS;
         ntok = rec[0];
         if (ntok <= 0) return;
@@ -116,7 +118,9 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
     uint16_t *__restrict__ y = static_cast<uint16_t *>(p.y[proj]);
     const uint16_t *__restrict__ arows = static_cast<const uint16_t *>(p.a_rows[proj]);
     const uint16_t *__restrict__ brows = static_cast<const uint16_t *>(p.b_rows[proj]);
-    const int ncc_out = hout >> 3;
+    // the 16-byte chunks of a row of y that this workgroup makes
+    const int per_part = WORK ? ((hout >> 3) + p.parts - 1) / p.parts : hout >> 3;
+    const int cc0 = part * per_part, cc1 = cc0 + per_part < (hout >> 3) ? cc0 + per_part : hout >> 3;
 
     if (adapter < 0) {
         // No adapter: y = delta mode must still define the row (zeros).  The reference-layout
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
 #pragma unroll
             for (int k = 0; k < G; k++)
                 if (tok[k] >= 0)
-                    for (int cc = tid; cc < ncc_out; cc += NT) stg16(y + (size_t)tok[k] * hout + (size_t)cc * 8, zero16());
+                    for (int cc = cc0 + tid; cc < cc1; cc += NT) stg16(y + (size_t)tok[k] * hout + (size_t)cc * 8, zero16());
         }
         return;
     }
@@ -190,50 +194,59 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
 #pragma unroll
         for (int i = 0; i < RPG; i++) acc[k][i] = 0.f;
 
-#pragma unroll 1
-    for (int it0 = 0; it0 < n_it; it0 += U) {
-        uint4 xv[G][U];
-        uint4 av[RPG][U];
-        bool cv[U];
+    uint4 xv[G][U];
+    uint4 av[RPG][U];
+    auto request = [&](int it0) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int c = c0 + (it0 + u) * 16;
-            cv[u] = (it0 + u) < n_it && c < ncc_in;
-            const int cs = c < ncc_in ? c : ncc_in - 1;
+            const int c = c0 + (it0 + u) * 16, cs = c < ncc_in ? c : ncc_in - 1;
 #pragma unroll
             for (int k = 0; k < G; k++) xv[k][u] = ldg16_stream(xp[k] + cs);
 #pragma unroll
             for (int i = 0; i < RPG; i++) av[i][u] = ldg16_stream(ap[i] + cs);
         }
+    };
+    auto multiply = [&](int it0) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
+            const bool cv = (it0 + u) < n_it && c0 + (it0 + u) * 16 < ncc_in;
 #pragma unroll
             for (int k = 0; k < G; k++) {
-                xv[k][u].x = cv[u] ? xv[k][u].x : 0u; xv[k][u].y = cv[u] ? xv[k][u].y : 0u;
-                xv[k][u].z = cv[u] ? xv[k][u].z : 0u; xv[k][u].w = cv[u] ? xv[k][u].w : 0u;
+                xv[k][u].x = cv ? xv[k][u].x : 0u; xv[k][u].y = cv ? xv[k][u].y : 0u;
+                xv[k][u].z = cv ? xv[k][u].z : 0u; xv[k][u].w = cv ? xv[k][u].w : 0u;
             }
 #pragma unroll
             for (int i = 0; i < RPG; i++)
 #pragma unroll
                 for (int k = 0; k < G; k++) acc[k][i] = dot8<DT>(av[i][u], xv[k][u], acc[k][i]);
         }
-    }
-
-    // First expand step requested now: its latency runs under the reduction and the two barriers.
+    };
+    // First expand step: its rows and y are requested behind the first A rows of an item of one or two tokens, and arrive while
+    // those are multiplied; with more tokens, when the A rows have left their registers.
+    constexpr bool EARLY = PF && G <= 2;
     uint4 bpre[PF ? EB : 1];
     uint4 ypre[PF ? G : 1];
-    if constexpr (PF) {
-        if (tid < ncc_out) {
+    auto request_expand = [&]() {
+        if (cc0 + tid < cc1) {
             int br[EB];
             b_rows_of(0, br);
 #pragma unroll
             for (int jj = 0; jj < EB; jj++)
-                bpre[jj] = br[jj] >= 0 ? ldg16_stream(brows + (size_t)br[jj] * hout + (size_t)tid * 8) : zero16();
+                bpre[jj] = br[jj] >= 0 ? ldg16_stream(brows + (size_t)br[jj] * hout + (size_t)(cc0 + tid) * 8) : zero16();
 #pragma unroll
             for (int k = 0; k < G; k++)
-                ypre[k] = (p.accumulate && tok[k] >= 0) ? ldg16_stream(y + (size_t)tok[k] * hout + (size_t)tid * 8) : zero16();
+                ypre[k] = (p.accumulate && tok[k] >= 0) ? ldg16_stream(y + (size_t)tok[k] * hout + (size_t)(cc0 + tid) * 8) : zero16();
         }
+    };
+    request(0);
+    if constexpr (EARLY) {
+        request_expand();
+        asm volatile("" ::: "memory");                          // the compiler leaves the requests there
     }
+    multiply(0);
+#pragma unroll 1
+    for (int it0 = U; it0 < n_it; it0 += U) { request(it0); multiply(it0); }
+    if constexpr (PF && !EARLY) request_expand();
 
 #pragma unroll
     for (int k = 0; k < G; k++)
@@ -256,8 +269,8 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
     // ---------------------------------------------------------------- expand
     if constexpr (!BT) {
 #pragma unroll 1
-        for (int cc = tid; cc < ncc_out; cc += NT) {
-            const bool pre = PF && cc == tid;            // this step's first rows and y are already in registers
+        for (int cc = cc0 + tid; cc < cc1; cc += NT) {
+            const bool pre = PF && cc == cc0 + tid;            // this step's first rows and y are already in registers
             float o[G][8];
 #pragma unroll
             for (int k = 0; k < G; k++) {
@@ -361,17 +374,34 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
     }
 }
 
-template <int DT, int G, int RMAX, bool BT, bool WORK>
-static int launch_one(const BgmvArgs &a, hipStream_t s)
+// Workgroups that share the output columns of an item: each repeats the shrink (the A rows come from L2, the items of a
+// record run on one XCD) and takes a quarter or half of the expand, while all of them fit the device at once.  A unit pulls
+// 256 KiB of an item's rows in about 4.5 us, so fewer bytes a unit is what shortens the launch.  Attention projections of
+// Llama-7B in a graph, 1 / 2 / 4 / 8 workgroups an item, us a call: rank 16, one token 6.2 / 5.3 / 5.3 / 5.4, 32 tokens x 1 projection
+// 8.6 / 7.2 / 6.6 / 6.7 (two launches 7.5), 16 x 3 9.3 / 7.8 / 7.2 / 11.7 (384 workgroups), 32 x 3 9.4 / 8.0 / 12.7 (384) / 17.7;
+// rank 8, 8 x 4 7.1 / 6.1 / 6.2 / 6.3.
+static int column_parts(const BgmvArgs &a)
 {
+    int widest = 0, parts = 1;
+    for (int q = 0; q < a.n_proj; q++) widest = a.hout[q] > widest ? a.hout[q] : widest;
+    while (parts < 4 && 2LL * parts * a.n_proj * a.items_cap <= device_compute_units() && 2 * parts * 512 <= widest) parts *= 2;
+    return parts;
+}
+
+template <int DT, int G, int RMAX, bool BT, bool WORK>
+static int launch_one(const BgmvArgs &a0, hipStream_t s)
+{
+    BgmvArgs a = a0;
+    a.parts = WORK ? column_parts(a) : 1;
     // Work items of one or two tokens are the small-batch form: a launch of at most about one
     // workgroup per CU, bound by the chain launch -> record -> page table -> rows -> y.  Twice the
     // threads halve the shrink's load rounds and the early expand requests overlap the reduction
-    // (8.5 vs 9.9 us per call at 64 tokens, 10.8 vs 13.2 us at 128, three projections).
+    // (8.5 vs 9.9 us per call at 64 tokens, 10.8 vs 13.2 us at 128, three projections; before the requests moved ahead of
+    // the shrink and items were shared).
     constexpr bool WIDE = WORK && !BT && G <= 2;
     constexpr int NT = WIDE ? 512 : 256;
     const long long per_proj = WORK ? a.items_cap : a.T;
-    const long long total = (long long)a.n_proj * per_proj;
+    const long long total = (long long)a.n_proj * per_proj * a.parts;
     if (total <= 0) return 0;
     if (total > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     // Early expand requests pay for their registers when a work item carries several tokens, or when

@@ -536,3 +536,17 @@ def test_bgmv_default_form_is_the_one_the_rule_names(T, ranks, hin, hout, form):
     got = _run(pp, x, tok, y0, group)
     assert_close_bits(got, oracle_apply(pp, x, tok, y0), FP16, form)
     assert np.array_equal(got, _run_form(pp, x, tok, y0, group, getattr(_ext, "FORM_" + form)))
+
+
+@pytest.mark.parametrize("accumulate", [True, False])
+@pytest.mark.parametrize("T,group,hout", [(1, 1, 1032), (32, 1, 1024), (33, 1, 2056), (64, 2, 2048), (61, 2, 5128), (120, 1, 1016), (100, 4, 4104)])
+def test_bgmv_fused_items_shared_by_workgroups(T, group, hout, accumulate):
+    """One, two and four workgroups an item, with column counts that leave the last one less."""
+    rng = np.random.default_rng(T + hout)
+    pp = PagedPool(rng, rng.choice([8, 16, 5], 9), 712, hout, page_rows=8, dtype=BF16 if T % 2 else FP16)
+    tok = rng.integers(-1, 9, T).astype(np.int32)
+    x = bits_of(rng.standard_normal((T, 712)).astype(np.float32), pp.dtype)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), pp.dtype) if accumulate else None
+    say(f"bgmv fused, shared items T={T} group={group} hout={hout} accumulate={accumulate}")
+    got = _run(pp, x, tok, y0, group, accumulate=accumulate, fused=True)
+    assert_close_bits(got, oracle_apply(pp, x, tok, y0), pp.dtype, f"T={T} hout={hout}")
