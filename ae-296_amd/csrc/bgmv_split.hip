@@ -60,15 +60,40 @@ __device__ __forceinline__ typename RecPtr<BIG>::type record_at(const int32_t *w
 
 constexpr int FINE_CHUNKS = 64;                                // slice width of a small launch, shrink and expand (512 columns)
 
-struct ItemId { int b, q; };
-
-__device__ __forceinline__ ItemId split_id(unsigned id, int nq)
+// Projection and slice of number q of a record, from the ends of the projections' numbers.  All ends are read at once: looking
+// them up one after the other is a chain of scalar loads in front of everything else.  (The record is the grid's second
+// dimension, which saves a division.)  Four layers: 125 tokens of mixed ranks, seven projections 255.6 -> 249.3 us, 256
+// tokens of rank 16, four projections 91.8 -> 90.2.
+struct SliceId { int proj, slice; };
+__device__ __forceinline__ SliceId slice_at(const int (&end)[MAX_PROJ], int q)
 {
-    ItemId r;
-    r.b = (int)(id / (unsigned)nq);
-    r.q = (int)(id - (unsigned)r.b * (unsigned)nq);
+    SliceId r = {0, q};
+#pragma unroll
+    for (int i = 0; i + 1 < MAX_PROJ; i++)
+        if (q >= end[i]) { r.proj = i + 1; r.slice = q - end[i]; }
     return r;
 }
+
+// Rows of a record's rank rows.  In a small launch (EARLY) every lane requests one of the 64 with the header, so that the rows
+// do not wait for the rank first, and the others get it from its register; in larger ones, where other workgroups fill the
+// wait, they are read where they are needed (the 125 tokens above 249 us that way, 259 with the lanes' rows; a graph of seven
+// tokens, small launches, 59.4 -> 58.7 with them).  pin() comes before any branch that part of a wavefront takes: a lane's row is
+// also read by the others.
+template <bool BIG, bool EARLY>
+struct Rows {
+    typename RecPtr<BIG>::type at;
+    __device__ __forceinline__ Rows(typename RecPtr<BIG>::type rec) : at(rec + WORK_ROWS_AT) {}
+    __device__ __forceinline__ void pin() {}
+    __device__ __forceinline__ int of_lane(int j) const { return at[j]; }
+};
+template <>
+struct Rows<false, true> {
+    int mine;
+    __device__ __forceinline__ Rows(RecPtr<false>::type rec) : mine(rec[WORK_ROWS_AT + (threadIdx.x & 63)]) {}
+    __device__ __forceinline__ void pin() { asm volatile("" : "+v"(mine)); }
+    __device__ __forceinline__ int of_lane(int j) const { return __shfl(mine, j); }
+    __device__ __forceinline__ int uniform(int j) const { return __builtin_amdgcn_readlane(mine, j); }     // j the same in all lanes
+};
 
 // Slices of the launch's width (Slices<RMAX>::KSC) that one shrink workgroup takes, by the rank bucket of
 // its item (more than 32, 17..32, 9..16, at most 8 rank rows): the bytes of a workgroup grow with
@@ -87,8 +112,8 @@ __device__ __forceinline__ int slice_factor(int r)
 // Shrink of one (item, projection, column slice) over the first 4 * NR rank rows (NR per 16-lane
 // row).  The caller picks the smallest NR that covers the item's rank, so an adapter of rank 8 in a
 // pool that goes up to rank 64 issues loads for 8 rows, not 64.
-template <int DT, int G, int RMAX, int KSC, int NR, bool HOT, class RowsPtr>
-__device__ __forceinline__ void shrink_rows(const BgmvArgs &p, RowsPtr rows, const int (&tok)[G],
+template <int DT, int G, int RMAX, int KSC, int NR, bool HOT, class Rows>
+__device__ __forceinline__ void shrink_rows(const BgmvArgs &p, const Rows &rows, const int (&tok)[G],
                                             int r, int proj, int ks, int slot, float (&s_part)[4][G][RMAX])
 {
     constexpr int NW = 4;
@@ -116,7 +141,7 @@ __device__ __forceinline__ void shrink_rows(const BgmvArgs &p, RowsPtr rows, con
     unsigned row_ok = 0;
 #pragma unroll
     for (int i = 0; i < NR; i++) {
-        int row = rows[rg + 4 * i];
+        int row = rows.of_lane(rg + 4 * i);
         row = (row >= 0 && row < pv.n_rows_a) ? row : -1;
         row_ok |= (row >= 0 ? 1u : 0u) << i;
         ap[i] = reinterpret_cast<const uint4 *>(arows + (size_t)(row >= 0 ? row : 0) * hin) + (whole ? c_first : 0);
@@ -200,19 +225,19 @@ __global__ __launch_bounds__(256) void bgmv_shrink_kernel(const BgmvArgs p)
     __shared__ float s_part[4][G][RMAX];
 
     // workgroup -> (record, projection, slice): only the slices a projection has are numbered
-    const ItemId id = split_id(blockIdx.x, p.sh_end[p.n_proj - 1]);
-    int proj = 0;
-    while (proj + 1 < p.n_proj && id.q >= p.sh_end[proj]) proj++;
-    const int ks = id.q - (proj ? p.sh_end[proj - 1] : 0);
-    // A workgroup serves records id.b, id.b + stride, ...: the launch covers `rec_stride` records, not the
+    const SliceId id = slice_at(p.sh_end, (int)blockIdx.x);
+    const int proj = id.proj, ks = id.slice;
+    // A workgroup serves records blockIdx.y, blockIdx.y + stride, ...: the launch covers `rec_stride` records, not the
     // host's upper bound on them (the records in use of one XCD residue are a prefix, so the first empty one ends
     // the walk).  Most batches need one pass; what a grid over the whole bound would spend on dispatching
     // workgroups of empty records is saved.
-    int b = id.b;
+    int b = (int)blockIdx.y;
     do {
         const typename RecPtr<BIG>::type rec = record_at<BIG>(p.work, b);
+        Rows<BIG, KSC == FINE_CHUNKS> rows(rec);
         int ntok = rec[0];
         if (ntok <= 0) break;
+        rows.pin();
         ntok = ntok < G ? ntok : G;
         const int adapter = rec[1];
         if (adapter < 0) continue;
@@ -224,7 +249,6 @@ __global__ __launch_bounds__(256) void bgmv_shrink_kernel(const BgmvArgs p)
             const int t = k < ntok ? rec[4 + k] : -1;
             tok[k] = (t >= 0 && t < p.T) ? t : -1;
         }
-        const typename RecPtr<BIG>::type rows = rec + WORK_ROWS_AT;
 
         // r is uniform over the workgroup: a scalar branch, no divergence.  An item of a lower rank bucket
         // takes F consecutive slices in one workgroup (the others of the F skip it) and stores its sums
@@ -257,10 +281,8 @@ __global__ __launch_bounds__(NTE) void bgmv_expand_kernel(const BgmvArgs p)
     const int tid = threadIdx.x;
     const PoolView &pv = p.pool;
 
-    const ItemId id = split_id(blockIdx.x, p.ex_end[p.n_proj - 1]);
-    int proj = 0;
-    while (proj + 1 < p.n_proj && id.q >= p.ex_end[proj]) proj++;
-    const int cs = id.q - (proj ? p.ex_end[proj - 1] : 0);
+    const SliceId id = slice_at(p.ex_end, (int)blockIdx.x);
+    const int proj = id.proj, cs = id.slice;
     const int hout = p.hout[proj];
     const int ncc_out = hout >> 3;
     const int cc = cs * NTE + tid;
@@ -270,8 +292,8 @@ __global__ __launch_bounds__(NTE) void bgmv_expand_kernel(const BgmvArgs p)
     const unsigned voff = (unsigned)(active ? cc : 0) * 16u;
     const int n_ks = ((p.hin[proj] >> 3) + KSC - 1) / KSC;
 
-    // records id.b, id.b + stride, ... (see the shrink kernel)
-    int b = id.b;
+    // records blockIdx.y, blockIdx.y + stride, ... (see the shrink kernel)
+    int b = (int)blockIdx.y;
     do {
         const typename RecPtr<BIG>::type rec = record_at<BIG>(p.work, b);
         int ntok = rec[0];
@@ -287,6 +309,7 @@ __global__ __launch_bounds__(NTE) void bgmv_expand_kernel(const BgmvArgs p)
             const int t = k < ntok ? rec[4 + k] : -1;
             tok[k] = (t >= 0 && t < p.T) ? t : -1;
         }
+
         const typename RecPtr<BIG>::type rows = rec + WORK_ROWS_AT;
 
         if (adapter < 0) {
@@ -412,10 +435,8 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const ItemId id = split_id(blockIdx.x, p.ex_end[p.n_proj - 1]);
-    int proj = 0;
-    while (proj + 1 < p.n_proj && id.q >= p.ex_end[proj]) proj++;
-    const int cs = id.q - (proj ? p.ex_end[proj - 1] : 0);
+    const SliceId id = slice_at(p.ex_end, (int)blockIdx.x);
+    const int proj = id.proj, cs = id.slice;
     const int hout = p.hout[proj];
     const int ncc_out = hout >> 3;
     const int cc = cs * FINE_CHUNKS + lane;
@@ -424,9 +445,11 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
     const uint16_t *__restrict__ brows = static_cast<const uint16_t *>(p.b_rows[proj]);
     const int n_ks = ((p.hin[proj] >> 3) + KSC - 1) / KSC;
 
-    const int32_t *__restrict__ rec = p.work + (size_t)id.b * WORK_WORDS;
+    const int32_t *__restrict__ rec = p.work + (size_t)blockIdx.y * WORK_WORDS;
+    Rows<false, true> rows(rec);
     int ntok = rec[0];
     if (ntok <= 0) return;
+    rows.pin();
     ntok = ntok < G ? ntok : G;
     const int adapter = rec[1];
     int r = rec[2];
@@ -445,7 +468,6 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
         if (!p.accumulate && active && ytok >= 0) stg16(yp, zero16());
         return;
     }
-    const int32_t *__restrict__ rows = rec + WORK_ROWS_AT;
     uint4 yv = zero16();
     float o[G][8];
 #pragma unroll
@@ -460,7 +482,7 @@ __global__ __launch_bounds__(256) void bgmv_expand_fine_kernel(const BgmvArgs p)
         uint4 bv[N];
 #pragma unroll
         for (int i = 0; i < N; i++) {
-            const int row = rows[j0 + i];
+            const int row = rows.uniform(j0 + i);
             const bool ok = active && row >= 0 && row < p.pool.n_rows_b;
             bv[i] = ok ? ldg16_stream(brows + (size_t)row * hout + (size_t)cc * 8) : zero16();
         }
@@ -580,16 +602,14 @@ __global__ __launch_bounds__(256) void bgmv_expand_bt_kernel(const BgmvArgs p)
     __shared__ __attribute__((aligned(16))) float s_out[G][COLS];
 
     const int tid = threadIdx.x;
-    const ItemId id = split_id(blockIdx.x, p.ex_end[p.n_proj - 1]);
-    int proj = 0;
-    while (proj + 1 < p.n_proj && id.q >= p.ex_end[proj]) proj++;
-    const int cs = id.q - (proj ? p.ex_end[proj - 1] : 0);
+    const SliceId id = slice_at(p.ex_end, (int)blockIdx.x);
+    const int proj = id.proj, cs = id.slice;
     const int hout = p.hout[proj];
     uint16_t *__restrict__ y = static_cast<uint16_t *>(p.y[proj]);
     const int col0 = cs * COLS;
     const int n_ks = ((p.hin[proj] >> 3) + KSC - 1) / KSC;
 
-    const int32_t *__restrict__ rec = p.work + (size_t)id.b * WORK_WORDS;
+    const int32_t *__restrict__ rec = p.work + (size_t)blockIdx.y * WORK_WORDS;
     int ntok = rec[0];
     if (ntok <= 0) return;
     ntok = ntok < G ? ntok : G;
@@ -688,6 +708,7 @@ __global__ __launch_bounds__(256) void bgmv_expand_bt_kernel(const BgmvArgs p)
 // (that many records are in use whenever every token has an adapter entry) and large enough for the launch to
 // hold a few rounds of workgroups, so that small batches keep one workgroup per record.
 constexpr int GRID_TARGET = 3072;                               // (record, slice) pairs a many-round launch covers at least
+constexpr int MAX_STRIDE = 65528;                               // the grid's second dimension
 template <int G>
 static int record_stride(const BgmvArgs &a, int slices, bool big)
 {
@@ -696,6 +717,7 @@ static int record_stride(const BgmvArgs &a, int slices, bool big)
     const long long fill = (GRID_TARGET + slices - 1) / slices;
     want = want > fill ? want : fill;
     want = (want + 7) / 8 * 8;
+    want = want < MAX_STRIDE ? want : MAX_STRIDE;
     return want < a.items_cap ? (int)want : a.items_cap;
 }
 
@@ -707,14 +729,12 @@ static int launch_pair_bt(const BgmvArgs &a0, hipStream_t s)
     a.rec_stride_ex = record_stride<G>(a, a.ex_end[a.n_proj - 1], false);
     constexpr int RMAX = R <= 16 ? 16 : (R <= 32 ? 32 : 64);
     constexpr int KSC = Slices<RMAX>::KSC;
-    const long long n_sh = (long long)a.sh_end[a.n_proj - 1] * a.rec_stride_sh;
-    const long long n_ex = (long long)a.ex_end[a.n_proj - 1] * a.rec_stride_ex;
-    if (n_sh <= 0 || n_ex <= 0) return 0;
-    if (n_sh > 0x7fffffffLL || n_ex > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, false>), dim3((unsigned)n_sh), dim3(256), 0, s, a);
+    const int n_sh = a.sh_end[a.n_proj - 1], n_ex = a.ex_end[a.n_proj - 1];
+    if (n_sh <= 0 || n_ex <= 0 || a.rec_stride_sh <= 0 || a.rec_stride_ex <= 0) return 0;
+    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, false>), dim3((unsigned)n_sh, (unsigned)a.rec_stride_sh), dim3(256), 0, s, a);
     int rc = (int)hipGetLastError();
     if (rc) return rc;
-    hipLaunchKernelGGL((bgmv_expand_bt_kernel<DT, G, R, KSC>), dim3((unsigned)n_ex), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((bgmv_expand_bt_kernel<DT, G, R, KSC>), dim3((unsigned)n_ex, (unsigned)a.rec_stride_ex), dim3(256), 0, s, a);
     return (int)hipGetLastError();
 }
 
@@ -747,28 +767,24 @@ static int launch_pair(const BgmvArgs &a0, hipStream_t s)
     BgmvArgs a = a0;
     a.rec_stride_sh = record_stride<G>(a, a.sh_end[a.n_proj - 1], BIG);
     a.rec_stride_ex = record_stride<G>(a, a.ex_end[a.n_proj - 1], BIG);
-    const long long n_sh = (long long)a.sh_end[a.n_proj - 1] * a.rec_stride_sh;
-    const long long n_ex = (long long)a.ex_end[a.n_proj - 1] * a.rec_stride_ex;
-    if (n_sh <= 0 || n_ex <= 0) return 0;
-    if (n_sh > 0x7fffffffLL || n_ex > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, BIG>), dim3((unsigned)n_sh), dim3(256), 0, s, a);
+    const int n_sh = a.sh_end[a.n_proj - 1], n_ex = a.ex_end[a.n_proj - 1];
+    if (n_sh <= 0 || n_ex <= 0 || a.rec_stride_sh <= 0 || a.rec_stride_ex <= 0) return 0;
+    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, BIG>), dim3((unsigned)n_sh, (unsigned)a.rec_stride_sh), dim3(256), 0, s, a);
     int rc = (int)hipGetLastError();
     if (rc) return rc;
-    hipLaunchKernelGGL((bgmv_expand_kernel<DT, G, RMAX, KSC, NTE, BIG>), dim3((unsigned)n_ex), dim3(NTE), 0, s, a);
+    hipLaunchKernelGGL((bgmv_expand_kernel<DT, G, RMAX, KSC, NTE, BIG>), dim3((unsigned)n_ex, (unsigned)a.rec_stride_ex), dim3(NTE), 0, s, a);
     return (int)hipGetLastError();
 }
 
 template <int DT, int G, int RMAX>
 static int launch_fine(const BgmvArgs &a, hipStream_t s)
 {
-    const long long n_sh = (long long)a.sh_end[a.n_proj - 1] * a.items_cap;
-    const long long n_ex = (long long)a.ex_end[a.n_proj - 1] * a.items_cap;
-    if (n_sh <= 0 || n_ex <= 0) return 0;
-    if (n_sh > 0x7fffffffLL || n_ex > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, FINE_CHUNKS, false>), dim3((unsigned)n_sh), dim3(256), 0, s, a);
+    const int n_sh = a.sh_end[a.n_proj - 1], n_ex = a.ex_end[a.n_proj - 1];
+    if (n_sh <= 0 || n_ex <= 0 || a.items_cap <= 0) return 0;
+    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, FINE_CHUNKS, false>), dim3((unsigned)n_sh, (unsigned)a.items_cap), dim3(256), 0, s, a);
     const int rc = (int)hipGetLastError();
     if (rc) return rc;
-    hipLaunchKernelGGL((bgmv_expand_fine_kernel<DT, G, RMAX, FINE_CHUNKS>), dim3((unsigned)n_ex), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((bgmv_expand_fine_kernel<DT, G, RMAX, FINE_CHUNKS>), dim3((unsigned)n_ex, (unsigned)a.items_cap), dim3(256), 0, s, a);
     return (int)hipGetLastError();
 }
 

@@ -450,6 +450,7 @@ static int bgmv_multi_impl(int form, int n_proj, void *const *y, const void *con
             ex += (hout[p] + nte * 8 - 1) / (nte * 8);
             a.sh_end[p] = sh; a.ex_end[p] = ex;
         }
+        for (int p = n_proj; p < mlora::MAX_PROJ; p++) a.sh_end[p] = a.ex_end[p] = 0x7fffffff;
         rc = mlora::launch_bgmv_split(a, dtype, group, max_rank, static_cast<hipStream_t>(stream));
     } else {
         rc = mlora::launch_bgmv(a, dtype, group, max_rank, false, static_cast<hipStream_t>(stream));
@@ -649,6 +650,7 @@ int mlora_bgmv_reflayout_multi(int n_proj, void *const *y, const void *const *x,
         ex += (hout[p] + nte * 8 - 1) / (nte * 8);
         a.sh_end[p] = sh; a.ex_end[p] = ex;
     }
+    for (int p = n_proj; p < mlora::MAX_PROJ; p++) a.sh_end[p] = a.ex_end[p] = 0x7fffffff;
     const int rc = mlora::launch_bgmv_split(a, dtype, group, r, static_cast<hipStream_t>(stream));
     if (rc) return fail(MLORA_ELAUNCH, "bgmv launch failed: %s", hipGetErrorString((hipError_t)rc));
     return MLORA_OK;

@@ -56,7 +56,7 @@ struct BgmvArgs {
     int ks_max;                    // shrink slices of the widest hin (stride of the partial sums)
     int cs_max;                    // expand slices of the widest hout
     // two-launch form: the (projection, slice) pairs that exist, numbered consecutively; sh_end[p] / ex_end[p] is
-    // the number of shrink / expand slices of projections 0..p
+    // the number of shrink / expand slices of projections 0..p, and past the last projection a number that no slice has
     int sh_end[MAX_PROJ];
     int ex_end[MAX_PROJ];
     // two-launch form: records the shrink / expand grid covers; a workgroup walks records b, b + stride, ... < items_cap
