@@ -138,7 +138,7 @@ struct SgmvArgs {
     int n_grp;
     int grp_first[MAX_PROJ], grp_n[MAX_PROJ];
     unsigned grp_end[MAX_PROJ];
-    unsigned ex_end[MAX_PROJ];     // expand launch: first workgroup id after projection p
+    unsigned ex_end[MAX_PROJ];     // expand launch: first workgroup id after projection p (few: first column block), ~0 past the last
     PoolView pool;
     const int32_t *seg_start;
     const int32_t *seg_len;

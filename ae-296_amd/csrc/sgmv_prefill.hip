@@ -100,6 +100,18 @@ __host__ __device__ inline long long expand_grid(int max_tiles, int ncb)
     return tile_major(ncb) && !few_tiles(max_tiles) ? (long long)max_tiles * ((ncb + 7) & ~7) : place_grid(max_tiles, ncb);
 }
 
+// Group (or projection) of workgroup w, and its number there, from the groups' first numbers behind them.  All ends are read at once:
+// looking them up in turn is a chain of scalar loads in front of everything else.
+struct GroupId { int group, rest; };
+__device__ __forceinline__ GroupId group_at(const unsigned (&end)[MAX_PROJ], unsigned w)
+{
+    GroupId r = {0, (int)w};
+#pragma unroll
+    for (int i = 0; i + 1 < MAX_PROJ; i++)
+        if (w >= end[i]) { r.group = i + 1; r.rest = (int)(w - end[i]); }
+    return r;
+}
+
 // What a workgroup needs to know about its tile: from the plan's record, or, for equally long segments on a dense
 // pool (the reference's prefill, segment s = adapter s), computed, which needs no plan at all.
 // (A compile-time choice: a branch on it around the row lookups made the shrink wait for each of its twelve in turn,
@@ -800,13 +812,10 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p
     __shared__ __attribute__((aligned(16))) uint16_t s_v[2][16][VPITCH];
     static_assert(16 * OPITCH * 4 <= WBYTES, "a wavefront's result fits its B tile");
 
-    int proj = 0;
-    while (proj + 1 < p.n_proj && blockIdx.x >= p.ex_end[proj]) proj++;
-    const SgmvProj &pj = p.pr[proj];
-    const int w = (int)(blockIdx.x - (proj ? p.ex_end[proj - 1] : 0u));
-    const int ncb = (pj.hout + FEW_COLS - 1) / FEW_COLS;
-    const int piece = w / ncb, colblk = w - piece * ncb, tile = piece >> 2, sub = piece & 3;
-    if (tile >= p.max_tiles) return;
+    // grid: column blocks of all projections x pieces
+    const GroupId at = group_at(p.ex_end, blockIdx.x);
+    const SgmvProj &pj = p.pr[at.group];
+    const int colblk = at.rest, tile = (int)blockIdx.y >> 2, sub = (int)blockIdx.y & 3;
     const Tile<BT> tl = tile_of<BT>(p, tile);
     const int ntok = tl.ntok - sub * 16 < 16 ? tl.ntok - sub * 16 : 16, tok0 = tl.tok0 + sub * 16;
     if (ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
@@ -825,42 +834,75 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p
                 if (q * 8 + (lane >> 3) < ntok) stg16(y + (size_t)(tok0 + q * 8 + (lane >> 3)) * hout + yc, zero16());
         return;
     }
+    // Row of rank row `lane`, requested with the partial sums; a B load gets its row from another lane.
+    int mine = -1;
+    if constexpr (!BT) mine = tl.row(lane, p.pool.n_rows_a);
+    const int nsplit = pj.ksplit;
+    const bool fold = p.fold && nsplit > 1;
+    const int ft = tid / (KP / 4), fc = (tid % (KP / 4)) * 4;           // folding: 16 tokens x 16 quads
+    float4_t part[SGMV_SPLITS];                                         // (requested also where there is nothing to fold: no branch)
+    {
+        const float *src = pj.v + (size_t)(tok0 + (ft < ntok ? ft : ntok - 1)) * VSTRIDE + fc;
+        const size_t stride = (size_t)p.T * VSTRIDE;
+#pragma unroll
+        for (int u = 0; u < SGMV_SPLITS; u++) part[u] = *reinterpret_cast<const float4_t *>(src + (u < nsplit ? u : 0) * stride);
+    }
+    // B and y: every load is made, at an address inside the operand, and what is not wanted becomes zero when it has arrived
     const uint16_t *__restrict__ brows = static_cast<const uint16_t *>(pj.b_rows);
     uint4 bv[BQ];
+    bool bok[BQ];
+    if constexpr (!BT) {
+        int row[BQ];
 #pragma unroll
-    for (int q = 0; q < BQ; q++) {
-        if constexpr (!BT) {
-            const int row = tl.row(q * 8 + (lane >> 3), p.pool.n_rows_a);
-            bv[q] = (row >= 0 && row < p.pool.n_rows_b && yc < hout) ? ldg16(brows + (size_t)row * hout + yc) : zero16();
-        } else {
+        for (int q = 0; q < BQ; q++) row[q] = __shfl(mine, q * 8 + (lane >> 3));
+#pragma unroll
+        for (int q = 0; q < BQ; q++) {
+            bok[q] = row[q] >= 0 && row[q] < p.pool.n_rows_b && yc < hout;
+            bv[q] = ldg16(brows + (bok[q] ? (size_t)row[q] * hout + yc : 0));
+        }
+    } else {
+        const uint16_t *__restrict__ bt = brows + (size_t)tl.adapter * (size_t)p.pool.b_dense_stride;
+#pragma unroll
+        for (int q = 0; q < BQ; q++) {
             const int e = q * 64 + lane, col = col0 + e / (KP / 8), k0 = (e % (KP / 8)) * 8;
-            bv[q] = (col < hout && k0 < r) ? ldg16(brows + (size_t)tl.adapter * (size_t)p.pool.b_dense_stride + (size_t)col * r + k0) : zero16();
+            bok[q] = col < hout && k0 < r;
+            bv[q] = ldg16(bt + (bok[q] ? (size_t)col * r + k0 : 0));
         }
     }
-    uint4 yv[2];
+    uint4 yv[2] = {zero16(), zero16()};
+    if (p.accumulate) {
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
-        const int t = q * 8 + (lane >> 3);
-        yv[q] = (p.accumulate && t < ntok && yc < hout) ? ldg16_stream(y + (size_t)(tok0 + t) * hout + yc) : zero16();
+        for (int q = 0; q < 2; q++) {
+            const int t = q * 8 + (lane >> 3);
+            yv[q] = ldg16_stream(y + (size_t)(tok0 + (t < ntok ? t : ntok - 1)) * hout + (yc < hout ? yc : 0));
+        }
     }
-    const bool fold = p.fold && pj.ksplit > 1;
     const int trow = m < ntok ? m : ntok - 1;
     uint4 vhi[KS], vlo[KS];
     if (fold) {
-        const int t = tid / (KP / 4), c0 = (tid % (KP / 4)) * 4;        // 16 tokens x 16 quads
         float v[4];
-        sum_splits4(pj.v + (size_t)(tok0 + (t < ntok ? t : ntok - 1)) * VSTRIDE + c0, (size_t)p.T * VSTRIDE, pj.ksplit, v);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[e] = 0.f;
+#pragma unroll
+            for (int u = 0; u < SGMV_SPLITS; u++) v[e] += u < nsplit ? part[u][e] : 0.f;
+        }
         uint32_t hi[2], lo[2];
         split_hi_lo<DT>(v, hi, lo);
-        *reinterpret_cast<uint2 *>(&s_v[0][t][c0]) = make_uint2(hi[0], hi[1]);
-        *reinterpret_cast<uint2 *>(&s_v[1][t][c0]) = make_uint2(lo[0], lo[1]);
+        *reinterpret_cast<uint2 *>(&s_v[0][ft][fc]) = make_uint2(hi[0], hi[1]);
+        *reinterpret_cast<uint2 *>(&s_v[1][ft][fc]) = make_uint2(lo[0], lo[1]);
         __syncthreads();
-    }
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        const int c0 = ks * 32 + 8 * g;
-        vhi[ks] = fold ? *reinterpret_cast<const uint4 *>(&s_v[0][trow][c0]) : ldg16(pj.vhi + (size_t)(tok0 + trow) * VSTRIDE + c0);
-        vlo[ks] = fold ? *reinterpret_cast<const uint4 *>(&s_v[1][trow][c0]) : ldg16(pj.vlo + (size_t)(tok0 + trow) * VSTRIDE + c0);
+        for (int ks = 0; ks < KS; ks++) {
+            vhi[ks] = *reinterpret_cast<const uint4 *>(&s_v[0][trow][ks * 32 + 8 * g]);
+            vlo[ks] = *reinterpret_cast<const uint4 *>(&s_v[1][trow][ks * 32 + 8 * g]);
+        }
+    } else {
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            vhi[ks] = ldg16(pj.vhi + (size_t)(tok0 + trow) * VSTRIDE + ks * 32 + 8 * g);
+            vlo[ks] = ldg16(pj.vlo + (size_t)(tok0 + trow) * VSTRIDE + ks * 32 + 8 * g);
+        }
     }
     // the wavefront's B tile through its own LDS, then its result: operations of one wavefront on LDS complete in order
     unsigned char *sb = s_b[wave];
@@ -868,7 +910,8 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p
     for (int q = 0; q < BQ; q++) {
         const int e = q * 64 + lane;
         unsigned char *at = BT ? sb + e / (KP / 8) * TPITCH + e % (KP / 8) * 16 : sb + e / 8 * BPITCH + e % 8 * 16;
-        *reinterpret_cast<uint4 *>(at) = bv[q];
+        const uint32_t keep = bok[q] ? ~0u : 0u;
+        *reinterpret_cast<uint4 *>(at) = make_uint4(bv[q].x & keep, bv[q].y & keep, bv[q].z & keep, bv[q].w & keep);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -955,11 +998,11 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     }
     const unsigned sgrid = end;
     end = 0;
-    for (int q = 0; q < g.n_proj; q++) {
-        end += g.few ? (unsigned)g.max_tiles * 4u * (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
-        g.ex_end[q] = end;
+    for (int q = 0; q < MAX_PROJ; q++) {
+        if (q < g.n_proj) end += g.few ? (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
+        g.ex_end[q] = q < g.n_proj ? end : ~0u;
     }
-    const unsigned egrid = end;
+    const dim3 egrid(end, g.few ? (unsigned)g.max_tiles * 4u : 1u);
     if ((g.seg_uniform_len > 0) != (g.b_transposed != 0)) return (int)hipErrorInvalidValue;
     if (g.seg_uniform_len > 0 && g.share_x) return (int)hipErrorInvalidValue;
     const dim3 threads(SG_NT * (g.share_x ? SH_KG<true> : SH_KG<false>));
@@ -976,15 +1019,15 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     }
     if constexpr (RMAX > 32) {
         if (g.few) {
-            if (g.b_transposed) hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, true>), dim3(egrid), dim3(SG_NT), 0, s, g);
-            else hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, false>), dim3(egrid), dim3(SG_NT), 0, s, g);
+            if (g.b_transposed) hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, true>), egrid, dim3(SG_NT), 0, s, g);
+            else hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, false>), egrid, dim3(SG_NT), 0, s, g);
             return (int)hipGetLastError();
         }
     }
     if (g.b_transposed)
-        hipLaunchKernelGGL((sgmv_expand_kernel<DT, RMAX, true>), dim3(egrid), dim3(SG_NT), 0, s, g);
+        hipLaunchKernelGGL((sgmv_expand_kernel<DT, RMAX, true>), egrid, dim3(SG_NT), 0, s, g);
     else
-        hipLaunchKernelGGL((sgmv_expand_kernel<DT, RMAX, false>), dim3(egrid), dim3(SG_NT), 0, s, g);
+        hipLaunchKernelGGL((sgmv_expand_kernel<DT, RMAX, false>), egrid, dim3(SG_NT), 0, s, g);
     return (int)hipGetLastError();
 }
 
