@@ -790,27 +790,37 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     }
 }
 
-// The expand of a launch of few tiles above rank 32.  The kernel above takes 64 tokens at a time, one 128-column step after the other, so a
+// The expand of a launch of few tiles.  The kernel above takes 64 tokens at a time, one 128-column step after the other, so a
 // prompt of a tile or two is a chain of a few long steps on a part of the chip.  Here a workgroup takes 16 tokens and 256
-// columns, 64 per wavefront, in one step, everything requested at once; B is read by four workgroups instead of one.
-// Two layers and the plan in a graph, that kernel -> this one, us: 64 tokens, q/k/v, rank 64 36.8 -> 33.6 (192 workgroups);
-// the reference's call, 64 tokens, 41.1 -> 32.4, 2 x 200 tokens 44.7 -> 37.2 (512); 4 x 300 tokens 60.5 -> 60.0 (1280); 200 tokens,
-// seven projections 64.4 -> 86.0 (2560).  So up to 512 workgroups, and not up to rank 32, where there is little B and less to sum:
-// 64 tokens, rank 16 28.2 -> 27.3, two prompts of 20 and 60, four projections 27.2 -> 29.6.
+// columns, 64 per wavefront, in one step, everything requested at once: the partial sums and the row table first, then B
+// and y; B is read by four workgroups instead of one.  What bounds it is the chain record -> row table -> B -> y; with each B load
+// waiting for its own row lookup 3.9 us of 8.8 went by before the last was requested.
+// Two layers and the plan in a graph, Llama-7B widths, that kernel -> this one, us, by workgroups: rank 64, q/k/v, 64 tokens 37.2 ->
+// 27.7 (192), 2 x 100 43.3 -> 36.6 (768), 8 x 64 60.7 -> 51.6 (2304), 2 x 512 69.1 -> 68.2 (3264), 8 x 128 73.1 -> 77.4 (3840); seven
+// projections, 2 x 100 72.9 -> 66.7 (2656), 4 x 64 77.2 -> 79.7 (3984).  Rank 32, q/k/v, 64 tokens 31.0 -> 25.0, 8 x 128 63.3 -> 62.0
+// (3840); q/k/v/o 8 x 128 74.6 -> 71.6 (5120); seven projections 8 x 64 85.1 -> 95.9 (7968).  Rank 16, q/k/v/o 16 x 64 71.5 -> 70.9 (6144);
+// seven 8 x 64 78.2 -> 83.0 (7968).  The reference's call, whose B is four times as many lines from L2, rank 64: 4 x 128 91.3 -> 76.3
+// (512), 8 x 128 100.2 -> 99.2 (1024), 16 x 64 102.3 -> 104.2 (1024); rank 16, 8 x 512 134.6 -> 128.8 (4096), 16 x 512 203.5 -> 214.0 (8192).
+// With one K split there is no reduce launch to save: rank 64, q/k/v, 2 x 100 59.9 -> 58.3 (768), 8 x 64 71.9 -> 71.7 (2304); at that rank the
+// line lies where four projections of 128 tokens do (512), as before.
 constexpr int FEW_COLS = 256;
-constexpr int FEW_EXPAND = 512;             // workgroups up to which it is taken
-template <int DT, bool BT>
+static int few_expand(int max_rank, bool bt, int splits)                // workgroups up to which it is taken
+{
+    if (max_rank <= 32) return 6144;
+    return splits == 1 ? 512 : (bt ? 1023 : 3200);
+}
+template <int DT, int RMAX, bool BT>
 __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p)
 {
-    constexpr int KP = MAX_RANK, KS = KP / 32;                  // K of the MFMAs (rank padded with zeros)
+    constexpr int KP = RMAX <= 32 ? 32 : 64, KS = KP / 32;      // K of the MFMAs (rank padded with zeros)
     constexpr int CW = FEW_COLS / 4, NBC = CW / 16;             // columns of a wavefront
     constexpr int BPITCH = CW * 2 + 16, TPITCH = KP * 2 + 16;   // bytes per LDS row of B: a rank row, or (reference layout) an output column
     constexpr int BQ = KP / 8;                                  // B loads per lane
     constexpr int VPITCH = KP + 8, OPITCH = CW + 4;
-    constexpr int WBYTES = BT ? CW * TPITCH : KP * BPITCH;
+    constexpr int BBYTES = BT ? CW * TPITCH : KP * BPITCH, WBYTES = BBYTES > 16 * OPITCH * 4 ? BBYTES : 16 * OPITCH * 4;
     __shared__ __attribute__((aligned(16))) unsigned char s_b[4][WBYTES];       // private to a wavefront: B, then its result
     __shared__ __attribute__((aligned(16))) uint16_t s_v[2][16][VPITCH];
-    static_assert(16 * OPITCH * 4 <= WBYTES, "a wavefront's result fits its B tile");
+    static_assert(16 * OPITCH * 4 <= sizeof(s_b[0]), "a wavefront's result fits its B tile");
 
     // grid: column blocks of all projections x pieces
     const GroupId at = group_at(p.ex_end, blockIdx.x);
@@ -839,10 +849,11 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p
     if constexpr (!BT) mine = tl.row(lane, p.pool.n_rows_a);
     const int nsplit = pj.ksplit;
     const bool fold = p.fold && nsplit > 1;
-    const int ft = tid / (KP / 4), fc = (tid % (KP / 4)) * 4;           // folding: 16 tokens x 16 quads
+    // folding: 16 tokens x KP / 4 quads; the shrink has filled RMAX columns
+    const int ft = tid / (KP / 4) & 15, fc = (tid % (KP / 4)) * 4, fs = fc < RMAX ? fc : 0;
     float4_t part[SGMV_SPLITS];                                         // (requested also where there is nothing to fold: no branch)
     {
-        const float *src = pj.v + (size_t)(tok0 + (ft < ntok ? ft : ntok - 1)) * VSTRIDE + fc;
+        const float *src = pj.v + (size_t)(tok0 + (ft < ntok ? ft : ntok - 1)) * VSTRIDE + fs;
         const size_t stride = (size_t)p.T * VSTRIDE;
 #pragma unroll
         for (int u = 0; u < SGMV_SPLITS; u++) part[u] = *reinterpret_cast<const float4_t *>(src + (u < nsplit ? u : 0) * stride);
@@ -886,6 +897,7 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p
             v[e] = 0.f;
 #pragma unroll
             for (int u = 0; u < SGMV_SPLITS; u++) v[e] += u < nsplit ? part[u][e] : 0.f;
+            v[e] = fc < RMAX ? v[e] : 0.f;
         }
         uint32_t hi[2], lo[2];
         split_hi_lo<DT>(v, hi, lo);
@@ -900,8 +912,9 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_few_kernel(const SgmvArgs p
     } else {
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-            vhi[ks] = ldg16(pj.vhi + (size_t)(tok0 + trow) * VSTRIDE + ks * 32 + 8 * g);
-            vlo[ks] = ldg16(pj.vlo + (size_t)(tok0 + trow) * VSTRIDE + ks * 32 + 8 * g);
+            const int c0 = ks * 32 + 8 * g;
+            vhi[ks] = c0 < RMAX ? ldg16(pj.vhi + (size_t)(tok0 + trow) * VSTRIDE + c0) : zero16();
+            vlo[ks] = c0 < RMAX ? ldg16(pj.vlo + (size_t)(tok0 + trow) * VSTRIDE + c0) : zero16();
         }
     }
     // the wavefront's B tile through its own LDS, then its result: operations of one wavefront on LDS complete in order
@@ -969,7 +982,7 @@ void sgmv_launch_shape(SgmvArgs &a, int max_rank, int phases)
         few_wgs += (long long)a.tiles * 4 * ((a.pr[q].hout + FEW_COLS - 1) / FEW_COLS);
         most = a.pr[q].ksplit > most ? a.pr[q].ksplit : most;
     }
-    a.few = max_rank > 32 && few_wgs <= FEW_EXPAND;
+    a.few = few_wgs <= few_expand(max_rank, a.seg_uniform_len > 0, most);
     // The expand sums the splits itself up to rank 32 and in launches of few tiles; rows outside every segment are zeroed by the reduce launch only.
     a.fold = (max_rank <= 32 || a.few) && (a.accumulate || a.seg_uniform_len > 0);
     // Without splits the shrink has stored the halves itself, and the launch would only read the cover flags: two projections
@@ -1017,12 +1030,10 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
         rc = (int)hipGetLastError();
         if (rc) return rc;
     }
-    if constexpr (RMAX > 32) {
-        if (g.few) {
-            if (g.b_transposed) hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, true>), egrid, dim3(SG_NT), 0, s, g);
-            else hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, false>), egrid, dim3(SG_NT), 0, s, g);
-            return (int)hipGetLastError();
-        }
+    if (g.few) {
+        if (g.b_transposed) hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, RMAX, true>), egrid, dim3(SG_NT), 0, s, g);
+        else hipLaunchKernelGGL((sgmv_expand_few_kernel<DT, RMAX, false>), egrid, dim3(SG_NT), 0, s, g);
+        return (int)hipGetLastError();
     }
     if (g.b_transposed)
         hipLaunchKernelGGL((sgmv_expand_kernel<DT, RMAX, true>), egrid, dim3(SG_NT), 0, s, g);

@@ -474,6 +474,43 @@ def test_sgmv_few_tiles(lens, gap, ranks, hin, hout, n_proj, shape, dtype):
             assert_close_bits(torch_to_bits(y), want, dtype)
 
 
+@pytest.mark.parametrize("lens,ranks,hin,hout,n_proj,few,many", [
+    ([64] * 11 + [30, 1], [64, 40], 1096, 4096, 3, 0, True),       # 18 tiles by the estimate, 3456 workgroups
+    ([64] * 9 + [30, 1], [64, 40], 1096, 4096, 3, 1, True),        # 2880
+    ([64] * 13 + [30], [64], 1096, 5128, 2, 0, True),              # 3360
+    ([64] * 22, [48], 4096, 4104, 3, 0, True),
+    ([700], [16, 5], 72, 4104, 7, 1, False),                       # 11 tiles, 5236 workgroups
+    ([700], [16], 1096, 6152, 7, 0, True),                         # 7700
+    ([33, 640], [32, 20], 1096, 4104, 7, 1, True),
+    ([1000], [24], 72, 4104, 7, 0, False),
+])
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+def test_sgmv_both_expands(lens, ranks, hin, hout, n_proj, few, many, dtype):
+    """Both kernels at the ranks of every instance, on either side of the number of workgroups at which they change."""
+    from mlora import sgmv_multi
+    rng = np.random.default_rng(sum(lens) + hout)
+    pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
+    names = [f"p{i}" for i in range(n_proj)]
+    pool = upload_pool(pp, projections={nm: (hin, hout) for nm in names})
+    for nm in names:
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, dtype))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, dtype))
+    seg = _segments(lens, rng.integers(0, len(ranks), len(lens)))
+    T = sum(lens)
+    shape = sgmv_shape([(hin, hout)] * n_proj, [0] * n_proj, T, len(lens), pool.max_rank)
+    assert shape["few"] == few and (max(shape["splits"]) > 1) == many, shape
+    plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in seg), T, pool, n_proj=n_proj)
+    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
+    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
+    say(f"sgmv both expands lens={lens[:2]}x{len(lens)} ranks={ranks} {hin}->{hout} n_proj={n_proj} dtype={dtype}")
+    ys = [bits_to_torch(y0, dtype, "cuda") for _ in names]
+    sgmv_multi(ys, [bits_to_torch(x, dtype, "cuda")] * n_proj, pool, 0, names, plan)
+    torch.cuda.synchronize()
+    want = oracle_apply(pp, x, _tok_of(*seg, T), y0)
+    for y in ys:
+        assert_close_bits(torch_to_bits(y), want, dtype)
+
+
 @pytest.mark.parametrize("aligned", [False, True])
 @pytest.mark.parametrize("n_seg,longest", [(300, 5), (17, 1100), (1, 1)])
 def test_plan_over_several_workgroups(n_seg, longest, aligned):
