@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace mlora {
 
@@ -199,6 +200,22 @@ __device__ __forceinline__ float wave_sum(float v)
     v = row16_sum(v);
     v += __shfl_xor(v, 16);
     v += __shfl_xor(v, 32);
+    return v;
+}
+
+// Inclusive sum over the lanes of a wavefront, all of which are active.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v)
+{
+    auto take = [](uint32_t x, auto ctrl, auto rows) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    };
+    using std::integral_constant;
+    v += take(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});       // row_shr:1, 2, 4, 8
+    v += take(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
+    v += take(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
+    v += take(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
+    v += take(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});       // row_bcast:15, 31
+    v += take(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});
     return v;
 }
 

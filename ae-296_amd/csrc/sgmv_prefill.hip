@@ -34,13 +34,6 @@ constexpr int VSTRIDE = MAX_RANK;
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4;
 
-__device__ __forceinline__ int sg_pool_row(const int32_t *__restrict__ tbl, int adapter, int j, const PoolView &pv, long long n_rows)
-{
-    const int pg = tbl[(long long)adapter * pv.max_pages + (j >> pv.page_shift)];
-    const long long row = pg < 0 ? -1 : (((long long)pg << pv.page_shift) + (j & ((1 << pv.page_shift) - 1)));
-    return (row < 0 || row >= n_rows) ? -1 : (int)row;
-}
-
 __device__ __forceinline__ void seg_of(const SgmvArgs &p, int s, int &start, int &len, int &adapter)
 {
     start = p.seg_start[s]; len = p.seg_len[s]; adapter = p.seg_adapter[s];
@@ -158,8 +151,9 @@ __device__ __forceinline__ Tile<UNIFORM> tile_of(const SgmvArgs &p, int tile)
 //
 // A workgroup writes the list entries and records of PLAN_TILES tiles and the cover flags of PLAN_TOKENS tokens; every one
 // counts the tiles of all segments itself, a few steps, so that none waits for another.  What bounds it is the start of a
-// launch and the chain segments -> counts -> adapter -> page table -> record, most of it on lines that no cache holds any
-// more: 3.9 us for one prompt of 64 tokens, 12 for sixteen of 9216 (18 with one workgroup for all of it).
+// launch and the chain segments -> adapter -> rank, scaling, page table -> record, most of it on lines that no cache holds any
+// more; the counting runs beside it.  One prompt of 64
+// tokens 4.0 -> 3.7 us, sixteen of 9216 12.0 -> 11.2 (before, the rank and the page table were asked for behind the headers).
 constexpr int PLAN_NT = 256;
 constexpr int PLAN_TILES = 16;
 constexpr int PLAN_TOKENS = 4 * PLAN_NT;
@@ -178,16 +172,20 @@ __global__ __launch_bounds__(PLAN_NT) void sgmv_plan_kernel(const SgmvArgs p)
         const int s = s0 + tid;
         int start = 0, len = 0, adapter = -1;
         if (s < p.n_seg) seg_of(p, s, start, len, adapter);
+        // what the records of the segment's tiles will need, requested with nothing else to wait for; the page table's line
+        // for the rows
+        const bool real = adapter >= 0 && adapter < pv.n_adapters;
+        int rk = 0, sc = 0, pg = 0;
+        if (real) {
+            rk = pv.rank[adapter];
+            sc = __builtin_bit_cast(int, pv.scaling[adapter]);
+            pg = pv.a_tbl[(long long)adapter * pv.max_pages];
+        }
         // tiles of a segment: every TM tokens from its start, or (aligned) the pieces between multiples of TM
         const int lead = p.tile_aligned ? start % TM : 0;
         const int nt = len > 0 ? (lead + len + TM - 1) / TM : 0;
-        int v = nt;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(v, d);
-            if (lane >= d) v += o;
-        }
-        __syncthreads();                               // the previous batch of segments has been looked at
+        const int v = (int)wave_scan((uint32_t)nt);
+        if (s0 > 0) __syncthreads();                   // the previous batch of segments has been looked at
         if (lane == 63) s_wave[wave] = v;
         __syncthreads();
         int first = carry + v - nt, all = carry;
@@ -196,13 +194,16 @@ __global__ __launch_bounds__(PLAN_NT) void sgmv_plan_kernel(const SgmvArgs p)
         s_start[tid] = start; s_end[tid] = start + len; s_first[tid] = first;
         // this workgroup's tiles of the segment
         const int i0 = t0 - first > 0 ? t0 - first : 0, i1 = t0 + PLAN_TILES - first < nt ? t0 + PLAN_TILES - first : nt;
+        const int cap = pv.max_pages << pv.page_shift < MAX_RANK ? pv.max_pages << pv.page_shift : MAX_RANK;
+        rk = rk < 0 ? 0 : (rk > cap ? cap : rk);
         for (int i = i0; i < i1; i++) {
             if (first + i >= p.max_tiles) break;
             const int b = i == 0 ? start : start - lead + i * TM;
             const int e = start - lead + (i + 1) * TM < start + len ? start - lead + (i + 1) * TM : start + len;
             int *h = s_hdr[first + i - t0];
-            h[0] = e - b; h[1] = adapter; h[4] = b; h[5] = s;
+            h[0] = e - b; h[1] = real ? adapter : -1; h[2] = rk; h[3] = sc; h[4] = b; h[5] = s;
         }
+        asm volatile("" :: "v"(pg));                   // the page table's line has arrived
         __syncthreads();
         // Which tokens belong to a tile at all: y = delta mode must define the rows of the others (zeros).
         const int ns = p.n_seg - s0 < PLAN_NT ? p.n_seg - s0 : PLAN_NT;
@@ -217,45 +218,36 @@ __global__ __launch_bounds__(PLAN_NT) void sgmv_plan_kernel(const SgmvArgs p)
             }
         carry = all;
     }
+    // Per-tile records: everything a shrink / expand workgroup needs, so that it starts from one load.  Records beyond the
+    // tiles in use are marked empty, so that a workgroup starts from its record alone and does not wait for the count first.
+    constexpr int WPT = PLAN_TILES * TILE_WORDS / PLAN_NT;
+    static_assert(WPT * PLAN_NT == PLAN_TILES * TILE_WORDS, "every thread writes as many words");
+    int page[WPT];
+#pragma unroll
+    for (int u = 0; u < WPT; u++) {                    // all table lookups leave together: each is made, at entry 0 where there is none
+        const int idx = u * PLAN_NT + tid, lt = idx / TILE_WORDS, j = idx - lt * TILE_WORDS - TILE_ROWS_AT;
+        const int *h = s_hdr[lt];
+        const bool has = j >= 0 && h[0] > 0 && h[1] >= 0 && j < h[2];
+        page[u] = pv.a_tbl[has ? (long long)h[1] * pv.max_pages + (j >> pv.page_shift) : 0];
+        page[u] = has ? page[u] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < WPT; u++) {
+        const int idx = u * PLAN_NT + tid, lt = idx / TILE_WORDS, w = idx - lt * TILE_WORDS, j = w - TILE_ROWS_AT;
+        const int *h = s_hdr[lt];
+        int val = h[0] <= 0 ? -w : (w < 6 ? h[w] : 0); // an empty record: no tokens, no adapter
+        if (j >= 0) {
+            const long long row = ((long long)page[u] << pv.page_shift) + (j & ((1 << pv.page_shift) - 1));
+            val = page[u] < 0 || row >= pv.n_rows_a ? -1 : (int)row;
+        }
+        if (t0 + lt < p.max_tiles && (h[0] > 0 || w < 2)) p.tile_rec[(size_t)(t0 + lt) * TILE_WORDS + w] = val;
+    }
+    if (tid < PLAN_TILES && s_hdr[tid][0] > 0) { p.tile_seg[t0 + tid] = s_hdr[tid][5]; p.tile_tok0[t0 + tid] = s_hdr[tid][4]; p.tile_ntok[t0 + tid] = s_hdr[tid][0]; }
+    if (blockIdx.x == 0 && tid == 0) p.n_tiles[0] = carry < p.max_tiles ? carry : p.max_tiles;
 #pragma unroll
     for (int u = 0; u < PLAN_TOKENS / PLAN_NT; u++) {
         const int t = k0 + u * PLAN_NT + tid;
         if (t < p.T) p.tok_cover[t] = cover[u] ? 1 : 0;
-    }
-    if (blockIdx.x == 0 && tid == 0) p.n_tiles[0] = carry < p.max_tiles ? carry : p.max_tiles;
-    // Per-tile records: everything a shrink / expand workgroup needs, so that it starts from one load.  Records beyond the
-    // tiles in use are marked empty, so that a workgroup starts from its record alone and does not wait for the count first.
-    __syncthreads();
-    if (tid < PLAN_TILES) {
-        int *h = s_hdr[tid];
-        const int adapter = h[0] > 0 ? h[1] : -1;
-        const bool real = adapter >= 0 && adapter < pv.n_adapters;
-        int rk = 0, sc = 0;
-        if (real) {
-            const int cap = pv.max_pages << pv.page_shift;
-            rk = pv.rank[adapter];
-            rk = rk < 0 ? 0 : (rk > MAX_RANK ? MAX_RANK : rk);
-            rk = rk > cap ? cap : rk;
-            sc = __builtin_bit_cast(int, pv.scaling[adapter]);
-        }
-        h[1] = real ? adapter : -1; h[2] = rk; h[3] = sc;
-        if (h[0] > 0) { p.tile_seg[t0 + tid] = h[5]; p.tile_tok0[t0 + tid] = h[4]; p.tile_ntok[t0 + tid] = h[0]; }
-    }
-    __syncthreads();
-    constexpr int WPT = PLAN_TILES * TILE_WORDS / PLAN_NT;
-    static_assert(WPT * PLAN_NT == PLAN_TILES * TILE_WORDS, "every thread writes as many words");
-    int val[WPT];
-#pragma unroll
-    for (int u = 0; u < WPT; u++) {                    // all table lookups leave together
-        const int idx = u * PLAN_NT + tid, lt = idx / TILE_WORDS, w = idx - lt * TILE_WORDS, j = w - TILE_ROWS_AT;
-        const int *h = s_hdr[lt];
-        val[u] = h[0] <= 0 ? -w : (w < 6 ? h[w] : 0);  // an empty record: no tokens, no adapter
-        if (j >= 0) val[u] = (h[0] > 0 && h[1] >= 0 && j < h[2]) ? sg_pool_row(pv.a_tbl, h[1], j, pv, pv.n_rows_a) : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < WPT; u++) {
-        const int idx = u * PLAN_NT + tid, lt = idx / TILE_WORDS, w = idx - lt * TILE_WORDS;
-        if (t0 + lt < p.max_tiles && (s_hdr[lt][0] > 0 || w < 2)) p.tile_rec[(size_t)(t0 + lt) * TILE_WORDS + w] = val[u];
     }
 }
 
