@@ -642,22 +642,17 @@ __global__ __launch_bounds__(256) void gemm_lora_sum_kernel(const GemmLoraArgs p
 // hundred tiles or fewer: most units idle, the longest K (the MLP's second product) is a chain several times as long as
 // the rest, and rows past T are multiplied for nothing.  The rule estimates, for every tile height and number of
 // ranges, rounds of workgroups x mean time of one (or the longest chain) plus the cost of the partial sums, and takes
-// the least; the plain shape is kept where it comes within 5 %, which the estimate does not tell apart.  Base products at Llama-7B
-// widths, fp16, weights of two layers in turn, us, plain -> chosen (best of the 25 shapes): q/k/v 16 tokens 76 -> 24 (24),
-// 120 tokens 74 -> 33 (30), 192 tokens 73 -> 41 (33), 351 tokens 74 -> 53 (45), 700 tokens 79 -> 72 (71), 1500 tokens 182 -> 148
-// (145), 2000 tokens 185 -> 193 (179); all seven 16 tokens 191 -> 77 (77; 5.3 TB/s of weights), 192 tokens 205 -> 100 (100), 351
-// tokens 239 -> 166 (166), 500 tokens 242 -> 229 (217), 900 tokens 368 -> 371 (345), 1500 tokens 529 (529).
-// Step times are those of one workgroup on each unit when x came in stages of 32 columns; x in whole lines shortened every step,
-// and the estimate now cuts K too early: where it is 10 to 25 % off (q/k/v at 120 to 384 tokens), 64 or 128 rows with K whole
-// are the best shape.
-// K is cut up to 384 tokens; the plain shape is chosen for the seven from 577 tokens on, but for
-// 1025..1152 and 1793..1920, and for q/k/v at 961..1280, at 1921..2560 and from 3073 on but for 6657..7104: in between, the
-// estimate has 256 rows leave a last round nearly empty (1500 tokens above, 192 rows).
+// the least; the plain shape is kept where it comes within 1 %.  Fitted to 25 shapes of 165 batches (24 to 4500 tokens, three
+// prompts; q/k/v, with o, all seven; Llama-7B and -13B widths, whole and halves; rank 16, bf16, weights of two or three layers in turn, card
+// under load): the shape it names is 1.6 % off the best on average and 17 % at worst (2.4 % with the constants from before x came in
+// whole lines).  A layer with its LoRA launches, us, plain -> chosen (best): Llama-7B, q/k/v 24 tokens 86 -> 36 (36), 161 tokens 88 -> 53
+// (53), 768 tokens 96 -> 85 (85); q/k/v/o 192 tokens 92 -> 72 (68), 300 tokens 95 -> 72 (72); all seven 24 tokens 207 -> 90 (90), 351 tokens
+// 262 -> 194 (191), 450 tokens 265 -> 251 (223), 900 tokens 378 (361); halves, q/k/v 768 tokens 89 -> 58 (58).
 // Tiles of 256 rows are never cut: with the ranges the compiler spills accumulators.
 int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out)
 {
-    static const double step_us[4] = {0.42, 0.55, 0.68, 0.85};                // one K step, by mi
-    const double ends_us = 6.0, launch_us = 4.0, byte_us = 2.0 / 4.0e6;         // a workgroup's start and end; one more launch; a byte written and read
+    static const double step_us[4] = {0.435, 0.541, 0.652, 0.81};             // one K step, by mi
+    const double ends_us = 6.63, launch_us = 2.38, byte_us = 6.78e-7;           // a workgroup's start and end; one more launch; a byte written and read
     const double cus = device_compute_units();
     int longest = 1;
     for (int q = 0; q < a.n_proj; q++) longest = a.pr[q].hin / GK > longest ? a.pr[q].hin / GK : longest;
@@ -689,7 +684,7 @@ int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out)
             us = us > chain ? us : chain;
             if (bytes > 0) us += launch_us + (double)bytes * byte_us;
             if (mi == 4) {
-                *out = cand; best = 0.95 * us;
+                *out = cand; best = 0.99 * us;
                 if (items >= 8 * cus) return 0;                                 // many rounds: nothing to gain
             } else if (us < best) { best = us; *out = cand; best_bytes = bytes; }
         }
