@@ -542,8 +542,11 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
 // launches of few tiles below (sgmv_launch_shape): 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing, 55.4 and a reduce
 // of 5.2 not; at rank 16 the whole call of 8 x 512 tokens 185 -> 179.
 
+// The reference's call (BT) only writes y, and its whole batch is about one round of workgroups: no registers for y, and a staging
+// tile of half a step, so that four workgroups fit a unit instead of three (16 x 512 tokens,
+// rank 64, 1024 workgroups: q, k and v 124.5 us with three, 118.9 with four).
 template <int DT, int RMAX, bool BT>
-__global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
+__global__ __launch_bounds__(SG_NT, BT ? 4 : 1) void sgmv_expand_kernel(const SgmvArgs p)
 {
     // One workgroup: 64 tokens (16 per wavefront) x cols_per_block output columns, 128 columns per step.
     // The B tile of a step is parked in LDS row-major and read back column-wise with the transposing LDS
@@ -555,24 +558,25 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     constexpr int KS = KP / 32;
     constexpr int NBC = TN / 16;               // 16-column blocks per step
     constexpr int BPITCH = TN * 2 + 16;        // bytes per rank row of the LDS B tile (16-byte aligned rows)
-    constexpr int OPITCH = TN + 4;             // floats per token row of the staging tile
+    constexpr int ON = BT ? TN / 2 : TN;       // columns staged at a time
+    constexpr int OPITCH = ON + 4;             // floats per token row of the staging tile
     constexpr int TPITCH = KP * 2 + 16;        // reference layout: bytes per output column of the LDS tile (K contiguous)
     constexpr int BQ = KP * (TN / 8) / SG_NT;  // B-tile loads per thread and step (either layout: KP x TN values)
     __shared__ __attribute__((aligned(16))) unsigned char s_b[BT ? TN * TPITCH : KP * BPITCH];
     __shared__ __attribute__((aligned(16))) float s_out[SG_NT / 64][16][OPITCH];
     __shared__ int s_brow[BT ? 1 : KP];
-    constexpr int VPITCH = KP + 8;             // 16-bit values per token row of the folded intermediate, which lies in s_out for a while
-    static_assert(2 * TM * VPITCH * 2 <= (int)sizeof(s_out), "the folded intermediate fits the staging tiles");
+    constexpr int VPITCH = KP + 8;             // 16-bit values per token row of the folded intermediate, which lies in s_out (BT: s_b) for a while
+    uint16_t *const s_v = BT ? reinterpret_cast<uint16_t *>(s_b) : reinterpret_cast<uint16_t *>(&s_out[0][0][0]);
+    static_assert(2 * TM * VPITCH * 2 <= (int)(BT ? sizeof(s_b) : sizeof(s_out)), "the folded intermediate fits there");
     typedef __attribute__((address_space(3))) volatile float lds_vfloat;
     typedef __attribute__((address_space(3))) volatile float4_t lds_vfloat4;
 
-    int proj = 0;
-    while (proj + 1 < p.n_proj && blockIdx.x >= p.ex_end[proj]) proj++;
-    const SgmvProj &pj = p.pr[proj];
+    const GroupId at = group_at(p.ex_end, blockIdx.x);
+    const SgmvProj &pj = p.pr[at.group];
     const int cols_per_block = pj.cols;
     int tile, colblk;
     {
-        const int w = (int)(blockIdx.x - (proj ? p.ex_end[proj - 1] : 0u));
+        const int w = at.rest;
         if (tile_major(pj.ncb) && !few_tiles(p.max_tiles)) {
             const int ncb8 = (pj.ncb + 7) & ~7;
             tile = w / ncb8;
@@ -623,7 +627,6 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     const bool fold = p.fold && pj.ksplit > 1;
     if (fold) {
         // whole rows of the partial sums, four ranks a thread; the operands are read back from LDS behind the barrier
-        uint16_t *s_v = reinterpret_cast<uint16_t *>(&s_out[0][0][0]);
         constexpr int RQ = RMAX / 4;
 #pragma unroll
         for (int i = 0; i < TM * RQ / SG_NT; i++) {
@@ -650,7 +653,6 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     const uint16_t *__restrict__ bt = brows + (BT ? (size_t)adapter * (size_t)pv.b_dense_stride : 0);
     __syncthreads();
     if (fold) {
-        const uint16_t *s_v = reinterpret_cast<const uint16_t *>(&s_out[0][0][0]);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const int c0 = ks * 32 + 8 * g;
@@ -663,8 +665,9 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
     // Loads of a step (this thread's share of the B tile and of the y rows) are issued one step ahead.
     // y rows of this wavefront: lane handles (token p / 16, 16-byte chunk p % 16), p = lane + 64 q.
     uint4 y_nx[4], b_nx[BQ];
+    const bool accumulate = !BT && p.accumulate;
     auto prefetch = [&](int col0) {
-        if (p.accumulate) {
+        if (accumulate) {
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const int pp = lane + 64 * q, t = pp >> 4, c = pp & 15;
@@ -752,31 +755,32 @@ __global__ __launch_bounds__(SG_NT) void sgmv_expand_kernel(const SgmvArgs p)
         // barrier is needed; the accesses are volatile so that the compiler keeps them in program order and
         // emits one ds_write_b32 per element (left to itself it pairs these stores into ds_write2_b32 and,
         // in the variant without the B tile, gets two of the paired offsets wrong).
-        {
+#pragma unroll
+        for (int h = 0; h < TN / ON; h++) {
             lds_vfloat *so = (lds_vfloat *)&s_out[wave][4 * g][m];
 #pragma unroll
-            for (int nb = 0; nb < NBC; nb++)
+            for (int nb = 0; nb < ON / 16; nb++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) so[i * OPITCH + nb * 16] = acc[nb][i];
-        }
+                for (int i = 0; i < 4; i++) so[i * OPITCH + nb * 16] = acc[h * (ON / 16) + nb][i];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int pp = lane + 64 * q, t = pp >> 4, c = pp & 15;
-            const int col = col0 + c * 8;
-            const float4_t d0 = *(lds_vfloat4 *)&s_out[wave][t][c * 8];
-            const float4_t d1 = *(lds_vfloat4 *)&s_out[wave][t][c * 8 + 4];
-            if (wave * 16 + t < ntok && col < col_end) {
-                float o[8];
-                if (p.accumulate) unpack8<DT>(y0[q], o);
-                else {
+            for (int q = 0; q < ON / 32; q++) {
+                const int pp = lane + 64 * q, t = pp / (ON / 8), c = pp % (ON / 8);
+                const int col = col0 + h * ON + c * 8;
+                const float4_t d0 = *(lds_vfloat4 *)&s_out[wave][t][c * 8];
+                const float4_t d1 = *(lds_vfloat4 *)&s_out[wave][t][c * 8 + 4];
+                if (wave * 16 + t < ntok && col < col_end) {
+                    float o[8];
+                    if (accumulate) unpack8<DT>(y0[q], o);
+                    else {
 #pragma unroll
-                    for (int e = 0; e < 8; e++) o[e] = 0.f;
+                        for (int e = 0; e < 8; e++) o[e] = 0.f;
+                    }
+                    o[0] = fmaf(scale, d0[0], o[0]); o[1] = fmaf(scale, d0[1], o[1]);
+                    o[2] = fmaf(scale, d0[2], o[2]); o[3] = fmaf(scale, d0[3], o[3]);
+                    o[4] = fmaf(scale, d1[0], o[4]); o[5] = fmaf(scale, d1[1], o[5]);
+                    o[6] = fmaf(scale, d1[2], o[6]); o[7] = fmaf(scale, d1[3], o[7]);
+                    stg16_stream(y + (size_t)(tok0 + wave * 16 + t) * hout + col, pack8<DT>(o));
                 }
-                o[0] = fmaf(scale, d0[0], o[0]); o[1] = fmaf(scale, d0[1], o[1]);
-                o[2] = fmaf(scale, d0[2], o[2]); o[3] = fmaf(scale, d0[3], o[3]);
-                o[4] = fmaf(scale, d1[0], o[4]); o[5] = fmaf(scale, d1[1], o[5]);
-                o[6] = fmaf(scale, d1[2], o[6]); o[7] = fmaf(scale, d1[3], o[7]);
-                stg16_stream(y + (size_t)(tok0 + wave * 16 + t) * hout + col, pack8<DT>(o));
             }
         }
     }
