@@ -306,22 +306,33 @@ __global__ __launch_bounds__(SG_NT *SH_KG<SHARE>) void sgmv_shrink_kernel(const 
     constexpr int CH = SH_CH, ROWB = SH_ROWB;
     constexpr int RPL = 1024 / ROWB;                            // rows one load of a wavefront fills
     __shared__ __attribute__((aligned(16))) unsigned char s_ring[KG * GROUP_BYTES];
-    int grp = 0;
-    while (grp + 1 < p.n_grp && blockIdx.x >= p.grp_end[grp]) grp++;
     // SHARE: a workgroup per (tile, split) of a group; otherwise one per projection, the projections of a group being the
-    // fastest index, so that they run side by side on one XCD and find x in its L2
-    int tile, split;
-    const int w = (int)(blockIdx.x - (grp ? p.grp_end[grp - 1] : 0u)), ng = SHARE ? 1 : p.grp_n[grp];
+    // fastest index, so that they run side by side on one XCD and find x in its L2.  Few tiles: the tile is the grid's second
+    // dimension, and nothing is divided but by the projections of a group.
+    const GroupId at = group_at(p.grp_end, blockIdx.x);
+    const int grp = at.group, w = at.rest, ng = SHARE ? 1 : p.grp_n[grp];
+    auto by_group = [&](int v) { return ng == 1 ? v : (ng == 2 ? v >> 1 : (int)((unsigned)v * 43691u >> 17)); };      // v / ng, v < 2^16
     const bool few = few_tiles(p.max_tiles);
-    const int wq = few ? w / ng : (w >> 3) / ng * 8 + (w & 7);
-    const int p0 = p.grp_first[grp] + (few ? w - wq * ng : (w >> 3) % ng);
+    int tile = (int)blockIdx.y, split, p0 = p.grp_first[grp];
+    if (few) {
+        split = by_group(w);
+        p0 += w - split * ng;
+    } else {
+        const int q = (w >> 3) / ng;
+        p0 += (w >> 3) - q * ng;
+        place(q * 8 + (w & 7), p.pr[p0].ksplit, p.max_tiles, grp * 3, tile, split);
+        if (tile >= p.max_tiles) return;                        // records beyond the tiles in use hold no tokens
+    }
     const int nm = SHARE ? p.grp_n[grp] : 1;
     const SgmvProj &pj = p.pr[p0];
-    place(wq, pj.ksplit, p.max_tiles, grp * 3, tile, split);
-    if (tile >= p.max_tiles) return;                            // records beyond the tiles in use hold no tokens
     const Tile<UNIFORM> tl = tile_of<UNIFORM>(p, tile);
+    // Row of rank row `lane`, requested with the record's header; the loads get theirs from the other lanes, and the end of the
+    // kernel asks the mask which of them exist.
+    int mine = tl.row((int)threadIdx.x & 63, p.pool.n_rows_a);
     const int ntok = tl.ntok, tok0 = tl.tok0;
     if (tl.adapter < 0 || ntok <= 0 || tok0 < 0 || tok0 + ntok > p.T) return;
+    asm volatile("" : "+v"(mine));                              // loaded by all lanes
+    const unsigned long long have = __ballot(mine >= 0);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -361,7 +372,7 @@ __global__ __launch_bounds__(SG_NT *SH_KG<SHARE>) void sgmv_shrink_kernel(const 
             if (u < XU) {
                 row = reinterpret_cast<const char *>(static_cast<const uint16_t *>(pj.x) + (size_t)(tok0 + (r < ntok ? r : ntok - 1)) * hin);
             } else {
-                const int mm = i * RPL / RMAX, at = tl.row(r - mm * RMAX, p.pool.n_rows_a);
+                const int mm = i * RPL / RMAX, at = __shfl(mine, r - mm * RMAX);
                 row = reinterpret_cast<const char *>(static_cast<const uint16_t *>(p.pr[p0 + mm].a_rows) + (size_t)(at >= 0 ? at : 0) * hin);
             }
             src[u] = row + (size_t)g0 * ROWB + c * 16;
@@ -472,7 +483,7 @@ __global__ __launch_bounds__(SG_NT *SH_KG<SHARE>) void sgmv_shrink_kernel(const 
             const int c0 = (rw * NBW + nb) * 16 + 4 * g;
             bool real[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) real[e] = tl.row(c0 + e, p.pool.n_rows_a) >= 0;
+            for (int e = 0; e < 4; e++) real[e] = (have >> (c0 + e) & 1ull) != 0;
 #pragma unroll
             for (int mm = 0; mm < NM; mm++) {
                 const SgmvProj &pm = p.pr[p0 + mm];
@@ -1001,11 +1012,15 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     SgmvArgs g = a;
     sgmv_launch_shape(g, RMAX, phases);
     unsigned end = 0;
-    for (int q = 0; q < g.n_grp; q++) {
-        end += (unsigned)(place_grid(g.max_tiles, g.pr[g.grp_first[q]].ksplit) * (g.share_x ? 1 : g.grp_n[q]));
-        g.grp_end[q] = end;
+    const bool few = few_tiles(g.max_tiles);
+    for (int q = 0; q < MAX_PROJ; q++) {
+        if (q < g.n_grp) {
+            const long long splits = g.pr[g.grp_first[q]].ksplit;
+            end += (unsigned)((few ? splits : place_grid(g.max_tiles, (int)splits)) * (g.share_x ? 1 : g.grp_n[q]));
+        }
+        g.grp_end[q] = q < g.n_grp ? end : ~0u;
     }
-    const unsigned sgrid = end;
+    const dim3 sgrid(end, few ? (unsigned)g.max_tiles : 1u);
     end = 0;
     for (int q = 0; q < MAX_PROJ; q++) {
         if (q < g.n_proj) end += g.few ? (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
@@ -1015,9 +1030,9 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     if ((g.seg_uniform_len > 0) != (g.b_transposed != 0)) return (int)hipErrorInvalidValue;
     if (g.seg_uniform_len > 0 && g.share_x) return (int)hipErrorInvalidValue;
     const dim3 threads(SG_NT * (g.share_x ? SH_KG<true> : SH_KG<false>));
-    if (g.seg_uniform_len > 0) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, true, false>), dim3(sgrid), threads, 0, s, g);
-    else if (g.share_x) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, false, true>), dim3(sgrid), threads, 0, s, g);
-    else hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, false, false>), dim3(sgrid), threads, 0, s, g);
+    if (g.seg_uniform_len > 0) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, true, false>), sgrid, threads, 0, s, g);
+    else if (g.share_x) hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, false, true>), sgrid, threads, 0, s, g);
+    else hipLaunchKernelGGL((sgmv_shrink_kernel<DT, RMAX, false, false>), sgrid, threads, 0, s, g);
     rc = (int)hipGetLastError();
     if (rc || !(phases & SGMV_APPLY)) return rc;
     if (g.reduce) {
