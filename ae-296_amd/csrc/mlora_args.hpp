@@ -132,8 +132,8 @@ struct SgmvArgs {
     SgmvProj pr[MAX_PROJ];
     int n_proj;
     // Shrink launch: up to three consecutive projections that read the same x form a group, served by one workgroup per
-    // (tile, K split) where share_x is set and by neighbouring ones otherwise.  grp_end[g] = first workgroup id after group g (in a launch of
-    // few tiles, of each tile), ~0 past the last.
+    // (tile, K split) where share_x is set and by neighbouring ones otherwise.  grp_end[g] = first workgroup id after group g (of
+    // each tile, where the tile is the grid's second dimension), ~0 past the last.
     int share_x;
     int stream_x;          // x by streaming loads
     int n_grp;

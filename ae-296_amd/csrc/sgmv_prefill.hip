@@ -79,6 +79,11 @@ __host__ __device__ inline long long place_grid(int max_tiles, int n_second)
     return few_tiles(max_tiles) ? (long long)max_tiles * n_second : xcd_grid(max_tiles, n_second);
 }
 
+// Shrink launches of a few tiles have them as the grid's second dimension, one tile's groups behind each other: nothing to divide by.
+// With more, the longest groups of all tiles go first: 1536 workgroups of 47 tiles, rank 32, q/k/v/o, 21.9 us, 25.5 tile by tile; four layers
+// of one tile 47.9 us, 47.0 as the second dimension.
+__host__ __device__ inline bool tile_rows(int max_tiles) { return max_tiles <= 2 * XRUN; }
+
 // Expand launches use a second order where it fits: tile-major, the column blocks of a tile next to each other, so
 // that the eight workgroups running side by side (one per XCD) update one contiguous stretch of 64 y rows instead
 // of the same 1 KiB column block of 64 different tiles (DRAM pages stay open: a bare read-modify-write walk over
@@ -307,16 +312,18 @@ __global__ __launch_bounds__(SG_NT *SH_KG<SHARE>) void sgmv_shrink_kernel(const 
     constexpr int RPL = 1024 / ROWB;                            // rows one load of a wavefront fills
     __shared__ __attribute__((aligned(16))) unsigned char s_ring[KG * GROUP_BYTES];
     // SHARE: a workgroup per (tile, split) of a group; otherwise one per projection, the projections of a group being the
-    // fastest index, so that they run side by side on one XCD and find x in its L2.  Few tiles: the tile is the grid's second
-    // dimension, and nothing is divided but by the projections of a group.
+    // fastest index, so that they run side by side on one XCD and find x in its L2.
     const GroupId at = group_at(p.grp_end, blockIdx.x);
     const int grp = at.group, w = at.rest, ng = SHARE ? 1 : p.grp_n[grp];
     auto by_group = [&](int v) { return ng == 1 ? v : (ng == 2 ? v >> 1 : (int)((unsigned)v * 43691u >> 17)); };      // v / ng, v < 2^16
-    const bool few = few_tiles(p.max_tiles);
     int tile = (int)blockIdx.y, split, p0 = p.grp_first[grp];
-    if (few) {
+    if (tile_rows(p.max_tiles)) {
         split = by_group(w);
         p0 += w - split * ng;
+    } else if (few_tiles(p.max_tiles)) {
+        const int q = w / ng;
+        p0 += w - q * ng;
+        place(q, p.pr[p0].ksplit, p.max_tiles, grp * 3, tile, split);
     } else {
         const int q = (w >> 3) / ng;
         p0 += (w >> 3) - q * ng;
@@ -1012,15 +1019,15 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     SgmvArgs g = a;
     sgmv_launch_shape(g, RMAX, phases);
     unsigned end = 0;
-    const bool few = few_tiles(g.max_tiles);
+    const bool rows = tile_rows(g.max_tiles);
     for (int q = 0; q < MAX_PROJ; q++) {
         if (q < g.n_grp) {
-            const long long splits = g.pr[g.grp_first[q]].ksplit;
-            end += (unsigned)((few ? splits : place_grid(g.max_tiles, (int)splits)) * (g.share_x ? 1 : g.grp_n[q]));
+            const int splits = g.pr[g.grp_first[q]].ksplit;
+            end += (unsigned)((rows ? splits : place_grid(g.max_tiles, splits)) * (g.share_x ? 1 : g.grp_n[q]));
         }
         g.grp_end[q] = q < g.n_grp ? end : ~0u;
     }
-    const dim3 sgrid(end, few ? (unsigned)g.max_tiles : 1u);
+    const dim3 sgrid(end, rows ? (unsigned)g.max_tiles : 1u);
     end = 0;
     for (int q = 0; q < MAX_PROJ; q++) {
         if (q < g.n_proj) end += g.few ? (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
