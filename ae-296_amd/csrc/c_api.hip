@@ -321,9 +321,20 @@ static int64_t fine_workgroups(int n_proj, const int32_t *hin, const int32_t *ho
 // workgroups per compute unit, the wider slices beyond.  Measured on Llama-7B widths, wide -> fine, us per call: 8
 // tokens x 7 projections (560 workgroups) 26.6 -> 21.9 at rank 64, 12.5 -> 11.7 at rank 16; 32 tokens x 3 (768)
 // 23.5 -> 20.8; 16 x 7 (1120) 34.6 -> 34.8; 32 x 7 (2240) 52.4 -> 59.6.
-static bool prefer_sliced(int n_proj, const int32_t *hin, const int32_t *hout, int items, int group)
+//
+// Items of four tokens are far fewer than the host's bound where adapters have several tokens, so they also take the narrow slices while
+// about T/4 and two pieces for every fifth adapter make at most three workgroups per unit above rank 32 (2.5 above 16).  One projection, 100
+// adapters, Zipf 0.8, wide -> fine, us: 160 tokens of ranks 8 to 64 26.2 -> 18.2, of rank 64 29.9 -> 24.6, of rank 32 18.0 -> 16.8, of rank 16
+// 12.4 -> 12.4; 256 tokens (3.25 a unit) of ranks 8 to 64 26.5 -> 21.2, of rank 64 33.1 -> 33.7, of rank 32 18.5 -> 19.0; 100 tokens x 3 of rank 64 43.7
+// -> 46.4.
+static bool prefer_sliced(int n_proj, const int32_t *hin, const int32_t *hout, int T, int n_adapters, int max_rank, int group)
 {
-    return group > 4 || fine_workgroups(n_proj, hin, hout, items) > 4LL * mlora::device_compute_units();
+    if (group > 4) return true;
+    const int64_t cus = mlora::device_compute_units();
+    if (fine_workgroups(n_proj, hin, hout, items_bound(T, n_adapters, group)) <= 4 * cus) return false;
+    if (group < 4 || max_rank <= 16) return true;
+    const int items = (T + 3) / 4 + 2 * (T < n_adapters ? T : n_adapters) / 5;
+    return 4 * fine_workgroups(n_proj, hin, hout, (items + 7) / 8 * 8) > (max_rank > 32 ? 12 : 10) * cus;
 }
 
 // How a planned decode call runs best, and the workspace its two-launch form takes (mlora_bgmv_form).
@@ -351,7 +362,7 @@ static int decode_form(int n_proj, const int32_t *hin, const int32_t *hout, int 
     // groups of two leave one odd item for about every other adapter
     const int64_t items = group == 1 ? T : (T + 1) / 2 + segs / 2;
     const bool one_round = group <= 2 && items * n_proj <= cus;
-    const bool sliced = prefer_sliced(n_proj, hin, hout, items_bound(T, n_adapters, group), group);
+    const bool sliced = prefer_sliced(n_proj, hin, hout, T, n_adapters, max_rank, group);
     if (one_round && widest <= 8192 && item_bytes <= (sliced ? 640 << 10 : 320 << 10)) return MLORA_FORM_FUSED;
     return sliced ? MLORA_FORM_SLICED : MLORA_FORM_FINE;
 }
@@ -372,7 +383,7 @@ int mlora_bgmv_form(int n_proj, const int32_t *hin, const int32_t *hout, int T, 
     }
     *workspace_bytes = 0;
     if (T == 0) return MLORA_FORM_FUSED;
-    const bool sliced = prefer_sliced(n_proj, hin, hout, items_bound(T, n_adapters, group), group);
+    const bool sliced = prefer_sliced(n_proj, hin, hout, T, n_adapters, max_rank, group);
     const int64_t coarse = mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
     const int64_t fine = sliced ? 0 : fine_workspace_bytes(n_proj, T, max_hin, max_rank);
     *workspace_bytes = coarse > fine ? coarse : fine;
@@ -432,7 +443,7 @@ static int bgmv_multi_impl(int form, int n_proj, void *const *y, const void *con
         workspace_bytes = (int64_t)SCRATCH_BYTES;
     }
     if (form != MLORA_FORM_FUSED) {
-        a.fine = form == MLORA_FORM_FINE || (form == MLORA_FORM_PAIR && !prefer_sliced(n_proj, hin, hout, a.items_cap, group));
+        a.fine = form == MLORA_FORM_FINE || (form == MLORA_FORM_PAIR && !prefer_sliced(n_proj, hin, hout, T, n_adapters, max_rank, group));
         const int64_t need = a.fine ? fine_workspace_bytes(n_proj, T, max_hin, max_rank)
                                     : mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
         if (!workspace) return fail(MLORA_EINVAL, "the two-launch form needs a workspace");

@@ -248,3 +248,15 @@ def test_decode_form_on_both_sides_of_its_lines():
     assert (form(1, 1024, 512, 40, 16, group=4, slots=8), form(1, 1024, 512, 40, 16, group=8, slots=8)) == (FINE, SLICED)
     assert form(0, 512, 512, 4, 16) == _ext.MLORA_ERANGE and form(1, 512, 512, 4, 65) == _ext.MLORA_ERANGE
     assert form(1, 512, 512, 4, 16, group=3) == _ext.MLORA_EINVAL
+
+
+def test_decode_form_of_four_token_items():
+    """Items of four tokens by their likely number, 8 slices of 512 columns each: 96 make 768 workgroups, 80 make 640."""
+    lib = _ext.lib()
+
+    def form(T, slots, rank, hout=4096):
+        return lib.mlora_bgmv_form(1, (C.c_int32 * 8)(4096), (C.c_int32 * 8)(hout), T, slots, rank, 4, C.byref(C.c_int64()))
+
+    assert (form(224, 100, 64), form(225, 100, 64)) == (_ext.FORM_FINE, _ext.FORM_SLICED)
+    assert (form(160, 100, 32), form(161, 100, 32)) == (_ext.FORM_FINE, _ext.FORM_SLICED)
+    assert (form(160, 100, 16), form(160, 100, 17)) == (_ext.FORM_SLICED, _ext.FORM_FINE)
