@@ -341,7 +341,7 @@ static bool prefer_sliced(int n_proj, const int32_t *hin, const int32_t *hout, i
 //
 // Fused, one launch: every item on one compute unit, whose chain of loads grows with the bytes of an item; it saves
 // a launch, which is 1.6 us of a graph and 2.6 us of host time of an eager call.  Eight layers of Llama-7B attention
-// projections in a graph, fused (several workgroups an item where they fit, column_parts) / two fine launches, us: rank 16
+// projections in a graph, fused (several workgroups an item where they fit, column_part_shift) / two fine launches, us: rank 16
 // (256 KiB an item), 32 tokens x 1 projection 53 / 60, 8 x 3 55 / 61, 64 x 1 55 / 65, 64 x 3 82 / 101; rank 32 (512 KiB), 8 x 1
 // 74 / 64, 32 x 1 87 / 67; with one workgroup an item 32 x 3 126 / 109, 64 x 3 (more workgroups than the fine form likes)
 // 136 / 152.  So: fused up to 320 KiB an item, up to 640 KiB where the slices have filled the chip, and never where one item

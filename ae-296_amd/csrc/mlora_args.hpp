@@ -62,7 +62,7 @@ struct BgmvArgs {
     // two-launch form: records the shrink / expand grid covers; a workgroup walks records b, b + stride, ... < items_cap
     // (set by the launcher)
     int rec_stride_sh, rec_stride_ex;
-    int parts;                     // fused form: workgroups that share the output columns of a work item (set by the launcher)
+    int part_shift;                // fused form: 2^part_shift workgroups share the output columns of a work item (set by the launcher)
     int fine;                      // two-launch form of a small batch: 512-column slices, rank rows split over wavefronts
 };
 
