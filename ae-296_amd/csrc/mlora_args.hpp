@@ -126,6 +126,9 @@ struct SgmvProj {
     int hin, hout;
     int ksplit;            // K splits of the shrink
     int cols, ncb;         // expand: columns per workgroup, column blocks
+    // set by the launcher: stages of 64 columns in a K split, and inverses (inverse_of) of the numbers a workgroup id is divided by
+    int kper;
+    unsigned ksplit_inv, ncb_inv;
 };
 
 struct SgmvArgs {
@@ -139,6 +142,8 @@ struct SgmvArgs {
     int n_grp;
     int grp_first[MAX_PROJ], grp_n[MAX_PROJ];
     unsigned grp_end[MAX_PROJ];
+    int seg_tiles;                 // equally long segments: tiles of one, and the inverse of that (set by the launcher)
+    unsigned seg_tiles_inv;
     unsigned ex_end[MAX_PROJ];     // expand launch: first workgroup id after projection p (few: first column block), ~0 past the last
     PoolView pool;
     const int32_t *seg_start;
