@@ -380,9 +380,15 @@ __global__ __launch_bounds__(NT) void bgmv_kernel(const BgmvArgs p)
 // Llama-7B in a graph, 1 / 2 / 4 / 8 workgroups an item, us a call: rank 16, one token 6.2 / 5.3 / 5.3 / 5.4, 32 tokens x 1 projection
 // 8.6 / 7.2 / 6.6 / 6.7 (two launches 7.5), 16 x 3 9.3 / 7.8 / 7.2 / 11.7 (384 workgroups), 32 x 3 9.4 / 8.0 / 12.7 (384) / 17.7;
 // rank 8, 8 x 4 7.1 / 6.1 / 6.2 / 6.3.
+// Not where y lies over x: a workgroup that has stored its columns would have changed what the others of the item still read.
 static int column_part_shift(const BgmvArgs &a)
 {
     int widest = 0, shift = 0;
+    for (int q = 0; q < a.n_proj; q++)
+        for (int k = 0; k < a.n_proj; k++) {
+            const uintptr_t y = (uintptr_t)a.y[q], x = (uintptr_t)a.x[k];
+            if (y < x + (uintptr_t)a.T * a.hin[k] * 2 && x < y + (uintptr_t)a.T * a.hout[q] * 2) return 0;
+        }
     for (int q = 0; q < a.n_proj; q++) widest = a.hout[q] > widest ? a.hout[q] : widest;
     while (shift < 2 && (2LL << shift) * a.n_proj * a.items_cap <= device_compute_units() && (2 << shift) * 512 <= widest) shift++;
     return shift;

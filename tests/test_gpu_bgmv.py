@@ -550,3 +550,30 @@ def test_bgmv_fused_items_shared_by_workgroups(T, group, hout, accumulate):
     say(f"bgmv fused, shared items T={T} group={group} hout={hout} accumulate={accumulate}")
     got = _run(pp, x, tok, y0, group, accumulate=accumulate, fused=True)
     assert_close_bits(got, oracle_apply(pp, x, tok, y0), pp.dtype, f"T={T} hout={hout}")
+
+
+@pytest.mark.parametrize("T,n_proj,group,width", [(1, 1, 1, 1024), (1, 1, 1, 4096), (32, 1, 1, 4096), (10, 3, 1, 2048), (96, 1, 2, 4096)])
+@pytest.mark.parametrize("accumulate", [True, False])
+def test_bgmv_in_place(T, n_proj, group, width, accumulate):
+    """y over x, in launches small enough for several workgroups an item: each of them reads all of x and stores a part of y, so
+    such a call keeps one workgroup an item; bit for bit the call with a y of its own."""
+    rng = np.random.default_rng(T + width)
+    pp = PagedPool(rng, [16, 9, 4, 16], width, width, page_rows=8, dtype=FP16)
+    names = [f"p{i}" for i in range(n_proj)]
+    pool = upload_pool(pp, projections={nm: (width, width) for nm in names})
+    for nm in names:
+        pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, FP16))
+        pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, FP16))
+    tok = rng.integers(-1, 4, T).astype(np.int32)
+    t = torch.from_numpy(tok).cuda()
+    plan = plan_decode(t, pool, group=group)
+    xs = [torch.from_numpy(rng.standard_normal((T, width)).astype(np.float32)).cuda().half() for _ in names]
+    ys, inplace = [x.clone() for x in xs], [x.clone() for x in xs]
+    say(f"bgmv in place T={T} n_proj={n_proj} group={group} width={width} accumulate={accumulate}")
+    bgmv(ys, xs, pool, 0, names, t, plan=plan, accumulate=accumulate, fused=True)
+    bgmv(inplace, inplace, pool, 0, names, t, plan=plan, accumulate=accumulate, fused=True)
+    torch.cuda.synchronize()
+    for x, y, z in zip(xs, ys, inplace):
+        x_bits = torch_to_bits(x)
+        assert_close_bits(torch_to_bits(y), oracle_apply(pp, x_bits, tok, x_bits if accumulate else None), FP16)
+        assert torch.equal(y, z)
