@@ -824,14 +824,17 @@ __global__ __launch_bounds__(SG_NT, BT ? 4 : 1) void sgmv_expand_kernel(const Sg
 // 27.7 (192), 2 x 100 43.3 -> 36.6 (768), 8 x 64 60.7 -> 51.6 (2304), 2 x 512 69.1 -> 68.2 (3264), 8 x 128 73.1 -> 77.4 (3840); seven
 // projections, 2 x 100 72.9 -> 66.7 (2656), 4 x 64 77.2 -> 79.7 (3984).  Rank 32, q/k/v, 64 tokens 31.0 -> 25.0, 8 x 128 63.3 -> 62.0
 // (3840); q/k/v/o 8 x 128 74.6 -> 71.6 (5120); seven projections 8 x 64 85.1 -> 95.9 (7968).  Rank 16, q/k/v/o 16 x 64 71.5 -> 70.9 (6144);
-// seven 8 x 64 78.2 -> 83.0 (7968).  The reference's call, whose B is four times as many lines from L2, rank 64: 4 x 128 91.3 -> 76.3
-// (512), 8 x 128 100.2 -> 99.2 (1024), 16 x 64 102.3 -> 104.2 (1024); rank 16, 8 x 512 134.6 -> 128.8 (4096), 16 x 512 203.5 -> 214.0 (8192).
-// With one K split there is no reduce launch to save: rank 64, q/k/v, 2 x 100 59.9 -> 58.3 (768), 8 x 64 71.9 -> 71.7 (2304); at that rank the
-// line lies where four projections of 128 tokens do (512), as before.
+// seven 8 x 64 78.2 -> 83.0 (7968).  With one K split there is no reduce launch to save: rank 64, q/k/v, 2 x 100 59.9 -> 58.3 (768),
+// 8 x 64 71.9 -> 71.7 (2304); at that rank the line lies where four projections of 128 tokens do (512), as before.
+// The reference's call, whose B is four times as many lines from L2, against the kernel above with four workgroups a unit; three
+// calls on one x, several inputs in turn, hidden 4096: rank 16, 4 x 256 34.4 -> 32.1 (1024), 6 x 256 41.3 -> 40.8 (1536), 16 x 100
+// 42.5 -> 46.9 (2048), 8 x 512 59.7 -> 63.3 (4096), 12 x 512 80.7 -> 86.6 (6144); rank 32, 6 x 256 45.4 -> 45.7 (1536), 8 x 256
+// 48.4 -> 50.9 (2048); hidden 5120, rank 16, 6 x 256 45.0 -> 43.5 (1920), 8 x 256 49.1 -> 52.2 (2560).  Rank 64, 16 x 64 54.7 -> 52.9
+// (1024) and 63.1 -> 59.6 (1280, hidden 5120), 4 x 512 59.8 -> 65.2 (2048).
 constexpr int FEW_COLS = 256;
 static int few_expand(int max_rank, bool bt, int splits)                // workgroups up to which it is taken
 {
-    if (max_rank <= 32) return 6144;
+    if (max_rank <= 32) return bt ? 2047 : 6144;
     return splits == 1 ? 512 : (bt ? 1023 : 3200);
 }
 template <int DT, int RMAX, bool BT>

@@ -207,6 +207,16 @@ def test_the_reduce_launch_is_made_where_it_has_something_to_do(hin, T, n_seg, r
     assert s["reduce"] == (max(s["splits"]) > 1 and rank > 32 and not s["few"]), s
 
 
+@pytest.mark.parametrize("rank,most", [(8, 2047), (16, 2047), (32, 2047), (64, 1023)])
+def test_the_reference_call_takes_the_short_expand_up_to_its_own_line(rank, most):
+    """64 workgroups a tile of 4096 columns, 68 of 4104: the last call below the line and the first above, with several K splits."""
+    for width, per_tile in ((4096, 64), (4104, 68)):
+        n = most // per_tile
+        for tiles, few in ((n, 1), (n + 1, 0)):
+            s = sgmv_shape([(4096, width)], [0], 64 * tiles, tiles, rank, False, seg_len=64)
+            assert s["few"] == few and max(s["splits"]) > 1, (width, tiles, s)
+
+
 def test_x_is_streamed_by_large_calls_only():
     """From 100 MB of x and y on for the reference's call, whose three are measured so, and from 200 MB on for paged ones."""
     for T, paged, ref in ((5920, 0, 0), (6400, 0, 1), (12000, 0, 1), (12800, 1, 1)):        # 4096 + 4096 columns: 16 KiB a token
