@@ -244,6 +244,35 @@ def test_prefill_ref_tiles_without_a_plan(B, Lpad, r, hin, hout, dtype):
     assert_close_bits(torch_to_bits(y), orc.prefill_bmm_ref(x, A_T, B_T, 1, dtype, round_mid=False), dtype)
 
 
+@pytest.mark.parametrize("dtype", [FP16, BF16])
+@pytest.mark.parametrize("B,Lpad,r,hin,hout,splits,reduce", [
+    (33, 64, 8, 4096, 4184, True, 0),           # the expand sums the splits
+    (12, 130, 16, 4104, 4184, True, 0),
+    (16, 512, 16, 4096, 4096, True, 0),         # a batch of the reference's own prompts: whole steps
+    (33, 65, 24, 2056, 2136, True, 0),          # a rank between those of the kernel's instances
+    (12, 190, 32, 4096, 4184, True, 0),
+    (26, 65, 64, 1096, 1368, True, 1),          # behind the reduce launch
+    (44, 130, 64, 128, 216, False, 0),          # one split: the halves come from the shrink
+    (44, 130, 56, 128, 4184, False, 0),
+])
+def test_prefill_ref_of_64_token_tiles(B, Lpad, r, hin, hout, splits, reduce, dtype):
+    """The expand of 64 tokens a workgroup on the reference layout, which stages a step's result in two halves of 64 columns: widths
+    that end in the second of them, tiles of one and two tokens, several splits summed by it and by the reduce launch, and one."""
+    shape = sgmv_shape([(hin, hout)], [0], B * Lpad, B, r, False, seg_len=Lpad)
+    assert shape["few"] == 0 and shape["reduce"] == reduce and (max(shape["splits"]) > 1) == splits, shape
+    assert hout % 128 > 64 or hout == 4096
+    rng = np.random.default_rng(B + r)
+    A_T = bits_of((rng.standard_normal((B, 1, r, hin)) * 0.02).astype(np.float32), dtype)
+    B_T = bits_of((rng.standard_normal((B, 1, hout, r)) * 0.02).astype(np.float32), dtype)
+    x = bits_of(rng.standard_normal((B, Lpad, hin)).astype(np.float32), dtype)
+    say(f"prefill ref 64-token tiles B={B} Lpad={Lpad} r={r} {hin}x{hout} dtype={dtype}")
+    y = lora_prefill_ref(*(bits_to_torch(t, dtype, "cuda") for t in (x, A_T, B_T)), 0)
+    torch.cuda.synchronize()
+    rows = np.unique(np.concatenate([rng.choice(Lpad, min(Lpad, 40), replace=False), [0, 15, 16, 63, Lpad - 1]]))
+    want = orc.prefill_bmm_ref(np.ascontiguousarray(x[:, rows]), A_T, B_T, 0, dtype, round_mid=False)
+    assert_close_bits(torch_to_bits(y).reshape(B, Lpad, hout)[:, rows], want, dtype)
+
+
 def test_lora_gpu_keeps_its_workspace_for_a_shorter_prefill():
     """One prompt of 300 tokens, then one of 250: the workspace that a captured call may still use is not replaced, and both
     results meet the reference."""
