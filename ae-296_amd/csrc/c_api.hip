@@ -383,9 +383,11 @@ int mlora_bgmv_form(int n_proj, const int32_t *hin, const int32_t *hout, int T, 
     }
     *workspace_bytes = 0;
     if (T == 0) return MLORA_FORM_FUSED;
-    const bool sliced = prefer_sliced(n_proj, hin, hout, T, n_adapters, max_rank, group);
+    // Narrow slices take more room a token than wide ones, so a shorter batch that takes them can need more than a longer one:
+    // the size covers every batch up to T (prefer_sliced allows them at most four workgroups a unit).
     const int64_t coarse = mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
-    const int64_t fine = sliced ? 0 : fine_workspace_bytes(n_proj, T, max_hin, max_rank);
+    const int64_t most = group > 4 ? 0 : 4LL * mlora::device_compute_units() * group / fine_workgroups(n_proj, hin, hout, 1);
+    const int64_t fine = most > 0 ? fine_workspace_bytes(n_proj, most < T ? (int)most : T, max_hin, max_rank) : 0;
     *workspace_bytes = coarse > fine ? coarse : fine;
     return decode_form(n_proj, hin, hout, T, n_adapters, max_rank, group);
 }
@@ -443,9 +445,10 @@ static int bgmv_multi_impl(int form, int n_proj, void *const *y, const void *con
         workspace_bytes = (int64_t)SCRATCH_BYTES;
     }
     if (form != MLORA_FORM_FUSED) {
-        a.fine = form == MLORA_FORM_FINE || (form == MLORA_FORM_PAIR && !prefer_sliced(n_proj, hin, hout, T, n_adapters, max_rank, group));
-        const int64_t need = a.fine ? fine_workspace_bytes(n_proj, T, max_hin, max_rank)
-                                    : mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
+        const int64_t need_fine = fine_workspace_bytes(n_proj, T, max_hin, max_rank);
+        a.fine = form == MLORA_FORM_FINE || (form == MLORA_FORM_PAIR && workspace_bytes >= need_fine &&
+                                             !prefer_sliced(n_proj, hin, hout, T, n_adapters, max_rank, group));
+        const int64_t need = a.fine ? need_fine : mlora_bgmv_workspace_bytes(n_proj, T, max_hin, max_rank);
         if (!workspace) return fail(MLORA_EINVAL, "the two-launch form needs a workspace");
         if (workspace_bytes < need)
             return fail(MLORA_ENOSPACE, "workspace holds %lld bytes, %lld needed", (long long)workspace_bytes, (long long)need);

@@ -194,11 +194,12 @@ int mlora_bgmv_multi(int n_proj, void *const *y, const void *const *x,
 /*
  * Which form of mlora_bgmv_multi_form is fastest for a batch of these sizes, or a negative error code.  Arguments as
  * for that call (host arrays hin, hout).  *workspace_bytes receives what its two-launch forms take, whichever form
- * is returned.
+ * is returned, for this batch and for every shorter one in the form that this call names for it.
  *   MLORA_FORM_FUSED   one launch, no workspace
  *   MLORA_FORM_SLICED  two launches over slices of 1024 or 2048 columns, as mlora_bgmv_multi with a workspace
  *   MLORA_FORM_FINE    two launches over 512-column slices with the rank rows split over wavefronts (group <= 4): small batches
- *   MLORA_FORM_PAIR    two launches, fine or sliced by the sizes (mlora_bgmv_form does not return it)
+ *   MLORA_FORM_PAIR    two launches, fine or sliced by the sizes (mlora_bgmv_form does not return it); sliced where the workspace
+ *                      holds no more than that takes (mlora_bgmv_workspace_bytes)
  * The forms differ in the order the fp32 sums are added.
  */
 #define MLORA_FORM_FUSED 0

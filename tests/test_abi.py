@@ -260,6 +260,26 @@ def test_decode_form_on_both_sides_of_its_lines():
     assert form(1, 512, 512, 4, 16, group=3) == _ext.MLORA_EINVAL
 
 
+@pytest.mark.parametrize("group", [1, 2, 4, 8])
+def test_the_room_of_a_decode_batch_serves_every_shorter_one(group):
+    """A workspace sized for the longest batch of a pool holds what shorter ones take, narrow slices or wide."""
+    lib = _ext.lib()
+    need = C.c_int64()
+    forms = set()
+    for n, hin, hout, rank, slots in ((1, 4096, 4096, 64, 100), (1, 4096, 4096, 32, 100), (3, 4096, 2048, 16, 8), (1, 4096, 11008, 64, 1000),
+                                      (1, 11008, 4096, 24, 64), (7, 512, 520, 64, 300), (1, 64, 64, 8, 4)):
+        had = 0
+        for T in list(range(1, 330)) + [511, 512, 1024, 4097, 8192]:
+            form = lib.mlora_bgmv_form(n, (C.c_int32 * 8)(*[hin] * n), (C.c_int32 * 8)(*[hout] * n), T, slots, rank, group, C.byref(need))
+            forms.add(form)
+            stride = 16 if rank <= 16 else 32 if rank <= 32 else 64
+            fine = n * T * ((hin + 511) // 512) * stride * 4
+            assert need.value >= lib.mlora_bgmv_workspace_bytes(n, T, hin, rank) and (form != _ext.FORM_FINE or need.value >= fine)
+            assert need.value >= had, (n, hin, rank, T)
+            had = need.value
+    assert group == 8 or _ext.FORM_FINE in forms
+
+
 def test_decode_form_of_four_token_items():
     """Items of four tokens by their likely number, 8 slices of 512 columns each: 96 make 768 workgroups, 80 make 640."""
     lib = _ext.lib()

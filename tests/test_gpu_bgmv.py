@@ -577,3 +577,45 @@ def test_bgmv_in_place(T, n_proj, group, width, accumulate):
         x_bits = torch_to_bits(x)
         assert_close_bits(torch_to_bits(y), oracle_apply(pp, x_bits, tok, x_bits if accumulate else None), FP16)
         assert torch.equal(y, z)
+
+
+@pytest.mark.parametrize("T", [104, 160, 224])
+def test_bgmv_pair_in_the_room_of_wide_slices(T):
+    """The two-launch form by sizes would take narrow slices here; in a workspace of mlora_bgmv_workspace_bytes it takes the wide
+    ones, bit for bit mlora_bgmv_multi's, and one byte less is refused."""
+    import ctypes as C
+    from mlora import _ext
+    lib = _ext.lib()
+    rng = np.random.default_rng(T)
+    N, H = 100, 4096
+    pp = PagedPool(rng, [64] * N, H, H, page_rows=8, dtype=FP16)
+    pool = upload_pool(pp)
+    tok = rng.integers(0, N, T).astype(np.int32)
+    t = torch.from_numpy(tok).cuda()
+    plan = plan_decode(t, pool, group=4)
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).cuda().half()
+    widths = (C.c_int32 * 8)(H)
+    full = C.c_int64()
+    assert lib.mlora_bgmv_form(1, widths, widths, T, N, 64, 4, C.byref(full)) == _ext.FORM_FINE
+    bytes_wide = lib.mlora_bgmv_workspace_bytes(1, T, H, 64)
+    assert full.value > bytes_wide
+    room = torch.empty(full.value, dtype=torch.uint8, device="cuda")
+
+    def run(form, nbytes):
+        y = torch.zeros(T, H, device="cuda").half()
+        ptr = lambda p: (C.c_void_p * 8)(p)  # noqa: E731
+        a, b = pool.slab_ptrs(0, "p")
+        rc = lib.mlora_bgmv_multi_form(form, 1, ptr(y.data_ptr()), ptr(x.data_ptr()), ptr(a), ptr(b), widths, widths, t.data_ptr(), T,
+                                       pool.page_tbl.data_ptr(), pool.rank.data_ptr(), pool.scaling.data_ptr(), N, pool.max_pages,
+                                       pool.page_rows, pool.n_pages, 64, plan.work.data_ptr(), 4, room.data_ptr(), nbytes, 0, 1,
+                                       _ext.current_stream_ptr())
+        torch.cuda.synchronize()
+        return rc, y
+
+    say(f"bgmv pair in the room of wide slices T={T}")
+    assert run(_ext.FORM_PAIR, bytes_wide - 1)[0] == _ext.MLORA_ENOSPACE
+    (rc, pair), (rw, wide), (rf, fine) = run(_ext.FORM_PAIR, bytes_wide), run(_ext.FORM_SLICED, bytes_wide), run(_ext.FORM_PAIR, full.value)
+    assert rc == rw == rf == _ext.MLORA_OK and torch.equal(pair, wide)
+    want = oracle_apply(pp, torch_to_bits(x), tok, np.zeros((T, H), np.uint16))
+    for y in (pair, fine):
+        assert_close_bits(torch_to_bits(y), want, FP16)
