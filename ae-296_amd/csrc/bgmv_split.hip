@@ -777,15 +777,23 @@ static int launch_pair(const BgmvArgs &a0, hipStream_t s)
 }
 
 template <int DT, int G, int RMAX>
-static int launch_fine(const BgmvArgs &a, hipStream_t s)
+static int launch_fine(const BgmvArgs &a0, hipStream_t s)
 {
+    BgmvArgs a = a0;
     const int n_sh = a.sh_end[a.n_proj - 1], n_ex = a.ex_end[a.n_proj - 1];
-    if (n_sh <= 0 || n_ex <= 0 || a.items_cap <= 0) return 0;
-    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, FINE_CHUNKS, false>), dim3((unsigned)n_sh, (unsigned)a.items_cap), dim3(256), 0, s, a);
-    const int rc = (int)hipGetLastError();
-    if (rc) return rc;
-    hipLaunchKernelGGL((bgmv_expand_fine_kernel<DT, G, RMAX, FINE_CHUNKS>), dim3((unsigned)n_ex, (unsigned)a.items_cap), dim3(256), 0, s, a);
-    return (int)hipGetLastError();
+    if (n_sh <= 0 || n_ex <= 0) return 0;
+    // every workgroup has one record, so a batch beyond the grid's second dimension goes in pieces
+    for (int b0 = 0; b0 < a0.items_cap; b0 += MAX_STRIDE) {
+        const unsigned n_rec = (unsigned)(a0.items_cap - b0 < MAX_STRIDE ? a0.items_cap - b0 : MAX_STRIDE);
+        a.work = a0.work + (size_t)b0 * WORK_WORDS;
+        hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, FINE_CHUNKS, false>), dim3((unsigned)n_sh, n_rec), dim3(256), 0, s, a);
+        int rc = (int)hipGetLastError();
+        if (rc) return rc;
+        hipLaunchKernelGGL((bgmv_expand_fine_kernel<DT, G, RMAX, FINE_CHUNKS>), dim3((unsigned)n_ex, n_rec), dim3(256), 0, s, a);
+        rc = (int)hipGetLastError();
+        if (rc) return rc;
+    }
+    return 0;
 }
 
 template <int DT, int G, int RMAX>

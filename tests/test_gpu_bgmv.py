@@ -619,3 +619,44 @@ def test_bgmv_pair_in_the_room_of_wide_slices(T):
     want = oracle_apply(pp, torch_to_bits(x), tok, np.zeros((T, H), np.uint16))
     for y in (pair, fine):
         assert_close_bits(torch_to_bits(y), want, FP16)
+
+
+@pytest.mark.parametrize("fine", [True, False])
+def test_bgmv_more_records_than_the_grids_second_dimension(fine):
+    """65600 one-token records that the caller has written, which is more than a launch row of them; integer inputs, bit for bit."""
+    import ctypes as C
+    from mlora import _ext
+    lib = _ext.lib()
+    rng = np.random.default_rng(8)
+    T, hin, hout, N = 65600, 64, 72, 3
+    pp = PagedPool(rng, [8, 5, 2], hin, hout, page_rows=8, dtype=FP16, integer=True)
+    pp.scaling[:] = [1, 2, 0.5]
+    pool = upload_pool(pp)
+    tok = rng.integers(0, N, T).astype(np.int32)
+    x = rng.integers(-1, 2, (T, hin)).astype(np.float32)
+    rec = np.zeros((T, _ext.WORK_WORDS), np.int32)
+    rec[:, 0], rec[:, 1], rec[:, 2], rec[:, 3] = 1, tok, pp.ranks[tok], pp.scaling[tok].view(np.int32)
+    rec[:, 4:12], rec[:, 16:] = -1, -1
+    rec[:, 4] = np.arange(T)
+    for a in range(N):
+        rec[np.ix_(tok == a, 16 + np.arange(pp.ranks[a]))] = pp.rows(a)
+    want = np.zeros((T, hout))
+    for a in range(N):
+        want[tok == a] = x[tok == a].astype(np.float64) @ pp.A(a) @ pp.B(a) * pp.scaling[a]
+    assert np.abs(want).max() < 2048
+    work, t, xt = (torch.from_numpy(v).cuda() for v in (rec, tok, x))
+    xt = xt.half()
+    y = torch.zeros(T, hout, device="cuda").half()
+    hi, ho = (C.c_int32 * 8)(hin), (C.c_int32 * 8)(hout)
+    ptr = lambda p: (C.c_void_p * 8)(p)  # noqa: E731
+    a, b = pool.slab_ptrs(0, "p")
+    nbytes = T * 16 * 4
+    assert lib.mlora_bgmv_workspace_bytes(1, T, hin, pool.max_rank) == nbytes        # one slice in either form
+    room = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    say(f"bgmv with 65600 records, fine={fine}")
+    _ext.check(lib.mlora_bgmv_multi_form(_ext.FORM_FINE if fine else _ext.FORM_SLICED, 1, ptr(y.data_ptr()), ptr(xt.data_ptr()), ptr(a), ptr(b),
+                                         hi, ho, t.data_ptr(), T, pool.page_tbl.data_ptr(), pool.rank.data_ptr(), pool.scaling.data_ptr(), N,
+                                         pool.max_pages, pool.page_rows, pool.n_pages, pool.max_rank, work.data_ptr(), 1, room.data_ptr(),
+                                         nbytes, 0, 1, _ext.current_stream_ptr()))
+    torch.cuda.synchronize()
+    assert np.array_equal(y.double().cpu().numpy(), want)
