@@ -14,6 +14,7 @@ the limits below.  The limits say what the kernels were designed around:
 * the decode shrink of a one-round launch needs at least four (rank <= 16) or three (rank 32) workgroups per
   compute unit, the expand three;
 * the prefill shrink keeps a workgroup of eight wavefronts, or one of four that shares x, on a compute unit (more up to rank 32);
+* four workgroups of the reference layout's prefill expand fit a compute unit, by their registers and by their LDS;
 * M0 in `gemm_lora_kernel`, `gemm_lora_short_kernel` and `sgmv_shrink_kernel` is written only by the kernel's own LDS-bound loads: one
   `s_mov_b32 m0` per such load and no other instruction that names M0.
 """
@@ -46,6 +47,7 @@ LIMITS = [
     ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, (32|64), (true|false), false>", {"occupancy": (2, 8), "lds": (0, 160 * 1024)}),
     ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, (16|32), false, true>", {"occupancy": (2, 8), "lds": (0, 80 * 1024)}),
     ("sgmv_prefill.hip", r"sgmv_shrink_kernel<\d, 64, false, true>", {"occupancy": (1, 8), "lds": (0, 160 * 1024)}),
+    ("sgmv_prefill.hip", r"sgmv_expand_kernel<\d, \d+, true>", {"occupancy": (4, 8), "lds": (0, 40 * 1024)}),
 ]
 
 FIELDS = {"TotalSGPRs": "sgprs", "VGPRs": "vgprs", "AGPRs": "agprs", "ScratchSize [bytes/lane]": "scratch",
