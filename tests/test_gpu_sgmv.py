@@ -281,11 +281,12 @@ def test_sgmv_multi_projection_call():
 @pytest.mark.parametrize("dtype", [FP16, BF16])
 @pytest.mark.parametrize("lens,ranks,hin,hout,n_proj,shape", [
     ([1], [64], 4096, 640, 3, dict(share=0, few=1, most=8)),                # one tile, eight K splits, projections kept apart
-    ([65, 3], [16, 32], 264, 1032, 3, dict(most=1)),                        # a short K; a width that ends inside a column block
+    ([65, 3], [16, 32], 264, 1032, 3, dict(few=1, most=1)),                 # a short K; a width that ends inside a column block
     ([64] * 20 + [17], [33, 8], 4096, 128, 1, dict(few=1, most=8)),         # eight splits, one column block
-    ([300, 150], [32, 24, 8], 1024, 2048, 7, dict(reduce=0, most=2)),       # the expand sums the splits
+    ([300, 150], [32, 24, 8], 1024, 2048, 7, dict(few=1, reduce=0, most=2)),    # the expand of 16-token pieces sums the splits
+    ([300, 400], [32, 24, 8], 1096, 5128, 7, dict(few=0, reduce=0, most=2)),    # so does that of 64-token tiles
     ([64] * 25, [64], 512, 512, 2, dict(few=0, reduce=0, most=1)),          # 76 tiles at most: the numbering in runs
-    ([64] * 30, [16], 384, 256, 3, dict(share=1)),                          # projections that share x in one workgroup
+    ([64] * 30, [16], 384, 256, 3, dict(share=1, few=1)),                   # projections that share x in one workgroup
 ])
 def test_sgmv_launch_shapes(lens, ranks, hin, hout, n_proj, shape, dtype):
     """Both sides of the size rules of the prefill launches: K splits, column blocks, numbering of the workgroups,
@@ -483,10 +484,12 @@ def test_sgmv_few_tiles(lens, gap, ranks, hin, hout, n_proj, shape, dtype):
     ([700], [16], 1096, 6152, 7, 0, True),                         # 7700
     ([33, 640], [32, 20], 1096, 4104, 7, 1, True),
     ([1000], [24], 72, 4104, 7, 0, False),
+    ([641], [32, 20], 1096, 6152, 7, 0, True),
 ])
 @pytest.mark.parametrize("dtype", [FP16, BF16])
 def test_sgmv_both_expands(lens, ranks, hin, hout, n_proj, few, many, dtype):
-    """Both kernels at the ranks of every instance, on either side of the number of workgroups at which they change."""
+    """Both kernels at the ranks of every instance, on either side of the number of workgroups at which they change, summing the
+    splits themselves (up to rank 32, or few) and behind the reduce launch (y = delta); rows at the end outside every segment."""
     from mlora import sgmv_multi
     rng = np.random.default_rng(sum(lens) + hout)
     pp = PagedPool(rng, ranks, hin, hout, page_rows=8, dtype=dtype)
@@ -496,19 +499,21 @@ def test_sgmv_both_expands(lens, ranks, hin, hout, n_proj, few, many, dtype):
         pool.a_rows[nm][0].copy_(bits_to_torch(pp.a_rows, dtype))
         pool.b_rows[nm][0].copy_(bits_to_torch(pp.b_rows, dtype))
     seg = _segments(lens, rng.integers(0, len(ranks), len(lens)))
-    T = sum(lens)
-    shape = sgmv_shape([(hin, hout)] * n_proj, [0] * n_proj, T, len(lens), pool.max_rank)
-    assert shape["few"] == few and (max(shape["splits"]) > 1) == many, shape
-    plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in seg), T, pool, n_proj=n_proj)
-    x = bits_of(rng.standard_normal((T, hin)).astype(np.float32), dtype)
-    y0 = bits_of(rng.standard_normal((T, hout)).astype(np.float32), dtype)
-    say(f"sgmv both expands lens={lens[:2]}x{len(lens)} ranks={ranks} {hin}->{hout} n_proj={n_proj} dtype={dtype}")
-    ys = [bits_to_torch(y0, dtype, "cuda") for _ in names]
-    sgmv_multi(ys, [bits_to_torch(x, dtype, "cuda")] * n_proj, pool, 0, names, plan)
-    torch.cuda.synchronize()
-    want = oracle_apply(pp, x, _tok_of(*seg, T), y0)
-    for y in ys:
-        assert_close_bits(torch_to_bits(y), want, dtype)
+    x = bits_of(rng.standard_normal((sum(lens) + 3, hin)).astype(np.float32), dtype)
+    y0 = bits_of(rng.standard_normal((sum(lens) + 3, hout)).astype(np.float32), dtype)
+    for gap, accumulate in ((0, True), (3, True), (3, False)):
+        T = sum(lens) + gap
+        shape = sgmv_shape([(hin, hout)] * n_proj, [0] * n_proj, T, len(lens), pool.max_rank, accumulate)
+        assert shape["few"] == few and (max(shape["splits"]) > 1) == many, shape
+        assert shape["reduce"] == (not accumulate or (many and pool.max_rank > 32 and not few)), shape
+        plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in seg), T, pool, n_proj=n_proj)
+        say(f"sgmv both expands lens={lens[:2]}x{len(lens)} ranks={ranks} {hin}->{hout} n_proj={n_proj} dtype={dtype} accumulate={accumulate}")
+        ys = [bits_to_torch(y0[:T], dtype, "cuda") for _ in names]
+        sgmv_multi(ys, [bits_to_torch(x[:T], dtype, "cuda")] * n_proj, pool, 0, names, plan, accumulate=accumulate)
+        torch.cuda.synchronize()
+        want = oracle_apply(pp, x[:T], _tok_of(*seg, T), y0[:T] if accumulate else None)
+        for y in ys:
+            assert_close_bits(torch_to_bits(y), want, dtype)
 
 
 @pytest.mark.parametrize("aligned", [False, True])
