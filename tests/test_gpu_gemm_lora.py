@@ -219,16 +219,17 @@ def test_plan_tile_list_matches_oracle(aligned):
     assert np.array_equal(words[2 * max_tiles:2 * max_tiles + n], want_n)
 
 
-@pytest.mark.parametrize("T,hin,hout,n_proj,ranks,dtype", [
-    (1, 2056, 264, 1, [64, 8], FP16),          # one row of a 64-row tile, uneven K ranges and a partial last step
-    (64, 2088, 4104, 3, [16, 8], BF16),        # a full 64-row tile, a column tile of eight columns
-    (65, 2056, 4096, 3, [64, 24], FP16),       # 128-row tiles, one row in the upper half's first block
-    (128, 3080, 4096, 3, [32, 17], BF16),
-    (129, 4104, 4096, 3, [32, 16], FP16),      # 192-row tiles, one row in the third block
-    (192, 4096, 4352, 3, [64, 40], BF16),
-    (351, 4104, 1288, 7, [16, 8], FP16),       # three tiles of 128 rows, the last with a ragged end
+@pytest.mark.parametrize("T,hin,hout,n_proj,ranks,dtype,splits", [
+    (1, 2056, 264, 1, [64, 8], FP16, 8),          # one row of a 64-row tile, uneven K ranges and a partial last step
+    (64, 2088, 4104, 3, [16, 8], BF16, 3),        # a full 64-row tile, a column tile of eight columns
+    (65, 2056, 4096, 3, [64, 24], FP16, 4),       # 128-row tiles, one row in the upper half's first block
+    (128, 3080, 4096, 3, [32, 17], BF16, 2),      # two full 64-row tiles
+    (128, 3592, 4104, 3, [32, 17], BF16, 4),      # a full 128-row tile
+    (129, 4104, 4096, 3, [32, 16], FP16, 4),      # 192-row tiles, one row in the third block
+    (192, 4096, 4352, 3, [64, 40], BF16, 4),
+    (351, 4104, 1288, 7, [16, 8], FP16, 2),       # three tiles of 128 rows, the last with a ragged end
 ])
-def test_gemm_lora_short_batches(T, hin, hout, n_proj, ranks, dtype):
+def test_gemm_lora_short_batches(T, hin, hout, n_proj, ranks, dtype, splits):
     """Tiles of 64 to 192 rows with K cut into ranges: the rows at the tiles' edges against the oracle, every projection
     alike, and the same result as the call without room for partial sums up to the last rounding."""
     from mlora import _ext
@@ -248,7 +249,7 @@ def test_gemm_lora_short_batches(T, hin, hout, n_proj, ranks, dtype):
     w = bits_of((rng.standard_normal((hin, hout)) / np.sqrt(hin)).astype(np.float32), dtype)
     xt, wt = bits_to_torch(x, dtype, "cuda"), bits_to_torch(w, dtype, "cuda")
     arr = [(C.c_int32 * 8)(*([v] * n_proj)) for v in (hin, hout)]
-    assert _ext.lib().mlora_gemm_lora_partial_bytes(n_proj, *arr, T) > 0          # K is cut
+    assert _ext.lib().mlora_gemm_lora_partial_bytes(n_proj, *arr, T) == splits * n_proj * T * hout * 4          # K ranges
     plan = plan_prefill(*(torch.from_numpy(a).cuda() for a in (ss, sl, sa)), T, pool, n_proj=n_proj)
     ys = [torch.full((T, hout), float("nan"), dtype=tdtype(dtype), device="cuda") for _ in names]
     say(f"gemm_lora short T={T} {hin}x{hout} n_proj={n_proj} ranks={ranks} dtype={dtype}")
