@@ -731,7 +731,8 @@ static int launch_pair_bt(const BgmvArgs &a0, hipStream_t s)
     constexpr int KSC = Slices<RMAX>::KSC;
     const int n_sh = a.sh_end[a.n_proj - 1], n_ex = a.ex_end[a.n_proj - 1];
     if (n_sh <= 0 || n_ex <= 0 || a.rec_stride_sh <= 0 || a.rec_stride_ex <= 0) return 0;
-    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, false>), dim3((unsigned)n_sh, (unsigned)a.rec_stride_sh), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, false>), dim3((unsigned)n_sh, (unsigned)a.rec_stride_sh), dim3(256),
+                       0, s, a);
     int rc = (int)hipGetLastError();
     if (rc) return rc;
     hipLaunchKernelGGL((bgmv_expand_bt_kernel<DT, G, R, KSC>), dim3((unsigned)n_ex, (unsigned)a.rec_stride_ex), dim3(256), 0, s, a);
@@ -769,10 +770,12 @@ static int launch_pair(const BgmvArgs &a0, hipStream_t s)
     a.rec_stride_ex = record_stride<G>(a, a.ex_end[a.n_proj - 1], BIG);
     const int n_sh = a.sh_end[a.n_proj - 1], n_ex = a.ex_end[a.n_proj - 1];
     if (n_sh <= 0 || n_ex <= 0 || a.rec_stride_sh <= 0 || a.rec_stride_ex <= 0) return 0;
-    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, BIG>), dim3((unsigned)n_sh, (unsigned)a.rec_stride_sh), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((bgmv_shrink_kernel<DT, G, RMAX, KSC, BIG>), dim3((unsigned)n_sh, (unsigned)a.rec_stride_sh), dim3(256),
+                       0, s, a);
     int rc = (int)hipGetLastError();
     if (rc) return rc;
-    hipLaunchKernelGGL((bgmv_expand_kernel<DT, G, RMAX, KSC, NTE, BIG>), dim3((unsigned)n_ex, (unsigned)a.rec_stride_ex), dim3(NTE), 0, s, a);
+    hipLaunchKernelGGL((bgmv_expand_kernel<DT, G, RMAX, KSC, NTE, BIG>), dim3((unsigned)n_ex, (unsigned)a.rec_stride_ex),
+                       dim3(NTE), 0, s, a);
     return (int)hipGetLastError();
 }
 

@@ -322,11 +322,14 @@ static int64_t fine_workgroups(int n_proj, const int32_t *hin, const int32_t *ho
 // tokens x 7 projections (560 workgroups) 26.6 -> 21.9 at rank 64, 12.5 -> 11.7 at rank 16; 32 tokens x 3 (768)
 // 23.5 -> 20.8; 16 x 7 (1120) 34.6 -> 34.8; 32 x 7 (2240) 52.4 -> 59.6.
 //
-// Items of four tokens are far fewer than the host's bound where adapters have several tokens, so they also take the narrow slices while
-// about T/4 and two pieces for every fifth adapter make at most three workgroups per unit above rank 32 (2.5 above 16).  One projection, 100
-// adapters, Zipf 0.8, wide -> fine, us: 160 tokens of ranks 8 to 64 26.2 -> 18.2, of rank 64 29.9 -> 24.6, of rank 32 18.0 -> 16.8, of rank 16
-// 12.4 -> 12.4; 256 tokens (3.25 a unit) of ranks 8 to 64 26.5 -> 21.2, of rank 64 33.1 -> 33.7, of rank 32 18.5 -> 19.0; 100 tokens x 3 of rank 64 43.7
-// -> 46.4.
+// Items of four tokens are far fewer than the host's bound where adapters have several tokens, so they also take the narrow
+// slices while about T/4 and two pieces for every fifth adapter make at most three workgroups per unit above rank 32 (2.5 above
+// 16).  One projection, 100 adapters, Zipf 0.8, wide -> fine, us: 160 tokens of ranks 8 to 64 26.2 -> 18.2, of rank 64 29.9 ->
+// 24.6, of rank 32 18.0 -> 16.8, of rank 16 12.4 -> 12.4; 256 tokens (3.25 a unit) of ranks 8 to 64 26.5 -> 21.2, of rank 64 33.1
+// -> 33.7, of rank 32 18.5 -> 19.0; 100 tokens x 3 of rank 64 43.7 -> 46.4.  The estimate of pieces is that popularity's; with
+// others the line holds: 162 batches below it (64 to 700 adapters, uniform, Zipf 0.8 and 1.2; 144 to 256 tokens, four widths,
+// ranks 24 to 64), fine / wide 0.63 to 1.006 times; of rank 64 and uniform 0.83 to 0.98, the last with 700 adapters and 144
+// tokens (134 pieces, 4.2 workgroups a unit).
 static bool prefer_sliced(int n_proj, const int32_t *hin, const int32_t *hout, int T, int n_adapters, int max_rank, int group)
 {
     if (group > 4) return true;

@@ -123,8 +123,8 @@ __device__ __forceinline__ void gemm_lora_body(const GemmLoraArgs &p)
     const int ntn = pj.ntn * nsplit, ntm = p.ntm;               // the K ranges of a column tile follow each other
     const int n_tiles_out = ntm * ntn;
     // Every id has a tile: an id without one would still take its turn in the dealing of workgroups inside an XCD, and in a launch
-    // of about one round some units would get two (248 tiles of
-    // 160 steps, seven projections of Llama-13B, 64 tokens: 190 us, 151 without such ids; halves of its layers, 192 tokens 165, 125).
+    // of about one round some units would get two (248 tiles of 160 steps, seven projections of Llama-13B, 64 tokens: 190 us, 151
+    // without such ids; halves of its layers, 192 tokens 165, 125).
     const int base = n_tiles_out >> 3, more = n_tiles_out & 7, xcd = w & 7;
     const int L = xcd * base + (xcd < more ? xcd : more) + (w >> 3);
     const int grp = L / (GROUP_M * ntn), within = L - grp * (GROUP_M * ntn);
@@ -643,16 +643,22 @@ __global__ __launch_bounds__(256) void gemm_lora_sum_kernel(const GemmLoraArgs p
 // the rest, and rows past T are multiplied for nothing.  The rule estimates, for every tile height and number of
 // ranges, rounds of workgroups x mean time of one (or the longest chain) plus the cost of the partial sums, and takes
 // the least; the plain shape is kept where it comes within 1 %.  Fitted to 25 shapes of 165 batches (24 to 4500 tokens, three
-// prompts; q/k/v, with o, all seven; Llama-7B and -13B widths, whole and halves; rank 16, bf16, weights of two or three layers in turn, card
-// under load): the shape it names is 1.6 % off the best on average and 17 % at worst (2.4 % with the constants from before x came in
-// whole lines).  A layer with its LoRA launches, us, plain -> chosen (best): Llama-7B, q/k/v 24 tokens 86 -> 36 (36), 161 tokens 88 -> 53
-// (53), 768 tokens 96 -> 85 (85); q/k/v/o 192 tokens 92 -> 72 (68), 300 tokens 95 -> 72 (72); all seven 24 tokens 207 -> 90 (90), 351 tokens
-// 262 -> 194 (191), 450 tokens 265 -> 251 (223), 900 tokens 378 (361); halves, q/k/v 768 tokens 89 -> 58 (58).
+// prompts; q/k/v, with o, all seven; Llama-7B and -13B widths, whole and halves; rank 16, bf16, weights of two or three layers in
+// turn, card under load): the shape it names is 1.6 % off the best on average and 17 % at worst (2.4 % with the constants from before
+// x came in whole lines).  A layer with its LoRA launches, us, plain -> chosen (best): Llama-7B, q/k/v 24 tokens 86 -> 36 (36), 161
+// tokens 88 -> 53 (53), 768 tokens 96 -> 85 (85); q/k/v/o 192 tokens 92 -> 72 (68), 300 tokens 95 -> 72 (72); all seven 24 tokens
+// 207 -> 90 (90), 351 tokens 262 -> 194 (191), 450 tokens 265 -> 251 (223), 900 tokens 378 (361); halves, q/k/v 768 tokens 89 -> 58
+// (58).  The worst lie where two shapes change places: all seven at 400 to 500 tokens, and q/k/v at 378 to 384, where the shape that
+// the earlier constants named is 3 % the faster (72.1, 74.1).
+// What it names at whole Llama-7B widths, rows of a tile and the last token of a range.  q/k/v, K cut: 64 to 64, 128 to 128, 192 to
+// 192, 128 to 256, and 192 at 321..377; K whole: 64 to 320, 128 to 640, 192 to 960, 256 to 1280, 192 to 1920, 256 to 2560, 192 to 3072
+// and 256 beyond, but 192 at 5377..6144 and 6657..7104.  All seven, K cut: 64 to 64, 128 to 128, 192 to 192, 128 to 256, 192 to 384; K
+// whole: 192 to 576 and 256 beyond, but 192 at 1025..1152, 1537..1728 and 1793..1920.
 // Tiles of 256 rows are never cut: with the ranges the compiler spills accumulators.
 int64_t gemm_lora_shape(const GemmLoraArgs &a, bool may_split, GemmShape *out)
 {
     static const double step_us[4] = {0.435, 0.541, 0.652, 0.81};             // one K step, by mi
-    const double ends_us = 6.63, launch_us = 2.38, byte_us = 6.78e-7;           // a workgroup's start and end; one more launch; a byte written and read
+    const double ends_us = 6.63, launch_us = 2.38, byte_us = 6.78e-7;   // a workgroup's start and end; a launch; a byte both ways
     const double cus = device_compute_units();
     int longest = 1;
     for (int q = 0; q < a.n_proj; q++) longest = a.pr[q].hin / GK > longest ? a.pr[q].hin / GK : longest;

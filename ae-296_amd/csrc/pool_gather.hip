@@ -471,7 +471,8 @@ __global__ __launch_bounds__(FEW_NT) void gather_few_kernel(const GatherArgs g, 
             const uint2 v = *reinterpret_cast<const uint2 *>(s_cnt[key[e]]);
             const int w = e * NW + wave;
             const uint32_t below = (1u << (8 * (w & 3))) - 1u;
-            const int idx = (int)__builtin_amdgcn_sad_u8(v.x & (w < 4 ? below : ~0u), 0u, __builtin_amdgcn_sad_u8(v.y & (w < 4 ? 0u : below), 0u, (uint32_t)in_wave[e]));
+            const int idx = (int)__builtin_amdgcn_sad_u8(v.x & (w < 4 ? below : ~0u), 0u,
+                                                         __builtin_amdgcn_sad_u8(v.y & (w < 4 ? 0u : below), 0u, (uint32_t)in_wave[e]));
             const int total = (int)__builtin_amdgcn_sad_u8(v.x, 0u, __builtin_amdgcn_sad_u8(v.y, 0u, 0u));
             const int at = (int)(b & 0x3fffu) + idx;
             s_perm[at] = (uint16_t)i;
@@ -480,7 +481,8 @@ __global__ __launch_bounds__(FEW_NT) void gather_few_kernel(const GatherArgs g, 
                 int eighth = 0;
 #pragma unroll
                 for (int k = 1; k < 8; k++) eighth += c >= k * per_xcd;
-                const int4 h = make_int4(at | (left < g.group ? left : g.group) << TOK_BITS, key[e], rk[e], __builtin_bit_cast(int, sc[e]));
+                const int4 h = make_int4(at | (left < g.group ? left : g.group) << TOK_BITS, key[e], rk[e],
+                                         __builtin_bit_cast(int, sc[e]));
                 s_chunk[c] = h;
                 if (by_rank) s_key[eighth][c - eighth * per_xcd] = (uint16_t)(rk[e] << 6 | (63 - (c - eighth * per_xcd)));
                 else s_rec[c] = h;
@@ -549,7 +551,8 @@ __global__ __launch_bounds__(FEW_NT) void gather_few_kernel(const GatherArgs g, 
             g.chunk_adapter[c] = h.y < n ? h.y : -1;
         }
         if (tid < 8)
-            g.counters[tid] = tid == 0 ? (int)(all_ts >> 16) : tid == 1 ? T - (int)tokens_of(n) : tid == 2 ? n_chunks : tid == 3 ? s_bad : 0;
+            g.counters[tid] = tid == 0 ? (int)(all_ts >> 16) : tid == 1 ? T - (int)tokens_of(n)
+                              : tid == 2 ? n_chunks : tid == 3 ? s_bad : 0;
     }
 }
 

@@ -1,6 +1,7 @@
 // SGMV prefill kernels for gfx950: tokens are packed per segment (one adapter per segment)
 //     y[t] (+)= s_a * (x[t] . A_a) . B_a
-// computed on v_mfma_f32_16x16x32_{f16,bf16} tiles in two to four launches on one stream (the first can be shared by all projections and layers of a batch):
+// computed on v_mfma_f32_16x16x32_{f16,bf16} tiles in two to four launches on one stream (the first can be shared by all projections
+// and layers of a batch):
 //   plan   : cuts every segment into tiles of at most 64 tokens (work list in the workspace);
 //   shrink : V[split][t][0..R) = x[t, Kslice] . A_a[:, Kslice]^T   (split-K, fp32 partials), or with one
 //            split the result itself as a hi + lo pair of 16-bit values, so that the intermediate keeps
@@ -89,9 +90,11 @@ __host__ __device__ inline long long place_grid(int max_tiles, int n_second)
     return few_tiles(max_tiles) ? (long long)max_tiles * n_second : xcd_grid(max_tiles, n_second);
 }
 
-// Shrink launches of a few tiles have them as the grid's second dimension, one tile's groups behind each other: nothing to divide by.
-// With more, the longest groups of all tiles go first: 1536 workgroups of 47 tiles, rank 32, q/k/v/o, 21.9 us, 25.5 tile by tile; four layers
-// of one tile 47.9 us, 47.0 as the second dimension.
+// Shrink launches of a few tiles have them as the grid's second dimension, one tile's groups behind each other: nothing to divide
+// by. With more, the longest groups of all tiles go first.  Whole calls of 1 to 24 prompts of 1 to 1000 tokens, two layers of
+// Llama-7B, one, three, four and seven projections, ranks 16 to 64, second dimension against longest first: up to 16 tiles (of
+// the host's bound) 1 % faster on average (0.92 to 1.06 times, one tile 47.9 -> 47.0 us), 17 to 32 0.99 to 1.005 times on average
+// and up to 1.08, 33 to 56 1.01 to 1.02 times at rank 64 and up to 1.11 (seven projections, 4 x 400 tokens 211 -> 234 us).
 __host__ __device__ inline bool tile_rows(int max_tiles) { return max_tiles <= 2 * XRUN; }
 
 // Expand launches use a second order where it fits: tile-major, the column blocks of a tile next to each other, so
@@ -167,8 +170,8 @@ __device__ __forceinline__ Tile<UNIFORM> tile_of(const SgmvArgs &p, int tile)
 // A workgroup writes the list entries and records of PLAN_TILES tiles and the cover flags of PLAN_TOKENS tokens; every one
 // counts the tiles of all segments itself, a few steps, so that none waits for another.  What bounds it is the start of a
 // launch and the chain segments -> adapter -> rank, scaling, page table -> record, most of it on lines that no cache holds any
-// more; the counting runs beside it.  One prompt of 64
-// tokens 4.0 -> 3.7 us, sixteen of 9216 12.0 -> 11.2 (before, the rank and the page table were asked for behind the headers).
+// more; the counting runs beside it.  One prompt of 64 tokens 4.0 -> 3.7 us, sixteen of 9216 12.0 -> 11.2 (before, the rank and the
+// page table were asked for behind the headers).
 constexpr int PLAN_NT = 256;
 constexpr int PLAN_TILES = 16;
 constexpr int PLAN_TOKENS = 4 * PLAN_NT;
@@ -257,7 +260,9 @@ __global__ __launch_bounds__(PLAN_NT) void sgmv_plan_kernel(const SgmvArgs p)
         }
         if (t0 + lt < p.max_tiles && (h[0] > 0 || w < 2)) p.tile_rec[(size_t)(t0 + lt) * TILE_WORDS + w] = val;
     }
-    if (tid < PLAN_TILES && s_hdr[tid][0] > 0) { p.tile_seg[t0 + tid] = s_hdr[tid][5]; p.tile_tok0[t0 + tid] = s_hdr[tid][4]; p.tile_ntok[t0 + tid] = s_hdr[tid][0]; }
+    if (tid < PLAN_TILES && s_hdr[tid][0] > 0) {
+        p.tile_seg[t0 + tid] = s_hdr[tid][5]; p.tile_tok0[t0 + tid] = s_hdr[tid][4]; p.tile_ntok[t0 + tid] = s_hdr[tid][0];
+    }
     if (blockIdx.x == 0 && tid == 0) p.n_tiles[0] = carry < p.max_tiles ? carry : p.max_tiles;
 #pragma unroll
     for (int u = 0; u < PLAN_TOKENS / PLAN_NT; u++) {
@@ -325,7 +330,9 @@ __global__ __launch_bounds__(SG_NT *SH_KG<SHARE>) void sgmv_shrink_kernel(const 
     // fastest index, so that they run side by side on one XCD and find x in its L2.
     const GroupId at = group_at(p.grp_end, blockIdx.x);
     const int grp = at.group, w = at.rest, ng = SHARE ? 1 : p.grp_n[grp];
-    auto by_group = [&](int v) { return ng == 1 ? v : (ng == 2 ? v >> 1 : (int)(__umulhi((unsigned)v, 0xaaaaaaabu) >> 1)); };      // v / ng
+    auto by_group = [&](int v) {                                // v / ng
+        return ng == 1 ? v : (ng == 2 ? v >> 1 : (int)(__umulhi((unsigned)v, 0xaaaaaaabu) >> 1));
+    };
     int tile = (int)blockIdx.y, split, p0 = p.grp_first[grp];
     if (tile_rows(p.max_tiles)) {
         split = by_group(w);
@@ -363,7 +370,8 @@ __global__ __launch_bounds__(SG_NT *SH_KG<SHARE>) void sgmv_shrink_kernel(const 
     const int half = (st1 - st0 + KG - 1) / KG;                 // every group walks this many steps, the last one may have fewer stages
     const int g0 = st0 + kg * half < st1 ? st0 + kg * half : st1;
     const int n = st1 - g0 < half ? st1 - g0 : half;
-    const bool tail = whole < nstage && split * per <= whole && whole < split * per + per;   // this range ends with a stage of fewer columns
+    // whether this range ends with a stage of fewer columns
+    const bool tail = whole < nstage && split * per <= whole && whole < split * per + per;
     unsigned char *ring = s_ring + kg * GROUP_BYTES;
     typedef __attribute__((address_space(3))) unsigned char lds_byte;
     const unsigned ring_at = (unsigned)(__UINTPTR_TYPE__)(lds_byte *)ring;
@@ -567,12 +575,12 @@ __global__ __launch_bounds__(256) void sgmv_reduce_kernel(const SgmvArgs p)
 // ------------------------------------------------------------------ expand
 // Up to rank 32 the K splits are summed by the expand itself and the reduce launch falls away.  At rank 64 the sums are
 // four times as long as at 16 and every column block of a tile repeats them, so the reduce launch stays there but for the
-// launches of few tiles below (sgmv_launch_shape): 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing, 55.4 and a reduce
-// of 5.2 not; at rank 16 the whole call of 8 x 512 tokens 185 -> 179.
+// launches of few tiles below (sgmv_launch_shape): 1280 tokens, seven projections, rank 64, two splits 62.6 us of expand summing,
+// 55.4 and a reduce of 5.2 not; at rank 16 the whole call of 8 x 512 tokens 185 -> 179.
 
 // The reference's call (BT) only writes y, and its whole batch is about one round of workgroups: no registers for y, and a staging
-// tile of half a step, so that four workgroups fit a unit instead of three (16 x 512 tokens,
-// rank 64, 1024 workgroups: q, k and v 124.5 us with three, 118.9 with four).
+// tile of half a step, so that four workgroups fit a unit instead of three (16 x 512 tokens, rank 64, 1024 workgroups: q, k and v
+// 124.5 us with three, 118.9 with four).
 template <int DT, int RMAX, bool BT>
 __global__ __launch_bounds__(SG_NT, BT ? 4 : 1) void sgmv_expand_kernel(const SgmvArgs p)
 {
@@ -593,7 +601,7 @@ __global__ __launch_bounds__(SG_NT, BT ? 4 : 1) void sgmv_expand_kernel(const Sg
     __shared__ __attribute__((aligned(16))) unsigned char s_b[BT ? TN * TPITCH : KP * BPITCH];
     __shared__ __attribute__((aligned(16))) float s_out[SG_NT / 64][16][OPITCH];
     __shared__ int s_brow[BT ? 1 : KP];
-    constexpr int VPITCH = KP + 8;             // 16-bit values per token row of the folded intermediate, which lies in s_out (BT: s_b) for a while
+    constexpr int VPITCH = KP + 8;             // 16-bit values per token row of the folded intermediate, which lies in s_out (BT: s_b)
     uint16_t *const s_v = BT ? reinterpret_cast<uint16_t *>(s_b) : reinterpret_cast<uint16_t *>(&s_out[0][0][0]);
     static_assert(2 * TM * VPITCH * 2 <= (int)(BT ? sizeof(s_b) : sizeof(s_out)), "the folded intermediate fits there");
     typedef __attribute__((address_space(3))) volatile float lds_vfloat;
@@ -820,12 +828,23 @@ __global__ __launch_bounds__(SG_NT, BT ? 4 : 1) void sgmv_expand_kernel(const Sg
 // columns, 64 per wavefront, in one step, everything requested at once: the partial sums and the row table first, then B
 // and y; B is read by four workgroups instead of one.  What bounds it is the chain record -> row table -> B -> y; with each B load
 // waiting for its own row lookup 3.9 us of 8.8 went by before the last was requested.
-// Two layers and the plan in a graph, Llama-7B widths, that kernel -> this one, us, by workgroups: rank 64, q/k/v, 64 tokens 37.2 ->
-// 27.7 (192), 2 x 100 43.3 -> 36.6 (768), 8 x 64 60.7 -> 51.6 (2304), 2 x 512 69.1 -> 68.2 (3264), 8 x 128 73.1 -> 77.4 (3840); seven
-// projections, 2 x 100 72.9 -> 66.7 (2656), 4 x 64 77.2 -> 79.7 (3984).  Rank 32, q/k/v, 64 tokens 31.0 -> 25.0, 8 x 128 63.3 -> 62.0
-// (3840); q/k/v/o 8 x 128 74.6 -> 71.6 (5120); seven projections 8 x 64 85.1 -> 95.9 (7968).  Rank 16, q/k/v/o 16 x 64 71.5 -> 70.9 (6144);
-// seven 8 x 64 78.2 -> 83.0 (7968).  With one K split there is no reduce launch to save: rank 64, q/k/v, 2 x 100 59.9 -> 58.3 (768),
-// 8 x 64 71.9 -> 71.7 (2304); at that rank the line lies where four projections of 128 tokens do (512), as before.
+// Two layers and the plan in a graph, Llama-7B widths, that kernel -> this one, us, by workgroups: rank 64, q/k/v, 64 tokens
+// 37.2 -> 27.7 (192), 2 x 100 43.3 -> 36.6 (768), 8 x 64 60.7 -> 51.6 (2304), 2 x 512 69.1 -> 68.2 (3264), 8 x 128 73.1 -> 77.4 (3840);
+// seven projections, 2 x 100 72.9 -> 66.7 (2656), 4 x 64 77.2 -> 79.7 (3984).  Rank 32, q/k/v, 64 tokens 31.0 -> 25.0, 8 x 128
+// 63.3 -> 62.0 (3840); q/k/v/o 8 x 128 74.6 -> 71.6 (5120); seven projections 8 x 64 85.1 -> 95.9 (7968).  Rank 16, q/k/v/o 16 x 64
+// 71.5 -> 70.9 (6144); seven 8 x 64 78.2 -> 83.0 (7968).
+// The number is that of 64-token tiles the batch is likely to make (sgmv_launch_shape), four pieces each, and not that of the
+// grid, which covers the host's bound on tiles: many short prompts leave most of a grid empty and are where this kernel gains
+// most, one piece a prompt against a whole tile.  Seven projections, 16 x 4 tokens (5976 by the rule, 22576 dispatched, 2656 with
+// tokens) 70.8 -> 59.4 at rank 16, 76.2 -> 65.2 at 32; 32 x 8, beyond the line, 119 -> 102 (rank 16); q/k/v/o 24 x 8 52.2 ->
+// 45.8.  Over 1 to 32 prompts of 1 to 400 tokens, ranks 16 and 32, four sets of projections (whole, of the larger model, as one
+// of two shards, ragged), each batch alone or sixteen in turn, the rule is 0.1 to 1.0 % off the better kernel on average, at rank
+// 64 0.3 to 1.9 % (beyond its line prompts of up to 16 tokens would gain 6 to 20 %).  It is worst with all seven projections of
+// the whole layer at 40 to 100 tokens a prompt: 8 x 40 62.1 -> 69.2 at rank 16, 71.7 -> 80.4 at 32, 3 x 100 58.2 -> 60.6 and
+// 60.9 -> 65.4; any lower line would lose more on the narrower layers, where the same numbers gain up to 20 %.
+// One number up to rank 32, as both kernels sum the splits there whatever their number.  Above, this one saves the reduce launch,
+// but not with one K split: rank 64, q/k/v, 2 x 100 59.9 -> 58.3 (768), 8 x 64 71.9 -> 71.7 (2304); there the line lies where
+// four projections of 128 tokens do (512).
 // The reference's call, whose B is four times as many lines from L2, against the kernel above with four workgroups a unit; three
 // calls on one x, several inputs in turn, hidden 4096: rank 16, 4 x 256 34.4 -> 32.1 (1024), 6 x 256 41.3 -> 40.8 (1536), 16 x 100
 // 42.5 -> 46.9 (2048), 8 x 512 59.7 -> 63.3 (4096), 12 x 512 80.7 -> 86.6 (6144); rank 32, 6 x 256 45.4 -> 45.7 (1536), 8 x 256
@@ -1011,7 +1030,8 @@ void sgmv_launch_shape(SgmvArgs &a, int max_rank, int phases)
         most = a.pr[q].ksplit > most ? a.pr[q].ksplit : most;
     }
     a.few = few_wgs <= few_expand(max_rank, a.seg_uniform_len > 0, most);
-    // The expand sums the splits itself up to rank 32 and in launches of few tiles; rows outside every segment are zeroed by the reduce launch only.
+    // The expand sums the splits itself up to rank 32 and in launches of few tiles; rows outside every segment are zeroed by the
+    // reduce launch only.
     a.fold = (max_rank <= 32 || a.few) && (a.accumulate || a.seg_uniform_len > 0);
     // Without splits the shrink has stored the halves itself, and the launch would only read the cover flags: two projections
     // of 25 x 64 tokens, rank 64, hin 512 15.6 -> 14.0 us a call, q/k/v/o of 16 x 500 tokens at hidden 4096 153.4 -> 151.7.
@@ -1053,7 +1073,8 @@ static int launch_rmax(const SgmvArgs &a, int phases, hipStream_t s)
     const dim3 sgrid(end, rows ? (unsigned)g.max_tiles : 1u);
     end = 0;
     for (int q = 0; q < MAX_PROJ; q++) {
-        if (q < g.n_proj) end += g.few ? (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
+        if (q < g.n_proj)
+            end += g.few ? (unsigned)((g.pr[q].hout + FEW_COLS - 1) / FEW_COLS) : (unsigned)expand_grid(g.max_tiles, g.pr[q].ncb);
         g.ex_end[q] = q < g.n_proj ? end : ~0u;
     }
     const dim3 egrid(end, g.few ? (unsigned)g.max_tiles * 4u : 1u);
